@@ -1,0 +1,238 @@
+// Host side of the PyTorch operator: argument checks, output and workspace allocation, the autograd node and the
+// calls of the C ABI (include/dsdpa.h), in C++. The counterpart of the reference's autograd.Function
+// (ops/triton.py:377-466); ops/triton.py holds the Python entry point, which raises the exceptions.
+//
+// Why native: at the small end of the operator's range the GPU finishes long before the host has enqueued the next
+// launch. With the checks, torch.empty calls, ctypes conversions and autograd.Function of Python a training step
+// took 165 us of host time whatever its size (views x samples 2x2 of the sweep, 18x18, 32 heads: 162 us a step for
+// 86 us of kernels).
+//
+// apply(single_stream, q, k, v, coords, WIDTH, HEIGHT, sm_scale[, coords_grad]) -> out; None when an argument is
+// not what the kernels take as it is (wrong shape or type, layout that has to be copied first): nothing has
+// been done then, and the Python side says what is wrong or mends it; a number when the library refused the call (its
+// error code). No tensor is kept from one call for the next.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/Context.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <c10/core/DeviceGuard.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/dsdpa.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+struct Strides {
+    long long st[8];
+    bool given = false;                  // false: everything contiguous
+    const long long *ptr() const { return given ? st : nullptr; }
+};
+
+// Whether the kernels can read q, k, v where they lie: head dimension contiguous, k and v laid out alike, rows
+// 16-byte aligned, the views and pixels of one (batch, head) within 2^30 elements (the kernels address them in 32
+// bits). Fills the `strides` argument of the entry points.
+bool readable_in_place(const Tensor &q, const Tensor &k, const Tensor &v, Strides *out)
+{
+    if (q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) return true;
+    const int64_t align = 16 / (int64_t)q.element_size(), V = q.size(1), L = q.size(3), D = q.size(4);
+    for (const Tensor *t : {&q, &k, &v}) {
+        const auto st = t->strides();
+        if (st[4] != 1 || ((uintptr_t)t->data_ptr() & 15) || st[3] < D) return false;
+        for (int i = 0; i < 4; ++i)
+            if (st[i] < 0 || st[i] % align) return false;
+        if ((V - 1) * st[1] + (L - 1) * st[3] + D > (1ll << 30) || st[1] > (1ll << 30)) return false;
+    }
+    if (k.strides() != v.strides()) return false;
+    for (int i = 0; i < 4; ++i) {
+        out->st[i] = q.stride(i);
+        out->st[4 + i] = k.stride(i);
+    }
+    out->given = true;
+    return true;
+}
+
+// at::detail::empty_cuda: the caching allocator without the dispatcher, and without the fill that at::empty does under
+// torch.use_deterministic_algorithms (every element of every buffer made here is written by the kernels).
+Tensor fresh(at::IntArrayRef shape, at::ScalarType type, const at::Device &dev)
+{
+    return Tensor(at::detail::empty_cuda(shape, type, dev, std::nullopt));
+}
+
+void *stream_of(const at::Device &dev)
+{
+    return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream();
+}
+
+void check(int rc)
+{
+    TORCH_CHECK(rc == DSDPA_OK, "libdsdpa error ", rc, ": ", dsdpa_error_string(rc), " (hip error ", dsdpa_last_hip_error(), ")");
+}
+
+int dtype_code(at::ScalarType t)
+{
+    return t == at::kFloat ? DSDPA_F32 : t == at::kBFloat16 ? DSDPA_BF16 : DSDPA_F16;
+}
+
+struct Refused { int code; };            // the forward's error code on its way out of autograd
+
+struct Call {
+    int64_t W, H;
+    double scale;
+    bool coords_grad, single_stream;
+};
+
+// out and the log-sum-exp of every query row
+std::pair<Tensor, Tensor> forward(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &coords, const Call &c)
+{
+    const at::Device dev = q.device();
+    const c10::DeviceGuard guard(dev);
+    Strides st;
+    TORCH_CHECK(readable_in_place(q, k, v, &st));
+    const int B = (int)q.size(0), V = (int)q.size(1), H = (int)q.size(2), D = (int)q.size(4), P = (int)coords.size(4);
+    const int W = (int)c.W, Hi = (int)c.H, code = dtype_code(q.scalar_type());
+    Tensor out = fresh(q.sizes(), q.scalar_type(), dev);
+    Tensor lse = fresh({q.size(0), q.size(1), q.size(2), q.size(3)}, at::kFloat, dev);
+    Tensor ws;                                           // scratch, not kept for the backward
+    void *wsp = nullptr;
+    if (const size_t bytes = dsdpa_fwd_workspace_bytes(code, B, V, H, Hi, W, D, P)) {
+        ws = fresh({(int64_t)bytes}, at::kByte, dev);
+        wsp = ws.data_ptr();
+    }
+    const auto *cp = (const float *)coords.data_ptr();
+    auto *lp = (float *)lse.data_ptr();
+    void *s = stream_of(dev);
+    int rc;
+    if (code == DSDPA_F32)
+        rc = dsdpa_fwd_f32((const float *)q.data_ptr(), (const float *)k.data_ptr(), (const float *)v.data_ptr(), cp, (float *)out.data_ptr(), lp,
+                           wsp, B, V, H, Hi, W, D, P, (float)c.scale, st.ptr(), s);
+    else
+        rc = (code == DSDPA_BF16 ? dsdpa_fwd_bf16 : dsdpa_fwd_f16)(q.data_ptr(), k.data_ptr(), v.data_ptr(), cp, out.data_ptr(), lp, wsp, B, V,
+                                                                   H, Hi, W, D, P, (float)c.scale, st.ptr(), s);
+    if (rc != DSDPA_OK) throw Refused{rc};
+    return {out, lse};
+}
+
+struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &coords, const Call &c)
+    {
+        auto [out, lse] = ::forward(q, k, v, coords, c);
+        ctx->save_for_backward({q, k, v, coords, out, lse});
+        ctx->saved_data["W"] = c.W;
+        ctx->saved_data["H"] = c.H;
+        ctx->saved_data["scale"] = c.scale;
+        ctx->saved_data["flags"] = (int64_t)((c.coords_grad ? DSDPA_FLAG_COORDS_GRAD : 0) | (c.single_stream ? DSDPA_FLAG_SINGLE_STREAM : 0));
+        return out;
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &coords = saved[3], &out = saved[4], &lse = saved[5];
+        const at::Device dev = q.device();
+        const c10::DeviceGuard guard(dev);
+        Tensor dout = grads[0];
+        if (!dout.defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
+        dout = dout.contiguous();
+        unsigned flags = (unsigned)ctx->saved_data["flags"].toInt();
+        const bool want_dcoords = (flags & DSDPA_FLAG_COORDS_GRAD) != 0 && ctx->needs_input_grad(3);
+        flags &= DSDPA_FLAG_SINGLE_STREAM;
+        if (at::globalContext().deterministicAlgorithms()) {       // the bitwise reproducible backward
+            TORCH_CHECK(!want_dcoords, "deform_sdpa_triton: the coordinate gradient has no deterministic implementation "
+                                       "(it sums over heads with float atomics); turn one of the two off");
+            flags |= DSDPA_FLAG_DETERMINISTIC;
+        }
+        if (want_dcoords) flags |= DSDPA_FLAG_COORDS_GRAD;
+        const int B = (int)q.size(0), V = (int)q.size(1), H = (int)q.size(2), D = (int)q.size(4), P = (int)coords.size(4);
+        const int W = (int)ctx->saved_data["W"].toInt(), Hi = (int)ctx->saved_data["H"].toInt(), code = dtype_code(q.scalar_type());
+        const float scale = (float)ctx->saved_data["scale"].toDouble();
+        Strides st;
+        TORCH_CHECK(readable_in_place(q, k, v, &st));
+        Tensor dq = fresh(q.sizes(), q.scalar_type(), dev), dk = fresh(q.sizes(), q.scalar_type(), dev), dv = fresh(q.sizes(), q.scalar_type(), dev);
+        Tensor dcoords = want_dcoords ? fresh(coords.sizes(), at::kFloat, dev) : Tensor();
+        Tensor ws = fresh({(int64_t)dsdpa_bwd_workspace_bytes(code, B, V, H, Hi, W, D, P, flags)}, at::kByte, dev);
+        const auto *cp = (const float *)coords.data_ptr(), *lp = (const float *)lse.data_ptr();
+        float *dcp = want_dcoords ? (float *)dcoords.data_ptr() : nullptr;
+        void *s = stream_of(dev);
+        int rc;
+        if (code == DSDPA_F32)
+            rc = dsdpa_bwd_f32((const float *)q.data_ptr(), (const float *)k.data_ptr(), (const float *)v.data_ptr(), cp, (const float *)out.data_ptr(),
+                               lp, (const float *)dout.data_ptr(), (float *)dq.data_ptr(), (float *)dk.data_ptr(), (float *)dv.data_ptr(), dcp,
+                               ws.data_ptr(), B, V, H, Hi, W, D, P, scale, st.ptr(), flags, s);
+        else
+            rc = (code == DSDPA_BF16 ? dsdpa_bwd_bf16 : dsdpa_bwd_f16)(q.data_ptr(), k.data_ptr(), v.data_ptr(), cp, out.data_ptr(), lp,
+                                                                       dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dcp,
+                                                                       ws.data_ptr(), B, V, H, Hi, W, D, P, scale, st.ptr(), flags, s);
+        check(rc);
+        return {dq, dk, dv, dcoords, Tensor()};
+    }
+};
+
+// The reference's preconditions (ops/triton.py:375,385-388) and this build's: true when the call can go ahead as it is.
+bool acceptable(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &coords, const Call &c)
+{
+    const at::ScalarType t = q.scalar_type();
+    if (t != at::kFloat && t != at::kBFloat16 && t != at::kHalf) return false;
+    if (q.dim() != 5 || k.sizes() != q.sizes() || v.sizes() != q.sizes() || k.scalar_type() != t || v.scalar_type() != t) return false;
+    const int64_t D = q.size(4), L = q.size(3);
+    if (!(D == 16 || D == 32 || D == 64 || D == 128 || D == 256) || c.W < 1 || c.H < 1 || c.W > L || c.H > L || c.W * c.H != L) return false;
+    if (q.size(0) < 1 || q.size(1) < 1 || q.size(2) < 1 || coords.dim() != 6 || coords.size(4) < 1) return false;
+    if (q.size(0) > INT_MAX || q.size(1) > INT_MAX || q.size(2) > INT_MAX || L > INT_MAX) return false;
+    if (coords.scalar_type() != at::kFloat || !coords.is_contiguous() || coords.size(0) != q.size(0) ||
+        coords.size(1) != q.size(1) || coords.size(2) != L || coords.size(3) != q.size(1) || coords.size(5) != 2 || coords.size(4) > INT_MAX)
+        return false;
+    if (!q.is_cuda() || k.device() != q.device() || v.device() != q.device() || coords.device() != q.device()) return false;
+    Strides st;
+    return readable_in_place(q, k, v, &st);
+}
+
+PyObject *apply(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    if (n != 8 && n != 9) Py_RETURN_NONE;
+    for (int i = 1; i <= 4; ++i)
+        if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
+    if (!PyLong_Check(args[5]) || !PyLong_Check(args[6]) || !(PyFloat_Check(args[7]) || PyLong_Check(args[7]))) Py_RETURN_NONE;
+    Call c;
+    c.single_stream = PyObject_IsTrue(args[0]) == 1;
+    c.W = PyLong_AsLongLong(args[5]);
+    c.H = PyLong_AsLongLong(args[6]);
+    c.scale = PyFloat_AsDouble(args[7]);
+    const int cg = n == 9 ? PyObject_IsTrue(args[8]) : 0;
+    if (PyErr_Occurred() || cg < 0) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    c.coords_grad = cg == 1;
+    const Tensor &q = THPVariable_Unpack(args[1]), &k = THPVariable_Unpack(args[2]), &v = THPVariable_Unpack(args[3]),
+                 &coords = THPVariable_Unpack(args[4]);
+    if (!acceptable(q, k, v, coords, c)) Py_RETURN_NONE;
+    Tensor out;
+    try {
+        pybind11::gil_scoped_release no_gil;
+        const bool graph = at::GradMode::is_enabled() &&
+                           (q.requires_grad() || k.requires_grad() || v.requires_grad() || coords.requires_grad());
+        out = graph ? DeformSdpa::apply(q, k, v, coords, c) : forward(q, k, v, coords, c).first;
+    } catch (const Refused &r) {
+        return PyLong_FromLong(r.code);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {
+    {"apply", (PyCFunction)(void (*)(void))apply, METH_FASTCALL, "one call of the operator; None when the arguments need the Python side"},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_dsdpa_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__dsdpa_torch(void) { return PyModule_Create(&module); }

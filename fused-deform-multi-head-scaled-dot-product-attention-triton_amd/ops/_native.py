@@ -1,14 +1,16 @@
 """ctypes binding of libdsdpa.so (the C ABI declared in ``include/dsdpa.h``).
 
-The library is loaded from ``lib/libdsdpa.so`` next to this package. There is
-no fallback: if the library is missing, or a call returns an error code, an
-exception is raised.
+The library is loaded from ``lib/libdsdpa.so`` next to this package, and the operator's native host side from
+``lib/_dsdpa_torch.so``, which calls the same library. There is no fallback: if one is missing, or a call returns an
+error code, an exception is raised.
 """
 import ctypes
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libdsdpa.so")
+TORCH_LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "_dsdpa_torch.so")
 
 # every symbol include/dsdpa.h declares
 SYMBOLS = (
@@ -23,6 +25,7 @@ PATH_AUTO, PATH_GATHER, PATH_LDS = 0, 1, 2
 FLAG_DETERMINISTIC = 1
 FLAG_COORDS_GRAD = 2
 FLAG_SINGLE_STREAM = 4
+ERR_BAD_SHAPE = 2
 ERR_SCRATCH = 8
 ERR_BAD_STRIDES = 9
 NOALLOC_SCRATCH_BYTES = 32 << 20
@@ -75,6 +78,19 @@ def load():
     lib.dsdpa_timer_collect.restype = i
     _lib = lib
     return lib
+
+
+def load_torch():
+    """The extension module of csrc/dsdpa_torch.cpp. Raises if it is not built."""
+    load()
+    if not os.path.exists(TORCH_LIB_PATH):
+        raise ImportError(f"{TORCH_LIB_PATH} is missing: build it with `python build.py`. "
+                          "There is no fallback path for the fused operator.")
+    import torch  # noqa: F401  (its libraries have to be loaded first)
+    spec = importlib.util.spec_from_file_location("_dsdpa_torch", TORCH_LIB_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
 
 
 def strides_arg(q, k, v):
