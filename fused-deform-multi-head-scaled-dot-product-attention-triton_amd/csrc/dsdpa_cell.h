@@ -323,8 +323,14 @@ struct CellGrid {
 // in the order of the row's coordinates): an entry then costs a gather of that pair and the two rank-1 updates --
 // no taps in registers, no dot products, no exponential. Only with the work list (colour < 0) and with
 // records (the positions beside the ids).
-// RECORDS: the lists hold 12-byte records (sample id and position in the cell); without, ids alone, and every
-// entry's coordinate pair is read again (the deterministic backward, whose lists are sorted id arrays).
+// RECORDS: the lists hold 12-byte records (sample id and position in the cell), and the launch goes by the work list
+// (colour < 0); without, ids alone, and every entry's coordinate pair is read again (the deterministic backward,
+// whose lists are sorted id arrays, in its four colour launches).
+// What an item costs beside its entries is about 300 vector instructions (bounds, taps, tables, the sum over the
+// slots, the flush), which is most of the kernel where lists are short: 18x18, D = 32, 2 views x 2 samples (3.6
+// entries a list, fp32) 43.2 -> 39.0 us, 6 x 6 (32 entries, bf16) 170 -> 157, 14x14 with 8 x 32 (223, fp32) 247 -> 241,
+// with the slots summed on a quarter of the values where the step that halves them comes first, and no tables made
+// for a block that is not there.
 template <typename S, int D, int DC, bool HANDED, bool RECORDS>
 __global__ __launch_bounds__(kCellWaves *kWave, HANDED ? (DC <= 4 ? 5 : (S::kBytes == 2 ? 3 : 4))
                                                        : DC <= 4 ? (S::kBytes == 2 && D >= 64 ? 5 : 4) : (S::kBytes == 2 ? 3 : 2))
@@ -351,7 +357,6 @@ void bwd_dkdv_cell_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;   // wave index is uniform: keep it in an SGPR
     const unsigned work = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x) * kCellWaves + wave;
     if (work >= cg.nwork) return;
-    const int colour = cg.colour;
     // plane-major: (b, h, s2, cell or work item)
     unsigned t = cg.div_cells.div(work);
     const int ci = (int)(work - t * (unsigned)cg.ncells);
@@ -363,7 +368,7 @@ void bwd_dkdv_cell_kernel(
     const size_t grp = (size_t)b * dm.V + s2;
     int cy, cx, cell;
     unsigned lo, hi;
-    if (colour < 0) {
+    if constexpr (RECORDS) {
         const uint4 item = items[grp * (size_t)cg.ncells + ci];              // (cell, first entry, end)
         cell = (int)item.x;
         cy = (int)cg.div_ncx.div(item.x);                      // div_ncx: by Wimg + 1 in this mode
@@ -567,7 +572,7 @@ void bwd_dkdv_cell_kernel(
             e_a = load_entry_q(lo + 2 * kWave);
             const float2 pd0 = load_pair(e0.id), pd1 = load_pair(e1.id);
             tail = prepare(lo, 0, e0.id, make_float2(e0.fx, e0.fy), pd0);
-            tail += prepare(lo + kWave, tail, e1.id, make_float2(e1.fx, e1.fy), pd1);
+            if (lo + kWave < hi) tail += prepare(lo + kWave, tail, e1.id, make_float2(e1.fx, e1.fy), pd1);
         }
         wave_lds_sync();
         issue_q(0);
@@ -752,9 +757,13 @@ void bwd_dkdv_cell_kernel(
                 e_c = load_entry_c(c0 + 2 * kWave);
             }
             __builtin_amdgcn_sched_barrier(0);         // (requested here, not where they are used)
-            wave_lds_sync();
-            tables(c0 + kWave, cur ^ 1, e_a, pd_a);
-            wave_lds_sync();
+            // (a list of one block, the common case where lists are short, makes no second set of tables; plain ids
+            // bring their coordinate reads along, which may not sit under a branch)
+            if (has_next || !RECORDS) {
+                wave_lds_sync();
+                tables(c0 + kWave, cur ^ 1, e_a, pd_a);
+                wave_lds_sync();
+            }
             const int cnt = (int)min((unsigned)kWave, hi - c0);
             int j0 = 0;
             do {
@@ -799,22 +808,11 @@ void bwd_dkdv_cell_kernel(
             aV[2][d] -= aV[3][d];
         }
     }
-    // Sum the NS slots. Slots that differ in lane bits below 16 are summed by butterflies (every lane ends
-    // up with the sum); the last two steps (lane bits 16 and 32) are reduce-scatters on the lane-swap
-    // instructions: a step adds the two halves and leaves each half with one half of the taps, so that in
+    // Sum the NS slots. First the steps that halve what a lane holds (lane bits 16 and 32), reduce-scatters on the
+    // lane-swap instructions: a step adds the two halves and leaves each half with one half of the taps, so that in
     // the end lane bit 16 and lane bit 32 select the tap a lane holds (G <= 16), or bit 32 the tap pair
-    // (G = 32), and all 64 lanes carry sums that go to memory.
-#pragma unroll
-    for (int off = G; off < 16; off <<= 1) {
-#pragma unroll
-        for (int tpi = 0; tpi < 4; ++tpi) {
-#pragma unroll
-            for (int d = 0; d < DC; ++d) {
-                aK[tpi][d] += __shfl_xor(aK[tpi][d], off, kWave);
-                aV[tpi][d] += __shfl_xor(aV[tpi][d], off, kWave);
-            }
-        }
-    }
+    // (G = 32), and all 64 lanes carry sums that go to memory. Then, on the quarter that is left, slots that differ
+    // in lane bits below 16 by rotations of the 16 lanes (by 8, and by 4 once the lanes 8 apart agree).
     static_assert(G <= 32, "at least two slots");
     constexpr int kTapsHeld = G <= 16 ? 1 : 2;             // taps a lane holds after the reduce-scatters
     float hK[kTapsHeld][DC], hV[kTapsHeld][DC];
@@ -826,6 +824,8 @@ void bwd_dkdv_cell_kernel(
             const float v0 = swap_add_16(aV[0][d], aV[2][d]), v1 = swap_add_16(aV[1][d], aV[3][d]);
             hK[0][d] = swap_add_32(k0, k1);
             hV[0][d] = swap_add_32(v0, v1);
+            if constexpr (G < 16) { hK[0][d] += row_rotate<8>(hK[0][d]); hV[0][d] += row_rotate<8>(hV[0][d]); }
+            if constexpr (G < 8) { hK[0][d] += row_rotate<4>(hK[0][d]); hV[0][d] += row_rotate<4>(hV[0][d]); }
         }
     } else {
 #pragma unroll
@@ -869,7 +869,7 @@ void bwd_dkdv_cell_kernel(
             const float val = fl[idx];
             if (ok) {
                 float *pa = acc + (size_t)pix * D + dd;
-                if (colour < 0) atomicAdd(pa, val);
+                if constexpr (RECORDS) atomicAdd(pa, val);
                 else *pa += val;
             }
         }

@@ -488,6 +488,13 @@ __device__ __forceinline__ float swap_add_16(float x, float y)
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// The value N lanes on, round the row of 16 (DPP row rotation: part of the instruction that uses it).
+template <int N>
+__device__ __forceinline__ float row_rotate(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + N, 0xf, 0xf, false));
+}
+
 // Orders this wave's LDS writes before its later LDS reads (and the reverse):
 // waits for the wave's outstanding LDS traffic and stops the compiler from
 // moving LDS accesses across. No workgroup barrier is involved.
