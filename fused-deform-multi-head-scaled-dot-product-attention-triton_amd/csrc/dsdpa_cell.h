@@ -38,9 +38,11 @@ __device__ __forceinline__ int cell_of(const Taps &tp, int Wimg) { return (tp.y0
 // instead of gathering the coordinate pair again (a random 8-byte read per entry, per head).
 __device__ __forceinline__ float2 cell_fraction(float2 xy, const Dims &dm)
 {
-    const float x = ((xy.x * 2.0f - 1.0f) + 1.0f) * ((float)(dm.Wimg - 1) * 0.5f);
-    const float y = ((xy.y * 2.0f - 1.0f) + 1.0f) * ((float)(dm.Himg - 1) * 0.5f);
-    return make_float2(x - floorf(x), y - floorf(y));
+    // (fused, so that the position keeps the bits that the rounded pixel coordinate drops, whatever the compiler
+    // would contract where this is inlined)
+    const float ax = (xy.x * 2.0f - 1.0f) + 1.0f, kx = (float)(dm.Wimg - 1) * 0.5f;
+    const float ay = (xy.y * 2.0f - 1.0f) + 1.0f, ky = (float)(dm.Himg - 1) * 0.5f;
+    return make_float2(fmaf(ax, kx, -floorf(ax * kx)), fmaf(ay, ky, -floorf(ay * ky)));
 }
 
 __device__ __forceinline__ bool taps_any(const Taps &tp)
@@ -177,6 +179,62 @@ __global__ __launch_bounds__(kBinLdsThreads) void bin_samples_lds_kernel(
 // sums by lane shifts inside a wave and over the 16 waves' totals in LDS, two barriers per 4096 keys.
 // (8450 keys, 8 workgroups: 29.4 -> 15.3 us against a scan of 1024 keys at a time with 20 barriers; 2401 keys 10.4 -> 6.0.)
 constexpr int kScanKeys = 4;
+struct ScanCarry { unsigned entries, pieces; };
+// One turn of the scan for a workgroup of 1024 threads: keys [c0, c0 + 4) of each thread, v their list lengths;
+// returns the first key's start in `first`, writes start and items, advances the carry. s_wave: 16 places.
+__device__ __forceinline__ void scan_keys(const unsigned (&v)[kScanKeys], int c0, int NC, int grid_cells, unsigned piece,
+                                          unsigned wmax, unsigned *__restrict__ st, uint4 *__restrict__ it,
+                                          uint2 *s_wave, ScanCarry &carry, unsigned &first)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned np[kScanKeys], sum = 0, psum = 0;
+#pragma unroll
+    for (int i = 0; i < kScanKeys; ++i) {
+        np[i] = (v[i] + piece - 1) / piece;                        // pieces of this list
+        sum += v[i];
+        psum += np[i];
+    }
+    unsigned incl = sum, pincl = psum;                             // inclusive scans over the wave
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const unsigned add = (unsigned)__shfl_up((int)incl, off, kWave), padd = (unsigned)__shfl_up((int)pincl, off, kWave);
+        incl += lane >= off ? add : 0u;
+        pincl += lane >= off ? padd : 0u;
+    }
+    __syncthreads();                                               // (the totals of the keys before have been read)
+    if (lane == kWave - 1) s_wave[wave] = make_uint2(incl, pincl);
+    __syncthreads();
+    unsigned excl = carry.entries + incl - sum, pexcl = carry.pieces + pincl - psum;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        const uint2 t = s_wave[w];
+        excl += w < wave ? t.x : 0u;
+        pexcl += w < wave ? t.y : 0u;
+        carry.entries += t.x;
+        carry.pieces += t.y;
+    }
+    first = excl;
+#pragma unroll
+    for (int i = 0; i < kScanKeys; ++i) {
+        if (c0 + i < NC) {
+            st[c0 + i] = excl;
+            const unsigned cell = (unsigned)((c0 + i) % grid_cells);
+            for (unsigned j = 0; j < np[i]; ++j)
+                if (pexcl + j < wmax)
+                    it[pexcl + j] = make_uint4(cell, excl + j * piece, min(excl + v[i], excl + (j + 1) * piece), 0u);
+        }
+        excl += v[i];
+        pexcl += np[i];
+    }
+}
+
+// after the last turn: the total, and the empty slots behind the items
+__device__ __forceinline__ void scan_end(const ScanCarry &carry, int NC, unsigned wmax, unsigned *__restrict__ st, uint4 *__restrict__ it)
+{
+    if (threadIdx.x == 0) st[NC] = carry.entries;
+    for (unsigned i = min(carry.pieces, wmax) + threadIdx.x; i < wmax; i += 1024) it[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 static __global__ __launch_bounds__(1024) void bin_scan_kernel(unsigned *__restrict__ counters,
                                                         unsigned *__restrict__ start, int NC, int grid_cells,
                                                         unsigned piece, unsigned wmax, uint4 *__restrict__ items)
@@ -185,54 +243,86 @@ static __global__ __launch_bounds__(1024) void bin_scan_kernel(unsigned *__restr
     unsigned *cnt = counters + (size_t)blockIdx.x * NC;
     unsigned *st = start + (size_t)blockIdx.x * (NC + 1);
     uint4 *it = items + (size_t)blockIdx.x * wmax;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned carry = 0, pcarry = 0;
+    ScanCarry carry{0u, 0u};
     for (int base = 0; base < NC; base += 1024 * kScanKeys) {
         const int c0 = base + (int)threadIdx.x * kScanKeys;
-        unsigned v[kScanKeys], np[kScanKeys], sum = 0, psum = 0;
+        unsigned v[kScanKeys], at;
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NC ? cnt[c0 + i] : 0u;
+        scan_keys(v, c0, NC, grid_cells, piece, wmax, st, it, s_wave, carry, at);
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) {
-            np[i] = (v[i] + piece - 1) / piece;                    // pieces of this list
-            sum += v[i];
-            psum += np[i];
-        }
-        unsigned incl = sum, pincl = psum;                         // inclusive scans over the wave
-#pragma unroll
-        for (int off = 1; off < kWave; off <<= 1) {
-            const unsigned add = (unsigned)__shfl_up((int)incl, off, kWave), padd = (unsigned)__shfl_up((int)pincl, off, kWave);
-            incl += lane >= off ? add : 0u;
-            pincl += lane >= off ? padd : 0u;
-        }
-        __syncthreads();                                           // (the totals of the keys before have been read)
-        if (lane == kWave - 1) s_wave[wave] = make_uint2(incl, pincl);
-        __syncthreads();
-        unsigned excl = carry + incl - sum, pexcl = pcarry + pincl - psum;
-#pragma unroll
-        for (int w = 0; w < 16; ++w) {
-            const uint2 t = s_wave[w];
-            excl += w < wave ? t.x : 0u;
-            pexcl += w < wave ? t.y : 0u;
-            carry += t.x;
-            pcarry += t.y;
-        }
-#pragma unroll
-        for (int i = 0; i < kScanKeys; ++i) {
-            if (c0 + i < NC) {
-                st[c0 + i] = excl;
-                cnt[c0 + i] = excl;
-                const unsigned cell = (unsigned)((c0 + i) % grid_cells);
-                for (unsigned j = 0; j < np[i]; ++j)
-                    if (pexcl + j < wmax)
-                        it[pexcl + j] = make_uint4(cell, excl + j * piece, min(excl + v[i], excl + (j + 1) * piece), 0u);
-            }
-            excl += v[i];
-            pexcl += np[i];
+            if (c0 + i < NC) cnt[c0 + i] = at;
+            at += v[i];
         }
     }
-    if (threadIdx.x == 0) st[NC] = carry;
-    for (unsigned i = min(pcarry, wmax) + threadIdx.x; i < wmax; i += 1024) it[i] = make_uint4(0u, 0u, 0u, 0u);
+    scan_end(carry, NC, wmax, st, it);
+}
+
+// Count, scan and fill in one launch, for lists short enough that one workgroup holds all samples of a (b, s2) in
+// its registers, PER of them a thread: every sample's rank in its list comes from the counting atomic itself, so
+// the coordinates are read once and there is one round of LDS atomics, no counters in memory (nothing to clear)
+// and no wait between launches. Bound by that chain of latencies (a few workgroups on the whole chip), as the three
+// launches are: 1296 samples a list group (18x18, 2 views x 2 samples) 6.4 us against 13.2 for the three and the gaps
+// between them. One workgroup's throughput then takes over: 5184 (4 x 4, six samples a thread) 13.9 against 17.4, a step
+// no faster; 11664 34.8 against 24.1, 17871 59 against 19.
+// Keys: at most kBinOneKeys, in LDS.
+constexpr int kBinOneKeys = 8192, kBinOneSamples = 2 * 1024;
+template <int PER>
+__global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__ coords_, Dims dm, int NC, int NK, int vpg,
+                                                       unsigned *__restrict__ start, unsigned piece, unsigned wmax,
+                                                       uint4 *__restrict__ items, unsigned *__restrict__ sorted, int records)
+{
+    __shared__ unsigned s_hist[kBinOneKeys];                       // list lengths, then starts
+    __shared__ uint2 s_wave[16];
+    const int s2 = blockIdx.x % dm.V, b = blockIdx.x / dm.V;       // blockIdx.x = (b, s2), as the scan's
+    const unsigned M = (unsigned)dm.V * (unsigned)dm.L * (unsigned)dm.P;
+    const float2 *crd = reinterpret_cast<const float2 *>(coords_) + ((size_t)b * dm.V * dm.L * dm.V + s2) * (size_t)dm.P;
+    float2 xy[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const unsigned id = min((unsigned)i * 1024u + threadIdx.x, M - 1u);            // id = ql * P + p
+        const unsigned ql = dm.divP.div(id), p = id - ql * (unsigned)dm.P;
+        xy[i] = crd[(size_t)ql * dm.N + p];
+    }
+    for (int i = threadIdx.x; i < NK; i += 1024) s_hist[i] = 0u;
+    __syncthreads();
+    unsigned key_rank[PER];                                        // key in 13 bits, rank above; all ones: in no list
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const unsigned id = (unsigned)i * 1024u + threadIdx.x;
+        const Taps tp = make_taps(xy[i].x, xy[i].y, dm.Wimg, dm.Himg);
+        key_rank[i] = 0xffffffffu;
+        if (id < M && taps_any(tp)) {
+            const unsigned s1 = dm.divL.div(dm.divP.div(id));
+            const unsigned key = (s1 / (unsigned)vpg) * (unsigned)NC + (unsigned)cell_of(tp, dm.Wimg);
+            key_rank[i] = key | (atomicAdd(&s_hist[key], 1u) << 13);
+        }
+    }
+    __syncthreads();
+    ScanCarry carry{0u, 0u};
+    unsigned *st = start + (size_t)blockIdx.x * (NK + 1);
+    uint4 *it = items + (size_t)blockIdx.x * wmax;
+    for (int base = 0; base < NK; base += 1024 * kScanKeys) {
+        const int c0 = base + (int)threadIdx.x * kScanKeys;
+        unsigned v[kScanKeys], at;
+#pragma unroll
+        for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NK ? s_hist[c0 + i] : 0u;
+        scan_keys(v, c0, NK, NC, piece, wmax, st, it, s_wave, carry, at);
+#pragma unroll
+        for (int i = 0; i < kScanKeys; ++i) {
+            if (c0 + i < NK) s_hist[c0 + i] = at;                  // (this thread's own keys)
+            at += v[i];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        if (key_rank[i] != 0xffffffffu)
+            store_cell_entry(sorted, (size_t)blockIdx.x * M + s_hist[key_rank[i] & (kBinOneKeys - 1)] + (key_rank[i] >> 13),
+                             (unsigned)i * 1024u + threadIdx.x, cell_fraction(xy[i], dm), records);
+    }
+    scan_end(carry, NK, wmax, st, it);
 }
 
 // Deterministic backward: begin / end of every cell list as positions in the flat id array
