@@ -1,16 +1,17 @@
 // Host side of the PyTorch operator: argument checks, output and workspace allocation, the autograd node and the
 // calls of the C ABI (include/dsdpa.h), in C++. The counterpart of the reference's autograd.Function
-// (ops/triton.py:377-466); ops/triton.py holds the Python entry point, which raises the exceptions.
+// (ops/triton.py:377-466) for ordinary calls; ops/triton.py holds the Python entry point and an autograd.Function,
+// the general route of every call that is handed back to it here.
 //
 // Why native: at the small end of the operator's range the GPU finishes long before the host has enqueued the next
 // launch. With the checks, torch.empty calls, ctypes conversions and autograd.Function of Python a training step
 // took 165 us of host time whatever its size (views x samples 2x2 of the sweep, 18x18, 32 heads: 162 us a step for
 // 86 us of kernels).
 //
-// apply(single_stream, q, k, v, coords, WIDTH, HEIGHT, sm_scale[, coords_grad]) -> out; None when an argument is
-// not what the kernels take as it is (wrong shape or type, layout that has to be copied first): nothing has
-// been done then, and the Python side says what is wrong or mends it; a number when the library refused the call (its
-// error code). No tensor is kept from one call for the next.
+// apply(single_stream, q, k, v, coords, WIDTH, HEIGHT, sm_scale[, coords_grad]) -> out; None when the arguments
+// are wrong, or when PyTorch follows the call in a way that goes by an autograd.Function (followed()): nothing has been
+// done then, and the call takes the general route, which raises or is followed; a number when the library refused the call (its error code). No tensor is kept from one
+// call for the next.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -18,6 +19,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -175,7 +177,18 @@ struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
     }
 };
 
-// The reference's preconditions (ops/triton.py:375,385-388) and this build's: true when the call can go ahead as it is.
+// Whether the call has to be an autograd.Function's: an input carries a forward-mode tangent, or a torch.func transform
+// is active. The kernels read the values alone, and neither shows in requires_grad: from here the tangent would be
+// dropped without a word. The Function has no rule for them and raises.
+bool followed(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &coords)
+{
+    if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) return true;
+    for (const Tensor *t : {&q, &k, &v, &coords})
+        if (t->_fw_grad(/*level=*/0).defined()) return true;
+    return false;
+}
+
+// The reference's preconditions (ops/triton.py:375,385-388) and this build's own.
 bool acceptable(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &coords, const Call &c)
 {
     const at::ScalarType t = q.scalar_type();
@@ -185,12 +198,10 @@ bool acceptable(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor 
     if (!(D == 16 || D == 32 || D == 64 || D == 128 || D == 256) || c.W < 1 || c.H < 1 || c.W > L || c.H > L || c.W * c.H != L) return false;
     if (q.size(0) < 1 || q.size(1) < 1 || q.size(2) < 1 || coords.dim() != 6 || coords.size(4) < 1) return false;
     if (q.size(0) > INT_MAX || q.size(1) > INT_MAX || q.size(2) > INT_MAX || L > INT_MAX) return false;
-    if (coords.scalar_type() != at::kFloat || !coords.is_contiguous() || coords.size(0) != q.size(0) ||
-        coords.size(1) != q.size(1) || coords.size(2) != L || coords.size(3) != q.size(1) || coords.size(5) != 2 || coords.size(4) > INT_MAX)
+    if (!coords.is_contiguous() || coords.size(0) != q.size(0) || coords.size(1) != q.size(1) || coords.size(2) != L ||
+        coords.size(3) != q.size(1) || coords.size(5) != 2 || coords.size(4) > INT_MAX)
         return false;
-    if (!q.is_cuda() || k.device() != q.device() || v.device() != q.device() || coords.device() != q.device()) return false;
-    Strides st;
-    return readable_in_place(q, k, v, &st);
+    return q.is_cuda() && k.device() == q.device() && v.device() == q.device() && coords.device() == q.device();
 }
 
 PyObject *apply(PyObject *, PyObject *const *args, Py_ssize_t n)
@@ -199,36 +210,45 @@ PyObject *apply(PyObject *, PyObject *const *args, Py_ssize_t n)
     if (n != 8 && n != 9) Py_RETURN_NONE;
     for (int i = 1; i <= 4; ++i)
         if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
-    if (!PyLong_Check(args[5]) || !PyLong_Check(args[6]) || !(PyFloat_Check(args[7]) || PyLong_Check(args[7]))) Py_RETURN_NONE;
+    Tensor q = THPVariable_Unpack(args[1]), k = THPVariable_Unpack(args[2]), v = THPVariable_Unpack(args[3]),
+           coords = THPVariable_Unpack(args[4]);
+    if (followed(q, k, v, coords)) Py_RETURN_NONE;
     Call c;
-    c.single_stream = PyObject_IsTrue(args[0]) == 1;
-    c.W = PyLong_AsLongLong(args[5]);
-    c.H = PyLong_AsLongLong(args[6]);
-    c.scale = PyFloat_AsDouble(args[7]);
-    const int cg = n == 9 ? PyObject_IsTrue(args[8]) : 0;
-    if (PyErr_Occurred() || cg < 0) {
+    c.W = PyNumber_AsSsize_t(args[5], PyExc_OverflowError);
+    c.H = PyErr_Occurred() ? 0 : PyNumber_AsSsize_t(args[6], PyExc_OverflowError);
+    PyObject *scale = PyErr_Occurred() ? nullptr : PyNumber_Float(args[7]);
+    const int cg = scale && n == 9 ? PyObject_IsTrue(args[8]) : 0, ss = scale ? PyObject_IsTrue(args[0]) : 0;
+    if (scale) {
+        c.scale = PyFloat_AS_DOUBLE(scale);
+        Py_DECREF(scale);
+    }
+    if (!scale || cg < 0 || ss < 0) {
         PyErr_Clear();
         Py_RETURN_NONE;
     }
     c.coords_grad = cg == 1;
-    const Tensor &q = THPVariable_Unpack(args[1]), &k = THPVariable_Unpack(args[2]), &v = THPVariable_Unpack(args[3]),
-                 &coords = THPVariable_Unpack(args[4]);
-    if (!acceptable(q, k, v, coords, c)) Py_RETURN_NONE;
+    c.single_stream = ss == 1;
     Tensor out;
     try {
         pybind11::gil_scoped_release no_gil;
-        const bool graph = at::GradMode::is_enabled() &&
-                           (q.requires_grad() || k.requires_grad() || v.requires_grad() || coords.requires_grad());
-        out = graph ? DeformSdpa::apply(q, k, v, coords, c) : forward(q, k, v, coords, c).first;
+        if (acceptable(q, k, v, coords, c)) {
+            Strides st;
+            if (!readable_in_place(q, k, v, &st)) q = q.contiguous(), k = k.contiguous(), v = v.contiguous();
+            if (coords.scalar_type() != at::kFloat) coords = coords.to(at::kFloat);
+            const bool graph = at::GradMode::is_enabled() &&
+                               (q.requires_grad() || k.requires_grad() || v.requires_grad() || coords.requires_grad());
+            out = graph ? DeformSdpa::apply(q, k, v, coords, c) : forward(q, k, v, coords, c).first;
+        }
     } catch (const Refused &r) {
         return PyLong_FromLong(r.code);
     }
+    if (!out.defined()) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef methods[] = {
-    {"apply", (PyCFunction)(void (*)(void))apply, METH_FASTCALL, "one call of the operator; None when the arguments need the Python side"},
+    {"apply", (PyCFunction)(void (*)(void))apply, METH_FASTCALL, "one call of the operator; None when it has to take the general route"},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_dsdpa_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

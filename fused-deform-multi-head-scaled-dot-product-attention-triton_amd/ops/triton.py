@@ -16,8 +16,9 @@ Contract mirrored from ``_fused_deform_sdpa`` (``ops/triton.py:377-466``):
   ``NotImplementedError`` for an unsupported dtype;
 * fp32 storage, or bf16/fp16 storage with fp32 accumulation.
 
-The call itself -- checks, allocations, the autograd node -- is native (``csrc/dsdpa_torch.cpp``); what follows here
-is what it does not take as it is: the errors, and the layouts and types that are copied first.
+An ordinary call -- checks, allocations, the autograd node -- is native (``csrc/dsdpa_torch.cpp``). Every other call
+takes the ``torch.autograd.Function`` below, the general route: the errors, and the callers that PyTorch follows or
+refuses by way of that class (forward-mode AD and the ``torch.func`` transforms, for which the operator has no rule).
 
 Differences, all on purpose: coords are not cloned or pre-scaled (the kernels
 un-normalise), ``out``/``dq`` are not zero-filled first, no scaled copy of K is
@@ -27,13 +28,13 @@ q/k/v are read in place where the head dimension is contiguous (and copied
 otherwise) instead of asserted, dout is made contiguous, and only the
 log-sum-exp is saved on top of the inputs and output.
 """
-import operator
-
 import torch
 
 from . import _native
 
-_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
+_SUFFIX = {torch.float32: "f32", torch.bfloat16: "bf16", torch.float16: "f16"}
+_DTYPE_CODE = {torch.float32: _native.DSDPA_F32, torch.bfloat16: _native.DSDPA_BF16,
+               torch.float16: _native.DSDPA_F16}
 
 # The backward runs its dk/dv side beside the dq side on a second stream of the library's (forked from and joined
 # to the caller's stream inside the call). True keeps every launch on the caller's stream (same results).
@@ -44,7 +45,7 @@ _apply = None
 
 def _check_inputs(q, k, v, coords, WIDTH, HEIGHT):
     """Raises what the reference raises (``ops/triton.py:367-375,385-388``), and this build's own errors."""
-    if q.dtype not in _DTYPES:
+    if q.dtype not in _SUFFIX:
         raise NotImplementedError(f"unsupported dtype {q.dtype}")
     assert q.dim() == 5 and k.shape == q.shape and v.shape == q.shape, "q, k, v must share (B, V, H, L, D)"
     assert q.shape[-1] == k.shape[-1] == v.shape[-1]
@@ -61,22 +62,75 @@ def _check_inputs(q, k, v, coords, WIDTH, HEIGHT):
                            "use ops.torch.deform_sdpa_torch for an eager operator")
     if not (k.device == q.device and v.device == q.device and coords.device == q.device):
         raise RuntimeError("q, k, v, coords must be on one device")
-    if B < 1 or V < 1 or H < 1 or L < 1 or coords.shape[4] < 1:
-        _native.check(_native.ERR_BAD_SHAPE)
 
 
-def _mend_and_apply(q, k, v, coords, WIDTH, HEIGHT, sm_scale, *extra):
-    _check_inputs(q, k, v, coords, WIDTH, HEIGHT)
-    # strided q, k, v are read in place where the kernels can (the reference's forward takes their strides,
-    # ops/triton.py:396-405): head dimension contiguous, rows 16-byte aligned, k and v laid out alike
-    if _native.strides_arg(q, k, v) is False:
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-    if coords.dtype != torch.float32:
-        coords = coords.float()
-    out = _apply(SINGLE_STREAM, q, k, v, coords, operator.index(WIDTH), operator.index(HEIGHT), float(sm_scale), *extra)
-    if out is None:
-        raise RuntimeError("deform_sdpa_triton: the arguments are not ones the library takes")
-    return out
+class _fused_deform_sdpa(torch.autograd.Function):
+    """The general route. Every buffer comes from ``torch.empty``, so that dispatch modes see it."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, coords, WIDTH, HEIGHT, sm_scale, *extra):
+        if len(extra) > 1:
+            raise TypeError("deform_sdpa_triton takes 7 arguments and an optional coords_grad flag")
+        ctx.n_inputs = 7 + len(extra)
+        ctx.coords_grad = bool(extra[0]) if extra else False
+        _check_inputs(q, k, v, coords, WIDTH, HEIGHT)
+        lib = _native.load()
+        B, V, H, L, D = q.shape
+        P = coords.shape[-2]
+        # strided q, k, v are read in place where the kernels can (the reference's forward takes their strides,
+        # ops/triton.py:396-405): head dimension contiguous, rows 16-byte aligned, k and v laid out alike
+        strides = _native.strides_arg(q, k, v)
+        if strides is False:
+            q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+            strides = None
+        if coords.dtype != torch.float32:
+            coords = coords.float()
+        out = torch.empty(q.shape, device=q.device, dtype=q.dtype)          # contiguous whatever q's layout
+        lse = torch.empty((B, V, H, L), device=q.device, dtype=torch.float32)
+        ws_bytes = lib.dsdpa_fwd_workspace_bytes(_DTYPE_CODE[q.dtype], B, V, H, HEIGHT, WIDTH, D, P)
+        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)     # scratch, not saved for backward
+        with torch.cuda.device(q.device):
+            rc = getattr(lib, "dsdpa_fwd_" + _SUFFIX[q.dtype])(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), coords.data_ptr(), out.data_ptr(), lse.data_ptr(),
+                ws.data_ptr() if ws_bytes else None, B, V, H, HEIGHT, WIDTH, D, P, float(sm_scale), strides,
+                torch.cuda.current_stream(q.device).cuda_stream)
+        _native.check(rc)
+        ctx.save_for_backward(q, k, v, coords, out, lse)
+        ctx.sm_scale = float(sm_scale)
+        ctx.WIDTH, ctx.HEIGHT = WIDTH, HEIGHT
+        return out
+
+    @staticmethod
+    def backward(ctx, do):
+        q, k, v, coords, out, lse = ctx.saved_tensors
+        lib = _native.load()
+        B, V, H, L, D = q.shape
+        P = coords.shape[-2]
+        do = do.contiguous()
+        if do.dtype != q.dtype:
+            do = do.to(q.dtype)
+        dq, dk, dv = (torch.empty(q.shape, device=q.device, dtype=q.dtype) for _ in range(3))
+        strides = _native.strides_arg(q, k, v)          # (what forward saved: contiguous, or readable in place)
+        dcoords = torch.empty_like(coords) if ctx.coords_grad and ctx.needs_input_grad[3] else None
+        # torch.use_deterministic_algorithms(True) selects the bitwise reproducible backward
+        flags = _native.FLAG_DETERMINISTIC if torch.are_deterministic_algorithms_enabled() else 0
+        if flags and dcoords is not None:
+            raise RuntimeError("deform_sdpa_triton: the coordinate gradient has no deterministic implementation "
+                               "(it sums over heads with float atomics); turn one of the two off")
+        if dcoords is not None:
+            flags |= _native.FLAG_COORDS_GRAD
+        if SINGLE_STREAM:
+            flags |= _native.FLAG_SINGLE_STREAM
+        ws_bytes = lib.dsdpa_bwd_workspace_bytes(_DTYPE_CODE[q.dtype], B, V, H, ctx.HEIGHT, ctx.WIDTH, D, P, flags)
+        ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
+        with torch.cuda.device(q.device):
+            rc = getattr(lib, "dsdpa_bwd_" + _SUFFIX[q.dtype])(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), coords.data_ptr(), out.data_ptr(), lse.data_ptr(),
+                do.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                dcoords.data_ptr() if dcoords is not None else None, ws.data_ptr(), B, V, H, ctx.HEIGHT, ctx.WIDTH, D, P,
+                ctx.sm_scale, strides, flags, torch.cuda.current_stream(q.device).cuda_stream)
+        _native.check(rc)
+        return (dq, dk, dv, dcoords) + (None,) * (ctx.n_inputs - 4)
 
 
 def deform_sdpa_triton(*args):
@@ -88,11 +142,9 @@ def deform_sdpa_triton(*args):
     global _apply
     if _apply is None:
         _apply = _native.load_torch().apply
-    if not 7 <= len(args) <= 8:
-        raise TypeError("deform_sdpa_triton takes 7 arguments and an optional coords_grad flag")
     out = _apply(SINGLE_STREAM, *args)
     if out is None:
-        out = _mend_and_apply(*args)
+        return _fused_deform_sdpa.apply(*args)
     if isinstance(out, int):
         _native.check(out)
     return out

@@ -1,0 +1,44 @@
+"""The operator under the ways PyTorch follows a call other than by requires_grad, and what its backward reads and
+raises at the time it runs: where the autograd node is native, nothing of that may be passed by."""
+import pytest
+import torch
+from torch.autograd import forward_ad
+
+from ops import triton as op
+
+pytestmark = pytest.mark.gpu
+
+B, V, H, HIMG, WIMG, D, P = 1, 2, 2, 3, 4, 32, 3
+
+
+def inputs(seed=0, dtype=torch.float32):
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn(B, V, H, HIMG * WIMG, D, generator=g).to(dtype).cuda() for _ in range(3))
+    return [q, k, v, torch.rand(B, V, HIMG * WIMG, V, P, 2, generator=g).cuda()]
+
+
+def call(q, k, v, c):
+    return op.deform_sdpa_triton(q, k, v, c, WIMG, HIMG, 0.3)
+
+
+@pytest.mark.parametrize("which", [0, 3])
+@pytest.mark.parametrize("requires_grad", [False, True])
+@pytest.mark.parametrize("grad_mode", [False, True])
+def test_forward_mode_is_refused(which, requires_grad, grad_mode):
+    print(f"[case] dual {which} {requires_grad} {grad_mode}", flush=True)
+    args = inputs()
+    args[0].requires_grad_(requires_grad)
+    with forward_ad.dual_level(), torch.set_grad_enabled(grad_mode):
+        args[which] = forward_ad.make_dual(args[which], torch.ones_like(args[which]))
+        with pytest.raises(NotImplementedError, match="jvp"):
+            call(*args)
+
+
+def test_function_transforms_are_refused():
+    print("[case] transforms", flush=True)
+    q, k, v, c = inputs()
+    for f in (lambda x: call(q * x, k, v, c), lambda x: call(q, k, v, c) * x):
+        with pytest.raises(RuntimeError, match="functorch"):
+            torch.func.vmap(f)(torch.ones(2, device="cuda"))
+        with pytest.raises(RuntimeError, match="functorch"):
+            torch.func.grad(lambda x: f(x).sum())(torch.ones((), device="cuda"))
