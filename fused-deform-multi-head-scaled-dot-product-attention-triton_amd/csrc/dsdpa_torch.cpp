@@ -22,6 +22,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/dsdpa.h"
 
@@ -179,9 +180,11 @@ struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
 
 // Whether the call has to be an autograd.Function's: an input carries a forward-mode tangent, or a torch.func transform
 // is active. The kernels read the values alone, and neither shows in requires_grad: from here the tangent would be
-// dropped without a word. The Function has no rule for them and raises.
+// dropped without a word. The Function has no rule for them and raises. Under torch.jit.trace the Function is recorded
+// as a node; a call from here would be invisible, and its output a constant of the traced module.
 bool followed(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &coords)
 {
+    if (torch::jit::tracer::isTracing()) return true;
     if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) return true;
     for (const Tensor *t : {&q, &k, &v, &coords})
         if (t->_fw_grad(/*level=*/0).defined()) return true;

@@ -18,7 +18,8 @@ Contract mirrored from ``_fused_deform_sdpa`` (``ops/triton.py:377-466``):
 
 An ordinary call -- checks, allocations, the autograd node -- is native (``csrc/dsdpa_torch.cpp``). Every other call
 takes the ``torch.autograd.Function`` below, the general route: the errors, and the callers that PyTorch follows or
-refuses by way of that class (forward-mode AD and the ``torch.func`` transforms, for which the operator has no rule).
+refuses by way of that class (``torch.jit.trace``, which records it; forward-mode AD and the ``torch.func``
+transforms, for which the operator has no rule).
 
 Differences, all on purpose: coords are not cloned or pre-scaled (the kernels
 un-normalise), ``out``/``dq`` are not zero-filled first, no scaled copy of K is
@@ -28,6 +29,8 @@ q/k/v are read in place where the head dimension is contiguous (and copied
 otherwise) instead of asserted, dout is made contiguous, and only the
 log-sum-exp is saved on top of the inputs and output.
 """
+import contextlib
+
 import torch
 
 from . import _native
@@ -64,6 +67,19 @@ def _check_inputs(q, k, v, coords, WIDTH, HEIGHT):
         raise RuntimeError("q, k, v, coords must be on one device")
 
 
+@contextlib.contextmanager
+def _not_traced():
+    """Inside, sizes are plain ints also while ``torch.jit.trace`` records the caller. (It records the Function as a
+    node that calls it again, so nothing depends on a size having been read. The buffers are made outside: the output has
+    to be one that the tracer knows.)"""
+    state = torch._C._get_tracing_state()
+    torch._C._set_tracing_state(None)
+    try:
+        yield
+    finally:
+        torch._C._set_tracing_state(state)
+
+
 class _fused_deform_sdpa(torch.autograd.Function):
     """The general route. Every buffer comes from ``torch.empty``, so that dispatch modes see it."""
 
@@ -73,19 +89,20 @@ class _fused_deform_sdpa(torch.autograd.Function):
             raise TypeError("deform_sdpa_triton takes 7 arguments and an optional coords_grad flag")
         ctx.n_inputs = 7 + len(extra)
         ctx.coords_grad = bool(extra[0]) if extra else False
-        _check_inputs(q, k, v, coords, WIDTH, HEIGHT)
         lib = _native.load()
-        B, V, H, L, D = q.shape
-        P = coords.shape[-2]
-        # strided q, k, v are read in place where the kernels can (the reference's forward takes their strides,
-        # ops/triton.py:396-405): head dimension contiguous, rows 16-byte aligned, k and v laid out alike
-        strides = _native.strides_arg(q, k, v)
+        with _not_traced():
+            _check_inputs(q, k, v, coords, WIDTH, HEIGHT)
+            B, V, H, L, D = q.shape
+            P = coords.shape[-2]
+            # strided q, k, v are read in place where the kernels can (the reference's forward takes their strides,
+            # ops/triton.py:396-405): head dimension contiguous, rows 16-byte aligned, k and v laid out alike
+            strides = _native.strides_arg(q, k, v)
         if strides is False:
             q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
             strides = None
         if coords.dtype != torch.float32:
             coords = coords.float()
-        out = torch.empty(q.shape, device=q.device, dtype=q.dtype)          # contiguous whatever q's layout
+        out = torch.empty((B, V, H, L, D), device=q.device, dtype=q.dtype)  # contiguous whatever q's layout
         lse = torch.empty((B, V, H, L), device=q.device, dtype=torch.float32)
         ws_bytes = lib.dsdpa_fwd_workspace_bytes(_DTYPE_CODE[q.dtype], B, V, H, HEIGHT, WIDTH, D, P)
         ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)     # scratch, not saved for backward

@@ -42,3 +42,24 @@ def test_function_transforms_are_refused():
             torch.func.vmap(f)(torch.ones(2, device="cuda"))
         with pytest.raises(RuntimeError, match="functorch"):
             torch.func.grad(lambda x: f(x).sum())(torch.ones((), device="cuda"))
+
+
+@pytest.mark.parametrize("requires_grad", [False, True])
+@pytest.mark.parametrize("layout", ["plain", "copied"])
+def test_traced_module_follows_its_inputs(requires_grad, layout):
+    print(f"[case] trace {requires_grad} {layout}", flush=True)
+
+    def f(q, k, v, c):
+        if layout == "copied":
+            q, c = q.transpose(3, 4).contiguous().transpose(3, 4), c.double()
+        return call(q, k, v, c) * 2.0
+    first, second = inputs(0), inputs(1)
+    for args in (first, second):
+        args[0].requires_grad_(requires_grad)
+    traced = torch.jit.trace(f, tuple(first))
+    for _ in range(3):                                   # (the executor specialises on the first runs)
+        got, want = traced(*second), f(*second)
+        assert torch.equal(got, want)
+        if requires_grad:
+            dout = torch.ones_like(want)
+            assert torch.equal(*(torch.autograd.grad(o, second[0], dout)[0] for o in (got, want)))
