@@ -20,6 +20,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -181,13 +182,15 @@ struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
 // Whether the call has to be an autograd.Function's: an input carries a forward-mode tangent, or a torch.func transform
 // is active. The kernels read the values alone, and neither shows in requires_grad: from here the tangent would be
 // dropped without a word. The Function has no rule for them and raises. Under torch.jit.trace the Function is recorded
-// as a node; a call from here would be invisible, and its output a constant of the traced module.
+// as a node; a call from here would be invisible, and its output a constant of the traced module. And under a dispatch
+// mode, or with tensors that are a subclass's, the general route makes its buffers where these see them (fake tensors
+// among them, which the kernels cannot read: refused there).
 bool followed(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &coords)
 {
-    if (torch::jit::tracer::isTracing()) return true;
+    if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set()) return true;
     if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) return true;
     for (const Tensor *t : {&q, &k, &v, &coords})
-        if (t->_fw_grad(/*level=*/0).defined()) return true;
+        if (t->_fw_grad(/*level=*/0).defined() || t->unsafeGetTensorImpl()->is_python_dispatch()) return true;
     return false;
 }
 

@@ -19,7 +19,7 @@ Contract mirrored from ``_fused_deform_sdpa`` (``ops/triton.py:377-466``):
 An ordinary call -- checks, allocations, the autograd node -- is native (``csrc/dsdpa_torch.cpp``). Every other call
 takes the ``torch.autograd.Function`` below, the general route: the errors, and the callers that PyTorch follows or
 refuses by way of that class (``torch.jit.trace``, which records it; forward-mode AD and the ``torch.func``
-transforms, for which the operator has no rule).
+transforms, for which the operator has no rule; dispatch modes and tensor subclasses).
 
 Differences, all on purpose: coords are not cloned or pre-scaled (the kernels
 un-normalise), ``out``/``dq`` are not zero-filled first, no scaled copy of K is

@@ -63,3 +63,23 @@ def test_traced_module_follows_its_inputs(requires_grad, layout):
         if requires_grad:
             dout = torch.ones_like(want)
             assert torch.equal(*(torch.autograd.grad(o, second[0], dout)[0] for o in (got, want)))
+
+
+def test_dispatch_mode_sees_the_buffers():
+    print("[case] dispatch mode", flush=True)
+    from torch._subclasses import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        n = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.n += 1
+            return func(*args, **(kwargs or {}))
+    args = inputs()
+    want = call(*args)
+    with Seen() as seen:
+        assert torch.equal(call(*args), want)
+    assert seen.n > 0
+    with FakeTensorMode(allow_non_fake_inputs=True), pytest.raises(RuntimeError):
+        call(*args)
