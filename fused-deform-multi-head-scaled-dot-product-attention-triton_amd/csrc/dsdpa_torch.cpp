@@ -8,10 +8,11 @@
 // took 165 us of host time whatever its size (views x samples 2x2 of the sweep, 18x18, 32 heads: 162 us a step for
 // 86 us of kernels).
 //
+// bind(check) -> apply: check(code) is the Python function that raises for a library error code.
 // apply(single_stream, q, k, v, coords, WIDTH, HEIGHT, sm_scale[, coords_grad]) -> out; None when the arguments
 // are wrong, or when PyTorch follows the call in a way that goes by an autograd.Function (followed()): nothing has been
-// done then, and the call takes the general route, which raises or is followed; a number when the library refused the call (its error code). No tensor is kept from one
-// call for the next.
+// done then, and the call takes the general route, which raises or is followed. No tensor is kept from one call for
+// the next.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -21,6 +22,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -74,9 +76,17 @@ void *stream_of(const at::Device &dev)
     return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream();
 }
 
-void check(int rc)
+// Raises the library's error in Python, by the bound check(), on the thread whose HIP error it reports. With the lock
+// held; a C++ exception that carries the Python one, as autograd expects it from a node.
+[[noreturn]] void raise_error(PyObject *check, int rc)
 {
-    TORCH_CHECK(rc == DSDPA_OK, "libdsdpa error ", rc, ": ", dsdpa_error_string(rc), " (hip error ", dsdpa_last_hip_error(), ")");
+    if (PyObject *r = PyObject_CallFunction(check, "i", rc)) {
+        Py_DECREF(r);
+        PyErr_Format(PyExc_SystemError, "no exception for libdsdpa error %d", rc);
+    }
+    python_error err;
+    err.persist();
+    throw std::move(err);
 }
 
 int dtype_code(at::ScalarType t)
@@ -84,13 +94,19 @@ int dtype_code(at::ScalarType t)
     return t == at::kFloat ? DSDPA_F32 : t == at::kBFloat16 ? DSDPA_BF16 : DSDPA_F16;
 }
 
-struct Refused { int code; };            // the forward's error code on its way out of autograd
-
 struct Call {
     int64_t W, H;
     double scale;
     bool coords_grad, single_stream;
+    PyObject *check;                     // kept for the process's lifetime by bind()
 };
+
+void check(int rc, PyObject *checker)
+{
+    if (rc == DSDPA_OK) return;
+    pybind11::gil_scoped_acquire gil;
+    raise_error(checker, rc);
+}
 
 // out and the log-sum-exp of every query row
 std::pair<Tensor, Tensor> forward(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &coords, const Call &c)
@@ -119,7 +135,7 @@ std::pair<Tensor, Tensor> forward(const Tensor &q, const Tensor &k, const Tensor
     else
         rc = (code == DSDPA_BF16 ? dsdpa_fwd_bf16 : dsdpa_fwd_f16)(q.data_ptr(), k.data_ptr(), v.data_ptr(), cp, out.data_ptr(), lp, wsp, B, V,
                                                                    H, Hi, W, D, P, (float)c.scale, st.ptr(), s);
-    if (rc != DSDPA_OK) throw Refused{rc};
+    check(rc, c.check);
     return {out, lse};
 }
 
@@ -131,6 +147,7 @@ struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
         ctx->saved_data["W"] = c.W;
         ctx->saved_data["H"] = c.H;
         ctx->saved_data["scale"] = c.scale;
+        ctx->saved_data["check"] = (int64_t)(intptr_t)c.check;
         ctx->saved_data["flags"] = (int64_t)((c.coords_grad ? DSDPA_FLAG_COORDS_GRAD : 0) | (c.single_stream ? DSDPA_FLAG_SINGLE_STREAM : 0));
         return out;
     }
@@ -174,7 +191,7 @@ struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
             rc = (code == DSDPA_BF16 ? dsdpa_bwd_bf16 : dsdpa_bwd_f16)(q.data_ptr(), k.data_ptr(), v.data_ptr(), cp, out.data_ptr(), lp,
                                                                        dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dcp,
                                                                        ws.data_ptr(), B, V, H, Hi, W, D, P, scale, st.ptr(), flags, s);
-        check(rc);
+        check(rc, (PyObject *)(intptr_t)ctx->saved_data["check"].toInt());
         return {dq, dk, dv, dcoords, Tensor()};
     }
 };
@@ -210,7 +227,7 @@ bool acceptable(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor 
     return q.is_cuda() && k.device() == q.device() && v.device() == q.device() && coords.device() == q.device();
 }
 
-PyObject *apply(PyObject *, PyObject *const *args, Py_ssize_t n)
+PyObject *apply(PyObject *check, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
     if (n != 8 && n != 9) Py_RETURN_NONE;
@@ -234,8 +251,9 @@ PyObject *apply(PyObject *, PyObject *const *args, Py_ssize_t n)
     }
     c.coords_grad = cg == 1;
     c.single_stream = ss == 1;
+    c.check = check;
     Tensor out;
-    try {
+    {
         pybind11::gil_scoped_release no_gil;
         if (acceptable(q, k, v, coords, c)) {
             Strides st;
@@ -245,16 +263,23 @@ PyObject *apply(PyObject *, PyObject *const *args, Py_ssize_t n)
                                (q.requires_grad() || k.requires_grad() || v.requires_grad() || coords.requires_grad());
             out = graph ? DeformSdpa::apply(q, k, v, coords, c) : forward(q, k, v, coords, c).first;
         }
-    } catch (const Refused &r) {
-        return PyLong_FromLong(r.code);
     }
     if (!out.defined()) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
 
+PyMethodDef apply_method = {"apply", (PyCFunction)(void (*)(void))apply, METH_FASTCALL,
+                            "one call of the operator; None when it has to take the general route"};
+
+PyObject *bind(PyObject *, PyObject *check)
+{
+    Py_INCREF(check);                    // never given back: a graph may outlive the bound function
+    return PyCFunction_New(&apply_method, check);
+}
+
 PyMethodDef methods[] = {
-    {"apply", (PyCFunction)(void (*)(void))apply, METH_FASTCALL, "one call of the operator; None when it has to take the general route"},
+    {"bind", bind, METH_O, "the operator, raising library errors through the given function"},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_dsdpa_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -158,10 +158,6 @@ def deform_sdpa_triton(*args):
     (``ops/torch.py:14-15``)."""
     global _apply
     if _apply is None:
-        _apply = _native.load_torch().apply
+        _apply = _native.load_torch().bind(_native.check)
     out = _apply(SINGLE_STREAM, *args)
-    if out is None:
-        return _fused_deform_sdpa.apply(*args)
-    if isinstance(out, int):
-        _native.check(out)
-    return out
+    return _fused_deform_sdpa.apply(*args) if out is None else out

@@ -4,6 +4,7 @@ import pytest
 import torch
 from torch.autograd import forward_ad
 
+from ops import _native
 from ops import triton as op
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +84,15 @@ def test_dispatch_mode_sees_the_buffers():
     assert seen.n > 0
     with FakeTensorMode(allow_non_fake_inputs=True), pytest.raises(RuntimeError):
         call(*args)
+
+
+@pytest.mark.parametrize("route", ["native", "general"])
+def test_backward_raises_the_librarys_error(route):
+    print(f"[case] backward error {route}", flush=True)
+    args = inputs()
+    args[0].requires_grad_(True)
+    # saved tensors come back with a head dimension that the library refuses
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t[..., :8].contiguous() if t.shape[-1] == D else t):
+        out = call(*args) if route == "native" else op._fused_deform_sdpa.apply(*args, WIMG, HIMG, 0.3)
+    with pytest.raises(_native.DsdpaError, match="head dim"):
+        out.backward(torch.ones_like(out))
