@@ -8,8 +8,9 @@
 // took 165 us of host time whatever its size (views x samples 2x2 of the sweep, 18x18, 32 heads: 162 us a step for
 // 86 us of kernels).
 //
-// bind(check) -> apply: check(code) is the Python function that raises for a library error code.
-// apply(single_stream, q, k, v, coords, WIDTH, HEIGHT, sm_scale[, coords_grad]) -> out; None when the arguments
+// bind(check, globals) -> apply: check(code) is the Python function that raises for a library error code, globals the
+// Python module's, whose SINGLE_STREAM every backward reads when it runs.
+// apply(q, k, v, coords, WIDTH, HEIGHT, sm_scale[, coords_grad]) -> out; None when the arguments
 // are wrong, or when PyTorch follows the call in a way that goes by an autograd.Function (followed()): nothing has been
 // done then, and the call takes the general route, which raises or is followed. No tensor is kept from one call for
 // the next.
@@ -76,6 +77,25 @@ void *stream_of(const at::Device &dev)
     return (void *)c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream();
 }
 
+// What bind() was given, as a tuple kept for the process's lifetime (a graph may outlive the bound function).
+PyObject *check_of(PyObject *bound) { return PyTuple_GET_ITEM(bound, 0); }
+
+// SINGLE_STREAM now
+bool single_stream(PyObject *bound)
+{
+    pybind11::gil_scoped_acquire gil;
+    PyObject *flag = PyDict_GetItemString(PyTuple_GET_ITEM(bound, 1), "SINGLE_STREAM");
+    Py_XINCREF(flag);
+    const int on = flag ? PyObject_IsTrue(flag) : 0;
+    Py_XDECREF(flag);
+    if (on < 0) {
+        python_error err;
+        err.persist();
+        throw std::move(err);
+    }
+    return on == 1;
+}
+
 // Raises the library's error in Python, by the bound check(), on the thread whose HIP error it reports. With the lock
 // held; a C++ exception that carries the Python one, as autograd expects it from a node.
 [[noreturn]] void raise_error(PyObject *check, int rc)
@@ -97,15 +117,15 @@ int dtype_code(at::ScalarType t)
 struct Call {
     int64_t W, H;
     double scale;
-    bool coords_grad, single_stream;
-    PyObject *check;                     // kept for the process's lifetime by bind()
+    bool coords_grad;
+    PyObject *bound;
 };
 
-void check(int rc, PyObject *checker)
+void check(int rc, PyObject *bound)
 {
     if (rc == DSDPA_OK) return;
     pybind11::gil_scoped_acquire gil;
-    raise_error(checker, rc);
+    raise_error(check_of(bound), rc);
 }
 
 // out and the log-sum-exp of every query row
@@ -135,7 +155,7 @@ std::pair<Tensor, Tensor> forward(const Tensor &q, const Tensor &k, const Tensor
     else
         rc = (code == DSDPA_BF16 ? dsdpa_fwd_bf16 : dsdpa_fwd_f16)(q.data_ptr(), k.data_ptr(), v.data_ptr(), cp, out.data_ptr(), lp, wsp, B, V,
                                                                    H, Hi, W, D, P, (float)c.scale, st.ptr(), s);
-    check(rc, c.check);
+    check(rc, c.bound);
     return {out, lse};
 }
 
@@ -147,8 +167,8 @@ struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
         ctx->saved_data["W"] = c.W;
         ctx->saved_data["H"] = c.H;
         ctx->saved_data["scale"] = c.scale;
-        ctx->saved_data["check"] = (int64_t)(intptr_t)c.check;
-        ctx->saved_data["flags"] = (int64_t)((c.coords_grad ? DSDPA_FLAG_COORDS_GRAD : 0) | (c.single_stream ? DSDPA_FLAG_SINGLE_STREAM : 0));
+        ctx->saved_data["bound"] = (int64_t)(intptr_t)c.bound;
+        ctx->saved_data["coords_grad"] = c.coords_grad;
         return out;
     }
 
@@ -162,9 +182,9 @@ struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
         if (!dout.defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
         if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
         dout = dout.contiguous();
-        unsigned flags = (unsigned)ctx->saved_data["flags"].toInt();
-        const bool want_dcoords = (flags & DSDPA_FLAG_COORDS_GRAD) != 0 && ctx->needs_input_grad(3);
-        flags &= DSDPA_FLAG_SINGLE_STREAM;
+        PyObject *bound = (PyObject *)(intptr_t)ctx->saved_data["bound"].toInt();
+        const bool want_dcoords = ctx->saved_data["coords_grad"].toBool() && ctx->needs_input_grad(3);
+        unsigned flags = single_stream(bound) ? DSDPA_FLAG_SINGLE_STREAM : 0;
         if (at::globalContext().deterministicAlgorithms()) {       // the bitwise reproducible backward
             TORCH_CHECK(!want_dcoords, "deform_sdpa_triton: the coordinate gradient has no deterministic implementation "
                                        "(it sums over heads with float atomics); turn one of the two off");
@@ -191,7 +211,7 @@ struct DeformSdpa : public torch::autograd::Function<DeformSdpa> {
             rc = (code == DSDPA_BF16 ? dsdpa_bwd_bf16 : dsdpa_bwd_f16)(q.data_ptr(), k.data_ptr(), v.data_ptr(), cp, out.data_ptr(), lp,
                                                                        dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dcp,
                                                                        ws.data_ptr(), B, V, H, Hi, W, D, P, scale, st.ptr(), flags, s);
-        check(rc, (PyObject *)(intptr_t)ctx->saved_data["check"].toInt());
+        check(rc, bound);
         return {dq, dk, dv, dcoords, Tensor()};
     }
 };
@@ -227,31 +247,30 @@ bool acceptable(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor 
     return q.is_cuda() && k.device() == q.device() && v.device() == q.device() && coords.device() == q.device();
 }
 
-PyObject *apply(PyObject *check, PyObject *const *args, Py_ssize_t n)
+PyObject *apply(PyObject *bound, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    if (n != 8 && n != 9) Py_RETURN_NONE;
-    for (int i = 1; i <= 4; ++i)
+    if (n != 7 && n != 8) Py_RETURN_NONE;
+    for (int i = 0; i < 4; ++i)
         if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
-    Tensor q = THPVariable_Unpack(args[1]), k = THPVariable_Unpack(args[2]), v = THPVariable_Unpack(args[3]),
-           coords = THPVariable_Unpack(args[4]);
+    Tensor q = THPVariable_Unpack(args[0]), k = THPVariable_Unpack(args[1]), v = THPVariable_Unpack(args[2]),
+           coords = THPVariable_Unpack(args[3]);
     if (followed(q, k, v, coords)) Py_RETURN_NONE;
     Call c;
-    c.W = PyNumber_AsSsize_t(args[5], PyExc_OverflowError);
-    c.H = PyErr_Occurred() ? 0 : PyNumber_AsSsize_t(args[6], PyExc_OverflowError);
-    PyObject *scale = PyErr_Occurred() ? nullptr : PyNumber_Float(args[7]);
-    const int cg = scale && n == 9 ? PyObject_IsTrue(args[8]) : 0, ss = scale ? PyObject_IsTrue(args[0]) : 0;
+    c.bound = bound;
+    c.W = PyNumber_AsSsize_t(args[4], PyExc_OverflowError);
+    c.H = PyErr_Occurred() ? 0 : PyNumber_AsSsize_t(args[5], PyExc_OverflowError);
+    PyObject *scale = PyErr_Occurred() ? nullptr : PyNumber_Float(args[6]);
+    const int cg = scale && n == 8 ? PyObject_IsTrue(args[7]) : 0;
     if (scale) {
         c.scale = PyFloat_AS_DOUBLE(scale);
         Py_DECREF(scale);
     }
-    if (!scale || cg < 0 || ss < 0) {
+    if (!scale || cg < 0) {
         PyErr_Clear();
         Py_RETURN_NONE;
     }
     c.coords_grad = cg == 1;
-    c.single_stream = ss == 1;
-    c.check = check;
     Tensor out;
     {
         pybind11::gil_scoped_release no_gil;
@@ -272,14 +291,16 @@ PyObject *apply(PyObject *check, PyObject *const *args, Py_ssize_t n)
 PyMethodDef apply_method = {"apply", (PyCFunction)(void (*)(void))apply, METH_FASTCALL,
                             "one call of the operator; None when it has to take the general route"};
 
-PyObject *bind(PyObject *, PyObject *check)
+PyObject *bind(PyObject *, PyObject *args)
 {
-    Py_INCREF(check);                    // never given back: a graph may outlive the bound function
-    return PyCFunction_New(&apply_method, check);
+    PyObject *check, *globals;
+    if (!PyArg_ParseTuple(args, "OO!", &check, &PyDict_Type, &globals)) return nullptr;
+    Py_INCREF(args);                     // never given back, see check_of()
+    return PyCFunction_New(&apply_method, args);
 }
 
 PyMethodDef methods[] = {
-    {"bind", bind, METH_O, "the operator, raising library errors through the given function"},
+    {"bind", bind, METH_VARARGS, "the operator for a module: bind(check, globals) -> apply"},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_dsdpa_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -40,7 +40,8 @@ _DTYPE_CODE = {torch.float32: _native.DSDPA_F32, torch.bfloat16: _native.DSDPA_B
                torch.float16: _native.DSDPA_F16}
 
 # The backward runs its dk/dv side beside the dq side on a second stream of the library's (forked from and joined
-# to the caller's stream inside the call). True keeps every launch on the caller's stream (same results).
+# to the caller's stream inside the call). True keeps every launch on the caller's stream (same results);
+# read when a backward runs.
 SINGLE_STREAM = False
 
 _apply = None
@@ -158,6 +159,6 @@ def deform_sdpa_triton(*args):
     (``ops/torch.py:14-15``)."""
     global _apply
     if _apply is None:
-        _apply = _native.load_torch().bind(_native.check)
-    out = _apply(SINGLE_STREAM, *args)
+        _apply = _native.load_torch().bind(_native.check, globals())
+    out = _apply(*args)
     return _fused_deform_sdpa.apply(*args) if out is None else out

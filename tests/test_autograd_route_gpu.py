@@ -96,3 +96,21 @@ def test_backward_raises_the_librarys_error(route):
         out = call(*args) if route == "native" else op._fused_deform_sdpa.apply(*args, WIMG, HIMG, 0.3)
     with pytest.raises(_native.DsdpaError, match="head dim"):
         out.backward(torch.ones_like(out))
+
+
+@pytest.mark.parametrize("route", ["native", "general"])
+def test_single_stream_is_read_when_the_backward_runs(route, monkeypatch):
+    print(f"[case] single stream {route}", flush=True)
+    args = inputs()
+    args[0].requires_grad_(True)
+    out = call(*args) if route == "native" else op._fused_deform_sdpa.apply(*args, WIMG, HIMG, 0.3)
+
+    class Asked:
+        times = 0
+
+        def __bool__(self):
+            self.times += 1
+            return True
+    monkeypatch.setattr(op, "SINGLE_STREAM", Asked())
+    out.backward(torch.ones_like(out))
+    assert op.SINGLE_STREAM.times == 1
