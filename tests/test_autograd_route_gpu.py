@@ -114,3 +114,16 @@ def test_single_stream_is_read_when_the_backward_runs(route, monkeypatch):
     monkeypatch.setattr(op, "SINGLE_STREAM", Asked())
     out.backward(torch.ones_like(out))
     assert op.SINGLE_STREAM.times == 1
+
+
+@pytest.mark.parametrize("route", ["native", "general"])
+def test_profile_carries_the_operators_name(route):
+    print(f"[case] profile {route}", flush=True)
+    args = inputs()
+    args[0].requires_grad_(True)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        out = call(*args) if route == "native" else op._fused_deform_sdpa.apply(*args, WIMG, HIMG, 0.3)
+        out.backward(torch.ones_like(out))
+    names = {e.key for e in prof.key_averages()}
+    assert {"_fused_deform_sdpa", "_fused_deform_sdpaBackward"} <= names
+    assert "fused_deform_sdpa" in out.grad_fn.name() and "fused_deform_sdpa" in repr(out)
