@@ -43,16 +43,26 @@ struct Strides {
     const long long *ptr() const { return given ? st : nullptr; }
 };
 
+bool aligned(const Tensor &t, uintptr_t bytes) { return ((uintptr_t)t.data_ptr() & (bytes - 1)) == 0; }
+
+// Contiguous, and at an address that the kernels' vector loads take (a contiguous view may begin at any element).
+Tensor packed(const Tensor &t, uintptr_t bytes = 16)
+{
+    Tensor c = t.contiguous();
+    return aligned(c, bytes) ? c : c.clone(at::MemoryFormat::Contiguous);
+}
+
 // Whether the kernels can read q, k, v where they lie: head dimension contiguous, k and v laid out alike, rows
 // 16-byte aligned, the views and pixels of one (batch, head) within 2^30 elements (the kernels address them in 32
 // bits). Fills the `strides` argument of the entry points.
 bool readable_in_place(const Tensor &q, const Tensor &k, const Tensor &v, Strides *out)
 {
+    if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16)) return false;
     if (q.is_contiguous() && k.is_contiguous() && v.is_contiguous()) return true;
     const int64_t align = 16 / (int64_t)q.element_size(), V = q.size(1), L = q.size(3), D = q.size(4);
     for (const Tensor *t : {&q, &k, &v}) {
         const auto st = t->strides();
-        if (st[4] != 1 || ((uintptr_t)t->data_ptr() & 15) || st[3] < D) return false;
+        if (st[4] != 1 || st[3] < D) return false;
         for (int i = 0; i < 4; ++i)
             if (st[i] < 0 || st[i] % align) return false;
         if ((V - 1) * st[1] + (L - 1) * st[3] + D > (1ll << 30) || st[1] > (1ll << 30)) return false;
@@ -188,7 +198,7 @@ struct fused_deform_sdpa : public torch::autograd::Function<fused_deform_sdpa> {
         Tensor dout = grads[0];
         if (!dout.defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
         if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
-        dout = dout.contiguous();
+        dout = packed(dout);
         PyObject *bound = (PyObject *)(intptr_t)ctx->saved_data["bound"].toInt();
         const bool want_dcoords = ctx->saved_data["coords_grad"].toBool() && ctx->needs_input_grad(3);
         unsigned flags = single_stream(bound) ? DSDPA_FLAG_SINGLE_STREAM : 0;
@@ -285,8 +295,9 @@ PyObject *apply(PyObject *bound, PyObject *const *args, Py_ssize_t n)
         pybind11::gil_scoped_release no_gil;
         if (acceptable(q, k, v, coords, c)) {
             Strides st;
-            if (!readable_in_place(q, k, v, &st)) q = q.contiguous(), k = k.contiguous(), v = v.contiguous();
+            if (!readable_in_place(q, k, v, &st)) q = packed(q), k = packed(k), v = packed(v);
             if (coords.scalar_type() != at::kFloat) coords = coords.to(at::kFloat);
+            coords = packed(coords, 8);                  // (read as pairs)
             const bool graph = at::GradMode::is_enabled() &&
                                (q.requires_grad() || k.requires_grad() || v.requires_grad() || coords.requires_grad());
             out = graph ? fused_deform_sdpa::apply(q, k, v, coords, c) : forward_pass(q, k, v, coords, c).first;

@@ -68,6 +68,12 @@ def _check_inputs(q, k, v, coords, WIDTH, HEIGHT):
         raise RuntimeError("q, k, v, coords must be on one device")
 
 
+def _packed(t, align=16):
+    """Contiguous, and at an address that the kernels' vector loads take (a contiguous view may begin at any element)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % align == 0 else t.clone(memory_format=torch.contiguous_format)
+
+
 @contextlib.contextmanager
 def _not_traced():
     """Inside, sizes are plain ints also while ``torch.jit.trace`` records the caller. (It records the Function as a
@@ -99,10 +105,11 @@ class _fused_deform_sdpa(torch.autograd.Function):
             # ops/triton.py:396-405): head dimension contiguous, rows 16-byte aligned, k and v laid out alike
             strides = _native.strides_arg(q, k, v)
         if strides is False:
-            q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+            q, k, v = _packed(q), _packed(k), _packed(v)
             strides = None
         if coords.dtype != torch.float32:
             coords = coords.float()
+        coords = _packed(coords, 8)                                         # (read as pairs)
         out = torch.empty((B, V, H, L, D), device=q.device, dtype=q.dtype)  # contiguous whatever q's layout
         lse = torch.empty((B, V, H, L), device=q.device, dtype=torch.float32)
         ws_bytes = lib.dsdpa_fwd_workspace_bytes(_DTYPE_CODE[q.dtype], B, V, H, HEIGHT, WIDTH, D, P)
@@ -124,9 +131,7 @@ class _fused_deform_sdpa(torch.autograd.Function):
         lib = _native.load()
         B, V, H, L, D = q.shape
         P = coords.shape[-2]
-        do = do.contiguous()
-        if do.dtype != q.dtype:
-            do = do.to(q.dtype)
+        do = _packed(do if do.dtype == q.dtype else do.to(q.dtype))
         dq, dk, dv = (torch.empty(q.shape, device=q.device, dtype=q.dtype) for _ in range(3))
         strides = _native.strides_arg(q, k, v)          # (what forward saved: contiguous, or readable in place)
         dcoords = torch.empty_like(coords) if ctx.coords_grad and ctx.needs_input_grad[3] else None

@@ -172,3 +172,13 @@ def test_operator_contract_errors_on_cpu():
         deform_sdpa_triton(q, q, q, c.transpose(3, 4).contiguous().transpose(3, 4), 4, 3, 0.5)
     with pytest.raises(RuntimeError):
         deform_sdpa_triton(q, q, q, c, 4, 3, 0.5)                      # CPU tensors: no fallback
+
+
+def test_contiguous_tensors_at_an_odd_address_are_copied():
+    import torch
+    a = torch.empty(1, 2, 2, 12, 32, dtype=torch.bfloat16)
+    odd = torch.empty(a.numel() + 1, dtype=a.dtype)[1:].view(a.shape)
+    assert a.data_ptr() % 16 == 0 and odd.is_contiguous()
+    assert _native.strides_arg(a, a, a) is None
+    for qkv in ((odd, a, a), (a, odd, a), (a, a, odd)):
+        assert _native.strides_arg(*qkv) is False

@@ -127,3 +127,26 @@ def test_profile_carries_the_operators_name(route):
     names = {e.key for e in prof.key_averages()}
     assert {"_fused_deform_sdpa", "_fused_deform_sdpaBackward"} <= names
     assert "fused_deform_sdpa" in out.grad_fn.name() and "fused_deform_sdpa" in repr(out)
+
+
+@pytest.mark.parametrize("route", ["native", "general"])
+@pytest.mark.parametrize("which", range(5))
+def test_views_at_an_odd_address_are_copied(route, which):
+    print(f"[case] odd address {route} {which}", flush=True)
+    args = inputs(dtype=torch.bfloat16) + inputs(1, torch.bfloat16)[:1]
+
+    def odd(t):                                          # contiguous, one element after an aligned address
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
+
+    def step(q, k, v, c, dout):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v, c)]
+        f = op.deform_sdpa_triton if route == "native" else op._fused_deform_sdpa.apply
+        out = f(*leaves, WIMG, HIMG, 0.3, True)
+        out.backward(dout)
+        return [out.detach()] + [t.grad for t in leaves]
+    want = step(*args)
+    args[which] = odd(args[which])
+    got = step(*args)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    for a, b in zip(got[2:], want[2:]):      # float atomics: sums in another order, one step of bf16 (2^-8) at most
+        assert (a.float() - b.float()).abs().max() <= 2.0 ** -7 * b.float().abs().max()
