@@ -171,6 +171,27 @@ std::pair<Tensor, Tensor> forward_pass(const Tensor &q, const Tensor &k, const T
     return {out, lse};
 }
 
+// Saved-tensor hooks may bring back other tensors than were saved: q, k, v, coords, out and lse as the kernels read them.
+// What does not fit dout's shape and device is refused here: the kernels would read beyond it.
+void usable(variable_list &saved, const Tensor &dout, PyObject *bound)
+{
+    Tensor &q = saved[0], &k = saved[1], &v = saved[2], &coords = saved[3], &out = saved[4], &lse = saved[5];
+    const int64_t D = q.dim() == 5 ? q.size(4) : 0;
+    if (!(D == 16 || D == 32 || D == 64 || D == 128 || D == 256)) check(DSDPA_ERR_HEAD_DIM, bound);
+    bool fits = q.sizes() == dout.sizes() && lse.sizes() == q.sizes().slice(0, 4) && lse.scalar_type() == at::kFloat;
+    for (const Tensor *t : {&k, &v, &out}) fits &= t->sizes() == q.sizes() && t->scalar_type() == q.scalar_type();
+    for (const Tensor &t : saved) fits &= t.device() == dout.device();
+    fits &= coords.dim() == 6 && coords.size(0) == q.size(0) && coords.size(1) == q.size(1) && coords.size(2) == q.size(3) &&
+            coords.size(3) == q.size(1) && coords.size(4) >= 1 && coords.size(5) == 2 && coords.scalar_type() == at::kFloat;
+    fits &= q.scalar_type() == at::kFloat || q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf;
+    TORCH_CHECK(fits, "deform_sdpa_triton: a tensor saved for the backward came back with another shape, type or device");
+    Strides st;
+    if (!readable_in_place(q, k, v, &st)) q = packed(q), k = packed(k), v = packed(v);
+    coords = packed(coords, 8);
+    out = packed(out);
+    lse = packed(lse);
+}
+
 }  // namespace
 
 // The autograd node. Outside the namespace for a plain name in graphs (torch::autograd::CppNode<fused_deform_sdpa>); the
@@ -191,15 +212,16 @@ struct fused_deform_sdpa : public torch::autograd::Function<fused_deform_sdpa> {
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
         RECORD_FUNCTION("_fused_deform_sdpaBackward", std::vector<c10::IValue>());
-        const variable_list saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &coords = saved[3], &out = saved[4], &lse = saved[5];
-        const at::Device dev = q.device();
-        const c10::DeviceGuard on_device(dev);
         Tensor dout = grads[0];
         if (!dout.defined()) return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        const at::Device dev = dout.device();
+        const c10::DeviceGuard on_device(dev);
+        PyObject *bound = (PyObject *)(intptr_t)ctx->saved_data["bound"].toInt();
+        variable_list saved = ctx->get_saved_variables();
+        usable(saved, dout, bound);
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &coords = saved[3], &out = saved[4], &lse = saved[5];
         if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
         dout = packed(dout);
-        PyObject *bound = (PyObject *)(intptr_t)ctx->saved_data["bound"].toInt();
         const bool want_dcoords = ctx->saved_data["coords_grad"].toBool() && ctx->needs_input_grad(3);
         unsigned flags = single_stream(bound) ? DSDPA_FLAG_SINGLE_STREAM : 0;
         if (at::globalContext().deterministicAlgorithms()) {       // the bitwise reproducible backward
@@ -212,7 +234,7 @@ struct fused_deform_sdpa : public torch::autograd::Function<fused_deform_sdpa> {
         const int W = (int)ctx->saved_data["W"].toInt(), Hi = (int)ctx->saved_data["H"].toInt(), code = dtype_code(q.scalar_type());
         const float scale = (float)ctx->saved_data["scale"].toDouble();
         Strides st;
-        TORCH_CHECK(readable_in_place(q, k, v, &st));
+        readable_in_place(q, k, v, &st);
         Tensor dq = fresh(q.sizes(), q.scalar_type(), dev), dk = fresh(q.sizes(), q.scalar_type(), dev), dv = fresh(q.sizes(), q.scalar_type(), dev);
         Tensor dcoords = want_dcoords ? fresh(coords.sizes(), at::kFloat, dev) : Tensor();
         Tensor ws = fresh({(int64_t)dsdpa_bwd_workspace_bytes(code, B, V, H, Hi, W, D, P, flags)}, at::kByte, dev);

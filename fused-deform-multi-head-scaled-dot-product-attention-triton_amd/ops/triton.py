@@ -74,6 +74,19 @@ def _packed(t, align=16):
     return t if t.data_ptr() % align == 0 else t.clone(memory_format=torch.contiguous_format)
 
 
+def _check_saved(q, k, v, coords, out, lse, do):
+    """Saved-tensor hooks may bring back other tensors than were saved. What does not fit the gradient's shape and device
+    is refused: the kernels would read beyond it."""
+    if q.dim() != 5 or q.shape[4] not in {16, 32, 64, 128, 256}:
+        _native.check(_native.ERR_HEAD_DIM)
+    B, V, H, L, D = q.shape
+    if not (all(t.shape == do.shape and t.dtype == q.dtype for t in (q, k, v, out)) and q.dtype in _SUFFIX
+            and lse.shape == (B, V, H, L) and coords.dim() == 6 and coords.shape[:4] == (B, V, L, V)
+            and coords.shape[4] >= 1 and coords.shape[5] == 2 and lse.dtype == coords.dtype == torch.float32
+            and all(t.device == do.device for t in (q, k, v, coords, out, lse))):
+        raise RuntimeError("deform_sdpa_triton: a tensor saved for the backward came back with another shape, type or device")
+
+
 @contextlib.contextmanager
 def _not_traced():
     """Inside, sizes are plain ints also while ``torch.jit.trace`` records the caller. (It records the Function as a
@@ -129,11 +142,17 @@ class _fused_deform_sdpa(torch.autograd.Function):
     def backward(ctx, do):
         q, k, v, coords, out, lse = ctx.saved_tensors
         lib = _native.load()
-        B, V, H, L, D = q.shape
-        P = coords.shape[-2]
+        with _not_traced():
+            _check_saved(q, k, v, coords, out, lse, do)
+            B, V, H, L, D = q.shape
+            P = coords.shape[-2]
+            strides = _native.strides_arg(q, k, v)
         do = _packed(do if do.dtype == q.dtype else do.to(q.dtype))
-        dq, dk, dv = (torch.empty(q.shape, device=q.device, dtype=q.dtype) for _ in range(3))
-        strides = _native.strides_arg(q, k, v)          # (what forward saved: contiguous, or readable in place)
+        dq, dk, dv = (torch.empty((B, V, H, L, D), device=q.device, dtype=q.dtype) for _ in range(3))
+        if strides is False:                            # (from a hook: forward saves contiguous, or readable in place)
+            q, k, v = _packed(q), _packed(k), _packed(v)
+            strides = None
+        coords, out, lse = _packed(coords, 8), _packed(out), _packed(lse)
         dcoords = torch.empty_like(coords) if ctx.coords_grad and ctx.needs_input_grad[3] else None
         # torch.use_deterministic_algorithms(True) selects the bitwise reproducible backward
         flags = _native.FLAG_DETERMINISTIC if torch.are_deterministic_algorithms_enabled() else 0

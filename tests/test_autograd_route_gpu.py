@@ -150,3 +150,22 @@ def test_views_at_an_odd_address_are_copied(route, which):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     for a, b in zip(got[2:], want[2:]):      # float atomics: sums in another order, one step of bf16 (2^-8) at most
         assert (a.float() - b.float()).abs().max() <= 2.0 ** -7 * b.float().abs().max()
+
+
+@pytest.mark.parametrize("route", ["native", "general"])
+def test_saved_tensors_from_hooks(route):
+    print(f"[case] hooks {route}", flush=True)
+    f = op.deform_sdpa_triton if route == "native" else op._fused_deform_sdpa.apply
+
+    def dq(unpack):
+        args = inputs()
+        args[0].requires_grad_(True)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            out = f(*args, WIMG, HIMG, 0.3)
+        out.backward(torch.ones_like(out))
+        return args[0].grad
+    want = dq(lambda t: t)
+    assert torch.equal(dq(lambda t: t.transpose(-1, -2).contiguous().transpose(-1, -2)), want)      # layouts are mended
+    for unpack in (torch.Tensor.cpu, torch.Tensor.double, lambda t: t[..., :1, :].contiguous()):
+        with pytest.raises(RuntimeError, match="saved for the backward"):
+            dq(unpack)
