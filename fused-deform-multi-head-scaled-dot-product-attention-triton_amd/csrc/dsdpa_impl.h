@@ -723,7 +723,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     // So do small problems: the fork and join cost about 0.05 ms of host time per call, which a backward of
     // under two million query*samples (0.15 ms of kernels) does not win back.
     hipStream_t bst = st;
-    const bool worth_forking = (long long)dm.rows * dm.N >= (2ll << 20);
+    const bool worth_forking = (long long)dm.rows * dm.N >= DSDPA_TWO_STREAMS_FROM;
     SideLane *side = cell_binned && staged && worth_forking && !(flags & DSDPA_FLAG_SINGLE_STREAM) ? side_lane() : nullptr;
     const size_t ncounters = cell_binned && !bin_in_one_launch(dm, wl) ? wl.counters_bytes / 4 : 0;
     SideJoin joiner;

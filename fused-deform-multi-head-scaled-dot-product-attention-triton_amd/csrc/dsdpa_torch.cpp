@@ -9,7 +9,7 @@
 // 86 us of kernels).
 //
 // bind(check, globals) -> apply: check(code) is the Python function that raises for a library error code, globals the
-// Python module's, whose SINGLE_STREAM every backward reads when it runs.
+// Python module's, whose SINGLE_STREAM a backward reads when it runs.
 // apply(q, k, v, coords, WIDTH, HEIGHT, sm_scale[, coords_grad]) -> out; None when the arguments
 // are wrong, or when PyTorch follows the call in a way that goes by an autograd.Function (followed()): nothing has been
 // done then, and the call takes the general route, which raises or is followed. No tensor is kept from one call for
@@ -223,7 +223,9 @@ struct fused_deform_sdpa : public torch::autograd::Function<fused_deform_sdpa> {
         if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
         dout = packed(dout);
         const bool want_dcoords = ctx->saved_data["coords_grad"].toBool() && ctx->needs_input_grad(3);
-        unsigned flags = single_stream(bound) ? DSDPA_FLAG_SINGLE_STREAM : 0;
+        // (asked only where it makes a difference: taking the interpreter's lock costs a small step 2 us)
+        const bool may_fork = lse.numel() * q.size(1) * coords.size(4) >= DSDPA_TWO_STREAMS_FROM;
+        unsigned flags = may_fork && single_stream(bound) ? DSDPA_FLAG_SINGLE_STREAM : 0;
         if (at::globalContext().deterministicAlgorithms()) {       // the bitwise reproducible backward
             TORCH_CHECK(!want_dcoords, "deform_sdpa_triton: the coordinate gradient has no deterministic implementation "
                                        "(it sums over heads with float atomics); turn one of the two off");

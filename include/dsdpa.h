@@ -123,11 +123,13 @@ int dsdpa_fwd_noalloc(int dtype, const void *q, const void *k, const void *v, co
  * stores (cells of one row/column parity share no pixel) instead of float atomics. Needs a larger
  * workspace (pass the same flags to dsdpa_bwd_workspace_bytes) and cannot be combined with dcoords. */
 enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SINGLE_STREAM = 4 };
+/* B*V*H*L * V*P from which the backward may use its second stream; below it DSDPA_FLAG_SINGLE_STREAM changes nothing */
+#define DSDPA_TWO_STREAMS_FROM (1ll << 21)
 /* DSDPA_FLAG_SINGLE_STREAM: enqueue every launch of the backward on `stream` itself. By default the dk/dv side
  * (clearing the accumulators, delta, the cell binning, the dk/dv kernel) runs on a second stream of the
  * library's beside the tap table and the dq kernel: neither side reads what the other writes, and the two
  * main kernels leave each other idle issue slots (C2: 7 % off the fwd+bwd step). Only on shapes whose K/V planes
- * fit in LDS, and only from 2^21 query*samples (B*V*H*L * V*P) up: below that the fork and join cost more host
+ * fit in LDS, and only from DSDPA_TWO_STREAMS_FROM query*samples (B*V*H*L * V*P) up: below that the fork and join cost more host
  * time than the overlap saves. Same results either way. */
 /* DSDPA_FLAG_COORDS_GRAD: the workspace has room for the coordinate gradient's part of the per-coordinate
  * table (16 more bytes per coordinate pair where the staged kernels run), so that a backward given dcoords

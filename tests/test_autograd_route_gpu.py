@@ -101,9 +101,11 @@ def test_backward_raises_the_librarys_error(route):
 @pytest.mark.parametrize("route", ["native", "general"])
 def test_single_stream_is_read_when_the_backward_runs(route, monkeypatch):
     print(f"[case] single stream {route}", flush=True)
-    args = inputs()
-    args[0].requires_grad_(True)
-    out = call(*args) if route == "native" else op._fused_deform_sdpa.apply(*args, WIMG, HIMG, 0.3)
+    n, p = 64, 8                                         # 4 * 64 * 32^2 * 8 query samples: the least that may fork
+    q, k, v = (torch.randn(4, 1, n, 32 * 32, 16, device="cuda") for _ in range(3))
+    args = [q.requires_grad_(True), k, v, torch.rand(4, 1, 32 * 32, 1, p, 2, device="cuda")]
+    f = op.deform_sdpa_triton if route == "native" else op._fused_deform_sdpa.apply
+    out = f(*args, 32, 32, 0.3)
 
     class Asked:
         times = 0
