@@ -296,6 +296,9 @@ PyObject *apply(PyObject *bound, PyObject *const *args, Py_ssize_t n)
     if (n != 7 && n != 8) Py_RETURN_NONE;
     for (int i = 0; i < 4; ++i)
         if (!THPVariable_Check(args[i])) Py_RETURN_NONE;
+    // (a scale or size in a tensor may require a gradient or carry a tangent, too: the Function knows it for an input)
+    for (Py_ssize_t i = 4; i < n; ++i)
+        if (THPVariable_Check(args[i])) Py_RETURN_NONE;
     Tensor q = THPVariable_Unpack(args[0]), k = THPVariable_Unpack(args[1]), v = THPVariable_Unpack(args[2]),
            coords = THPVariable_Unpack(args[3]);
     if (followed(q, k, v, coords)) Py_RETURN_NONE;

@@ -35,6 +35,22 @@ def test_forward_mode_is_refused(which, requires_grad, grad_mode):
             call(*args)
 
 
+@pytest.mark.parametrize("grad_mode", [False, True])
+def test_scale_in_a_tensor_is_an_input(grad_mode):
+    print(f"[case] tensor scale {grad_mode}", flush=True)
+    q, k, v, c = inputs()
+    want = call(q, k, v, c)
+    scale = torch.tensor(0.3, requires_grad=True)
+    with torch.set_grad_enabled(grad_mode):
+        out = op.deform_sdpa_triton(q, k, v, c, WIMG, HIMG, scale)
+    assert torch.equal(out, want) and out.requires_grad == grad_mode
+    if grad_mode:
+        out.backward(torch.ones_like(out))               # (as in the reference: it gets no gradient)
+        assert scale.grad is None
+    with forward_ad.dual_level(), torch.set_grad_enabled(grad_mode), pytest.raises(NotImplementedError, match="jvp"):
+        op.deform_sdpa_triton(q, k, v, c, WIMG, HIMG, forward_ad.make_dual(scale.detach(), torch.ones(())))
+
+
 def test_function_transforms_are_refused():
     print("[case] transforms", flush=True)
     q, k, v, c = inputs()
