@@ -77,9 +77,11 @@ bool readable_in_place(const Tensor &q, const Tensor &k, const Tensor &v, Stride
 }
 
 // at::detail::empty_cuda: the caching allocator without the dispatcher, and without the fill that at::empty does under
-// torch.use_deterministic_algorithms (every element of every buffer made here is written by the kernels).
+// torch.use_deterministic_algorithms (every element of every tensor handed out is written by the kernels, and nothing of a
+// workspace is read that they have not written). A dispatch mode entered around a backward alone sees the buffers.
 Tensor fresh(at::IntArrayRef shape, at::ScalarType type, const at::Device &dev)
 {
+    if (c10::impl::TorchDispatchModeTLS::any_modes_set()) return at::empty(shape, at::TensorOptions(dev).dtype(type));
     return Tensor(at::detail::empty_cuda(shape, type, dev, std::nullopt));
 }
 

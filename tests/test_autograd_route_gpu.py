@@ -103,6 +103,35 @@ def test_dispatch_mode_sees_the_buffers():
 
 
 @pytest.mark.parametrize("route", ["native", "general"])
+def test_dispatch_mode_around_the_backward_sees_its_buffers(route):
+    print(f"[case] dispatch mode backward {route}", flush=True)
+    from torch._subclasses import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Made(TorchDispatchMode):
+        n = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.n += func is torch.ops.aten.empty.memory_format
+            return func(*args, **(kwargs or {}))
+
+    def forward():
+        args = inputs()
+        args[0].requires_grad_(True)
+        f = op.deform_sdpa_triton if route == "native" else op._fused_deform_sdpa.apply
+        return args[0], f(*args, WIMG, HIMG, 0.3)
+    (q, out), (want, same) = forward(), forward()
+    dout = torch.ones_like(out)
+    same.backward(dout)
+    with Made() as made:
+        out.backward(dout)
+    assert made.n >= 4 and torch.equal(q.grad, want.grad)        # dq, dk, dv and the workspace
+    q, out = forward()
+    with FakeTensorMode(allow_non_fake_inputs=True), pytest.raises(RuntimeError):
+        out.backward(dout)
+
+
+@pytest.mark.parametrize("route", ["native", "general"])
 def test_backward_raises_the_librarys_error(route):
     print(f"[case] backward error {route}", flush=True)
     args = inputs()
