@@ -266,10 +266,13 @@ static __global__ __launch_bounds__(1024) void bin_scan_kernel(unsigned *__restr
 // launches are: 1296 samples a list group (18x18, 2 views x 2 samples) 6.4 us against 13.2 for the three and the gaps
 // between them. One workgroup's throughput then takes over: 5184 (4 x 4, six samples a thread) 13.9 against 17.4, a step
 // no faster; 11664 34.8 against 24.1, 17871 59 against 19.
-// Keys: at most kBinOneKeys, in LDS.
-constexpr int kBinOneKeys = 8192, kBinOneSamples = 2 * 1024;
+// Keys: one per cell, (Himg + 1)(Wimg + 1) <= 2 Himg Wimg + 2 of them, in LDS; the query views are one group (their rows
+// take at most 2 * 2048 * 256 * 4 bytes, below where views_per_group splits them).
+constexpr int kBinOneSamples = 2 * 1024, kBinOneKeys = 2 * kBinOneSamples + 2, kBinOneKeyBits = 13;
+static_assert(kBinOneKeys < (1 << kBinOneKeyBits), "a key fits below its rank");
+static_assert(2ull * kBinOneSamples * 256 * 4 <= kGroupRowsBytes, "one group of query views");
 template <int PER>
-__global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__ coords_, Dims dm, int NC, int NK, int vpg,
+__global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__ coords_, Dims dm, int NC,
                                                        unsigned *__restrict__ start, unsigned piece, unsigned wmax,
                                                        uint4 *__restrict__ items, unsigned *__restrict__ sorted, int records)
 {
@@ -285,33 +288,32 @@ __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__
         const unsigned ql = dm.divP.div(id), p = id - ql * (unsigned)dm.P;
         xy[i] = crd[(size_t)ql * dm.N + p];
     }
-    for (int i = threadIdx.x; i < NK; i += 1024) s_hist[i] = 0u;
+    for (int i = threadIdx.x; i < NC; i += 1024) s_hist[i] = 0u;
     __syncthreads();
-    unsigned key_rank[PER];                                        // key in 13 bits, rank above; all ones: in no list
+    unsigned key_rank[PER];                                        // key, rank above; all ones: in no list
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const unsigned id = (unsigned)i * 1024u + threadIdx.x;
         const Taps tp = make_taps(xy[i].x, xy[i].y, dm.Wimg, dm.Himg);
         key_rank[i] = 0xffffffffu;
         if (id < M && taps_any(tp)) {
-            const unsigned s1 = dm.divL.div(dm.divP.div(id));
-            const unsigned key = (s1 / (unsigned)vpg) * (unsigned)NC + (unsigned)cell_of(tp, dm.Wimg);
-            key_rank[i] = key | (atomicAdd(&s_hist[key], 1u) << 13);
+            const unsigned key = (unsigned)cell_of(tp, dm.Wimg);
+            key_rank[i] = key | (atomicAdd(&s_hist[key], 1u) << kBinOneKeyBits);
         }
     }
     __syncthreads();
     ScanCarry carry{0u, 0u};
-    unsigned *st = start + (size_t)blockIdx.x * (NK + 1);
+    unsigned *st = start + (size_t)blockIdx.x * (NC + 1);
     uint4 *it = items + (size_t)blockIdx.x * wmax;
-    for (int base = 0; base < NK; base += 1024 * kScanKeys) {
+    for (int base = 0; base < NC; base += 1024 * kScanKeys) {
         const int c0 = base + (int)threadIdx.x * kScanKeys;
         unsigned v[kScanKeys], at;
 #pragma unroll
-        for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NK ? s_hist[c0 + i] : 0u;
-        scan_keys(v, c0, NK, NC, piece, wmax, st, it, s_wave, carry, at);
+        for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NC ? s_hist[c0 + i] : 0u;
+        scan_keys(v, c0, NC, NC, piece, wmax, st, it, s_wave, carry, at);
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) {
-            if (c0 + i < NK) s_hist[c0 + i] = at;                  // (this thread's own keys)
+            if (c0 + i < NC) s_hist[c0 + i] = at;                  // (this thread's own keys)
             at += v[i];
         }
     }
@@ -319,10 +321,10 @@ __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         if (key_rank[i] != 0xffffffffu)
-            store_cell_entry(sorted, (size_t)blockIdx.x * M + s_hist[key_rank[i] & (kBinOneKeys - 1)] + (key_rank[i] >> 13),
+            store_cell_entry(sorted, (size_t)blockIdx.x * M + s_hist[key_rank[i] & ((1u << kBinOneKeyBits) - 1u)] + (key_rank[i] >> kBinOneKeyBits),
                              (unsigned)i * 1024u + threadIdx.x, cell_fraction(xy[i], dm), records);
     }
-    scan_end(carry, NK, wmax, st, it);
+    scan_end(carry, NC, wmax, st, it);
 }
 
 // Deterministic backward: begin / end of every cell list as positions in the flat id array

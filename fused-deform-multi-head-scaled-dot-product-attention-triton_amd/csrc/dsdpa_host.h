@@ -250,9 +250,10 @@ inline void work_list_geometry(size_t V, size_t L, size_t P, size_t NC, unsigned
 // use to one group's: groups of at most 4 MB (64x64, D = 128, 16-bit, V = 4: 8 MB, two groups: 2.31 -> 2.07 ms;
 // four groups 2.23 ms -- every group multiplies the items, each with its set-up and flush), as long as the lists
 // stay long enough to pay for that (an average of 48 entries over the whole grid).
+constexpr size_t kGroupRowsBytes = (size_t)4 << 20;
 inline int views_per_group(size_t V, size_t L, size_t D, size_t esize, size_t P, size_t NC, bool handed)
 {
-    const size_t rows_bytes = 2 * V * L * D * esize, M = V * L * P, cap = (size_t)4 << 20;
+    const size_t rows_bytes = 2 * V * L * D * esize, M = V * L * P, cap = kGroupRowsBytes;
     if (!handed || rows_bytes <= cap) return (int)V;
     size_t groups = (rows_bytes + cap - 1) / cap;
     if (groups > V) groups = V;

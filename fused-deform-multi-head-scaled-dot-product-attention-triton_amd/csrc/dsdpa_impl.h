@@ -508,9 +508,9 @@ template <typename S, int D> struct CellChunk {
 // Binning in one launch (bin_one_kernel): up to two samples a thread of one workgroup per (batch, key view), where the
 // three launches of the general way mostly wait for each other; beyond that one workgroup is the slower (figures at
 // the kernel).
-static inline bool bin_in_one_launch(const Dims &dm, const WorkspaceLayout &wl)
+static inline bool bin_in_one_launch(const Dims &dm)
 {
-    return (long long)dm.V * dm.L * dm.P <= kBinOneSamples && wl.NK <= kBinOneKeys;
+    return (long long)dm.V * dm.L * dm.P <= kBinOneSamples;
 }
 
 // records: the lists as 12-byte records (id and position in the cell) from wl.sorted on, through the room of
@@ -521,11 +521,11 @@ static inline int launch_binning(const float *coords, const Dims &dm, const Work
     unsigned *counters = (unsigned *)(ws + wl.counters);
     unsigned *start = (unsigned *)(ws + wl.start);
     unsigned *sorted = (unsigned *)(ws + wl.sorted);
-    if (bin_in_one_launch(dm, wl)) {
+    if (bin_in_one_launch(dm)) {
         ScopedKernelTimer timer(3, st);
         auto kern = bin_one_kernel<kBinOneSamples / 1024>;
         DSDPA_LAUNCH(kern, dim3((unsigned)(dm.B * dm.V)), dim3(1024), 0, st, timer.start(), timer.stop(),
-                     coords, dm, wl.NC, wl.NK, wl.vpg, start, wl.piece, wl.wmax, (uint4 *)(ws + wl.items), sorted, records);
+                     coords, dm, wl.NC, start, wl.piece, wl.wmax, (uint4 *)(ws + wl.items), sorted, records);
         return check_launch();
     }
     const size_t hist_bytes = (size_t)dm.V * wl.NC * sizeof(unsigned);
@@ -725,7 +725,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     hipStream_t bst = st;
     const bool worth_forking = (long long)dm.rows * dm.N >= DSDPA_TWO_STREAMS_FROM;
     SideLane *side = cell_binned && staged && worth_forking && !(flags & DSDPA_FLAG_SINGLE_STREAM) ? side_lane() : nullptr;
-    const size_t ncounters = cell_binned && !bin_in_one_launch(dm, wl) ? wl.counters_bytes / 4 : 0;
+    const size_t ncounters = cell_binned && !bin_in_one_launch(dm) ? wl.counters_bytes / 4 : 0;
     SideJoin joiner;
     if (side && hipEventRecord(side->fork, st) == hipSuccess &&
         hipStreamWaitEvent(side->stream, side->fork, 0) == hipSuccess) {
