@@ -398,14 +398,14 @@ __device__ __forceinline__ void widen_words(const uint32_t (&w)[DC * S::kBytes /
 // Which cells one launch of the dk/dv kernel covers, and the divisors that decode a work index into
 // (b, h, s2, cell) with multiply-shift instead of integer division (the decode is scalar code every
 // wave runs before it knows whether its cell is empty).
-// colour < 0: all cells, per-cell sums flushed with float atomics (a pixel belongs to four cells).
-// colour 0..3 (deterministic backward): only the cells with (row parity, column parity) = colour; no
-// two of them share a pixel, so the flush is a plain read-add-write, and the four launches, one
+// With RECORDS: all cells, by the work list that the binning made, work index -> (b, h, s2, item), `ncells` being the
+// list's capacity wmax per (b, s2) (empty slots leave at once) and ncx = Wimg + 1; per-cell sums are flushed with float
+// atomics (a pixel belongs to four cells).
+// Without (deterministic backward): four launches, each for the cells (oy + 2i, ox + 2j) of one (row parity, column
+// parity); no two of them share a pixel, so the flush is a plain read-add-write, and the launches, one
 // after the other, add every pixel's four contributions in a fixed order.
-// colour < 0 also switches the decode to the work list made by bin_scan_kernel: work index -> (b, h, s2, item),
-// `ncells` then being the list's capacity wmax per (b, s2); empty slots leave at once.
 struct CellGrid {
-    int colour, oy, ox, step, ncx, ncells;
+    int oy, ox, step, ncx, ncells;
     int bh0;                                // first (batch, head) pair of this launch (b * H + h)
     unsigned nwork;                         // pairs of this launch * V * ncells < 2^31
     FastDiv div_cells, div_ncx, div_v, div_h;
@@ -413,10 +413,9 @@ struct CellGrid {
 
 // HANDED: the dq kernel has left (p, sm_scale * ds) of every sample in `handed_` (per query row of this head,
 // in the order of the row's coordinates): an entry then costs a gather of that pair and the two rank-1 updates --
-// no taps in registers, no dot products, no exponential. Only with the work list (colour < 0) and with
-// records (the positions beside the ids).
-// RECORDS: the lists hold 12-byte records (sample id and position in the cell), and the launch goes by the work list
-// (colour < 0); without, ids alone, and every entry's coordinate pair is read again (the deterministic backward,
+// no taps in registers, no dot products, no exponential. Only with records (the positions beside the ids).
+// RECORDS: the lists hold 12-byte records (sample id and position in the cell), and the launch goes by the work
+// list; without, ids alone, and every entry's coordinate pair is read again (the deterministic backward,
 // whose lists are sorted id arrays, in its four colour launches).
 // What an item costs beside its entries is about 300 vector instructions (bounds, taps, tables, the sum over the
 // slots, the flush), which is most of the kernel where lists are short: 18x18, D = 32, 2 views x 2 samples (3.6

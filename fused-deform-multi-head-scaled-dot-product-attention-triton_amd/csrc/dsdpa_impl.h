@@ -582,11 +582,12 @@ static inline int launch_binning(const float *coords, const Dims &dm, const Work
     return check_launch();
 }
 
-// deterministic: four launches, one per (row parity, column parity) of the cells, each with plain stores
+// deterministic: lists of plain ids, four launches, one per (row parity, column parity) of the cells, each with plain
+// stores; else records, by the work list
 template <typename S, int D>
 int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const float *coords,
                          const float2 *stats, const void *dout, const unsigned *start, const unsigned *sorted,
-                         int records, const uint4 *items, unsigned wmax, const float2 *handed,
+                         const uint4 *items, unsigned wmax, const float2 *handed,
                          float *dk_acc, float *dv_acc, const Dims &dm, int NC, bool deterministic, int bh0, int nbh,
                          hipStream_t st)
 {
@@ -595,7 +596,6 @@ int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const floa
     for (int colour = deterministic ? 0 : -1; colour < (deterministic ? 4 : 0); ++colour) {
         const int cw = dm.Wimg + 1, ch = dm.Himg + 1;
         CellGrid cg;
-        cg.colour = colour;
         cg.oy = colour < 0 ? 0 : colour >> 1;
         cg.ox = colour < 0 ? 0 : colour & 1;
         cg.step = colour < 0 ? 1 : 2;
@@ -612,11 +612,11 @@ int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const floa
         cg.div_h = FastDiv::make((unsigned)dm.H);
         const unsigned blocks = (unsigned)((nwork + kCellWaves - 1) / kCellWaves);
         const bool first = colour <= 0, last = colour < 0 || colour == 3;
-        if (handed && colour < 0 && records)
+        if (handed && !deterministic)
             DSDPA_LAUNCH((bwd_dkdv_cell_kernel<S, D, DC, true, true>), dim3(blocks), dim3(kCellWaves * kWave), 0, st,
                                   first ? timer.start() : nullptr, last ? timer.stop() : nullptr, q, k, v, coords,
                                   stats, dout, start, sorted, items, handed, dk_acc, dv_acc, dm, NC, cg);
-        else if (records)
+        else if (!deterministic)
             DSDPA_LAUNCH((bwd_dkdv_cell_kernel<S, D, DC, false, true>), dim3(blocks), dim3(kCellWaves * kWave), 0, st,
                                   first ? timer.start() : nullptr, last ? timer.stop() : nullptr, q, k, v, coords,
                                   stats, dout, start, sorted, items, handed, dk_acc, dv_acc, dm, NC, cg);
@@ -705,7 +705,6 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     const unsigned *start = (const unsigned *)(ws + wl.start);
     const unsigned *sorted = (const unsigned *)(ws + (deterministic ? wl.sorted2 : wl.sorted));
     // (the reordered lists of the deterministic backward are ids without positions beside them: coordinates are read again)
-    const int records = deterministic ? 0 : 1;
     // (p, sm_scale * ds) per query*sample from the dq kernel to the dk/dv kernel, where the layout has room for it
     // (shapes on the gather dq kernel, which then runs before dk/dv on the same stream)
     float2 *handed = (wl.handed_bytes && cell_binned && !staged) ? (float2 *)(ws + wl.handed) : nullptr;
@@ -776,7 +775,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
                         : launch_bwd_dq_gather<S, DD>(q, k, v, coords, out, lse, dout, dq, dq_stats, dcoords,   \
                                                       handed, dm, bh0, nbh, st);                                \
             if (rc == DSDPA_OK && cell_binned)                                                                  \
-                rc = launch_bwd_dkdv_cell<S, DD>(q, k, v, coords, stats, dout, start, sorted, records,          \
+                rc = launch_bwd_dkdv_cell<S, DD>(q, k, v, coords, stats, dout, start, sorted,                   \
                                                  (const uint4 *)(ws + wl.items), wl.wmax, handed, dk_acc,       \
                                                  dv_acc, dm, wl.NK, deterministic, bh0, nbh, bst);              \
             else if (rc == DSDPA_OK)                                                                            \
