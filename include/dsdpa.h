@@ -78,6 +78,9 @@ enum { DSDPA_F32 = 0, DSDPA_BF16 = 1, DSDPA_F16 = 2 };
  * including the coords clone/scale (:381-383) and the zero-fill of `o` (:389).
  * Writes out (storage dtype) and lse (fp32).
  *
+ * Here and in the backward every tensor begins at a 16-byte aligned address, coords and dcoords at an 8-byte aligned
+ * one (the kernels load rows 16 bytes, positions 8 bytes at a time; addresses are not checked).
+ *
  * `workspace` must hold dsdpa_fwd_workspace_bytes(...) bytes (256-byte aligned; may be NULL when that is
  * 0). It is scratch for the duration of the call on `stream`. Shapes whose K and V planes fit in LDS: a
  * table of the bilinear weights and tap addresses of every coordinate pair, computed once from coords and
