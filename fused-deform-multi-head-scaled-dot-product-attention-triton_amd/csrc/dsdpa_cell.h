@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kBinLdsThreads) void bin_samples_lds_kernel(
 //
 // Bound by its chain of waits (one workgroup per (b, s2), a few of them on the whole chip): four keys a thread, both
 // sums by lane shifts inside a wave and over the 16 waves' totals in LDS, two barriers per 4096 keys.
-// (8450 keys, 8 workgroups: 29.4 -> 15.3 us against a scan of 1024 keys at a time with 20 barriers; 2401 keys 10.4 -> 6.0.)
+// (8450 keys, 8 workgroups: 29.4 -> 15.2 us against a scan of 1024 keys at a time with 20 barriers; 2401 keys 10.4 -> 6.0.)
 constexpr int kScanKeys = 4;
 struct ScanCarry { unsigned entries, pieces; };
 // One turn of the scan for a workgroup of 1024 threads: keys [c0, c0 + 4) of each thread, v their list lengths;
@@ -263,7 +263,7 @@ static __global__ __launch_bounds__(1024) void bin_scan_kernel(unsigned *__restr
 // its registers, PER of them a thread: every sample's rank in its list comes from the counting atomic itself, so
 // the coordinates are read once and there is one round of LDS atomics, no counters in memory (nothing to clear)
 // and no wait between launches. Bound by that chain of latencies (a few workgroups on the whole chip), as the three
-// launches are: 1296 samples a list group (18x18, 2 views x 2 samples) 6.4 us against 13.2 for the three and the gaps
+// launches are: 1296 samples a list group (18x18, 2 views x 2 samples) 6.2 us against 13.7 for the three and the gaps
 // between them. One workgroup's throughput then takes over: 5184 (4 x 4, six samples a thread) 13.9 against 17.4, a step
 // no faster; 11664 34.8 against 24.1, 17871 59 against 19.
 // Keys: one per cell, (Himg + 1)(Wimg + 1) <= 2 Himg Wimg + 2 of them, in LDS; the query views are one group (their rows
@@ -419,7 +419,7 @@ struct CellGrid {
 // whose lists are sorted id arrays, in its four colour launches).
 // What an item costs beside its entries is about 300 vector instructions (bounds, taps, tables, the sum over the
 // slots, the flush), which is most of the kernel where lists are short: 18x18, D = 32, 2 views x 2 samples (3.6
-// entries a list, fp32) 43.2 -> 39.0 us, 6 x 6 (32 entries, bf16) 170 -> 157, 14x14 with 8 x 32 (223, fp32) 247 -> 241,
+// entries a list, fp32) 43.0 -> 39.8 us, 6 x 6 (32 entries, bf16) 172 -> 161, 14x14 with 8 x 32 (223, fp32) 244.5 -> 241,
 // with the slots summed on a quarter of the values where the step that halves them comes first, and no tables made
 // for a block that is not there.
 template <typename S, int D, int DC, bool HANDED, bool RECORDS>
