@@ -228,27 +228,41 @@ __device__ __forceinline__ void scan_keys(const unsigned (&v)[kScanKeys], int c0
     }
 }
 
-// after the last turn: the total, and the empty slots behind the items
-__device__ __forceinline__ void scan_end(const ScanCarry &carry, int NC, unsigned wmax, unsigned *__restrict__ st, uint4 *__restrict__ it)
+// after the last turn: the total, the empty slots behind the items, and (where `spread` is asked for) whether the lists are
+// the patch kernel's (kSpreadLongest entries at most and `mean` or fewer on average): 0 if they are, else the number of items
+struct Spread { unsigned *items, mean; };
+constexpr unsigned kSpreadLongest = 1024;
+__device__ __forceinline__ void scan_end(const ScanCarry &carry, int NC, unsigned wmax, unsigned *__restrict__ st, uint4 *__restrict__ it,
+                                         const Spread &spread, unsigned longest)
 {
+    if (spread.items) {
+        const int any_long = __syncthreads_or(longest > kSpreadLongest);
+        if (threadIdx.x == 0)
+            spread.items[blockIdx.x] = !any_long && (unsigned long long)carry.entries <= (unsigned long long)spread.mean * carry.pieces
+                                     ? 0u : min(carry.pieces, wmax);
+    }
     if (threadIdx.x == 0) st[NC] = carry.entries;
     for (unsigned i = min(carry.pieces, wmax) + threadIdx.x; i < wmax; i += 1024) it[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
 static __global__ __launch_bounds__(1024) void bin_scan_kernel(unsigned *__restrict__ counters,
                                                         unsigned *__restrict__ start, int NC, int grid_cells,
-                                                        unsigned piece, unsigned wmax, uint4 *__restrict__ items)
+                                                        unsigned piece, unsigned wmax, uint4 *__restrict__ items,
+                                                        Spread spread)
 {
     __shared__ uint2 s_wave[16];                                   // (entries, pieces) of each wave's keys
     unsigned *cnt = counters + (size_t)blockIdx.x * NC;
     unsigned *st = start + (size_t)blockIdx.x * (NC + 1);
     uint4 *it = items + (size_t)blockIdx.x * wmax;
     ScanCarry carry{0u, 0u};
+    unsigned longest = 0u;
     for (int base = 0; base < NC; base += 1024 * kScanKeys) {
         const int c0 = base + (int)threadIdx.x * kScanKeys;
         unsigned v[kScanKeys], at;
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NC ? cnt[c0 + i] : 0u;
+#pragma unroll
+        for (int i = 0; i < kScanKeys; ++i) longest = max(longest, v[i]);
         scan_keys(v, c0, NC, grid_cells, piece, wmax, st, it, s_wave, carry, at);
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) {
@@ -256,7 +270,7 @@ static __global__ __launch_bounds__(1024) void bin_scan_kernel(unsigned *__restr
             at += v[i];
         }
     }
-    scan_end(carry, NC, wmax, st, it);
+    scan_end(carry, NC, wmax, st, it, spread, longest);
 }
 
 // Count, scan and fill in one launch, for lists short enough that one workgroup holds all samples of a (b, s2) in
@@ -274,7 +288,8 @@ static_assert(2ull * kBinOneSamples * 256 * 4 <= kGroupRowsBytes, "one group of 
 template <int PER>
 __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__ coords_, Dims dm, int NC,
                                                        unsigned *__restrict__ start, unsigned piece, unsigned wmax,
-                                                       uint4 *__restrict__ items, unsigned *__restrict__ sorted, int records)
+                                                       uint4 *__restrict__ items, unsigned *__restrict__ sorted, int records,
+                                                       Spread spread)
 {
     __shared__ unsigned s_hist[kBinOneKeys];                       // list lengths, then starts
     __shared__ uint2 s_wave[16];
@@ -303,6 +318,7 @@ __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__
     }
     __syncthreads();
     ScanCarry carry{0u, 0u};
+    unsigned longest = 0u;
     unsigned *st = start + (size_t)blockIdx.x * (NC + 1);
     uint4 *it = items + (size_t)blockIdx.x * wmax;
     for (int base = 0; base < NC; base += 1024 * kScanKeys) {
@@ -310,6 +326,8 @@ __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__
         unsigned v[kScanKeys], at;
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NC ? s_hist[c0 + i] : 0u;
+#pragma unroll
+        for (int i = 0; i < kScanKeys; ++i) longest = max(longest, v[i]);
         scan_keys(v, c0, NC, NC, piece, wmax, st, it, s_wave, carry, at);
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) {
@@ -324,7 +342,7 @@ __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__
             store_cell_entry(sorted, (size_t)blockIdx.x * M + s_hist[key_rank[i] & ((1u << kBinOneKeyBits) - 1u)] + (key_rank[i] >> kBinOneKeyBits),
                              (unsigned)i * 1024u + threadIdx.x, cell_fraction(xy[i], dm), records);
     }
-    scan_end(carry, NC, wmax, st, it);
+    scan_end(carry, NC, wmax, st, it, spread, longest);
 }
 
 // Deterministic backward: begin / end of every cell list as positions in the flat id array
@@ -423,14 +441,12 @@ struct CellGrid {
 // with the slots summed on a quarter of the values where the step that halves them comes first, and no tables made
 // for a block that is not there.
 template <typename S, int D, int DC, bool HANDED, bool RECORDS>
-__global__ __launch_bounds__(kCellWaves *kWave, HANDED ? (DC <= 4 ? 5 : (S::kBytes == 2 ? 3 : 4))
-                                                       : DC <= 4 ? (S::kBytes == 2 && D >= 64 ? 5 : 4) : (S::kBytes == 2 ? 3 : 2))
-void bwd_dkdv_cell_kernel(
-    const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_,
+__device__ __forceinline__ void cell_sums(
+    unsigned t, int ci, const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_,
     const float *__restrict__ coords_, const float2 *__restrict__ stats_,
     const void *__restrict__ dout_, const unsigned *__restrict__ start, const unsigned *__restrict__ sorted,
     const uint4 *__restrict__ items, const float2 *__restrict__ handed_,
-    float *__restrict__ dk_acc, float *__restrict__ dv_acc, Dims dm, int NC, CellGrid cg)
+    float *__restrict__ dk_acc, float *__restrict__ dv_acc, const Dims &dm, int NC, const CellGrid &cg)
 {
     constexpr int G = D / DC;
     constexpr int NS = kWave / G;
@@ -446,11 +462,7 @@ void bwd_dkdv_cell_kernel(
     __shared__ __attribute__((aligned(16))) unsigned s_rowq[kQuad ? kCellWaves : 1][2 * kWave], s_qrowq[kQuad ? kCellWaves : 1][2 * kWave];
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;   // wave index is uniform: keep it in an SGPR
-    const unsigned work = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x) * kCellWaves + wave;
-    if (work >= cg.nwork) return;
-    // plane-major: (b, h, s2, cell or work item)
-    unsigned t = cg.div_cells.div(work);
-    const int ci = (int)(work - t * (unsigned)cg.ncells);
+    // t = plane (b, h, s2) of the launch, ci = its cell or work item
     const unsigned bhl = cg.div_v.div(t);                      // pair within this launch
     const int s2 = (int)(t - bhl * (unsigned)dm.V);
     const unsigned bh = (unsigned)cg.bh0 + bhl;
@@ -964,6 +976,45 @@ void bwd_dkdv_cell_kernel(
                 else *pa += val;
             }
         }
+    }
+}
+
+#define DSDPA_CELL_ARGS                                                                                                    \
+    const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_, const float *__restrict__ coords_, \
+    const float2 *__restrict__ stats_, const void *__restrict__ dout_, const unsigned *__restrict__ start,                  \
+    const unsigned *__restrict__ sorted, const uint4 *__restrict__ items, const float2 *__restrict__ handed_,               \
+    float *__restrict__ dk_acc, float *__restrict__ dv_acc, Dims dm, int NC, CellGrid cg
+
+template <typename S, int D, int DC, bool HANDED, bool RECORDS>
+__global__ __launch_bounds__(kCellWaves *kWave, HANDED ? (DC <= 4 ? 5 : (S::kBytes == 2 ? 3 : 4))
+                                                       : DC <= 4 ? (S::kBytes == 2 && D >= 64 ? 5 : 4) : (S::kBytes == 2 ? 3 : 2))
+void bwd_dkdv_cell_kernel(DSDPA_CELL_ARGS)
+{
+    const unsigned work = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x) * kCellWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (work >= cg.nwork) return;
+    const unsigned t = cg.div_cells.div(work);                 // plane-major
+    cell_sums<S, D, DC, HANDED, RECORDS>(t, (int)(work - t * (unsigned)cg.ncells), q_, k_, v_, coords_, stats_, dout_, start, sorted,
+                                         items, handed_, dk_acc, dv_acc, dm, NC, cg);
+}
+
+// The planes that the patch kernel has left: a loop over their work lists, at once over where there are none. left[grp]:
+// items of the list, 0 where the patch kernel has done the planes of this (batch, key view). Every XCD takes one contiguous
+// part of the planes. (A loop costs registers and, over whole launches, time: one wave per SIMD less.)
+template <typename S, int D, int DC>
+__global__ __launch_bounds__(kCellWaves *kWave) void bwd_dkdv_cell_rest_kernel(const unsigned *__restrict__ left, DSDPA_CELL_ARGS)
+{
+    unsigned most = 0u;
+    for (int i = threadIdx.x & 63; i < dm.B * dm.V; i += kWave) most = max(most, left[i]);
+    most = (unsigned)__builtin_amdgcn_readfirstlane((int)wave_all(most, [](unsigned x, unsigned y) { return max(x, y); }));
+    if (most == 0u) return;
+    const unsigned planes = cg.nwork / (unsigned)cg.ncells, total = planes * most, parts = gridDim.x / kXcds;
+    const unsigned x = blockIdx.x % kXcds, end = (unsigned)((unsigned long long)total * (x + 1) / kXcds);
+    for (unsigned i = (unsigned)((unsigned long long)total * x / kXcds) + blockIdx.x / kXcds; i < end; i += parts) {
+        const unsigned t = i / most, ci = i - t * most;
+        const unsigned bhl = cg.div_v.div(t), b = cg.div_h.div((unsigned)cg.bh0 + bhl);
+        if (ci < left[b * (unsigned)dm.V + t - bhl * (unsigned)dm.V])
+            cell_sums<S, D, DC, true, true>(t, (int)ci, q_, k_, v_, coords_, stats_, dout_, start, sorted, items, handed_, dk_acc, dv_acc,
+                                            dm, NC, cg);
     }
 }
 

@@ -201,8 +201,8 @@ inline bool slab_path_fits(size_t V, size_t Himg, size_t Wimg, size_t D, size_t 
 //                                            deterministic backward keeps plain ids in `sorted` (and sorts them)
 //   items    B*V*wmax x 16 bytes             work list of the dk/dv kernel: (cell, first entry, end) per item
 //   handed   bhg*V*L*(V*P) x 8 bytes         (p, sm_scale*ds) per query*sample of one GROUP of bhg (batch, head) pairs,
-//                                            dq kernel -> dk/dv kernel (shapes on the gather kernels only); at most
-//                                            kHandedCapBytes whatever the shape
+//                                            dq kernel -> dk/dv kernel (shapes on the gather kernels, and short lists);
+//                                            at most kHandedCapBytes whatever the shape
 //   acc      2*n floats                      fp32 dk/dv accumulators (16-bit storage only)
 //   desc     20 bytes per coordinate pair    descriptor table (only when the plane kernels apply); 36 with
 //                                            the coordinate gradient
@@ -219,6 +219,8 @@ int sort_cell_lists(void *temp, size_t temp_bytes, const unsigned *ids_in, unsig
 struct WorkspaceLayout {
     size_t delta, counters, start, sorted, frac, items, handed, handed_bytes, acc, desc, sorted2, seg, sorttmp, sorttmp_bytes, total;
     int bh_group;               // (batch, head) pairs whose pairs the handed buffer holds at a time; 0: nothing is handed over
+    bool patch;                 // dk/dv by patches where the lists are short (DSDPA_PATH_AUTO)
+    unsigned spread_mean;       // ... up to so many entries a non-empty list on average
     DescLayout dl;
     size_t counters_bytes;
     int NC;                     // cells of the grid
@@ -266,13 +268,12 @@ inline int views_per_group(size_t V, size_t L, size_t D, size_t esize, size_t P,
 // cache holds. So the backward runs in GROUPS of (batch, head) pairs -- dq of a group, then dk/dv of the same
 // group, the cell lists being shared by all heads -- and the buffer holds one group's pairs: at most
 // kHandedCapBytes, which also stay in the memory-side cache between the two kernels. Returns the (batch, head)
-// pairs per group, 0 when nothing is handed over: shapes on the staged kernels (dq and dk/dv run side by side
-// there), the deterministic backward (its four colour launches recompute), one pair's samples beyond the cap or
-// beyond 32-bit byte offsets.
+// pairs per group, 0 when nothing is handed over: one pair's samples beyond the cap or beyond 32-bit byte offsets. Not asked
+// for by the deterministic backward (its four colour launches recompute) nor by shapes on the staged kernels (dq and
+// dk/dv run side by side there), short lists apart.
 constexpr size_t kHandedCapBytes = (size_t)128 << 20;
-inline int handed_group(size_t B, size_t V, size_t H, size_t L, size_t D, size_t P, size_t esize, bool deterministic)
+inline int handed_group(size_t B, size_t V, size_t H, size_t L, size_t P)
 {
-    if (deterministic || plane_path_fits(L, D, esize)) return 0;
     const size_t per_bh = V * L * (V * P) * 8;
     if (per_bh >= ((size_t)1 << 32) || per_bh > kHandedCapBytes) return 0;
     size_t g = kHandedCapBytes / per_bh;
@@ -280,6 +281,21 @@ inline int handed_group(size_t B, size_t V, size_t H, size_t L, size_t D, size_t
     // groups of equal size (the last one may be smaller by less than one pair per group)
     const size_t ngroups = (B * H + g - 1) / g;
     return (int)((B * H + ngroups - 1) / ngroups);
+}
+// dk/dv by patches of 4x4 pixels (dsdpa_patch.h) where the lists are short: what the cell kernel pays per list -- 300
+// instructions and 8*D float atomics, which the memory side takes at 0.3 a ns -- is then most of its time. Up to 48
+// entries a list over the whole grid in 16-bit storage, where the products run at 16 times the vector rate, and 12 in fp32,
+// where they run at twice; from 1024 patches, which fill the chip. us a step, cells / patches, 20x20, V = 4, P = 2, 6, 18 (7, 22,
+// 65 entries): bf16 D = 32 118 / 88, 150 / 129, 273 / 255; D = 64 178 / 123, 230 / 193, 474 / 413; D = 128 114 / 82, 142 / 113,
+// 234 / 227; fp32 D = 32 115 / 98, 150 / 153, 269 / 300; D = 64 185 / 147, 277 / 289, 612 / 704. At 184 entries (48x48, D = 64,
+// bf16) the kernels take 1150 / 1680, at 223 (14x14, D = 32, fp32) 235 / 500.
+// The lists are counted when they are made: spread_mean is the mean of the non-empty ones up to which the patches go ahead.
+inline unsigned spread_mean(size_t esize) { return esize == 2 ? 64u : 16u; }
+inline bool patch_path(size_t B, size_t V, size_t H, size_t Himg, size_t Wimg, size_t P, size_t esize, bool deterministic)
+{
+    const size_t L = Himg * Wimg, mean = V * L * P / ((Himg + 1) * (Wimg + 1));
+    return !deterministic && L >= 16 && mean <= (esize == 2 ? 48 : 12) && B * V * H * L * V * P >= ((size_t)1 << 15) &&
+           B * V * H * ((Himg + 3) / 4) * ((Wimg + 3) / 4) >= 1024;
 }
 inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Himg, size_t Wimg, size_t D, size_t P,
                                         bool storage16, bool deterministic, bool coords_grad)
@@ -289,10 +305,15 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
     w.NC = (int)((Himg + 1) * (Wimg + 1));
     size_t off = 0;
     w.delta = off; off += round256(rows * 8);           // (lse, delta) per row
-    w.bh_group = handed_group(B, V, H, Himg * Wimg, D, P, storage16 ? 2 : 4, deterministic);
-    const bool handed = w.bh_group > 0;
-    w.vpg = views_per_group(V, Himg * Wimg, D, storage16 ? 2 : 4, P, (size_t)w.NC, handed);
-    w.NK = w.NC * (int)((V + w.vpg - 1) / w.vpg);
+    const size_t L = Himg * Wimg, esize = storage16 ? 2 : 4, acc_bytes = storage16 ? round256(2 * rows * D * 4) : 0;
+    const bool planes = plane_path_fits(L, D, esize);
+    w.patch = patch_path(B, V, H, Himg, Wimg, P, esize, deterministic);
+    w.bh_group = (planes || deterministic) && !w.patch ? 0 : handed_group(B, V, H, L, P);
+    w.patch = w.patch && w.bh_group > 0;
+    w.spread_mean = spread_mean(esize);
+    const bool grouped = w.bh_group > 0 && !planes && !deterministic;
+    w.vpg = views_per_group(V, L, D, esize, P, (size_t)w.NC, grouped);
+    w.NK = w.NC * (int)((V + w.vpg - 1) / w.vpg);       // (short lists are never split: NK = NC where there are patches)
     w.counters = off; w.counters_bytes = round256(B * V * (size_t)w.NK * 4); off += w.counters_bytes;
     w.start = off; off += round256(B * V * ((size_t)w.NK + 1) * 4);
     w.sorted = off; off += round256(B * V * (V * Himg * Wimg * P) * 4);
@@ -302,9 +323,9 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
     // (p, sm_scale * ds) per query*sample of one group of (batch, head) pairs, handed from the dq kernel to the
     // dk/dv kernel (see handed_group)
     w.handed = off;
-    w.handed_bytes = round256((size_t)w.bh_group * V * Himg * Wimg * (V * P) * 8);
+    w.handed_bytes = round256((size_t)w.bh_group * V * L * (V * P) * 8);
     off += w.handed_bytes;
-    w.acc = off; if (storage16) off += round256(2 * rows * D * 4);
+    w.acc = off; off += acc_bytes;
     // with the coordinate gradient the staged dq kernel needs more LDS; where it no longer fits, dq takes the
     // gather kernel and no table is needed
     w.dl = desc_layout(B, V, Himg, Wimg, D, P, storage16 ? 2 : 4, coords_grad);

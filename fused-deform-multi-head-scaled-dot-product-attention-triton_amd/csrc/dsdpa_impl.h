@@ -9,6 +9,7 @@
 #include "dsdpa_plane.h"
 #include "dsdpa_dense.h"
 #include "dsdpa_slab.h"
+#include "dsdpa_patch.h"
 
 namespace dsdpa {
 
@@ -60,6 +61,25 @@ __global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ ds
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
         v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
         store_chunk<S, 8>((char *)dst + i * 16, v);
+    }
+}
+
+// The same for dk and dv of the planes (b, view) whose sums are in the accumulators: those with left[] items
+// (n8 = elements of a (batch, view, head) over 8). At once over where there are none.
+template <typename S>
+__global__ void cast_rest_kernel(const unsigned *__restrict__ left, const float *__restrict__ dk_acc, const float *__restrict__ dv_acc,
+                                 void *__restrict__ dk, void *__restrict__ dv, Dims dm, size_t n8)
+{
+    const size_t per = n8 * dm.H, stride = (size_t)gridDim.x * blockDim.x;
+    for (int g = 0; g < dm.B * dm.V; ++g) {
+        if (left[g] == 0u) continue;
+        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < 2 * per; i += stride) {
+            const size_t at = g * per + (i < per ? i : i - per);
+            const float4 *s4 = reinterpret_cast<const float4 *>(i < per ? dk_acc : dv_acc) + 2 * at;
+            const float4 a = s4[0], b = s4[1];
+            const float v[8] = { a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w };
+            store_chunk<S, 8>((char *)(i < per ? dk : dv) + at * 16, v);
+        }
     }
 }
 
@@ -419,26 +439,27 @@ template <typename S, int D>
 int launch_bwd_dq_plane(const void *q, const void *k, const void *v, const float4 *desc_w,
                         const uint32_t *desc_e, const void *out,
                         const float *lse, const void *dout, void *dq, float2 *stats, const float4 *desc_g,
-                        float *dcoords, const Dims &dm, hipStream_t st)
+                        float *dcoords, float2 *handed, const Dims &dm, int bh0, int nbh, hipStream_t st)
 {
     constexpr int DC = Chunk<S, D>::value;
     const size_t smem = (size_t)plane_lds_bytes<S, D>(dm.L) + kPlaneDescBytes + (dcoords ? kPlaneGradBytes : 0);
     int waves, row_blocks;
     // (two row blocks only without the coordinate gradient and up to 8 elements per lane: registers)
-    plane_config((long long)dm.B * dm.H, dm.V * dm.L, kWave / (D / DC), dm.P, device_cus(), (!dcoords && DC <= 8) ? 2 : 1,
+    plane_config(nbh, dm.V * dm.L, kWave / (D / DC), dm.P, device_cus(), (!dcoords && DC <= 8) ? 2 : 1,
                  &waves, &row_blocks);
     const int rows_per_block = row_blocks * waves * (kWave / (D / DC));
-    const long long blocks = (long long)dm.B * dm.H * ((dm.V * dm.L + rows_per_block - 1) / rows_per_block);
-    auto kern = dcoords ? bwd_dq_slot_kernel<S, D, DC, true, 1> : bwd_dq_slot_kernel<S, D, DC, false, 1>;
+    const long long blocks = (long long)nbh * ((dm.V * dm.L + rows_per_block - 1) / rows_per_block);
+    auto kern = handed ? (dcoords ? bwd_dq_slot_kernel<S, D, DC, true, 1, true> : bwd_dq_slot_kernel<S, D, DC, false, 1, true>)
+                       : (dcoords ? bwd_dq_slot_kernel<S, D, DC, true, 1, false> : bwd_dq_slot_kernel<S, D, DC, false, 1, false>);
     if constexpr (DC <= 8) {
-        if (row_blocks == 2) kern = bwd_dq_slot_kernel<S, D, DC, false, 2>;
+        if (row_blocks == 2) kern = handed ? bwd_dq_slot_kernel<S, D, DC, false, 2, true> : bwd_dq_slot_kernel<S, D, DC, false, 2, false>;
     }
-    static std::atomic<unsigned long long> lds_set[3];
-    if (int rc = allow_full_lds(kern, lds_set[dcoords ? 2 : row_blocks - 1])) return rc;
+    static std::atomic<unsigned long long> lds_set[6];
+    if (int rc = allow_full_lds(kern, lds_set[(handed ? 3 : 0) + (dcoords ? 2 : row_blocks - 1)])) return rc;
     ScopedKernelTimer timer(2, st);
     DSDPA_LAUNCH(kern, dim3((unsigned)blocks), dim3(waves * kWave), smem, st,
                           timer.start(), timer.stop(), q, k, v, desc_w, desc_e, out, lse, dout, dq, stats, desc_g,
-                          dcoords, dm);
+                          dcoords, handed, bh0, dm);
     return check_launch();
 }
 
@@ -513,10 +534,11 @@ static inline bool bin_in_one_launch(const Dims &dm)
     return (long long)dm.V * dm.L * dm.P <= kBinOneSamples;
 }
 
+// spread: flags to set for the patch kernel, or none.
 // records: the lists as 12-byte records (id and position in the cell) from wl.sorted on, through the room of
 // wl.frac behind it; else plain ids in wl.sorted (the deterministic backward, which sorts them).
 static inline int launch_binning(const float *coords, const Dims &dm, const WorkspaceLayout &wl, char *ws,
-                                 int records, hipStream_t st)
+                                 int records, const Spread &spread, hipStream_t st)
 {
     unsigned *counters = (unsigned *)(ws + wl.counters);
     unsigned *start = (unsigned *)(ws + wl.start);
@@ -525,7 +547,7 @@ static inline int launch_binning(const float *coords, const Dims &dm, const Work
         ScopedKernelTimer timer(3, st);
         auto kern = bin_one_kernel<kBinOneSamples / 1024>;
         DSDPA_LAUNCH(kern, dim3((unsigned)(dm.B * dm.V)), dim3(1024), 0, st, timer.start(), timer.stop(),
-                     coords, dm, wl.NC, start, wl.piece, wl.wmax, (uint4 *)(ws + wl.items), sorted, records);
+                     coords, dm, wl.NC, start, wl.piece, wl.wmax, (uint4 *)(ws + wl.items), sorted, records, spread);
         return check_launch();
     }
     const size_t hist_bytes = (size_t)dm.V * wl.NC * sizeof(unsigned);
@@ -561,7 +583,7 @@ static inline int launch_binning(const float *coords, const Dims &dm, const Work
                            coords, dm, wl.NC, wl.NK, wl.vpg, lchunk, nlc, counters, sorted, records);
         DSDPA_LAUNCH(bin_scan_kernel, dim3((unsigned)(dm.B * dm.V)), dim3(1024), 0, st,
                               t_scan.start(), t_scan.stop(), counters, start, wl.NK, wl.NC, wl.piece, wl.wmax,
-                              (uint4 *)(ws + wl.items));
+                              (uint4 *)(ws + wl.items), spread);
         DSDPA_LAUNCH(k1, dim3((unsigned)blocks), dim3(kBinLdsThreads), 2 * hist_bytes, st,
                               t_fill.start(), t_fill.stop(),
                            coords, dm, wl.NC, wl.NK, wl.vpg, lchunk, nlc, counters, sorted, records);
@@ -575,7 +597,7 @@ static inline int launch_binning(const float *coords, const Dims &dm, const Work
                        coords, dm, wl.NC, wl.NK, wl.vpg, counters, sorted, records);
     DSDPA_LAUNCH(bin_scan_kernel, dim3((unsigned)(dm.B * dm.V)), dim3(1024), 0, st,
                           t_scan.start(), t_scan.stop(), counters, start, wl.NK, wl.NC, wl.piece, wl.wmax,
-                              (uint4 *)(ws + wl.items));
+                              (uint4 *)(ws + wl.items), spread);
     DSDPA_LAUNCH(bin_samples_kernel<1>, dim3((unsigned)blocks), dim3(kBinThreads), 0, st,
                           t_fill.start(), t_fill.stop(),
                        coords, dm, wl.NC, wl.NK, wl.vpg, counters, sorted, records);
@@ -625,6 +647,54 @@ int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const floa
                                   first ? timer.start() : nullptr, last ? timer.stop() : nullptr, q, k, v, coords,
                                   stats, dout, start, sorted, items, handed, dk_acc, dv_acc, dm, NC, cg);
     }
+    return check_launch();
+}
+
+// dk/dv by patches: a workgroup of one to four waves per patch of 4x4 pixels of a plane (and per 128 columns); behind it
+// the cell kernel for the planes whose lists are not the patches'.
+// left (may be null: all planes are the patches'): see bwd_dkdv_cell_rest_kernel.
+template <typename S, int D>
+int launch_bwd_dkdv_patch(const void *q, const void *k, const void *v, const float *coords, const void *dout,
+                          const unsigned *start, const unsigned *sorted, const uint4 *items, unsigned wmax,
+                          const unsigned *left, const float2 *handed, void *dk, void *dv, float *dk_acc, float *dv_acc,
+                          const Dims &dm, int NC, int bh0, int nbh, hipStream_t st)
+{
+    constexpr int DP = D < 128 ? D : 128;
+    PatchGrid pg;
+    pg.npx = (dm.Wimg + kPatchSide - 1) / kPatchSide;
+    pg.npatch = pg.npx * ((dm.Himg + kPatchSide - 1) / kPatchSide);
+    pg.bh0 = bh0;
+    pg.div_patch = FastDiv::make((unsigned)pg.npatch);
+    pg.div_npx = FastDiv::make((unsigned)pg.npx);
+    pg.div_v = FastDiv::make((unsigned)dm.V);
+    pg.div_h = FastDiv::make((unsigned)dm.H);
+    const long long blocks = (long long)nbh * dm.V * pg.npatch;
+    if (blocks > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;
+    const long long visits = (long long)dm.V * dm.L * dm.P * 25 / 16 / pg.npatch;         // entries of an average patch
+    // (20x20 and 18x18, us with 1 / 2 / 4 waves: 54 entries a patch 17 / 18 / 24, 175 23 / 23 / 27, 700 107 / 100 / 105, 1600
+    // 97 / 85 / 79; without a second launch behind it, two for the patches that many samples may share)
+    const int waves = visits <= 128 && left ? 1 : visits <= 1280 ? 2 : 4;
+    CellGrid cg;
+    const long long nwork = (long long)nbh * dm.V * wmax;
+    if (nwork >= 0x7fffffffll - 65536) return DSDPA_ERR_TOO_LARGE;
+    cg.oy = cg.ox = 0;
+    cg.step = 1;
+    cg.ncx = dm.Wimg + 1;
+    cg.ncells = (int)wmax;
+    cg.bh0 = bh0;
+    cg.nwork = (unsigned)nwork;
+    cg.div_cells = FastDiv::make(wmax);
+    cg.div_ncx = FastDiv::make((unsigned)cg.ncx);
+    cg.div_v = pg.div_v;
+    cg.div_h = pg.div_h;
+    const unsigned rest = 32u * (unsigned)device_cus();
+    ScopedKernelTimer timer(1, st);
+    DSDPA_LAUNCH((bwd_dkdv_patch_kernel<S, D, DP>), dim3((unsigned)blocks, D / DP), dim3(waves * kWave), patch_lds_bytes(waves), st,
+                 timer.start(), left ? nullptr : timer.stop(), q, dout, start, sorted, left, handed, dk, dv, dk_acc, dv_acc, dm, NC, pg);
+    if (!left) return check_launch();
+    DSDPA_LAUNCH((bwd_dkdv_cell_rest_kernel<S, D, CellChunk<S, D>::value>), dim3(rest), dim3(kCellWaves * kWave), 0, st, nullptr,
+                 timer.stop(), left, q, k, v, coords, (const float2 *)nullptr, dout, start, sorted, items, handed, dk_acc, dv_acc,
+                 dm, NC, cg);
     return check_launch();
 }
 
@@ -707,7 +777,11 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     // (the reordered lists of the deterministic backward are ids without positions beside them: coordinates are read again)
     // (p, sm_scale * ds) per query*sample from the dq kernel to the dk/dv kernel, where the layout has room for it
     // (shapes on the gather dq kernel, which then runs before dk/dv on the same stream)
-    float2 *handed = (wl.handed_bytes && cell_binned && !staged) ? (float2 *)(ws + wl.handed) : nullptr;
+    const bool patch = wl.patch && path == DSDPA_PATH_AUTO;
+    // (neither dk/dv kernel needs the statistics then. The few samples that are binned in one launch are the patches' wherever
+    // they lie in 16-bit storage: 18x18, 2 views x 2 samples, clustered, step 58 us with cells, 49 with patches; fp32 50 / 60)
+    unsigned *left = patch && !(S::kBytes == 2 && bin_in_one_launch(dm)) ? (unsigned *)stats : nullptr;
+    float2 *handed = patch || (wl.handed_bytes && cell_binned && !staged) ? (float2 *)(ws + wl.handed) : nullptr;
     // fp32 storage: dk and dv are their own accumulators; 16-bit: fp32 accumulators in the workspace
     float *dk_acc = S::kBytes == 4 ? (float *)dk : (float *)(ws + wl.acc);
     float *dv_acc = S::kBytes == 4 ? (float *)dv : dk_acc + n;
@@ -723,7 +797,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     // under two million query*samples (0.15 ms of kernels) does not win back.
     hipStream_t bst = st;
     const bool worth_forking = (long long)dm.rows * dm.N >= DSDPA_TWO_STREAMS_FROM;
-    SideLane *side = cell_binned && staged && worth_forking && !(flags & DSDPA_FLAG_SINGLE_STREAM) ? side_lane() : nullptr;
+    SideLane *side = cell_binned && staged && !patch && worth_forking && !(flags & DSDPA_FLAG_SINGLE_STREAM) ? side_lane() : nullptr;
     const size_t ncounters = cell_binned && !bin_in_one_launch(dm) ? wl.counters_bytes / 4 : 0;
     SideJoin joiner;
     if (side && hipEventRecord(side->fork, st) == hipSuccess &&
@@ -737,11 +811,12 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     const size_t ndc = dcoords ? (size_t)dm.B * dm.V * dm.L * dm.N * 2 : 0;
     // what has to start at zero: on one stream everything in one job, which the tap-table launch (when
     // there is one) takes along; with the side lane the dk/dv side clears its own buffers there
-    const ZeroJob zero_all{{dk_acc, dv_acc, (float *)(ws + wl.counters), dcoords}, {n, n, ncounters, ndc}};
+    const size_t nacc = patch ? 0 : n;                 // (the patches are stored, not added)
+    const ZeroJob zero_all{{dk_acc, dv_acc, (float *)(ws + wl.counters), dcoords}, {nacc, nacc, ncounters, ndc}};
     const ZeroJob zero_main{{dcoords, nullptr, nullptr, nullptr}, {ndc, 0, 0, 0}};
     const ZeroJob &zero = side_on ? zero_main : zero_all;
     if (staged) rc = launch_plane_descriptors(coords, dm, ws + wl.desc, wl.dl, cg_table, zero, 4, st);
-    else if (!side_on || ndc) rc = zero_fill(zero, st);
+    else if (zero.n[0] + zero.n[1] + zero.n[2] + zero.n[3] > 0) rc = zero_fill(zero, st);
     if (rc != DSDPA_OK) return rc;
     if (side_on) {
         // the dk/dv side: its clears, and the (lse, delta) pairs that the dq kernel otherwise writes on the way
@@ -752,9 +827,10 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
                            stats, (size_t)dm.rows, D);
         if ((rc = check_launch()) != DSDPA_OK) return rc;
     }
-    if (cell_binned && (rc = launch_binning(coords, dm, wl, ws, deterministic ? 0 : 1, bst)) != DSDPA_OK) return rc;
+    if (cell_binned && (rc = launch_binning(coords, dm, wl, ws, deterministic ? 0 : 1, Spread{left, wl.spread_mean}, bst)) != DSDPA_OK)
+        return rc;
     if (deterministic && (rc = launch_list_ordering(dm, wl, ws, bst)) != DSDPA_OK) return rc;
-    float2 *dq_stats = side_on ? nullptr : stats;       // the dq kernel writes them only when dk/dv runs behind it
+    float2 *dq_stats = side_on || patch ? nullptr : stats;       // the dq kernel writes them only when dk/dv runs behind it
     // With the pairs handed over the two kernels go group by group of (batch, head) pairs: the buffer holds one
     // group's pairs (workspace_layout), and the dk/dv kernel of a group finds them where the dq kernel of the same
     // group has just left them. Otherwise one launch each covers all pairs.
@@ -769,12 +845,16 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
         for (int bh0 = 0; bh0 < nbh_all && rc == DSDPA_OK; bh0 += bh_step) {                                    \
             const int nbh = bh_step < nbh_all - bh0 ? bh_step : nbh_all - bh0;                                  \
             rc = staged ? launch_bwd_dq_plane<S, DD>(q, k, v, desc_w, desc_e, out, lse, dout, dq, dq_stats,     \
-                                                     desc_g, dcoords, dm, st)                                   \
+                                                     desc_g, dcoords, handed, dm, bh0, nbh, st)                 \
                  : slab ? launch_bwd_dq_slab<S, DD>(q, k, v, coords, out, lse, dout, dq, dq_stats, handed, dcoords,\
                                                     dm, bh0, nbh, st)                                           \
                         : launch_bwd_dq_gather<S, DD>(q, k, v, coords, out, lse, dout, dq, dq_stats, dcoords,   \
                                                       handed, dm, bh0, nbh, st);                                \
-            if (rc == DSDPA_OK && cell_binned)                                                                  \
+            if (rc == DSDPA_OK && patch)                                                                        \
+                rc = launch_bwd_dkdv_patch<S, DD>(q, k, v, coords, dout, start, sorted,                         \
+                                                  (const uint4 *)(ws + wl.items), wl.wmax, left, handed, dk,    \
+                                                  dv, dk_acc, dv_acc, dm, wl.NC, bh0, nbh, st);                 \
+            else if (rc == DSDPA_OK && cell_binned)                                                             \
                 rc = launch_bwd_dkdv_cell<S, DD>(q, k, v, coords, stats, dout, start, sorted,                   \
                                                  (const uint4 *)(ws + wl.items), wl.wmax, handed, dk_acc,       \
                                                  dv_acc, dm, wl.NK, deterministic, bh0, nbh, bst);              \
@@ -793,7 +873,13 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     }
 #undef DSDPA_BWD_CASE
     if (rc != DSDPA_OK) return rc;
-    if (S::kBytes != 4) {
+    if (S::kBytes != 4 && left) {
+        const size_t n8 = (size_t)dm.L * D / 8;                     // of a plane
+        size_t blocks = (n8 * B * V * H + 255) / 256;
+        if (blocks > 256 * 8) blocks = 256 * 8;
+        hipLaunchKernelGGL((cast_rest_kernel<S>), dim3((unsigned)blocks), dim3(256), 0, st, left, dk_acc, dv_acc, dk, dv, dm, n8);
+        rc = check_launch();
+    } else if (S::kBytes != 4 && !patch) {
         const size_t n8 = n / 8;
         const int threads = 256;
         size_t blocks = (n8 + threads - 1) / threads;

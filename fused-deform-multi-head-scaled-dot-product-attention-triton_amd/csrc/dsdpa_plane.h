@@ -139,13 +139,13 @@ struct PlaneBlock {
     int b, h, qbase;     // first query row (index over (s1, l)) of this workgroup
 };
 
-__device__ __forceinline__ PlaneBlock decode_plane_block(const Dims &dm, int rows_per_block)
+__device__ __forceinline__ PlaneBlock decode_plane_block(const Dims &dm, int rows_per_block, int bh0 = 0)
 {
     const int nq = dm.V * dm.L;
     const int chunks = (nq + rows_per_block - 1) / rows_per_block;
     const int bid = xcd_logical_block(blockIdx.x, gridDim.x);
     PlaneBlock pb;
-    const int bh = bid / chunks;
+    const int bh = bh0 + bid / chunks;
     pb.qbase = (bid % chunks) * rows_per_block;
     pb.h = bh % dm.H;
     pb.b = bh / dm.H;
@@ -159,12 +159,17 @@ __device__ __forceinline__ PlaneBlock decode_plane_block(const Dims &dm, int row
 // 2*q + (q & 1) (byte offset / ROW, so the table does not depend on the head width or storage type)
 // packed into one 32-bit word (13 bits each: a plane that fits in LDS has fewer than 2200 slots). Within
 // every run of up to 64 samples of one (b, s1, l, s2) the entries are stored in paired_position order.
-// For the coordinate gradient (desc_g not null) the word also carries which taps lie inside the image
+// The three bits above each code hold the sample's index inside its run, modulo 64 (low three bits, high three bits):
+// what the dq kernel knows about a sample goes back to the place of that sample (see sample_of).
+// For the coordinate gradient (desc_g not null) they carry which taps lie inside the image instead
 // -- bits 13, 14: columns x0, x0+1; bits 29, 30: rows y0, y0+1 -- and desc_g holds (fx, fy, the sample's
 // index n inside its run as an integer, unused): the entries are stored in a permuted order, and the
 // gradient has to go back to the sample it belongs to.
 constexpr int kDescThreads = 256;
 constexpr uint32_t kDescCodeMask = 0x1fffu;
+// the sample index inside its run of a table entry at place `pos` of the run with code word `c` (runs of more than 64
+// samples are permuted within pieces of 64)
+__device__ __forceinline__ int sample_of(int pos, uint32_t c) { return (pos & ~63) + (int)(((c >> 13) & 7u) | (((c >> 29) & 7u) << 3)); }
 
 static __global__ __launch_bounds__(kDescThreads) void plane_descriptor_kernel(
     const float *__restrict__ coords_, Dims dm, float4 *__restrict__ desc_w, uint32_t *__restrict__ desc_e,
@@ -199,6 +204,7 @@ static __global__ __launch_bounds__(kDescThreads) void plane_descriptor_kernel(
         const long long dst = blk * dm.P + pos;
         desc_w[dst] = make_float4(tp.w[0], tp.w[1], tp.w[2], tp.w[3]);
         uint32_t word = (uint32_t)(2 * qt + (qt & 1)) | ((uint32_t)(2 * qb + (qb & 1)) << 16);
+        if (!desc_g) word |= ((uint32_t)n & 7u) << 13 | (((uint32_t)n >> 3) & 7u) << 29;
         if (desc_g) {
             // same arithmetic as make_taps, so that fx, fy and the inside tests agree with the weights
             const float x = ((xy.x * 2.0f - 1.0f) + 1.0f) * ((float)(dm.Wimg - 1) * 0.5f);
@@ -231,7 +237,7 @@ static __global__ __launch_bounds__(kDescThreads) void plane_descriptor_kernel(
 // opposite halves of the bank line in every trip.
 // s_g (coordinate gradient only): fx, fy of the sample; the four inside bits then ride in the low bits
 // of the parked top address (ROW >= 32 bytes leaves them free): bit 0, 1: columns x0, x0+1; bit 2, 3: rows.
-// Returns the index inside its run of the sample this lane fetched (coordinate gradient only, else 0).
+// Returns the index inside its run of the sample this lane fetched.
 template <typename S, int D>
 __device__ __forceinline__ int stage_slot_descriptors(const float4 *__restrict__ desc_w,
                                                       const uint32_t *__restrict__ desc_e, size_t d_row, int P,
@@ -260,7 +266,7 @@ __device__ __forceinline__ int stage_slot_descriptors(const float4 *__restrict__
     s_e[slot * (G_ + 1) + trip] = make_int2(ex, ey);
     if (desc_g) s_g[slot * (G_ + 1) + trip] = make_float2(gw.x, gw.y);
     wave_lds_sync();
-    return __float_as_int(gw.z);
+    return desc_g ? __float_as_int(gw.z) : sample_of(n, c);
 }
 
 // ROWS: query-row blocks per workgroup. With two, a workgroup of W waves covers 2*W*NS rows: every staged plane is
@@ -424,12 +430,16 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
 // the sample's result, and after the pass every lane adds its own sample's pair to dcoords (zeroed before
 // the launch) with float atomics -- one wave-wide pair of atomics per pass, not one per trip.
 // ROWS: query-row blocks per workgroup, as in the forward.
-template <typename S, int D, int DC, bool CG, int ROWS>
+// HAND: (p, sm_scale * ds) of every sample goes to handed_, in the order of the coordinates of the (batch, head) pairs
+// of this launch, which begin at pair bh0: the lane that fetched a sample's table entry keeps its pair (all lanes of
+// the slot have it) and stores it after the pass.
+template <typename S, int D, int DC, bool CG, int ROWS, bool HAND>
 __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
     const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_,
     const float4 *__restrict__ desc_w, const uint32_t *__restrict__ desc_e, const void *__restrict__ out_,
     const float *__restrict__ lse_, const void *__restrict__ dout_, void *__restrict__ dq_,
-    float2 *__restrict__ stats_, const float4 *__restrict__ desc_g, float *__restrict__ dcoords_, Dims dm)
+    float2 *__restrict__ stats_, const float4 *__restrict__ desc_g, float *__restrict__ dcoords_,
+    float2 *__restrict__ handed_, int bh0, Dims dm)
 {
     constexpr int G = D / DC, NS = kWave / G;
     constexpr int kRow = D * S::kBytes;
@@ -444,7 +454,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
     float2 *s_g = reinterpret_cast<float2 *>(smem + img_bytes + kPlaneDescBytes) + wave * kPlaneDescPlaces;   // CG only
 
     const int rows_block = (int)(blockDim.x >> 6) * NS;                       // (workgroups of up to kPlaneWaves waves)
-    const PlaneBlock pb = decode_plane_block(dm, ROWS * rows_block);
+    const PlaneBlock pb = decode_plane_block(dm, ROWS * rows_block, bh0);
     const int nq = dm.V * dm.L;
     const int g = lane % G, slot = lane / G, lane_elem = g * DC, lane_byte = lane_elem * S::kBytes;
     const float qscale = dm.sm_scale * kLog2e;
@@ -454,7 +464,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
 
     // per row block: this slot's row and its state
     bool have_s[ROWS];
-    size_t crow_s[ROWS], roff_s[ROWS];
+    size_t crow_s[ROWS], roff_s[ROWS], hrow_s[ROWS];
     float qf_s[ROWS][DC], dof_s[ROWS][DC], dqa_s[ROWS][DC], delta_s[ROWS], lse_s[ROWS];
     uint32_t dop_s[ROWS][kPacked ? DC / 2 : 1];
 #pragma unroll
@@ -465,6 +475,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         const unsigned s1 = dm.divL.div(qc), l = qc - s1 * (unsigned)dm.L;
         const size_t row = (((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l;
         crow_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.L + l) * (size_t)dm.N;
+        hrow_s[rb] = ((size_t)(pb.b * dm.H + pb.h - bh0) * nq + qc) * (size_t)dm.N;
         const size_t roff = (row * D + lane_elem) * S::kBytes;
         roff_s[rb] = roff;
         float of[DC];
@@ -500,7 +511,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                                                           slot, G, s_w, s_e, CG ? desc_g : nullptr, s_g);
             const int cnt = min(G, dm.P - c0);
             const int my_trip = (cnt & 1) == 0 ? g ^ (slot & 1) : g;     // where this lane's sample was parked
-            float my_gx = 0.f, my_gy = 0.f;
+            float my_gx = 0.f, my_gy = 0.f, my_p = 0.f, my_ds = 0.f;
             for (int t = 0; t < cnt; ++t) {
                 const float4 w = s_w[slot * (G + 1) + t];
                 const int2 e = s_e[slot * (G + 1) + t];
@@ -551,7 +562,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                     float gy = fmaf(gf.x, (g3 - g1) - dy0, dy0) * (float)(dm.Himg - 1);
                     gx = group_sum<G>(gx);
                     gy = group_sum<G>(gy);
-                    if (t == my_trip) { my_gx = gx; my_gy = gy; }
+                    if (t == my_trip) { my_gx = gx; my_gy = gy; my_p = p; my_ds = ds; }
                     continue;
                 }
                 const uint32_t at = e.x + lbase, ab = e.y + lbase;
@@ -589,9 +600,14 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                 dp = group_sum<G>(dp);
                 const float p = __builtin_amdgcn_exp2f(dot * qscale - lse);
                 const float ds = p * (dp - delta);
+                if constexpr (HAND) {
+                    if (t == my_trip) { my_p = p; my_ds = ds; }
+                }
 #pragma unroll
                 for (int d = 0; d < DC; ++d) dqa[d] = fmaf(ds, kk[d], dqa[d]);
             }
+            if (HAND && have && c0 + g < dm.P)
+                handed_[hrow_s[rb] + (size_t)(s2 * dm.P + my_n)] = make_float2(my_p, my_ds * dm.sm_scale);
             if (CG && have && c0 + g < dm.P) {
                 float *dst = dcoords_ + 2 * (crow + (size_t)s2 * dm.P + (size_t)my_n);
                 atomicAdd(dst, my_gx);
