@@ -374,45 +374,6 @@ __device__ __forceinline__ void load_tap_or_zero(const char *base, int pix, int 
 // (lse, delta) pair.
 template <int WORDS> struct RowFetch { uint32_t qw[WORDS], dw[WORDS]; float2 ld; };
 
-template <int WORDS>
-__device__ __forceinline__ void load_words(const void *p, uint32_t (&w)[WORDS])
-{
-    static_assert(WORDS == 2 || WORDS % 4 == 0, "8 bytes, or multiples of 16");
-    if constexpr (WORDS == 2) {
-        const uint2 t = *reinterpret_cast<const uint2 *>(p);
-        w[0] = t.x; w[1] = t.y;
-    } else {
-#pragma unroll
-        for (int i = 0; i < WORDS / 4; ++i) {
-            const uint4 t = reinterpret_cast<const uint4 *>(p)[i];
-            w[4 * i + 0] = t.x; w[4 * i + 1] = t.y; w[4 * i + 2] = t.z; w[4 * i + 3] = t.w;
-        }
-    }
-}
-
-// the words of load_words as DC fp32 values
-template <typename S, int DC>
-__device__ __forceinline__ void widen_words(const uint32_t (&w)[DC * S::kBytes / 4], float (&dst)[DC])
-{
-    if constexpr (S::kBytes == 4) {
-#pragma unroll
-        for (int d = 0; d < DC; ++d) dst[d] = __uint_as_float(w[d]);
-    } else {
-#pragma unroll
-        for (int j = 0; j < DC / 2; ++j) {
-            if constexpr (S::kBf16) {
-                dst[2 * j + 0] = __uint_as_float(w[j] << 16);
-                dst[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-            } else {
-                union { uint32_t u; _Float16 h[2]; } cv;
-                cv.u = w[j];
-                dst[2 * j + 0] = (float)cv.h[0];
-                dst[2 * j + 1] = (float)cv.h[1];
-            }
-        }
-    }
-}
-
 // Which cells one launch of the dk/dv kernel covers, and the divisors that decode a work index into
 // (b, h, s2, cell) with multiply-shift instead of integer division (the decode is scalar code every
 // wave runs before it knows whether its cell is empty).

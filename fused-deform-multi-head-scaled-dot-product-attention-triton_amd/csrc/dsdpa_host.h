@@ -132,11 +132,32 @@ inline bool plane_path_fits(size_t L, size_t D, size_t esize, bool coords_grad =
     return (L + 2) * 2 * D * esize + kPlaneDescLdsBytes + (coords_grad ? kPlaneGradLdsBytes : 0) <= kLdsBytes;
 }
 
-// With very few samples per view the staged kernels mostly stage: every workgroup loads all V plane pairs for
-// P samples per row and view, while the gather kernels touch only the rows they sample. Measured on 18x18,
-// D = 32 (forward, staged / gather ms): V = 12: P = 2 0.344 / 0.245, P = 4 0.431 / 0.414, P = 5 0.485 / 0.516;
-// V = 8: P = 3 0.173 / 0.162, P = 4 0.195 / 0.200; V = 6: equal up to P = 2, staged ahead from there.
-inline bool few_samples_prefer_gather(size_t V, size_t P) { return P <= 3 && V >= 8; }
+// With very few samples per view the staged kernels mostly stage: every workgroup loads all V plane pairs for P samples
+// per row and view, while the row kernels touch only the rows they sample, and need no table. us a step, staged / rows, D = 32,
+// 18x14: fp32 V = 8: P = 1 114 / 92, P = 2 165 / 163, P = 3 185 / 195; V = 12: P = 1 242 / 178, 2 293 / 277, 3 341 / 357; V = 4: P = 2
+// 79 / 73, 3 89 / 86, 4 97 / 97; V = 2 (18x18): P = 3 85 / 78, 5 89 / 93; bf16 V = 8: P = 3 155 / 142, 4 177 / 172; V = 12: P = 3 276 /
+// 262, 4 321 / 327.
+inline bool few_samples_prefer_rows(size_t V, size_t P, size_t esize) { return P <= (esize == 2 ? 3 : 2) || V * P <= 6; }
+
+// Row kernels (dsdpa_rows.h) against the gather kernels, a wave per row, for fewer than 64 samples per view. The less samples
+// a row has the more the latter's empty lanes and the merge of its slots cost; the more it has the more its eight or four samples
+// in flight per row pay where the launch has few rows to fill the chip with. us, gather / rows, forward: 40x40, D = 32, fp32, N = 8
+// samples a row, 400 / 1600 waves of rows: 5 / 4, 10 / 6; N = 24, 1200 / 2400 / 4800: 12 / 16, 21 / 21, 37 / 34; N = 40, 400 / 1600: 9 / 14,
+// 21 / 22; 44x20, 14080 waves: N = 8 59 / 33, 24 94 / 84, 80 277 / 264. Beyond 64 samples 16-bit rows and narrow heads are even or
+// behind (56x50, N = 150: D = 16 fp32 801 / 840, dq 808 / 1019; D = 32 bf16 800 / 861; 48x48, N = 192, D = 64 bf16 1440 / 1450), dq with
+// D >= 64 and fp32 ahead (1716 / 1636 there; fp32 D = 64 1833 / 1364). Rows of a wave sample all views at once: with the K and
+// V planes of a (batch, head) well beyond an XCD's 4 MB of L2 that costs misses (D = 128, 56x50, V = 5: bf16, 7 MB, forward
+// 563 / 632, dq 930 / 689; fp32, 14 MB, 1851 / 2227 and 1023 / 2182).
+inline bool row_path(size_t rows, size_t V, size_t L, size_t D, size_t P, size_t esize, bool dq)
+{
+    const size_t N = V * P, lanes = D * esize >= 512 ? 32 : D * esize / 16, waves = rows * lanes / 64;
+    if (P >= 64) return false;
+    if (N <= 16) return true;
+    if (2 * V * L * D * esize > ((size_t)(dq ? 8 : 4) << 20)) return false;
+    if (N <= 32) return waves >= 2048;
+    if (N <= 64) return waves >= 4096 && (esize == 2 || D >= 32);
+    return waves >= 8192 && D >= 64 && (dq || esize == 4 || D == 256);
+}
 
 // Descriptor table of the plane kernels: per coordinate pair 16 bytes of weights and 4 of packed slot
 // codes (plus, for the coordinate gradient, 16 bytes of derivative weights), computed once per call by

@@ -1,0 +1,58 @@
+"""Row kernels (one query row per slot of lanes, taps from memory): every lane split, query rows that end inside a wave, a last pass
+of one sample, of an odd number and of a whole pass, strided inputs, the coordinate gradient and the pairs handed on to
+dk/dv. Against the CPU oracle at the bars of the other parity tests."""
+import math
+
+import pytest
+import torch
+
+from oracle import oracle_bwd, oracle_fwd
+from ops.triton import deform_sdpa_triton
+from parity_util import rel
+
+pytestmark = pytest.mark.gpu
+BAR = {torch.float32: (1e-4, 1e-3), torch.bfloat16: (2e-2, 2e-2), torch.float16: (2e-2, 2e-2)}
+
+
+def check(B, V, H, Himg, Wimg, D, P, dtype, coords_grad=False, projection=False):
+    print(f"[case] rows B{B} V{V} H{H} {Himg}x{Wimg} D{D} P{P} {dtype} {coords_grad} {projection}", flush=True)
+    g = torch.Generator().manual_seed(V * P + D)
+    L, scale = Himg * Wimg, 1.0 / math.sqrt(D)
+    shape = (B, V, L, H, D) if projection else (B, V, H, L, D)
+    leaves = [torch.randn(shape, generator=g).to(dtype) for _ in range(3)]
+    coords = torch.rand(B, V, L, V, P, 2, generator=g) * 1.2 - 0.1
+    dout = torch.randn(B, V, H, L, D, generator=g).to(dtype)
+    dev = [t.to("cuda:0").requires_grad_(True) for t in leaves]
+    cdev = coords.to("cuda:0").requires_grad_(coords_grad)
+    view = (lambda t: t.permute(0, 1, 3, 2, 4)) if projection else (lambda t: t)
+    out = deform_sdpa_triton(*(view(t) for t in dev), cdev, Wimg, Himg, scale, coords_grad)
+    out.backward(dout.to("cuda:0"))
+    torch.cuda.synchronize()
+    n = [view(t).float().contiguous().numpy() for t in leaves]
+    assert rel(out, oracle_fwd(*n, coords.numpy(), Wimg, Himg, scale)[0]) < BAR[dtype][0]
+    want = oracle_bwd(*n, coords.numpy(), dout.float().numpy(), Wimg, Himg, scale, with_coords=coords_grad)
+    got = [view(t.grad) for t in dev] + ([cdev.grad] if coords_grad else [])
+    for a, b, name in zip(got, want, ("dq", "dk", "dv", "dcoords")):
+        if V * P == 1 and name in ("dq", "dk", "dcoords"):       # one sample: p = 1, the others are zero
+            continue
+        assert rel(a, b) < BAR[dtype][1], name
+
+
+# 23x29: planes too large for LDS from D = 64 fp32 on, below that few samples of a staged shape
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("D", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("V,P", [(1, 1), (3, 2), (2, 3), (3, 5)])
+def test_rows_against_the_oracle(V, P, D, dtype):
+    check(1, V, 3, 23, 29, D, P, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=str)
+@pytest.mark.parametrize("D,P", [(32, 3), (64, 8), (128, 2), (256, 5)])
+def test_rows_with_the_coordinate_gradient(D, P, dtype):
+    check(2, 2, 3, 23, 29, D, P, dtype, coords_grad=True, projection=True)
+
+
+# more than 16 and more than 32 samples a row, from 2048 and 4096 waves of rows on
+@pytest.mark.parametrize("V,H,P,dtype", [(2, 10, 12, torch.float32), (2, 20, 10, torch.bfloat16), (3, 14, 21, torch.bfloat16)], ids=str)
+def test_many_rows(V, H, P, dtype):
+    check(1, V, H, 30, 31, 64, P, dtype)
