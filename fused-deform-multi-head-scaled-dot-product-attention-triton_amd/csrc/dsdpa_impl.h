@@ -456,55 +456,87 @@ static inline int launch_plane_descriptors(const float *coords, const Dims &dm, 
     return check_launch();
 }
 
+// Elements per lane of the staged kernels' second form (two pieces of 16 bytes; fp32, rows of 128 and 256 bytes), or 0.
+template <typename S, int D> struct WideChunk { static constexpr int value = S::kBytes == 4 && (D == 32 || D == 64) ? 8 : 0; };
+
 template <typename S, int D>
-int launch_fwd_plane(const void *q, const void *k, const void *v, const float4 *desc_w, const uint32_t *desc_e,
-                     void *out, float *lse, const Dims &dm, hipStream_t st)
+PlaneConfig staged_config(const Dims &dm, int nbh, int max_blocks)
 {
-    constexpr int DC = Chunk<S, D>::value;
+    constexpr int DC = Chunk<S, D>::value, WDC = WideChunk<S, D>::value;
+    return plane_config(nbh, dm.V * dm.L, kWave * DC / D, dm.P, device_cus(), max_blocks, WDC != 0);
+}
+
+template <typename S, int D, int DC>
+int launch_fwd_plane_as(const void *q, const void *k, const void *v, const float4 *desc_w, const uint32_t *desc_e, void *out,
+                        float *lse, const Dims &dm, const PlaneConfig &pc, hipStream_t st)
+{
     const size_t smem = (size_t)plane_lds_bytes<S, D>(dm.L) + kPlaneDescBytes;
-    int waves, row_blocks;
-    plane_config((long long)dm.B * dm.H, dm.V * dm.L, kWave / (D / DC), dm.P, device_cus(), DC <= 8 ? 2 : 1, &waves,
-                 &row_blocks);          // (16 elements per lane: two rows' state does not fit in the registers)
-    const int rows_per_block = row_blocks * waves * (kWave / (D / DC));
+    const int rows_per_block = pc.row_blocks * pc.waves * (kWave / (D / DC));
     const long long blocks = (long long)dm.B * dm.H * ((dm.V * dm.L + rows_per_block - 1) / rows_per_block);
     auto kern = fwd_slot_kernel<S, D, DC, 1>;
-    if constexpr (DC <= 8) {
-        if (row_blocks == 2) kern = fwd_slot_kernel<S, D, DC, 2>;
+    if constexpr (DC == Chunk<S, D>::value && DC <= 8) {      // (16 elements per lane: two rows' state does not fit in the registers)
+        if (pc.row_blocks == 2) kern = fwd_slot_kernel<S, D, DC, 2>;
     }
     static std::atomic<unsigned long long> lds_set[2];
-    if (int rc = allow_full_lds(kern, lds_set[row_blocks - 1])) return rc;
+    if (int rc = allow_full_lds(kern, lds_set[pc.row_blocks - 1])) return rc;
     ScopedKernelTimer timer(0, st);
-    DSDPA_LAUNCH(kern, dim3((unsigned)blocks), dim3(waves * kWave), smem, st,
+    DSDPA_LAUNCH(kern, dim3((unsigned)blocks), dim3(pc.waves * kWave), smem, st,
                           timer.start(), timer.stop(), q, k, v, desc_w, desc_e, out, lse, dm);
     return check_launch();
 }
 
 template <typename S, int D>
-int launch_bwd_dq_plane(const void *q, const void *k, const void *v, const float4 *desc_w,
-                        const uint32_t *desc_e, const void *out,
-                        const float *lse, const void *dout, void *dq, float2 *stats, const float4 *desc_g,
-                        float *dcoords, float2 *handed, const Dims &dm, int bh0, int nbh, hipStream_t st)
+int launch_fwd_plane(const void *q, const void *k, const void *v, const float4 *desc_w, const uint32_t *desc_e,
+                     void *out, float *lse, const Dims &dm, hipStream_t st)
 {
-    constexpr int DC = Chunk<S, D>::value;
+    constexpr int DC = Chunk<S, D>::value, WDC = WideChunk<S, D>::value;
+    const PlaneConfig pc = staged_config<S, D>(dm, dm.B * dm.H, DC <= 8 ? 2 : 1);
+    if constexpr (WDC != 0) {
+        if (pc.wide) return launch_fwd_plane_as<S, D, WDC>(q, k, v, desc_w, desc_e, out, lse, dm, pc, st);
+    }
+    return launch_fwd_plane_as<S, D, DC>(q, k, v, desc_w, desc_e, out, lse, dm, pc, st);
+}
+
+template <typename S, int D, int DC>
+int launch_bwd_dq_plane_as(const void *q, const void *k, const void *v, const float4 *desc_w, const uint32_t *desc_e,
+                           const void *out, const float *lse, const void *dout, void *dq, float2 *stats, const float4 *desc_g,
+                           float *dcoords, float2 *handed, const Dims &dm, int bh0, int nbh, const PlaneConfig &pc, hipStream_t st)
+{
     const size_t smem = (size_t)plane_lds_bytes<S, D>(dm.L) + kPlaneDescBytes + (dcoords ? kPlaneGradBytes : 0);
-    int waves, row_blocks;
-    // (two row blocks only without the coordinate gradient and up to 8 elements per lane: registers)
-    plane_config(nbh, dm.V * dm.L, kWave / (D / DC), dm.P, device_cus(), (!dcoords && DC <= 8) ? 2 : 1,
-                 &waves, &row_blocks);
-    const int rows_per_block = row_blocks * waves * (kWave / (D / DC));
+    const int rows_per_block = pc.row_blocks * pc.waves * (kWave / (D / DC));
     const long long blocks = (long long)nbh * ((dm.V * dm.L + rows_per_block - 1) / rows_per_block);
-    auto kern = handed ? (dcoords ? bwd_dq_slot_kernel<S, D, DC, true, 1, true> : bwd_dq_slot_kernel<S, D, DC, false, 1, true>)
-                       : (dcoords ? bwd_dq_slot_kernel<S, D, DC, true, 1, false> : bwd_dq_slot_kernel<S, D, DC, false, 1, false>);
-    if constexpr (DC <= 8) {
-        if (row_blocks == 2) kern = handed ? bwd_dq_slot_kernel<S, D, DC, false, 2, true> : bwd_dq_slot_kernel<S, D, DC, false, 2, false>;
+    auto kern = handed ? bwd_dq_slot_kernel<S, D, DC, false, 1, true> : bwd_dq_slot_kernel<S, D, DC, false, 1, false>;
+    if constexpr (DC == Chunk<S, D>::value) {
+        if (dcoords) kern = handed ? bwd_dq_slot_kernel<S, D, DC, true, 1, true> : bwd_dq_slot_kernel<S, D, DC, true, 1, false>;
+        if constexpr (DC <= 8) {
+            if (pc.row_blocks == 2) kern = handed ? bwd_dq_slot_kernel<S, D, DC, false, 2, true> : bwd_dq_slot_kernel<S, D, DC, false, 2, false>;
+        }
     }
     static std::atomic<unsigned long long> lds_set[6];
-    if (int rc = allow_full_lds(kern, lds_set[(handed ? 3 : 0) + (dcoords ? 2 : row_blocks - 1)])) return rc;
+    if (int rc = allow_full_lds(kern, lds_set[(handed ? 3 : 0) + (dcoords ? 2 : pc.row_blocks - 1)])) return rc;
     ScopedKernelTimer timer(2, st);
-    DSDPA_LAUNCH(kern, dim3((unsigned)blocks), dim3(waves * kWave), smem, st,
+    DSDPA_LAUNCH(kern, dim3((unsigned)blocks), dim3(pc.waves * kWave), smem, st,
                           timer.start(), timer.stop(), q, k, v, desc_w, desc_e, out, lse, dout, dq, stats, desc_g,
                           dcoords, handed, bh0, dm);
     return check_launch();
+}
+
+template <typename S, int D>
+int launch_bwd_dq_plane(const void *q, const void *k, const void *v, const float4 *desc_w, const uint32_t *desc_e, const void *out,
+                        const float *lse, const void *dout, void *dq, float2 *stats, const float4 *desc_g,
+                        float *dcoords, float2 *handed, const Dims &dm, int bh0, int nbh, hipStream_t st)
+{
+    constexpr int DC = Chunk<S, D>::value, WDC = WideChunk<S, D>::value;
+    // (two row blocks and the wide form only without the coordinate gradient, two blocks up to 8 elements per lane: registers)
+    PlaneConfig pc = staged_config<S, D>(dm, nbh, (!dcoords && DC <= 8) ? 2 : 1);
+    if constexpr (WDC != 0) {
+        if (pc.wide && !dcoords)
+            return launch_bwd_dq_plane_as<S, D, WDC>(q, k, v, desc_w, desc_e, out, lse, dout, dq, stats, desc_g, dcoords, handed, dm,
+                                                     bh0, nbh, pc, st);
+        if (pc.wide) pc = plane_config(nbh, dm.V * dm.L, kWave * DC / D, dm.P, device_cus(), 1, false);
+    }
+    return launch_bwd_dq_plane_as<S, D, DC>(q, k, v, desc_w, desc_e, out, lse, dout, dq, stats, desc_g, dcoords, handed, dm, bh0, nbh,
+                                            pc, st);
 }
 
 template <typename S>

@@ -111,28 +111,34 @@ __device__ __forceinline__ int paired_position(bool valid, int cls, int lane, un
     return valid ? pos_valid : n0 + n1 + __popcll(mi & below);
 }
 
-// Waves per workgroup and query-row blocks per workgroup of a staged launch. The planes in LDS allow one workgroup
-// per CU, so a launch runs in rounds of `cus` workgroups, and a round lasts about as long as its workgroups have
+// Waves per workgroup, query-row blocks per workgroup and lane split of a staged launch. The planes in LDS allow one
+// workgroup per CU, so a launch runs in rounds of `cus` workgroups, and a round lasts about as long as its workgroups have
 // waves times samples per view (the kernels are bound by instruction issue) plus the staging of the planes (about
 // two waves' worth at 32 samples per view: 64 in these units). 16 waves is the most rows per staged plane and
 // block; fewer waves can mean fewer idle CUs in the last round (2 x 8 x 16 planes of 14x14 pixels and 8 views
 // make 416 workgroups of 16 waves, 1.6 rounds of 256, but 512 of 13 waves, two full rounds of shorter
 // workgroups), and two row blocks per workgroup halve the staging of a launch of many rounds (few samples per
-// view: the reference's sweep). Picks the pair with the lowest rounds * (blocks * waves * P + 64).
-inline void plane_config(long long planes, int rows_per_plane, int rows_per_wave, int P, int cus, int max_blocks,
-                         int *waves, int *row_blocks)
+// view: the reference's sweep). The wide split (fp32, D = 32 and 64: eight elements a lane, twice the rows a wave) spends 97
+// instructions on 16 samples where the other spends 62 on eight, so a wave of it counts 8/5; under three waves a SIMD it no
+// longer hides the LDS (18x18, 16 planes of 1944 rows, 256 workgroups of eight waves: forward 93 us against 87). Picks the
+// least rounds * (blocks * waves * P + 64). Narrow / wide, us: 18x18, 12 views x 12 samples, forward 548 / 490; 14x14, 8 x 32, forward
+// 198 / 179 and the step, whose dq leaves dk/dv more room, 693 / 606; 12x13, D = 64, 6 x 8 53 / 42, 8 x 32 351 / 284.
+struct PlaneConfig { int waves, row_blocks; bool wide; };
+inline PlaneConfig plane_config(long long planes, int rows_per_plane, int rows_per_wave, int P, int cus, int max_blocks, bool wide_ok)
 {
+    PlaneConfig best{kPlaneWaves, 1, false};
     long long best_cost = -1;
-    *waves = kPlaneWaves;
-    *row_blocks = 1;
-    for (int rb = 1; rb <= max_blocks; ++rb) {
-        for (int w = kPlaneWaves; w >= 4; --w) {
-            const long long rows = (long long)rb * w * rows_per_wave;
+    for (int form = 1; form <= max_blocks + (wide_ok ? 1 : 0); ++form) {       // blocks of rows; the last one: wide
+        const bool wide = form > max_blocks;
+        const int row_blocks = wide ? 1 : form;
+        for (int w = kPlaneWaves; w >= (wide ? 12 : 4); --w) {
+            const long long rows = (long long)(wide ? 2 : row_blocks) * w * rows_per_wave;
             const long long blocks = planes * ((rows_per_plane + rows - 1) / rows);
-            const long long cost = ((blocks + cus - 1) / cus) * ((long long)rb * w * P + 64);
-            if (best_cost < 0 || cost < best_cost) { best_cost = cost; *waves = w; *row_blocks = rb; }
+            const long long cost = ((blocks + cus - 1) / cus) * ((long long)(wide ? 8 : 5 * row_blocks) * w * P + 5 * 64);
+            if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = PlaneConfig{w, row_blocks, wide}; }
         }
     }
+    return best;
 }
 
 struct PlaneBlock {
@@ -269,6 +275,48 @@ __device__ __forceinline__ int stage_slot_descriptors(const float4 *__restrict__
     return desc_g ? __float_as_int(gw.z) : sample_of(n, c);
 }
 
+// A lane's DC elements of a row. fp32 with eight elements and at most eight lanes a row: two pieces of 16 bytes half a row
+// apart, in an order that alternates every two slots, so that the four quarters of the banks -- which half of the bank line the
+// row lies in alternates with the slot already -- serve eight rows of 64 bytes evenly (a lane's eight elements side by side
+// would leave every other 16 bytes of the banks idle). Else DC elements in a row.
+template <typename S, int D, int DC> struct PlaneLane {
+    static constexpr bool kSplit = S::kBytes == 4 && DC == 8 && D <= 64;
+    static constexpr unsigned kHalf = kSplit ? D * S::kBytes / 2 : 0u;
+    static __device__ __forceinline__ unsigned first(int g, int slot)        // byte offset in the row of the lane's first piece
+    {
+        return kSplit ? 16u * g + ((slot & 2) ? kHalf : 0u) : (unsigned)(g * DC * S::kBytes);
+    }
+    // from the image: `a` is an LDS address in the first row of a pixel's two, `off` a whole number of rows
+    static __device__ __forceinline__ void read(uint32_t a, uint32_t off, float (&x)[DC])
+    {
+        if constexpr (kSplit) {
+            load_chunk<S, 4>(lds_at(a) + off, *reinterpret_cast<float (*)[4]>(&x[0]));
+            load_chunk<S, 4>(lds_at(a ^ kHalf) + off, *reinterpret_cast<float (*)[4]>(&x[4]));
+        } else {
+            load_chunk<S, DC>(lds_at(a) + off, x);
+        }
+    }
+    // from and to memory: `row` the row, `off` the lane's first()
+    static __device__ __forceinline__ void load(const char *row, unsigned off, float (&x)[DC])
+    {
+        if constexpr (kSplit) {
+            load_chunk<S, 4>(row + off, *reinterpret_cast<float (*)[4]>(&x[0]));
+            load_chunk<S, 4>(row + (off ^ kHalf), *reinterpret_cast<float (*)[4]>(&x[4]));
+        } else {
+            load_chunk<S, DC>(row + off, x);
+        }
+    }
+    static __device__ __forceinline__ void store(char *row, unsigned off, const float (&x)[DC])
+    {
+        if constexpr (kSplit) {
+            store_chunk<S, 4>(row + off, *reinterpret_cast<const float (*)[4]>(&x[0]));
+            store_chunk<S, 4>(row + (off ^ kHalf), *reinterpret_cast<const float (*)[4]>(&x[4]));
+        } else {
+            store_chunk<S, DC>(row + off, x);
+        }
+    }
+};
+
 // ROWS: query-row blocks per workgroup. With two, a workgroup of W waves covers 2*W*NS rows: every staged plane is
 // worked on for the first W*NS rows and then for the second, so a launch of several rounds of workgroups stages
 // half as often (at 12 views x 12 samples per view the staging is a third of a workgroup's time).
@@ -292,7 +340,9 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
     const int rows_block = (int)(blockDim.x >> 6) * NS;                       // (workgroups of up to kPlaneWaves waves)
     const PlaneBlock pb = decode_plane_block(dm, ROWS * rows_block);
     const int nq = dm.V * dm.L;
-    const int g = lane % G, slot = lane / G, lane_elem = g * DC, lane_byte = lane_elem * S::kBytes;
+    using Lane = PlaneLane<S, D, DC>;
+    const int g = lane % G, slot = lane / G;
+    const unsigned lane_byte = Lane::first(g, slot);
     const float qscale = dm.sm_scale * kLog2e;
     const uint32_t lbase = lds_offset(smem) + lane_byte;
 
@@ -312,9 +362,9 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
         row_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l;
         crow_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.L + l) * (size_t)dm.N;
         if constexpr (kPacked) {
-            load_packed<S, DC>((const char *)q_ + (dm.q_row(pb.b, (int)s1, pb.h, (int)l) + lane_elem) * S::kBytes, qp_s[rb]);
+            load_packed<S, DC>((const char *)q_ + dm.q_row(pb.b, (int)s1, pb.h, (int)l) * S::kBytes + lane_byte, qp_s[rb]);
         } else {
-            load_chunk<S, DC>((const char *)q_ + (dm.q_row(pb.b, (int)s1, pb.h, (int)l) + lane_elem) * S::kBytes, qf_s[rb]);
+            Lane::load((const char *)q_ + dm.q_row(pb.b, (int)s1, pb.h, (int)l) * S::kBytes, lane_byte, qf_s[rb]);
 #pragma unroll
             for (int d = 0; d < DC; ++d) qf_s[rb][d] *= qscale;
         }
@@ -356,17 +406,15 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
                     const int2 e = s_e[slot * (G + 1) + t];
                     const uint32_t at = e.x + lbase, ab = e.y + lbase;
                     if constexpr (kKeep) { wt[t] = w; att[t] = at; abt[t] = ab; }
-                    const unsigned char *top = lds_at(at), *bot = lds_at(ab);
-                    const unsigned char *topr = lds_at((at ^ kRow) + 2 * kRow), *botr = lds_at((ab ^ kRow) + 2 * kRow);
                     float dot = 0.f;
                     if constexpr (kPacked) {
-                        dot = qscale * tap_dot16<S, DC>(top, topr, bot, botr, w, qp);
+                        dot = qscale * tap_dot16<S, DC>(lds_at(at), lds_at((at ^ kRow) + 2 * kRow), lds_at(ab), lds_at((ab ^ kRow) + 2 * kRow), w, qp);
                     } else {
                         float t0[DC], t1[DC], t2[DC], t3[DC];
-                        load_chunk<S, DC>(top, t0);
-                        load_chunk<S, DC>(topr, t1);
-                        load_chunk<S, DC>(bot, t2);
-                        load_chunk<S, DC>(botr, t3);
+                        Lane::read(at, 0, t0);
+                        Lane::read(at ^ kRow, 2 * kRow, t1);
+                        Lane::read(ab, 0, t2);
+                        Lane::read(ab ^ kRow, 2 * kRow, t3);
 #pragma unroll
                         for (int d = 0; d < DC; ++d) {
                             const float kk = fmaf(w.x, t0[d], fmaf(w.y, t1[d], fmaf(w.z, t2[d], w.w * t3[d])));
@@ -398,10 +446,10 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
                         at = e.x + lbase; ab = e.y + lbase;
                     }
                     float t0[DC], t1[DC], t2[DC], t3[DC];
-                    load_chunk<S, DC>(lds_at(at ^ kRow), t0);                  // V, left taps
-                    load_chunk<S, DC>(lds_at(at + 2 * kRow), t1);              // V, right taps
-                    load_chunk<S, DC>(lds_at(ab ^ kRow), t2);
-                    load_chunk<S, DC>(lds_at(ab + 2 * kRow), t3);
+                    Lane::read(at ^ kRow, 0, t0);                              // V, left taps
+                    Lane::read(at, 2 * kRow, t1);                              // V, right taps
+                    Lane::read(ab ^ kRow, 0, t2);
+                    Lane::read(ab, 2 * kRow, t3);
                     const float c0w = p * w.x, c1w = p * w.y, c2w = p * w.z, c3w = p * w.w;
 #pragma unroll
                     for (int d = 0; d < DC; ++d)
@@ -418,7 +466,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
             const float inv = 1.0f / lsum_s[rb];
 #pragma unroll
             for (int d = 0; d < DC; ++d) acc_s[rb][d] *= inv;
-            store_chunk<S, DC>((char *)out_ + (row_s[rb] * D + lane_elem) * S::kBytes, acc_s[rb]);
+            Lane::store((char *)out_ + row_s[rb] * (size_t)kRow, lane_byte, acc_s[rb]);
             if (g == 0) lse_[row_s[rb]] = m_s[rb] + __log2f(lsum_s[rb]);
         }
     }
@@ -456,7 +504,9 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
     const int rows_block = (int)(blockDim.x >> 6) * NS;                       // (workgroups of up to kPlaneWaves waves)
     const PlaneBlock pb = decode_plane_block(dm, ROWS * rows_block, bh0);
     const int nq = dm.V * dm.L;
-    const int g = lane % G, slot = lane / G, lane_elem = g * DC, lane_byte = lane_elem * S::kBytes;
+    using Lane = PlaneLane<S, D, DC>;
+    const int g = lane % G, slot = lane / G;
+    const unsigned lane_byte = Lane::first(g, slot);
     const float qscale = dm.sm_scale * kLog2e;
     const uint32_t lbase = lds_offset(smem) + lane_byte;
 
@@ -476,13 +526,13 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         const size_t row = (((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l;
         crow_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.L + l) * (size_t)dm.N;
         hrow_s[rb] = ((size_t)(pb.b * dm.H + pb.h - bh0) * nq + qc) * (size_t)dm.N;
-        const size_t roff = (row * D + lane_elem) * S::kBytes;
+        const size_t roff = row * (size_t)kRow;
         roff_s[rb] = roff;
         float of[DC];
-        load_chunk<S, DC>((const char *)q_ + (dm.q_row(pb.b, (int)s1, pb.h, (int)l) + lane_elem) * S::kBytes, qf_s[rb]);
-        load_chunk<S, DC>((const char *)dout_ + roff, dof_s[rb]);
-        if constexpr (kPacked) load_packed<S, DC>((const char *)dout_ + roff, dop_s[rb]);
-        load_chunk<S, DC>((const char *)out_ + roff, of);
+        Lane::load((const char *)q_ + dm.q_row(pb.b, (int)s1, pb.h, (int)l) * S::kBytes, lane_byte, qf_s[rb]);
+        Lane::load((const char *)dout_ + roff, lane_byte, dof_s[rb]);
+        if constexpr (kPacked) load_packed<S, DC>((const char *)dout_ + roff + lane_byte, dop_s[rb]);
+        Lane::load((const char *)out_ + roff, lane_byte, of);
         float dl = 0.f;
 #pragma unroll
         for (int d = 0; d < DC; ++d) { dl = fmaf(dof_s[rb][d], of[d], dl); dqa_s[rb][d] = 0.f; }
@@ -518,10 +568,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                 if constexpr (CG) {
                     const uint32_t inside = (uint32_t)e.x & 15u;
                     const uint32_t at = (uint32_t)e.x - inside + lbase, ab = e.y + lbase;
-                    const unsigned char *kp[4] = { lds_at(at), lds_at((at ^ kRow) + 2 * kRow), lds_at(ab),
-                                                   lds_at((ab ^ kRow) + 2 * kRow) };
-                    const unsigned char *vp[4] = { lds_at(at ^ kRow), lds_at(at + 2 * kRow), lds_at(ab ^ kRow),
-                                                   lds_at(ab + 2 * kRow) };
+                    const uint32_t kp[4] = { at, at ^ kRow, ab, ab ^ kRow }, vp[4] = { at ^ kRow, at, ab ^ kRow, ab };
                     const float wt[4] = { w.x, w.y, w.z, w.w };
                     float kk[DC], dk_t[4], dv_t[4];
                     float dot = 0.f, dp = 0.f;
@@ -530,8 +577,8 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         float tk[DC], tv[DC];
-                        load_chunk<S, DC>(kp[i], tk);
-                        load_chunk<S, DC>(vp[i], tv);
+                        Lane::read(kp[i], (i & 1) * 2 * kRow, tk);
+                        Lane::read(vp[i], (i & 1) * 2 * kRow, tv);
                         dk_t[i] = 0.f;
                         dv_t[i] = 0.f;
 #pragma unroll
@@ -566,16 +613,15 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                     continue;
                 }
                 const uint32_t at = e.x + lbase, ab = e.y + lbase;
-                const unsigned char *top = lds_at(at), *bot = lds_at(ab);                      // K left; V right at +2*ROW
-                const unsigned char *topx = lds_at(at ^ kRow), *botx = lds_at(ab ^ kRow);      // V left; K right at +2*ROW
+                // at, ab: K left, and V right 2*ROW on; ^ ROW: V left, and K right 2*ROW on
                 float kk[DC];
                 float dot = 0.f, dp = 0.f;
                 {
                     float t0[DC], t1[DC], t2[DC], t3[DC];
-                    load_chunk<S, DC>(top, t0);
-                    load_chunk<S, DC>(topx + 2 * kRow, t1);
-                    load_chunk<S, DC>(bot, t2);
-                    load_chunk<S, DC>(botx + 2 * kRow, t3);
+                    Lane::read(at, 0, t0);
+                    Lane::read(at ^ kRow, 2 * kRow, t1);
+                    Lane::read(ab, 0, t2);
+                    Lane::read(ab ^ kRow, 2 * kRow, t3);
 #pragma unroll
                     for (int d = 0; d < DC; ++d) {
                         kk[d] = fmaf(w.x, t0[d], fmaf(w.y, t1[d], fmaf(w.z, t2[d], w.w * t3[d])));
@@ -583,13 +629,13 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                     }
                 }
                 if constexpr (kPacked) {
-                    dp = tap_dot16<S, DC>(topx, top + 2 * kRow, botx, bot + 2 * kRow, w, dop);
+                    dp = tap_dot16<S, DC>(lds_at(at ^ kRow), lds_at(at + 2 * kRow), lds_at(ab ^ kRow), lds_at(ab + 2 * kRow), w, dop);
                 } else {
                     float u0[DC], u1[DC], u2[DC], u3[DC];
-                    load_chunk<S, DC>(topx, u0);
-                    load_chunk<S, DC>(top + 2 * kRow, u1);
-                    load_chunk<S, DC>(botx, u2);
-                    load_chunk<S, DC>(bot + 2 * kRow, u3);
+                    Lane::read(at ^ kRow, 0, u0);
+                    Lane::read(at, 2 * kRow, u1);
+                    Lane::read(ab ^ kRow, 0, u2);
+                    Lane::read(ab, 2 * kRow, u3);
 #pragma unroll
                     for (int d = 0; d < DC; ++d) {
                         const float vv = fmaf(w.x, u0[d], fmaf(w.y, u1[d], fmaf(w.z, u2[d], w.w * u3[d])));
@@ -622,7 +668,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         if (have_s[rb]) {
 #pragma unroll
             for (int d = 0; d < DC; ++d) dqa_s[rb][d] *= dm.sm_scale;
-            store_chunk<S, DC>((char *)dq_ + roff_s[rb], dqa_s[rb]);
+            Lane::store((char *)dq_ + roff_s[rb], lane_byte, dqa_s[rb]);
         }
     }
 }
