@@ -370,6 +370,22 @@ __device__ __forceinline__ void load_tap_or_zero(const char *base, int pix, int 
     }
 }
 
+// Deterministic backward: the sorted ids as records, so that the dk/dv kernel finds the positions beside them there too (one
+// thread per list place; `total` = B*V*M, places beyond a group's lists are skipped).
+static __global__ __launch_bounds__(256) void records_kernel(const float *__restrict__ coords_, const unsigned *__restrict__ start,
+                                                             const unsigned *__restrict__ ids, unsigned *__restrict__ records,
+                                                             int NC, unsigned total, Dims dm)
+{
+    const unsigned M = (unsigned)dm.V * (unsigned)dm.L * (unsigned)dm.P;
+    const unsigned at = blockIdx.x * 256u + threadIdx.x;
+    const unsigned grp = at / M, i = at - grp * M;                                   // (b, s2), place
+    if (at >= total || i >= start[(size_t)grp * (NC + 1) + NC]) return;
+    const unsigned b = grp / (unsigned)dm.V, s2 = grp - b * (unsigned)dm.V;
+    const unsigned id = ids[at], ql = dm.divP.div(id), p = id - ql * (unsigned)dm.P;
+    const float2 xy = reinterpret_cast<const float2 *>(coords_)[((size_t)b * dm.V * dm.L + ql) * dm.N + s2 * (unsigned)dm.P + p];
+    store_cell_entry(records, at, id, cell_fraction(xy, dm), 1);
+}
+
 // A lane's part of one query row as it comes from memory: q and dout words (storage type), and the row's
 // (lse, delta) pair.
 template <int WORDS> struct RowFetch { uint32_t qw[WORDS], dw[WORDS]; float2 ld; };
@@ -377,34 +393,37 @@ template <int WORDS> struct RowFetch { uint32_t qw[WORDS], dw[WORDS]; float2 ld;
 // Which cells one launch of the dk/dv kernel covers, and the divisors that decode a work index into
 // (b, h, s2, cell) with multiply-shift instead of integer division (the decode is scalar code every
 // wave runs before it knows whether its cell is empty).
-// With RECORDS: all cells, by the work list that the binning made, work index -> (b, h, s2, item), `ncells` being the
-// list's capacity wmax per (b, s2) (empty slots leave at once) and ncx = Wimg + 1; per-cell sums are flushed with float
+// All cells by the work list that the binning made, work index -> (b, h, s2, item), `ncells` being the
+// list's capacity wmax per (b, s2) (empty slots leave at once); per-cell sums are flushed with float
 // atomics (a pixel belongs to four cells).
-// Without (deterministic backward): four launches, each for the cells (oy + 2i, ox + 2j) of one (row parity, column
-// parity); no two of them share a pixel, so the flush is a plain read-add-write, and the launches, one
-// after the other, add every pixel's four contributions in a fixed order.
+// FIXED (deterministic backward): every cell of the grid, one wave each and no pieces, and the sums are stored: a pixel's
+// four contributions come from four cells, as a different one of the four taps of each, so tap t of every cell has a
+// buffer of its own, [dk, dv][tap][plane][pixel][D], every place of which one wave writes (zeros from an empty list).
+// combine_taps_kernel then adds a pixel's four in a fixed order. (Four launches, each for the cells of one row and column parity
+// and with read-add-write into dk and dv, took 222 us at 18x18, 6 views x 32 samples, D = 32, where the one and the sums take 142: a quarter
+// of the cells are 8664 waves, a third of what the chip holds, four times.)
 struct CellGrid {
-    int oy, ox, step, ncx, ncells;
+    int ncells;
     int bh0;                                // first (batch, head) pair of this launch (b * H + h)
-    unsigned nwork;                         // pairs of this launch * V * ncells < 2^31
+    unsigned t0, nplanes;                   // deterministic: first plane (b, h, s2) of this launch, counted from pair bh0, and planes
+    unsigned nwork;                         // planes of this launch * ncells < 2^31
     FastDiv div_cells, div_ncx, div_v, div_h;
 };
 
 // HANDED: the dq kernel has left (p, sm_scale * ds) of every sample in `handed_` (per query row of this head,
 // in the order of the row's coordinates): an entry then costs a gather of that pair and the two rank-1 updates --
-// no taps in registers, no dot products, no exponential. Only with records (the positions beside the ids).
-// RECORDS: the lists hold 12-byte records (sample id and position in the cell), and the launch goes by the work
-// list; without, ids alone, and every entry's coordinate pair is read again (the deterministic backward,
-// whose lists are sorted id arrays, in its four colour launches).
+// no taps in registers, no dot products, no exponential.
+// The lists hold 12-byte records (sample id and position in the cell).
+// FIXED: the deterministic backward's launch (see CellGrid).
 // What an item costs beside its entries is about 300 vector instructions (bounds, taps, tables, the sum over the
 // slots, the flush), which is most of the kernel where lists are short: 18x18, D = 32, 2 views x 2 samples (3.6
 // entries a list, fp32) 43.0 -> 39.8 us, 6 x 6 (32 entries, bf16) 172 -> 161, 14x14 with 8 x 32 (223, fp32) 244.5 -> 241,
 // with the slots summed on a quarter of the values where the step that halves them comes first, and no tables made
 // for a block that is not there.
-template <typename S, int D, int DC, bool HANDED, bool RECORDS>
+template <typename S, int D, int DC, bool HANDED, bool FIXED>
 __device__ __forceinline__ void cell_sums(
     unsigned t, int ci, const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_,
-    const float *__restrict__ coords_, const float2 *__restrict__ stats_,
+    const float2 *__restrict__ stats_,
     const void *__restrict__ dout_, const unsigned *__restrict__ start, const unsigned *__restrict__ sorted,
     const uint4 *__restrict__ items, const float2 *__restrict__ handed_,
     float *__restrict__ dk_acc, float *__restrict__ dv_acc, const Dims &dm, int NC, const CellGrid &cg)
@@ -432,7 +451,7 @@ __device__ __forceinline__ void cell_sums(
     const size_t grp = (size_t)b * dm.V + s2;
     int cy, cx, cell;
     unsigned lo, hi;
-    if constexpr (RECORDS) {
+    if constexpr (!FIXED) {
         const uint4 item = items[grp * (size_t)cg.ncells + ci];              // (cell, first entry, end)
         cell = (int)item.x;
         cy = (int)cg.div_ncx.div(item.x);                      // div_ncx: by Wimg + 1 in this mode
@@ -440,19 +459,32 @@ __device__ __forceinline__ void cell_sums(
         lo = item.y;
         hi = item.z;
     } else {
-        const int cyi = (int)cg.div_ncx.div((unsigned)ci);
-        cy = cyi * cg.step + cg.oy;
-        cx = (ci - cyi * cg.ncx) * cg.step + cg.ox;            // on the (Himg+1) x (Wimg+1) grid
-        cell = cy * (dm.Wimg + 1) + cx;
+        cell = ci;
+        cy = (int)cg.div_ncx.div((unsigned)ci);
+        cx = ci - cy * (dm.Wimg + 1);                          // on the (Himg+1) x (Wimg+1) grid
         lo = start[grp * (NC + 1) + cell];
         hi = start[grp * (NC + 1) + cell + 1];
     }
-    if (lo >= hi) return;
+    if (!FIXED && lo >= hi) return;
 
     const int g = lane % G, slot = lane / G, lane_elem = g * DC;
     const int y0 = cy - 1, x0 = cx - 1;
     const bool vy0 = y0 >= 0, vy1 = y0 + 1 < dm.Himg, vx0 = x0 >= 0, vx1 = x0 + 1 < dm.Wimg;
     const bool tv[4] = { vy0 && vx0, vy0 && vx1, vy1 && vx0, vy1 && vx1 };
+    // where tap r of this cell goes (deterministic backward), `which` 0: dk, 1: dv; its pixel has to be inside the image
+    auto tap_place = [&](int which, int r, int pix) -> float * {
+        return (which == 0 ? dk_acc : dv_acc) + (((size_t)r * cg.nplanes + (t - cg.t0)) * dm.L + pix) * (size_t)D;
+    };
+    if constexpr (FIXED) {
+        if (lo >= hi) {
+            for (int idx = lane; idx < 8 * D; idx += kWave) {
+                const int r = (idx / D) & 3;
+                if (((r & 2) ? vy1 : vy0) && ((r & 1) ? vx1 : vx0))
+                    tap_place(idx / (4 * D), r, (y0 + (r >> 1)) * dm.Wimg + x0 + (r & 1))[idx & (D - 1)] = 0.f;
+            }
+            return;
+        }
+    }
     const int tpix[4] = { y0 * dm.Wimg + x0, y0 * dm.Wimg + x0 + 1, (y0 + 1) * dm.Wimg + x0,
                           (y0 + 1) * dm.Wimg + x0 + 1 };
     const size_t plane_base = ((grp * dm.H) + h) * (size_t)dm.L * D;          // elements in dk/dv; grp = b*V + s2
@@ -507,8 +539,7 @@ __device__ __forceinline__ void cell_sums(
     }
     const float qscale = dm.sm_scale * kLog2e;
     const size_t M = (size_t)dm.V * dm.L * dm.P;
-    static_assert(RECORDS || !HANDED, "the pairs are handed over to lists of records only");
-    const unsigned *list = sorted + grp * M * (RECORDS ? 3u : 1u);      // ids, or 12-byte records (id, fx, fy)
+    const unsigned *list = sorted + grp * M * 3u;                       // records (id, fx, fy)
     // Query rows of this wave's (b, h) are addressed as a uniform base plus a 32-bit byte offset
     // (s1*H*L + l) * ROW < V*H*L*D*e <= 2^32 (the shape limits keep one batch item of a tensor below 2^30
     // elements): one add per gather instead of 64-bit address arithmetic per lane.
@@ -521,7 +552,6 @@ __device__ __forceinline__ void cell_sums(
     const char *stats_bh = (const char *)(stats_ + bh_row0);                 // (lse, delta) per row
     const unsigned lane_byte = (unsigned)lane_elem * S::kBytes;
     const unsigned view_rows = (unsigned)dm.H * (unsigned)dm.L;
-    const float2 *coords = reinterpret_cast<const float2 *>(coords_);
 
     // HANDED: the entry's pair, gathered one chunk ahead (so the ids are fetched two chunks ahead). The pairs of
     // this launch's (batch, head) pairs lie as [pair][s1][l][sample]; those of this wave's pair are a uniform base
@@ -688,25 +718,15 @@ __device__ __forceinline__ void cell_sums(
         // younger requests instead of "everything" (a request under a branch, or a loop that may run zero times,
         // makes the wait at the join a wait for all outstanding loads, which undoes the overlap).
         auto load_entry_c = [&](unsigned cstart) -> CellEntry {
-            const unsigned at = min(cstart + (unsigned)lane, hi - 1u);
-            if constexpr (RECORDS) {
-                const unsigned *r = list + 3u * at;
-                return CellEntry{r[0], __uint_as_float(r[1]), __uint_as_float(r[2])};
-            } else {
-                return CellEntry{list[at], 0.f, 0.f};
-            }
+            const unsigned *r = list + 3u * min(cstart + (unsigned)lane, hi - 1u);
+            return CellEntry{r[0], __uint_as_float(r[1]), __uint_as_float(r[2])};
         };
         auto tables = [&](unsigned cstart, int buf, const CellEntry &e, const float2 &pdv) {
-            const unsigned ql = dm.divP.div(e.id), p = e.id - ql * (unsigned)dm.P;     // ql = s1*L + l
+            const unsigned ql = dm.divP.div(e.id);                     // ql = s1*L + l
             const unsigned s1 = dm.divL.div(ql), l = ql - s1 * (unsigned)dm.L;
-            float2 ff = make_float2(e.fx, e.fy);
-            if constexpr (!RECORDS) {
-                const size_t ci = (((size_t)b * dm.V * dm.L + ql) * dm.V + s2) * (size_t)dm.P + p;
-                ff = cell_fraction(coords[ci], dm);
-            }
             // Plain bilinear weights, not masked: every sample of this list lies in this cell, whose taps
             // outside the image were loaded as zeros above and are skipped by the flush below.
-            const float fx = ff.x, fy = ff.y;
+            const float fx = e.fx, fy = e.fy;
             const float gx = 1.0f - fx, gy = 1.0f - fy;
             const bool live = cstart + (unsigned)lane < hi;           // a dead entry adds nothing
             const int at = buf * kWave + lane;
@@ -821,9 +841,8 @@ __device__ __forceinline__ void cell_sums(
                 e_c = load_entry_c(c0 + 2 * kWave);
             }
             __builtin_amdgcn_sched_barrier(0);         // (requested here, not where they are used)
-            // (a list of one block, the common case where lists are short, makes no second set of tables; plain ids
-            // bring their coordinate reads along, which may not sit under a branch)
-            if (has_next || !RECORDS) {
+            // (a list of one block, the common case where lists are short, makes no second set of tables)
+            if (has_next) {
                 wave_lds_sync();
                 tables(c0 + kWave, cur ^ 1, e_a, pd_a);
                 wave_lds_sync();
@@ -932,21 +951,20 @@ __device__ __forceinline__ void cell_sums(
             const int pix = (y0 + (r >> 1)) * dm.Wimg + x0 + (r & 1);
             const float val = fl[idx];
             if (ok) {
-                float *pa = acc + (size_t)pix * D + dd;
-                if constexpr (RECORDS) atomicAdd(pa, val);
-                else *pa += val;
+                if constexpr (FIXED) tap_place(which, r, pix)[dd] = val;
+                else atomicAdd(acc + (size_t)pix * D + dd, val);
             }
         }
     }
 }
 
 #define DSDPA_CELL_ARGS                                                                                                    \
-    const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_, const float *__restrict__ coords_, \
+    const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_,                                 \
     const float2 *__restrict__ stats_, const void *__restrict__ dout_, const unsigned *__restrict__ start,                  \
     const unsigned *__restrict__ sorted, const uint4 *__restrict__ items, const float2 *__restrict__ handed_,               \
     float *__restrict__ dk_acc, float *__restrict__ dv_acc, Dims dm, int NC, CellGrid cg
 
-template <typename S, int D, int DC, bool HANDED, bool RECORDS>
+template <typename S, int D, int DC, bool HANDED, bool FIXED>
 __global__ __launch_bounds__(kCellWaves *kWave, HANDED ? (DC <= 4 ? 5 : (S::kBytes == 2 ? 3 : 4))
                                                        : DC <= 4 ? (S::kBytes == 2 && D >= 64 ? 5 : 4) : (S::kBytes == 2 ? 3 : 2))
 void bwd_dkdv_cell_kernel(DSDPA_CELL_ARGS)
@@ -954,8 +972,35 @@ void bwd_dkdv_cell_kernel(DSDPA_CELL_ARGS)
     const unsigned work = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x) * kCellWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (work >= cg.nwork) return;
     const unsigned t = cg.div_cells.div(work);                 // plane-major
-    cell_sums<S, D, DC, HANDED, RECORDS>(t, (int)(work - t * (unsigned)cg.ncells), q_, k_, v_, coords_, stats_, dout_, start, sorted,
-                                         items, handed_, dk_acc, dv_acc, dm, NC, cg);
+    cell_sums<S, D, DC, HANDED, FIXED>(t + cg.t0, (int)(work - t * (unsigned)cg.ncells), q_, k_, v_, stats_, dout_, start, sorted,
+                                       items, handed_, dk_acc, dv_acc, dm, NC, cg);
+}
+
+// dk and dv of the planes [t0, t0 + nplanes) of the (batch, head, key view) order from the four taps' sums of the deterministic
+// backward, in the order 00 + 01, 10 + 11, their sum. VE elements (16 bytes of the storage type) a thread. Bound by the
+// eight floats read per element of dk and dv.
+template <typename S, int D>
+__global__ __launch_bounds__(256) void combine_taps_kernel(const float *__restrict__ dk_taps, const float *__restrict__ dv_taps,
+                                                           void *__restrict__ dk_, void *__restrict__ dv_, Dims dm, CellGrid cg)
+{
+    constexpr int VE = S::kBytes == 4 ? 4 : 8;
+    const unsigned per = (unsigned)dm.L * (D / VE);                          // threads per plane
+    const unsigned at = blockIdx.x * 256u + threadIdx.x, t = blockIdx.y;     // of the plane t of this launch
+    if (at >= per) return;
+    const unsigned bhl = cg.div_v.div(t + cg.t0), s2 = t + cg.t0 - bhl * (unsigned)dm.V, bh = (unsigned)cg.bh0 + bhl;
+    const unsigned b = cg.div_h.div(bh), h = bh - b * (unsigned)dm.H;
+    const size_t dst = (((size_t)b * dm.V + s2) * dm.H + h) * dm.L * D + (size_t)at * VE;
+    const size_t tap = (size_t)cg.nplanes * dm.L * D;
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+        const float *src = (which == 0 ? dk_taps : dv_taps) + (size_t)t * dm.L * D + (size_t)at * VE;
+        float x[4][VE];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) load_chunk<F32, VE>(src + r * tap, x[r]);
+#pragma unroll
+        for (int d = 0; d < VE; ++d) x[0][d] = (x[0][d] + x[1][d]) + (x[2][d] + x[3][d]);
+        store_chunk<S, VE>((char *)(which == 0 ? dk_ : dv_) + dst * S::kBytes, x[0]);
+    }
 }
 
 // The planes that the patch kernel has left: a loop over their work lists, at once over where there are none. left[grp]:
@@ -974,7 +1019,7 @@ __global__ __launch_bounds__(kCellWaves *kWave) void bwd_dkdv_cell_rest_kernel(c
         const unsigned t = i / most, ci = i - t * most;
         const unsigned bhl = cg.div_v.div(t), b = cg.div_h.div((unsigned)cg.bh0 + bhl);
         if (ci < left[b * (unsigned)dm.V + t - bhl * (unsigned)dm.V])
-            cell_sums<S, D, DC, true, true>(t, (int)ci, q_, k_, v_, coords_, stats_, dout_, start, sorted, items, handed_, dk_acc, dv_acc,
+            cell_sums<S, D, DC, true, false>(t, (int)ci, q_, k_, v_, stats_, dout_, start, sorted, items, handed_, dk_acc, dv_acc,
                                             dm, NC, cg);
     }
 }

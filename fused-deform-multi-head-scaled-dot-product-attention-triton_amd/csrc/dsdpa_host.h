@@ -219,7 +219,7 @@ inline bool slab_path_fits(size_t V, size_t Himg, size_t Wimg, size_t D, size_t 
 //   start    B*V*(NC+1) u32                  exclusive scan of the counts
 //   sorted   B*V*(V*L*P) u32                 the cell lists: 12-byte records (sample id, its position (fx, fy) in the
 //   frac     B*V*(V*L*P) x 8 bytes           cell) that run from `sorted` on through `frac`, which follows it; the
-//                                            deterministic backward keeps plain ids in `sorted` (and sorts them)
+//                                            deterministic backward sorts plain ids first
 //   items    B*V*wmax x 16 bytes             work list of the dk/dv kernel: (cell, first entry, end) per item
 //   handed   bhg*V*L*(V*P) x 8 bytes         (p, sm_scale*ds) per query*sample of one GROUP of bhg (batch, head) pairs,
 //                                            dq kernel -> dk/dv kernel (shapes on the gather kernels, and short lists);
@@ -231,6 +231,7 @@ inline bool slab_path_fits(size_t V, size_t Himg, size_t Wimg, size_t D, size_t 
 //   sorted2  as sorted                       the lists with every cell's ids in ascending order
 //   seg      2*B*V*NC u32                    begin / end of every list in the flat id array
 //   sorttmp  sort_temp_bytes()               scratch of the segmented sort
+//   taps     8 * L * D floats per plane      the sums of every cell's four taps, of dk and of dv, of a group of planes (b, h, s2)
 // with NC = (Himg+1)*(Wimg+1) cells.
 size_t sort_temp_bytes(size_t n, size_t segments);                       // dsdpa_sort.hip
 int sort_cell_lists(void *temp, size_t temp_bytes, const unsigned *ids_in, unsigned *ids_out, size_t n,
@@ -238,7 +239,8 @@ int sort_cell_lists(void *temp, size_t temp_bytes, const unsigned *ids_in, unsig
                     hipStream_t st);
 
 struct WorkspaceLayout {
-    size_t delta, counters, start, sorted, frac, items, handed, handed_bytes, acc, desc, sorted2, seg, sorttmp, sorttmp_bytes, total;
+    size_t delta, counters, start, sorted, frac, items, handed, handed_bytes, acc, desc, sorted2, seg, sorttmp, sorttmp_bytes, taps, total;
+    int tap_planes;             // planes (b, h, s2) whose taps the buffer of the deterministic backward holds at a time
     int bh_group;               // (batch, head) pairs whose pairs the handed buffer holds at a time; 0: nothing is handed over
     bool patch;                 // dk/dv by patches where the lists are short (DSDPA_PATH_AUTO)
     unsigned spread_mean;       // ... up to so many entries a non-empty list on average
@@ -290,9 +292,11 @@ inline int views_per_group(size_t V, size_t L, size_t D, size_t esize, size_t P,
 // group, the cell lists being shared by all heads -- and the buffer holds one group's pairs: at most
 // kHandedCapBytes, which also stay in the memory-side cache between the two kernels. Returns the (batch, head)
 // pairs per group, 0 when nothing is handed over: one pair's samples beyond the cap or beyond 32-bit byte offsets. Not asked
-// for by the deterministic backward (its four colour launches recompute) nor by shapes on the staged kernels (dq and
-// dk/dv run side by side there), short lists apart.
+// for by shapes on the staged kernels (dq and dk/dv run side by side there), short lists apart.
 constexpr size_t kHandedCapBytes = (size_t)128 << 20;
+// The deterministic backward's taps (8 floats per element of dk): a launch covers the planes whose taps fit, and ends with its
+// longest list.
+constexpr size_t kTapsCapBytes = (size_t)256 << 20;
 inline int handed_group(size_t B, size_t V, size_t H, size_t L, size_t P)
 {
     const size_t per_bh = V * L * (V * P) * 8;
@@ -329,7 +333,7 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
     const size_t L = Himg * Wimg, esize = storage16 ? 2 : 4, acc_bytes = storage16 ? round256(2 * rows * D * 4) : 0;
     const bool planes = plane_path_fits(L, D, esize);
     w.patch = patch_path(B, V, H, Himg, Wimg, P, esize, deterministic);
-    w.bh_group = (planes || deterministic) && !w.patch ? 0 : handed_group(B, V, H, L, P);
+    w.bh_group = planes && !w.patch ? 0 : handed_group(B, V, H, L, P);
     w.patch = w.patch && w.bh_group > 0;
     w.spread_mean = spread_mean(esize);
     const bool grouped = w.bh_group > 0 && !planes && !deterministic;
@@ -351,7 +355,8 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
     // gather kernel and no table is needed
     w.dl = desc_layout(B, V, Himg, Wimg, D, P, storage16 ? 2 : 4, coords_grad);
     w.desc = off; off += w.dl.bytes;
-    w.sorted2 = w.seg = w.sorttmp = off;
+    w.sorted2 = w.seg = w.sorttmp = w.taps = off;
+    w.tap_planes = 0;
     w.sorttmp_bytes = 0;
     if (deterministic) {
         const size_t ids = B * V * (V * Himg * Wimg * P), segs = B * V * (size_t)w.NC;
@@ -359,6 +364,21 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
         w.seg = off; off += round256(2 * segs * 4);
         w.sorttmp_bytes = round256(sort_temp_bytes(ids, segs));
         w.sorttmp = off; off += w.sorttmp_bytes;
+        // dk and dv as four taps each: groups of equal size, at most kTapsCapBytes or one plane, in the place of the
+        // accumulators, which this backward does not use, as far as that goes
+        const size_t per = 8 * L * D * 4, planes_all = B * H * V;
+        size_t g = kTapsCapBytes / per;
+        g = g < 1 ? 1 : g > planes_all ? planes_all : g;
+        g = g > 32768 ? 32768 : g;                          // (a dimension of the grid)
+        const size_t ngroups = (planes_all + g - 1) / g;
+        w.tap_planes = (int)((planes_all + ngroups - 1) / ngroups);
+        const size_t taps_bytes = round256((size_t)w.tap_planes * per);
+        if (taps_bytes <= acc_bytes) {
+            w.taps = w.acc;
+        } else {
+            w.taps = off;
+            off += taps_bytes;
+        }
     }
     w.total = off;
     return w;

@@ -684,48 +684,62 @@ static inline int launch_binning(const float *coords, const Dims &dm, const Work
     return check_launch();
 }
 
-// deterministic: lists of plain ids, four launches, one per (row parity, column parity) of the cells, each with plain
-// stores; else records, by the work list
+// The cells of `planes` planes (b, h, s2) from the t0-th of pair bh0 on, `ncells` of them (or slots of the work list) each.
+static inline int make_cell_grid(const Dims &dm, int ncells, int bh0, long long t0, long long planes, CellGrid *cg)
+{
+    const long long nwork = planes * ncells;
+    if (nwork >= 0x7fffffffll - 65536) return DSDPA_ERR_TOO_LARGE;
+    cg->ncells = ncells;
+    cg->bh0 = bh0;
+    cg->t0 = (unsigned)t0;
+    cg->nplanes = (unsigned)planes;
+    cg->nwork = (unsigned)nwork;
+    cg->div_cells = FastDiv::make((unsigned)ncells);
+    cg->div_ncx = FastDiv::make((unsigned)dm.Wimg + 1);
+    cg->div_v = FastDiv::make((unsigned)dm.V);
+    cg->div_h = FastDiv::make((unsigned)dm.H);
+    return DSDPA_OK;
+}
+
+// dk/dv by cells, lists of records and the work list; sums added to the accumulators
 template <typename S, int D>
-int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const float *coords,
-                         const float2 *stats, const void *dout, const unsigned *start, const unsigned *sorted,
+int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const float2 *stats, const void *dout, const unsigned *start, const unsigned *sorted,
                          const uint4 *items, unsigned wmax, const float2 *handed,
-                         float *dk_acc, float *dv_acc, const Dims &dm, int NC, bool deterministic, int bh0, int nbh,
-                         hipStream_t st)
+                         float *dk_acc, float *dv_acc, const Dims &dm, int NC, int bh0, int nbh, hipStream_t st)
 {
     constexpr int DC = CellChunk<S, D>::value;
+    CellGrid cg;
+    if (int rc = make_cell_grid(dm, (int)wmax, bh0, 0, (long long)nbh * dm.V, &cg)) return rc;
+    const unsigned blocks = (cg.nwork + kCellWaves - 1) / kCellWaves;
+    auto kern = handed ? bwd_dkdv_cell_kernel<S, D, DC, true, false> : bwd_dkdv_cell_kernel<S, D, DC, false, false>;
     ScopedKernelTimer timer(1, st);
-    for (int colour = deterministic ? 0 : -1; colour < (deterministic ? 4 : 0); ++colour) {
-        const int cw = dm.Wimg + 1, ch = dm.Himg + 1;
+    DSDPA_LAUNCH(kern, dim3(blocks), dim3(kCellWaves * kWave), 0, st, timer.start(), timer.stop(), q, k, v, stats, dout, start,
+                 sorted, items, handed, dk_acc, dv_acc, dm, NC, cg);
+    return check_launch();
+}
+
+// dk/dv by cells, deterministic: lists in a fixed order, the sums of every cell's four taps stored and then added pixel by
+// pixel; as many planes of the (batch, head) pairs [bh0, bh0 + nbh) at a time as the taps' buffer holds
+template <typename S, int D>
+int launch_bwd_dkdv_fixed(const void *q, const void *k, const void *v, const float2 *stats, const void *dout, const unsigned *start,
+                          const unsigned *sorted, const float2 *handed, float *taps, int tap_planes, void *dk, void *dv,
+                          const Dims &dm, int NC, int bh0, int nbh, hipStream_t st)
+{
+    constexpr int DC = CellChunk<S, D>::value;
+    const long long all = (long long)nbh * dm.V;
+    const unsigned blocks = (unsigned)(((size_t)dm.L * D * S::kBytes / 16 + 255) / 256);
+    auto kern = handed ? bwd_dkdv_cell_kernel<S, D, DC, true, true> : bwd_dkdv_cell_kernel<S, D, DC, false, true>;
+    ScopedKernelTimer timer(1, st);
+    for (long long t0 = 0; t0 < all; t0 += tap_planes) {
+        const long long planes = all - t0 < tap_planes ? all - t0 : tap_planes;
         CellGrid cg;
-        cg.oy = colour < 0 ? 0 : colour >> 1;
-        cg.ox = colour < 0 ? 0 : colour & 1;
-        cg.step = colour < 0 ? 1 : 2;
-        cg.ncx = (cw - cg.ox + cg.step - 1) / cg.step;
-        cg.ncells = cg.ncx * ((ch - cg.oy + cg.step - 1) / cg.step);
-        if (colour < 0) cg.ncells = (int)wmax;          // work-list mode: one wave per item slot
-        const long long nwork = (long long)nbh * dm.V * cg.ncells;       // the pairs [bh0, bh0 + nbh) of (batch, head)
-        if (nwork >= 0x7fffffffll - kCellWaves) return DSDPA_ERR_TOO_LARGE;
-        cg.bh0 = bh0;
-        cg.nwork = (unsigned)nwork;
-        cg.div_cells = FastDiv::make((unsigned)cg.ncells);
-        cg.div_ncx = FastDiv::make((unsigned)cg.ncx);
-        cg.div_v = FastDiv::make((unsigned)dm.V);
-        cg.div_h = FastDiv::make((unsigned)dm.H);
-        const unsigned blocks = (unsigned)((nwork + kCellWaves - 1) / kCellWaves);
-        const bool first = colour <= 0, last = colour < 0 || colour == 3;
-        if (handed && !deterministic)
-            DSDPA_LAUNCH((bwd_dkdv_cell_kernel<S, D, DC, true, true>), dim3(blocks), dim3(kCellWaves * kWave), 0, st,
-                                  first ? timer.start() : nullptr, last ? timer.stop() : nullptr, q, k, v, coords,
-                                  stats, dout, start, sorted, items, handed, dk_acc, dv_acc, dm, NC, cg);
-        else if (!deterministic)
-            DSDPA_LAUNCH((bwd_dkdv_cell_kernel<S, D, DC, false, true>), dim3(blocks), dim3(kCellWaves * kWave), 0, st,
-                                  first ? timer.start() : nullptr, last ? timer.stop() : nullptr, q, k, v, coords,
-                                  stats, dout, start, sorted, items, handed, dk_acc, dv_acc, dm, NC, cg);
-        else
-            DSDPA_LAUNCH((bwd_dkdv_cell_kernel<S, D, DC, false, false>), dim3(blocks), dim3(kCellWaves * kWave), 0, st,
-                                  first ? timer.start() : nullptr, last ? timer.stop() : nullptr, q, k, v, coords,
-                                  stats, dout, start, sorted, items, handed, dk_acc, dv_acc, dm, NC, cg);
+        if (int rc = make_cell_grid(dm, NC, bh0, t0, planes, &cg)) return rc;
+        float *dv_taps = taps + 4 * (size_t)planes * dm.L * D;
+        DSDPA_LAUNCH(kern, dim3((cg.nwork + kCellWaves - 1) / kCellWaves), dim3(kCellWaves * kWave), 0, st,
+                     t0 == 0 ? timer.start() : nullptr, nullptr, q, k, v, stats, dout, start, sorted, (const uint4 *)nullptr, handed,
+                     taps, dv_taps, dm, NC, cg);
+        DSDPA_LAUNCH((combine_taps_kernel<S, D>), dim3(blocks, (unsigned)planes), dim3(256), 0, st, nullptr,
+                     t0 + planes == all ? timer.stop() : nullptr, taps, dv_taps, dk, dv, dm, cg);
     }
     return check_launch();
 }
@@ -734,8 +748,8 @@ int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const floa
 // the cell kernel for the planes whose lists are not the patches'.
 // left (may be null: all planes are the patches'): see bwd_dkdv_cell_rest_kernel.
 template <typename S, int D>
-int launch_bwd_dkdv_patch(const void *q, const void *k, const void *v, const float *coords, const void *dout,
-                          const unsigned *start, const unsigned *sorted, const uint4 *items, unsigned wmax,
+int launch_bwd_dkdv_patch(const void *q, const void *k, const void *v, const void *dout, const unsigned *start,
+                          const unsigned *sorted, const uint4 *items, unsigned wmax,
                           const unsigned *left, const float2 *handed, void *dk, void *dv, float *dk_acc, float *dv_acc,
                           const Dims &dm, int NC, int bh0, int nbh, hipStream_t st)
 {
@@ -755,32 +769,21 @@ int launch_bwd_dkdv_patch(const void *q, const void *k, const void *v, const flo
     // 97 / 85 / 79; without a second launch behind it, two for the patches that many samples may share)
     const int waves = visits <= 128 && left ? 1 : visits <= 1280 ? 2 : 4;
     CellGrid cg;
-    const long long nwork = (long long)nbh * dm.V * wmax;
-    if (nwork >= 0x7fffffffll - 65536) return DSDPA_ERR_TOO_LARGE;
-    cg.oy = cg.ox = 0;
-    cg.step = 1;
-    cg.ncx = dm.Wimg + 1;
-    cg.ncells = (int)wmax;
-    cg.bh0 = bh0;
-    cg.nwork = (unsigned)nwork;
-    cg.div_cells = FastDiv::make(wmax);
-    cg.div_ncx = FastDiv::make((unsigned)cg.ncx);
-    cg.div_v = pg.div_v;
-    cg.div_h = pg.div_h;
+    if (int rc = make_cell_grid(dm, (int)wmax, bh0, 0, (long long)nbh * dm.V, &cg)) return rc;
     const unsigned rest = 32u * (unsigned)device_cus();
     ScopedKernelTimer timer(1, st);
     DSDPA_LAUNCH((bwd_dkdv_patch_kernel<S, D, DP>), dim3((unsigned)blocks, D / DP), dim3(waves * kWave), patch_lds_bytes(waves), st,
                  timer.start(), left ? nullptr : timer.stop(), q, dout, start, sorted, left, handed, dk, dv, dk_acc, dv_acc, dm, NC, pg);
     if (!left) return check_launch();
     DSDPA_LAUNCH((bwd_dkdv_cell_rest_kernel<S, D, CellChunk<S, D>::value>), dim3(rest), dim3(kCellWaves * kWave), 0, st, nullptr,
-                 timer.stop(), left, q, k, v, coords, (const float2 *)nullptr, dout, start, sorted, items, handed, dk_acc, dv_acc,
+                 timer.stop(), left, q, k, v, (const float2 *)nullptr, dout, start, sorted, items, handed, dk_acc, dv_acc,
                  dm, NC, cg);
     return check_launch();
 }
 
 // Deterministic backward: order every cell list by sample id (the counting sort leaves the order inside a
-// cell to its atomics).
-static inline int launch_list_ordering(const Dims &dm, const WorkspaceLayout &wl, char *ws, hipStream_t st)
+// cell to its atomics), and make the ids records.
+static inline int launch_list_ordering(const float *coords, const Dims &dm, const WorkspaceLayout &wl, char *ws, hipStream_t st)
 {
     const size_t M = (size_t)dm.V * dm.L * dm.P, groups = (size_t)dm.B * dm.V;
     const size_t ids = groups * M, segs = groups * (size_t)wl.NC;
@@ -793,8 +796,12 @@ static inline int launch_list_ordering(const Dims &dm, const WorkspaceLayout &wl
     if (rc != DSDPA_OK) return rc;
     unsigned bits = 1;
     while (bits < 32 && (1ull << bits) < M) ++bits;
-    return sort_cell_lists(ws + wl.sorttmp, wl.sorttmp_bytes, (const unsigned *)(ws + wl.sorted),
-                           (unsigned *)(ws + wl.sorted2), ids, segs, seg_begin, seg_end, bits, st);
+    rc = sort_cell_lists(ws + wl.sorttmp, wl.sorttmp_bytes, (const unsigned *)(ws + wl.sorted),
+                         (unsigned *)(ws + wl.sorted2), ids, segs, seg_begin, seg_end, bits, st);
+    if (rc != DSDPA_OK) return rc;
+    hipLaunchKernelGGL(records_kernel, dim3((unsigned)((ids + 255) / 256)), dim3(256), 0, st, coords, (const unsigned *)(ws + wl.start),
+                       (const unsigned *)(ws + wl.sorted2), (unsigned *)(ws + wl.sorted), wl.NC, (unsigned)ids, dm);
+    return check_launch();
 }
 
 // Joins the backward's side lane to the caller's stream, once: by join() on the normal path, by the
@@ -853,8 +860,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     const uint32_t *desc_e = (const uint32_t *)(ws + wl.desc + wl.dl.e);
     const float4 *desc_g = (const float4 *)(ws + wl.desc + wl.dl.g);
     const unsigned *start = (const unsigned *)(ws + wl.start);
-    const unsigned *sorted = (const unsigned *)(ws + (deterministic ? wl.sorted2 : wl.sorted));
-    // (the reordered lists of the deterministic backward are ids without positions beside them: coordinates are read again)
+    const unsigned *sorted = (const unsigned *)(ws + wl.sorted);
     // (p, sm_scale * ds) per query*sample from the dq kernel to the dk/dv kernel, where the layout has room for it
     // (shapes on the gather dq kernel, which then runs before dk/dv on the same stream)
     const bool patch = wl.patch && path == DSDPA_PATH_AUTO;
@@ -891,7 +897,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     const size_t ndc = dcoords ? (size_t)dm.B * dm.V * dm.L * dm.N * 2 : 0;
     // what has to start at zero: on one stream everything in one job, which the tap-table launch (when
     // there is one) takes along; with the side lane the dk/dv side clears its own buffers there
-    const size_t nacc = patch ? 0 : n;                 // (the patches are stored, not added)
+    const size_t nacc = patch || deterministic ? 0 : n;      // (those are stored, not added)
     const ZeroJob zero_all{{dk_acc, dv_acc, (float *)(ws + wl.counters), dcoords}, {nacc, nacc, ncounters, ndc}};
     const ZeroJob zero_main{{dcoords, nullptr, nullptr, nullptr}, {ndc, 0, 0, 0}};
     const ZeroJob &zero = side_on ? zero_main : zero_all;
@@ -900,7 +906,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     if (rc != DSDPA_OK) return rc;
     if (side_on) {
         // the dk/dv side: its clears, and the (lse, delta) pairs that the dq kernel otherwise writes on the way
-        const ZeroJob zero_side{{dk_acc, dv_acc, (float *)(ws + wl.counters), nullptr}, {n, n, ncounters, 0}};
+        const ZeroJob zero_side{{dk_acc, dv_acc, (float *)(ws + wl.counters), nullptr}, {nacc, nacc, ncounters, 0}};
         if ((rc = zero_fill(zero_side, bst)) != DSDPA_OK) return rc;
         const size_t lanes = (size_t)dm.rows * 4;
         hipLaunchKernelGGL((delta_kernel<S>), dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, bst, out, dout, lse,
@@ -909,7 +915,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     }
     if (cell_binned && (rc = launch_binning(coords, dm, wl, ws, deterministic ? 0 : 1, Spread{left, wl.spread_mean}, bst)) != DSDPA_OK)
         return rc;
-    if (deterministic && (rc = launch_list_ordering(dm, wl, ws, bst)) != DSDPA_OK) return rc;
+    if (deterministic && (rc = launch_list_ordering(coords, dm, wl, ws, bst)) != DSDPA_OK) return rc;
     float2 *dq_stats = side_on || patch ? nullptr : stats;       // the dq kernel writes them only when dk/dv runs behind it
     // With the pairs handed over the two kernels go group by group of (batch, head) pairs: the buffer holds one
     // group's pairs (workspace_layout), and the dk/dv kernel of a group finds them where the dq kernel of the same
@@ -936,13 +942,17 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
                         : launch_bwd_dq_gather<S, DD>(q, k, v, coords, out, lse, dout, dq, dq_stats, dcoords,   \
                                                       handed, dm, bh0, nbh, st);                                \
             if (rc == DSDPA_OK && patch)                                                                        \
-                rc = launch_bwd_dkdv_patch<S, DD>(q, k, v, coords, dout, start, sorted,                         \
+                rc = launch_bwd_dkdv_patch<S, DD>(q, k, v, dout, start, sorted,                                 \
                                                   (const uint4 *)(ws + wl.items), wl.wmax, left, handed, dk,    \
                                                   dv, dk_acc, dv_acc, dm, wl.NC, bh0, nbh, st);                 \
+            else if (rc == DSDPA_OK && deterministic)                                                           \
+                rc = launch_bwd_dkdv_fixed<S, DD>(q, k, v, stats, dout, start, sorted, handed,                  \
+                                                  (float *)(ws + wl.taps), wl.tap_planes, dk, dv, dm, wl.NC,    \
+                                                  bh0, nbh, bst);                                               \
             else if (rc == DSDPA_OK && cell_binned)                                                             \
-                rc = launch_bwd_dkdv_cell<S, DD>(q, k, v, coords, stats, dout, start, sorted,                   \
+                rc = launch_bwd_dkdv_cell<S, DD>(q, k, v, stats, dout, start, sorted,                           \
                                                  (const uint4 *)(ws + wl.items), wl.wmax, handed, dk_acc,       \
-                                                 dv_acc, dm, wl.NK, deterministic, bh0, nbh, bst);              \
+                                                 dv_acc, dm, wl.NK, bh0, nbh, bst);                             \
             else if (rc == DSDPA_OK)                                                                            \
                 rc = launch_bwd_dkdv_tile<S, DD>(q, k, v, coords, stats, dout, dk_acc, dv_acc, dm, st);         \
         }                                                                                                       \
@@ -964,7 +974,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
         if (blocks > 256 * 8) blocks = 256 * 8;
         hipLaunchKernelGGL((cast_rest_kernel<S>), dim3((unsigned)blocks), dim3(256), 0, st, left, dk_acc, dv_acc, dk, dv, dm, n8);
         rc = check_launch();
-    } else if (S::kBytes != 4 && !patch) {
+    } else if (S::kBytes != 4 && !patch && !deterministic) {
         const size_t n8 = n / 8;
         const int threads = 256;
         size_t blocks = (n8 + threads - 1) / threads;
