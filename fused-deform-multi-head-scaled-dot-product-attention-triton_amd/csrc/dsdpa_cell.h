@@ -111,10 +111,11 @@ __global__ __launch_bounds__(kBinThreads) void bin_samples_kernel(const float *_
 // mode 0: global count[cell] += local count
 // mode 1: reserve [base, base+local count) from the global cursor of each cell,
 //         then place every sample at base + its local rank.
-constexpr int kBinLdsThreads = 1024;
-
-template <int MODE>
-__global__ __launch_bounds__(kBinLdsThreads) void bin_samples_lds_kernel(
+// THREADS: 1024 (48x48, 6 views x 32 samples of spread coordinates, batch 2: 148 us for count, scan and fill, 171 with 512), or
+// 512 beside the staged dq kernel, whose 14 to 16 waves on every CU leave a workgroup of 16 no place until dq ends, and dk/dv
+// behind it (14x14, 8 views x 32 samples: the count 217 us from start to end, 16 with 512 threads; the step 684 -> 634).
+template <int MODE, int THREADS>
+__global__ __launch_bounds__(THREADS) void bin_samples_lds_kernel(
     const float *__restrict__ coords_, Dims dm, int NC, int NK, int vpg, int lchunk, int nlc,
     unsigned *__restrict__ counters, unsigned *__restrict__ sorted, int records)
 {
@@ -125,11 +126,11 @@ __global__ __launch_bounds__(kBinLdsThreads) void bin_samples_lds_kernel(
     const int b = blockIdx.x / (nlc * dm.V);
     const int l0 = lc * lchunk, l1 = min(dm.L, l0 + lchunk);
     const int nhist = dm.V * NC;
-    for (int i = threadIdx.x; i < nhist; i += kBinLdsThreads) s_hist[i] = 0u;
+    for (int i = threadIdx.x; i < nhist; i += THREADS) s_hist[i] = 0u;
     __syncthreads();
     const float2 *crd = reinterpret_cast<const float2 *>(coords_) + (((size_t)b * dm.V + s1) * dm.L + l0) * dm.N;
     const int total = (l1 - l0) * dm.N;                  // samples of this workgroup, all key views
-    for (int i = threadIdx.x; i < total; i += kBinLdsThreads) {
+    for (int i = threadIdx.x; i < total; i += THREADS) {
         const float2 xy = crd[i];
         const Taps tp = make_taps(xy.x, xy.y, dm.Wimg, dm.Himg);
         if (taps_any(tp)) atomicAdd(&s_hist[((i / dm.P) % dm.V) * NC + cell_of(tp, dm.Wimg)], 1u);
@@ -138,19 +139,19 @@ __global__ __launch_bounds__(kBinLdsThreads) void bin_samples_lds_kernel(
     // [s2][key] of this batch item, at this workgroup's group of query views
     unsigned *gctr = counters + (size_t)b * dm.V * NK + (size_t)(s1 / vpg) * NC;
     if (MODE == 0) {
-        for (int i = threadIdx.x; i < nhist; i += kBinLdsThreads) {
+        for (int i = threadIdx.x; i < nhist; i += THREADS) {
             const unsigned c = s_hist[i];
             if (c) atomicAdd(gctr + (size_t)(i / NC) * NK + i % NC, c);
         }
     } else {
-        for (int i = threadIdx.x; i < nhist; i += kBinLdsThreads) {
+        for (int i = threadIdx.x; i < nhist; i += THREADS) {
             const unsigned c = s_hist[i];
             s_base[i] = c ? atomicAdd(gctr + (size_t)(i / NC) * NK + i % NC, c) : 0u;
             s_hist[i] = 0u;
         }
         __syncthreads();
         const size_t M = (size_t)dm.V * dm.L * dm.P;
-        for (int i = threadIdx.x; i < total; i += kBinLdsThreads) {
+        for (int i = threadIdx.x; i < total; i += THREADS) {
             const float2 xy = crd[i];
             const Taps tp = make_taps(xy.x, xy.y, dm.Wimg, dm.Himg);
             if (!taps_any(tp)) continue;
@@ -176,12 +177,13 @@ __global__ __launch_bounds__(kBinLdsThreads) void bin_samples_lds_kernel(
 // list's bounds would be a second, dependent one.
 //
 // Bound by its chain of waits (one workgroup per (b, s2), a few of them on the whole chip): four keys a thread, both
-// sums by lane shifts inside a wave and over the 16 waves' totals in LDS, two barriers per 4096 keys.
+// sums by lane shifts inside a wave and over the waves' totals in LDS, two barriers per THREADS * 4 keys.
 // (8450 keys, 8 workgroups: 29.4 -> 15.2 us against a scan of 1024 keys at a time with 20 barriers; 2401 keys 10.4 -> 6.0.)
 constexpr int kScanKeys = 4;
 struct ScanCarry { unsigned entries, pieces; };
-// One turn of the scan for a workgroup of 1024 threads: keys [c0, c0 + 4) of each thread, v their list lengths;
-// returns the first key's start in `first`, writes start and items, advances the carry. s_wave: 16 places.
+// One turn of the scan for a workgroup of THREADS threads: keys [c0, c0 + 4) of each thread, v their list lengths;
+// returns the first key's start in `first`, writes start and items, advances the carry. s_wave: a place per wave.
+template <int THREADS>
 __device__ __forceinline__ void scan_keys(const unsigned (&v)[kScanKeys], int c0, int NC, int grid_cells, unsigned piece,
                                           unsigned wmax, unsigned *__restrict__ st, uint4 *__restrict__ it,
                                           uint2 *s_wave, ScanCarry &carry, unsigned &first)
@@ -206,7 +208,7 @@ __device__ __forceinline__ void scan_keys(const unsigned (&v)[kScanKeys], int c0
     __syncthreads();
     unsigned excl = carry.entries + incl - sum, pexcl = carry.pieces + pincl - psum;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) {
+    for (int w = 0; w < THREADS / kWave; ++w) {
         const uint2 t = s_wave[w];
         excl += w < wave ? t.x : 0u;
         pexcl += w < wave ? t.y : 0u;
@@ -232,6 +234,7 @@ __device__ __forceinline__ void scan_keys(const unsigned (&v)[kScanKeys], int c0
 // the patch kernel's (kSpreadLongest entries at most and `mean` or fewer on average): 0 if they are, else the number of items
 struct Spread { unsigned *items, mean; };
 constexpr unsigned kSpreadLongest = 1024;
+template <int THREADS>
 __device__ __forceinline__ void scan_end(const ScanCarry &carry, int NC, unsigned wmax, unsigned *__restrict__ st, uint4 *__restrict__ it,
                                          const Spread &spread, unsigned longest)
 {
@@ -242,35 +245,36 @@ __device__ __forceinline__ void scan_end(const ScanCarry &carry, int NC, unsigne
                                      ? 0u : min(carry.pieces, wmax);
     }
     if (threadIdx.x == 0) st[NC] = carry.entries;
-    for (unsigned i = min(carry.pieces, wmax) + threadIdx.x; i < wmax; i += 1024) it[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (unsigned i = min(carry.pieces, wmax) + threadIdx.x; i < wmax; i += THREADS) it[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
-static __global__ __launch_bounds__(1024) void bin_scan_kernel(unsigned *__restrict__ counters,
-                                                        unsigned *__restrict__ start, int NC, int grid_cells,
-                                                        unsigned piece, unsigned wmax, uint4 *__restrict__ items,
-                                                        Spread spread)
+// (512 threads and at most 64 registers beside the staged dq kernel, as above)
+template <int THREADS>
+__global__ __launch_bounds__(THREADS, THREADS == 512 ? 8 : 4) void bin_scan_kernel(
+    unsigned *__restrict__ counters, unsigned *__restrict__ start, int NC, int grid_cells,
+    unsigned piece, unsigned wmax, uint4 *__restrict__ items, Spread spread)
 {
-    __shared__ uint2 s_wave[16];                                   // (entries, pieces) of each wave's keys
+    __shared__ uint2 s_wave[THREADS / kWave];                      // (entries, pieces) of each wave's keys
     unsigned *cnt = counters + (size_t)blockIdx.x * NC;
     unsigned *st = start + (size_t)blockIdx.x * (NC + 1);
     uint4 *it = items + (size_t)blockIdx.x * wmax;
     ScanCarry carry{0u, 0u};
     unsigned longest = 0u;
-    for (int base = 0; base < NC; base += 1024 * kScanKeys) {
+    for (int base = 0; base < NC; base += THREADS * kScanKeys) {
         const int c0 = base + (int)threadIdx.x * kScanKeys;
         unsigned v[kScanKeys], at;
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NC ? cnt[c0 + i] : 0u;
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) longest = max(longest, v[i]);
-        scan_keys(v, c0, NC, grid_cells, piece, wmax, st, it, s_wave, carry, at);
+        scan_keys<THREADS>(v, c0, NC, grid_cells, piece, wmax, st, it, s_wave, carry, at);
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) {
             if (c0 + i < NC) cnt[c0 + i] = at;
             at += v[i];
         }
     }
-    scan_end(carry, NC, wmax, st, it, spread, longest);
+    scan_end<THREADS>(carry, NC, wmax, st, it, spread, longest);
 }
 
 // Count, scan and fill in one launch, for lists short enough that one workgroup holds all samples of a (b, s2) in
@@ -328,7 +332,7 @@ __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__
         for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NC ? s_hist[c0 + i] : 0u;
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) longest = max(longest, v[i]);
-        scan_keys(v, c0, NC, NC, piece, wmax, st, it, s_wave, carry, at);
+        scan_keys<1024>(v, c0, NC, NC, piece, wmax, st, it, s_wave, carry, at);
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) {
             if (c0 + i < NC) s_hist[c0 + i] = at;                  // (this thread's own keys)
@@ -342,7 +346,7 @@ __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__
             store_cell_entry(sorted, (size_t)blockIdx.x * M + s_hist[key_rank[i] & ((1u << kBinOneKeyBits) - 1u)] + (key_rank[i] >> kBinOneKeyBits),
                              (unsigned)i * 1024u + threadIdx.x, cell_fraction(xy[i], dm), records);
     }
-    scan_end(carry, NC, wmax, st, it, spread, longest);
+    scan_end<1024>(carry, NC, wmax, st, it, spread, longest);
 }
 
 // Deterministic backward: begin / end of every cell list as positions in the flat id array

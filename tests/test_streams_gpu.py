@@ -84,6 +84,24 @@ def test_side_lane_matches_single_stream(shape):
         assert rel(two[2], one[2]) < tol and rel(two[3], one[3]) < tol
 
 
+# Beside the staged dq kernel the lists are made by workgroups of 512 threads, 2048 keys a turn of the scan: one turn that is
+# not full, several turns with a remainder of one and of a few keys a thread, a histogram of few cells and many samples
+@pytest.mark.parametrize("dims", [(2, 3, 32, 13, 20, 32, 16), (1, 9, 8, 21, 22, 32, 9), (2, 12, 8, 14, 13, 64, 7),
+                                  (1, 2, 32, 20, 24, 32, 40), (1, 1, 64, 5, 30, 64, 300)], ids=lambda d: "x".join(map(str, d)))
+def test_lists_made_beside_dq(dims):
+    B, V, H, Himg, Wimg, D, P = dims
+    dtype = torch.float32 if D == 32 else torch.bfloat16
+    say(f"[case] lists beside dq vs single stream {dims} {dtype}")
+    q, k, v, c, do = make(71, B, V, H, Himg, Wimg, D, P, dtype)
+    one = c_abi_backward(q, k, v, c, do, Himg, Wimg, _native.FLAG_SINGLE_STREAM)
+    torch.cuda.synchronize()
+    two = c_abi_backward(q, k, v, c, do, Himg, Wimg, 0)
+    torch.cuda.synchronize()
+    tol = 1e-5 if dtype == torch.float32 else 1e-2         # order of the float atomics / one rounding to 16 bits
+    assert torch.equal(one[1], two[1])
+    assert rel(two[2], one[2]) < tol and rel(two[3], one[3]) < tol
+
+
 def test_caller_stream_is_ordered_before_and_after():
     """Inputs are produced on the caller's stream right before the call and the gradients consumed on it right
     after, with no synchronisation in between: the side lane's fork and join carry the ordering."""
