@@ -103,63 +103,81 @@ __global__ __launch_bounds__(kBinThreads) void bin_samples_kernel(const float *_
     }
 }
 
-// LDS-aggregated variant of the two passes above, used when the V*NC counters of
-// one batch item fit in LDS. A workgroup takes a contiguous run of query rows of
-// one (b, s1) -- whose coordinates are one contiguous block covering all V key
-// views -- and histograms it in LDS first, so the contended global atomics drop
-// from one per sample to one per (workgroup, non-empty cell).
+// LDS-aggregated variant of the two passes above. A workgroup takes kBinRunThreads * PER consecutive samples of one (b, s2), PER
+// of them a thread, requested together and kept in registers, and histograms them in LDS first, so the contended global
+// atomics drop from one per sample to one per (workgroup, non-empty cell).
 // mode 0: global count[cell] += local count
-// mode 1: reserve [base, base+local count) from the global cursor of each cell,
-//         then place every sample at base + its local rank.
-// THREADS: 1024 (48x48, 6 views x 32 samples of spread coordinates, batch 2: 148 us for count, scan and fill, 171 with 512), or
-// 512 beside the staged dq kernel, whose 14 to 16 waves on every CU leave a workgroup of 16 no place until dq ends, and dk/dv
-// behind it (14x14, 8 views x 32 samples: the count 217 us from start to end, 16 with 512 threads; the step 684 -> 634).
-template <int MODE, int THREADS>
-__global__ __launch_bounds__(THREADS) void bin_samples_lds_kernel(
-    const float *__restrict__ coords_, Dims dm, int NC, int NK, int vpg, int lchunk, int nlc,
+// mode 1: every sample's rank among the workgroup's in its cell comes from the counting atomic; reserve
+//         [base, base+local count) from the global cursor of each cell, then place every sample at base + rank.
+// Bound by the chain load -> LDS atomic -> global atomic -> scattered store, and by the counters that every workgroup walks: one key
+// view's, not all V views' of a run of query rows (V * NC counters, twice that LDS, and each sample read and worked out twice in
+// the fill). Count, scan and fill, us, before / now: 48x48, 6 views x 32 samples, batch 2 148 / 72; 64x64, 4 x 64, batch 2,
+// clustered 165 / 95; 32x32, 6 x 16 38 / 21; 40x28, 4 x 8, batch 2 30 / 14; 18x18, 6 x 6, batch 2 22 / 13.
+// 512 threads: 1024 with half the samples each are even, but beside the staged dq kernel, whose 14 to 16 waves on every CU
+// leave workgroups of 16 waves or of more than 64 registers no place until dq ends, dk/dv would wait behind them (14x14, 8 views x
+// 32 samples: the three launches 41 us from first to last with four samples a thread, 194 with eight).
+constexpr int kBinRunThreads = 512, kBinRunKeys = 20 * 1024;
+template <int MODE, int PER>
+__global__ __launch_bounds__(kBinRunThreads, PER <= 4 ? 8 : 4) void bin_samples_lds_kernel(
+    const float *__restrict__ coords_, Dims dm, int NC, int NK, int vpg, int nlc,
     unsigned *__restrict__ counters, unsigned *__restrict__ sorted, int records)
 {
-    extern __shared__ unsigned s_hist[];                 // [V][NC]; mode 1 adds [V][NC] bases
-    unsigned *s_base = s_hist + (size_t)dm.V * NC;
-    const int lc = blockIdx.x % nlc;
-    const int s1 = (blockIdx.x / nlc) % dm.V;
-    const int b = blockIdx.x / (nlc * dm.V);
-    const int l0 = lc * lchunk, l1 = min(dm.L, l0 + lchunk);
-    const int nhist = dm.V * NC;
-    for (int i = threadIdx.x; i < nhist; i += THREADS) s_hist[i] = 0u;
+    constexpr int THREADS = kBinRunThreads;
+    extern __shared__ unsigned s_hist[];                 // [NC] local counts; mode 1: then the places reserved
+    // (b, s2, group of query views, run): the lists of a (b, s2) are filled by the workgroups of one XCD or two, whose L2 joins
+    // their stores. Sample ids (s1*L + l)*P + p of a group are consecutive.
+    const unsigned work = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x), ngrp = (unsigned)(NK / NC);
+    const unsigned t = work / (unsigned)nlc, lc = work - t * (unsigned)nlc;
+    const unsigned grp = t / ngrp, qg = t - grp * ngrp, b = grp / (unsigned)dm.V, s2 = grp - b * (unsigned)dm.V;
+    const unsigned n = (unsigned)dm.L * (unsigned)dm.P, end = min((qg + 1u) * (unsigned)vpg, (unsigned)dm.V) * n;
+    const unsigned first = qg * (unsigned)vpg * n + lc * (unsigned)(THREADS * PER) + threadIdx.x;
+    const float2 *crd = reinterpret_cast<const float2 *>(coords_) + (size_t)b * dm.V * dm.L * dm.N + (size_t)s2 * dm.P;
+    float2 xy[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const unsigned id = min(first + (unsigned)(j * THREADS), end - 1u), ql = dm.divP.div(id);
+        xy[j] = crd[(size_t)ql * dm.N + (id - ql * (unsigned)dm.P)];
+    }
+    for (int i = threadIdx.x; i < NC; i += THREADS) s_hist[i] = 0u;
     __syncthreads();
-    const float2 *crd = reinterpret_cast<const float2 *>(coords_) + (((size_t)b * dm.V + s1) * dm.L + l0) * dm.N;
-    const int total = (l1 - l0) * dm.N;                  // samples of this workgroup, all key views
-    for (int i = threadIdx.x; i < total; i += THREADS) {
-        const float2 xy = crd[i];
-        const Taps tp = make_taps(xy.x, xy.y, dm.Wimg, dm.Himg);
-        if (taps_any(tp)) atomicAdd(&s_hist[((i / dm.P) % dm.V) * NC + cell_of(tp, dm.Wimg)], 1u);
+    unsigned key[PER], rank[PER];                        // key NC: in no list
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const Taps tp = make_taps(xy[j].x, xy[j].y, dm.Wimg, dm.Himg);
+        const bool counted = first + (unsigned)(j * THREADS) < end && taps_any(tp);
+        key[j] = counted ? (unsigned)cell_of(tp, dm.Wimg) : (unsigned)NC;
+        rank[j] = 0u;
+        if (counted) rank[j] = atomicAdd(&s_hist[key[j]], 1u);
     }
     __syncthreads();
-    // [s2][key] of this batch item, at this workgroup's group of query views
-    unsigned *gctr = counters + (size_t)b * dm.V * NK + (size_t)(s1 / vpg) * NC;
-    if (MODE == 0) {
-        for (int i = threadIdx.x; i < nhist; i += THREADS) {
-            const unsigned c = s_hist[i];
-            if (c) atomicAdd(gctr + (size_t)(i / NC) * NK + i % NC, c);
+    // the keys of this (b, s2) and group, four counters a thread in flight
+    unsigned *gctr = counters + (size_t)grp * NK + (size_t)qg * NC;
+    for (int i0 = threadIdx.x; i0 < NC; i0 += 4 * THREADS) {
+        unsigned c[4], base[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = i0 + u * THREADS;
+            c[u] = i < NC ? s_hist[i] : 0u;
+            base[u] = 0u;
+            if (c[u]) {
+                if (MODE == 0) atomicAdd(gctr + i, c[u]);
+                else base[u] = atomicAdd(gctr + i, c[u]);
+            }
         }
-    } else {
-        for (int i = threadIdx.x; i < nhist; i += THREADS) {
-            const unsigned c = s_hist[i];
-            s_base[i] = c ? atomicAdd(gctr + (size_t)(i / NC) * NK + i % NC, c) : 0u;
-            s_hist[i] = 0u;
+        if (MODE == 1) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (c[u]) s_hist[i0 + u * THREADS] = base[u];
         }
+    }
+    if (MODE == 1) {
         __syncthreads();
-        const size_t M = (size_t)dm.V * dm.L * dm.P;
-        for (int i = threadIdx.x; i < total; i += THREADS) {
-            const float2 xy = crd[i];
-            const Taps tp = make_taps(xy.x, xy.y, dm.Wimg, dm.Himg);
-            if (!taps_any(tp)) continue;
-            const int p = i % dm.P, s2 = (i / dm.P) % dm.V, l = l0 + i / dm.N;
-            const int hidx = s2 * NC + cell_of(tp, dm.Wimg);
-            const unsigned pos = s_base[hidx] + atomicAdd(&s_hist[hidx], 1u);
-            store_cell_entry(sorted, ((size_t)b * dm.V + s2) * M + pos, ((unsigned)s1 * dm.L + l) * (unsigned)dm.P + (unsigned)p,
-                             cell_fraction(xy, dm), records);
+        const size_t place0 = (size_t)grp * ((size_t)dm.V * n);
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (key[j] == (unsigned)NC) continue;
+            store_cell_entry(sorted, place0 + s_hist[key[j]] + rank[j], first + (unsigned)(j * THREADS),
+                             cell_fraction(xy[j], dm), records);
         }
     }
 }

@@ -615,8 +615,7 @@ static inline bool bin_in_one_launch(const Dims &dm)
 }
 
 // spread: flags to set for the patch kernel, or none. beside_dq: the staged dq kernel runs at the same time and dk/dv is next, so
-// take workgroups that fit beside its waves (not where the ordering of the lists comes between: 18x18, D = 32, 6 views x 32 samples,
-// 415 us a step with the large ones, 418 with these).
+// take workgroups that fit beside its waves.
 // records: the lists as 12-byte records (id and position in the cell) from wl.sorted on, through the room of
 // wl.frac behind it; else plain ids in wl.sorted (the deterministic backward, which sorts them).
 static inline int launch_binning(const float *coords, const Dims &dm, const WorkspaceLayout &wl, char *ws,
@@ -632,56 +631,43 @@ static inline int launch_binning(const float *coords, const Dims &dm, const Work
                      coords, dm, wl.NC, start, wl.piece, wl.wmax, (uint4 *)(ws + wl.items), sorted, records, spread);
         return check_launch();
     }
-    const size_t hist_bytes = (size_t)dm.V * wl.NC * sizeof(unsigned);
+    const long long total = (long long)dm.B * dm.V * dm.L * dm.N;
     // each of the three launches carries its own pair of events: the timer's slot 3 adds up their busy time
     ScopedKernelTimer t_count(3, st), t_scan(3, st), t_fill(3, st);
-    if (2 * hist_bytes <= (size_t)kLdsBytes - 1024) {
-        // LDS-aggregated passes: a workgroup per run of about 4k samples of one (b, s1); more when the histogram
-        // is large, since every workgroup walks all of it twice: twice its counters, between 8k and 32k samples, as
-        // long as that leaves 128 workgroups (64x64, 4 views, 8.4 M samples: 0.203 ms for the three launches with
-        // runs of 8k, 0.179 with 16k or 32k, 0.229 with 64k; 48x48, 6 views, 5.3 M: 0.177 / 0.174 / 0.157 / 0.221;
-        // 32x32, 6 views, 0.6 M: 0.037 / 0.050 / 0.072)
-        const long long hist_entries = (long long)dm.V * wl.NC, total_samples = (long long)dm.B * dm.V * dm.L * dm.N;
-        long long run = 4096;
-        if (hist_entries >= 4096) {
-            run = 2 * hist_entries < 8192 ? 8192 : (2 * hist_entries > 32768 ? 32768 : 2 * hist_entries);
-            while (run > 8192 && total_samples / run < 128) run /= 2;
-            if (run < 8192) run = 8192;
-        }
-        int lchunk = (int)(run / dm.N);
-        if (lchunk < 1) lchunk = 1;
-        if (lchunk > dm.L) lchunk = dm.L;
-        const int nlc = (dm.L + lchunk - 1) / lchunk;
-        lchunk = (dm.L + nlc - 1) / nlc;
-        const long long blocks = (long long)dm.B * dm.V * nlc;
+    auto scan = beside_dq ? bin_scan_kernel<512> : bin_scan_kernel<1024>;
+    auto launch_scan = [&]() {
+        DSDPA_LAUNCH(scan, dim3((unsigned)(dm.B * dm.V)), dim3(beside_dq ? 512 : 1024), 0, st, t_scan.start(), t_scan.stop(), counters,
+                     start, wl.NK, wl.NC, wl.piece, wl.wmax, (uint4 *)(ws + wl.items), spread);
+    };
+    // LDS-aggregated passes, as long as two workgroups' counters fit on a CU. Count, scan and fill, us, one atomic a sample / these:
+    // 96x128, 2 views x 2 samples 35 / 35, x 16 119 / 65, clustered 190 / 44; 200x200, 1 x 4 (40401 cells) 70 / 86.
+    if (wl.NC <= kBinRunKeys) {
+        // Eight samples a thread where that leaves 1024 workgroups, else four (and beside the staged dq kernel, see the kernel): us
+        // with 4 / 8, 64x64, 4 views x 64 samples, batch 2 122 / 95; 48x48, 6 x 32 89 / 72; 64x64, 8 x 8 34 / 34; 32x32, 6 x 16
+        // 21 / 20; 40x28, 4 x 8 14 / 17; 37x23, 3 x 7 14 / 17.
+        const int per = !beside_dq && total >= 1024ll * 8 * kBinRunThreads ? 8 : 4;
+        const long long nlc = ((long long)wl.vpg * dm.L * dm.P + per * kBinRunThreads - 1) / (per * kBinRunThreads);
+        const long long blocks = (long long)dm.B * dm.V * (wl.NK / wl.NC) * nlc;
         if (blocks > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;
-        auto k0 = beside_dq ? bin_samples_lds_kernel<0, 512> : bin_samples_lds_kernel<0, 1024>;
-        auto k1 = beside_dq ? bin_samples_lds_kernel<1, 512> : bin_samples_lds_kernel<1, 1024>;
-        auto scan = beside_dq ? bin_scan_kernel<512> : bin_scan_kernel<1024>;
-        const int threads = beside_dq ? 512 : 1024;
+        auto k0 = per == 8 ? bin_samples_lds_kernel<0, 8> : bin_samples_lds_kernel<0, 4>;
+        auto k1 = per == 8 ? bin_samples_lds_kernel<1, 8> : bin_samples_lds_kernel<1, 4>;
+        const size_t hist_bytes = (size_t)wl.NC * sizeof(unsigned);
         static std::atomic<unsigned long long> lds_set[4];
-        if (int rc = allow_full_lds(k0, lds_set[beside_dq ? 2 : 0])) return rc;
-        if (int rc = allow_full_lds(k1, lds_set[beside_dq ? 3 : 1])) return rc;
-        DSDPA_LAUNCH(k0, dim3((unsigned)blocks), dim3(threads), hist_bytes, st,
-                              t_count.start(), t_count.stop(),
-                           coords, dm, wl.NC, wl.NK, wl.vpg, lchunk, nlc, counters, sorted, records);
-        DSDPA_LAUNCH(scan, dim3((unsigned)(dm.B * dm.V)), dim3(threads), 0, st,
-                              t_scan.start(), t_scan.stop(), counters, start, wl.NK, wl.NC, wl.piece, wl.wmax,
-                              (uint4 *)(ws + wl.items), spread);
-        DSDPA_LAUNCH(k1, dim3((unsigned)blocks), dim3(threads), 2 * hist_bytes, st,
-                              t_fill.start(), t_fill.stop(),
-                           coords, dm, wl.NC, wl.NK, wl.vpg, lchunk, nlc, counters, sorted, records);
+        if (int rc = allow_full_lds(k0, lds_set[per == 8 ? 2 : 0])) return rc;
+        if (int rc = allow_full_lds(k1, lds_set[per == 8 ? 3 : 1])) return rc;
+        DSDPA_LAUNCH(k0, dim3((unsigned)blocks), dim3(kBinRunThreads), hist_bytes, st, t_count.start(), t_count.stop(),
+                     coords, dm, wl.NC, wl.NK, wl.vpg, (int)nlc, counters, sorted, records);
+        launch_scan();
+        DSDPA_LAUNCH(k1, dim3((unsigned)blocks), dim3(kBinRunThreads), hist_bytes, st, t_fill.start(), t_fill.stop(),
+                     coords, dm, wl.NC, wl.NK, wl.vpg, (int)nlc, counters, sorted, records);
         return check_launch();
     }
-    const long long total = (long long)dm.B * dm.V * dm.L * dm.N;
     const long long blocks = (total + kBinThreads - 1) / kBinThreads;
     if (blocks > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;
     DSDPA_LAUNCH(bin_samples_kernel<0>, dim3((unsigned)blocks), dim3(kBinThreads), 0, st,
                           t_count.start(), t_count.stop(),
                        coords, dm, wl.NC, wl.NK, wl.vpg, counters, sorted, records);
-    DSDPA_LAUNCH((bin_scan_kernel<1024>), dim3((unsigned)(dm.B * dm.V)), dim3(1024), 0, st,
-                          t_scan.start(), t_scan.stop(), counters, start, wl.NK, wl.NC, wl.piece, wl.wmax,
-                              (uint4 *)(ws + wl.items), spread);
+    launch_scan();
     DSDPA_LAUNCH(bin_samples_kernel<1>, dim3((unsigned)blocks), dim3(kBinThreads), 0, st,
                           t_fill.start(), t_fill.stop(),
                        coords, dm, wl.NC, wl.NK, wl.vpg, counters, sorted, records);

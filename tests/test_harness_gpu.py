@@ -87,9 +87,9 @@ def test_non_default_stream_and_back_to_back_calls():
 
 
 def test_large_image_uses_global_binning_path():
-    """A 96x128 image with 2 views has too many cells for the LDS-aggregated binning (V*NC counters do not
-    fit in LDS), so the backward takes the global-atomic counting passes; planes are too big for LDS too."""
-    print("[case] large image, global binning", flush=True)
+    """A 96x128 image with 2 views: 12513 cells, more than a binning workgroup's samples (images beyond its counters in
+    LDS: test_binning_runs_gpu.py); planes are too big for LDS too."""
+    print("[case] large image", flush=True)
     g = torch.Generator().manual_seed(41)
     B, V, H, Himg, Wimg, D, P = 1, 2, 1, 96, 128, 16, 3
     L = Himg * Wimg
