@@ -445,7 +445,8 @@ static inline int launch_plane_descriptors(const float *coords, const Dims &dm, 
                                            bool coords_grad, const ZeroJob &zero, int timer_slot, hipStream_t st)
 {
     const long long nblk = (long long)dm.B * dm.V * dm.L * dm.V;
-    const long long waves = dm.P <= 32 ? (nblk + 1) / 2 : nblk * ((dm.P + 63) / 64);
+    const int per = kWave / dm.P;                                 // whole runs of a wave (P <= 32)
+    const long long waves = dm.P <= 32 ? (nblk + per - 1) / per : nblk * ((dm.P + 63) / 64);
     const long long blocks = (waves * kWave + kDescThreads - 1) / kDescThreads;
     if (blocks > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;
     ScopedKernelTimer timer(timer_slot, st);

@@ -171,6 +171,9 @@ __device__ __forceinline__ PlaneBlock decode_plane_block(const Dims &dm, int row
 // -- bits 13, 14: columns x0, x0+1; bits 29, 30: rows y0, y0+1 -- and desc_g holds (fx, fy, the sample's
 // index n inside its run as an integer, unused): the entries are stored in a permuted order, and the
 // gradient has to go back to the sample it belongs to.
+// A wave takes as many whole runs as fit its 64 lanes, side by side in memory (two at 32 lanes each left 40 of 64 empty at 12
+// samples a view): bound by latency, a load and the ranking before the stores, so the fewer waves the better. us, two runs a
+// wave / as many as fit: 18x18, batch 2: 12 views x 12 samples 17.0 / 10.9, 10 x 4 12.2 / 5.9, 6 x 6 5.6 / 4.5, 6 x 32 even.
 constexpr int kDescThreads = 256;
 constexpr uint32_t kDescCodeMask = 0x1fffu;
 // the sample index inside its run of a table entry at place `pos` of the run with code word `c` (runs of more than 64
@@ -188,14 +191,15 @@ static __global__ __launch_bounds__(kDescThreads) void plane_descriptor_kernel(
     long long blk;
     int n;                                                              // sample index inside the run
     unsigned long long group;                                           // lanes that share a run
-    if (dm.P <= 32) {                                                   // two runs per wave
-        blk = wave * 2 + (lane >> 5);
-        n = lane & 31;
-        group = lane < 32 ? 0xffffffffull : 0xffffffff00000000ull;
+    if (dm.P <= 32) {                                                   // as many whole runs per wave as there is room for
+        const unsigned per = dm.divP.div((unsigned)kWave), r = dm.divP.div((unsigned)lane);
+        blk = r < per ? wave * per + r : nblk;
+        n = lane - (int)r * dm.P;
+        group = ((1ull << dm.P) - 1ull) << (r < per ? r * (unsigned)dm.P : 0u);
     } else {                                                            // one 64-sample piece of a run per wave
         const int pieces = (dm.P + 63) / 64;
-        blk = wave / pieces;
-        n = (int)(wave % pieces) * 64 + lane;
+        blk = pieces == 1 ? wave : wave / pieces;
+        n = (int)(wave - blk * pieces) * 64 + lane;
         group = ~0ull;
     }
     const bool valid = blk < nblk && n < dm.P;
