@@ -122,8 +122,8 @@ int dsdpa_fwd_noalloc(int dtype, const void *q, const void *k, const void *v, co
 
 /* Flags of the backward. The reference has one backward, with float atomics (ops/triton.py:345-360).
  * DSDPA_FLAG_DETERMINISTIC: bitwise reproducible dq, dk, dv: the samples of every bilinear cell are
- * added up in ascending order of their index and the per-cell sums reach dk/dv in four passes of plain
- * stores (cells of one row/column parity share no pixel) instead of float atomics. Needs a larger
+ * added up in ascending order of their index, and the sums of every cell's four taps are stored apart and then
+ * added pixel by pixel in a fixed order instead of by float atomics. Needs a larger
  * workspace (pass the same flags to dsdpa_bwd_workspace_bytes) and cannot be combined with dcoords. */
 enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SINGLE_STREAM = 4 };
 /* B*V*H*L * V*P from which the backward may use its second stream; below it DSDPA_FLAG_SINGLE_STREAM changes nothing */
@@ -210,9 +210,10 @@ int dsdpa_version(void);
  * table, ops/triton.py:10-25.
  */
 /* Forward and backward-dq: AUTO and LDS stage each key view's K/V planes in LDS
- * when a plane pair fits (AUTO: unless there are at most 3 samples per view and 8
- * or more views, where staging costs more than it saves), GATHER always reads the
- * taps from global memory, one query at a time. AUTO alone lets the forward work on
+ * when a plane pair fits (AUTO: unless there are at most 2 samples per view, 3 in 16-bit storage, or
+ * at most 6 per query, where staging costs more than it saves), GATHER always reads the
+ * taps from global memory, one query at a time. AUTO alone gives a slot of lanes one query row each where a query has
+ * few samples and the planes are not staged, lets the forward work on
  * tiles of 16 queries with the matrix instructions where the shape allows it
  * (16-bit storage, D = 64 or 128, P >= 64, planes too large for LDS), and lets the
  * forward and dq walk the planes through LDS 16 columns at a time (fp32 storage,
