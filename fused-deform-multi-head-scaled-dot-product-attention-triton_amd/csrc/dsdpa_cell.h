@@ -458,7 +458,8 @@ __device__ __forceinline__ void cell_sums(
     __shared__ unsigned s_qrow[kCellWaves][2 * kWave];      // ... in q (which may be strided)
     __shared__ float2 s_f[S::kBytes == 2 ? kCellWaves : 1][2 * kWave];      // 16-bit storage: (fx, fy) of the entry
     __shared__ __attribute__((aligned(16))) float s_flush[kCellWaves][4 * D];                 // the flush: four rows of dk, then of dv
-    constexpr bool kQuad = HANDED && S::kBytes == 2 && DC >= 8;            // four-entry trips (below)
+    // four-entry trips (below), whose coefficients are two 16-bit parts; the deterministic backward keeps fp32 ones
+    constexpr bool kQuad = HANDED && !FIXED && S::kBytes == 2 && DC >= 8;
     // kQuad: a ring of merged entries; the coefficients as [tap][place]
     __shared__ __attribute__((aligned(16))) float s_ckq[kQuad ? kCellWaves : 1][2 * 4 * kWave], s_cvq[kQuad ? kCellWaves : 1][2 * 4 * kWave];
     __shared__ __attribute__((aligned(16))) unsigned s_rowq[kQuad ? kCellWaves : 1][2 * kWave], s_qrowq[kQuad ? kCellWaves : 1][2 * kWave];

@@ -1,0 +1,58 @@
+"""dk and dv of fp16 storage where the gradients that come in are far from one: down to what a training step without loss
+scaling sends (1e-5), and up to coefficients beyond fp16's largest number. Against the CPU oracle, whose inputs are the same
+fp16 values.
+
+The bar on the root mean square of the error is twice that of storing the oracle's result in fp16, which is all that the
+storage type takes (below 6e-5 its step no longer shrinks), and 1e-3 of the result's for sums and for the saved output, of which the
+row sums are taken (2^-12 of |dout| |out| beside logit gradients of |dout| |v|)."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle_bwd
+from ops.triton import deform_sdpa_triton
+
+pytestmark = pytest.mark.gpu
+
+
+def check(B, V, H, Himg, Wimg, D, P, scale, qk, v_size, dout_size, names=("dk", "dv")):
+    print(f"[case] range B{B} V{V} H{H} {Himg}x{Wimg} D{D} P{P} qk {qk} dout {dout_size}", flush=True)
+    g = torch.Generator().manual_seed(D + P)
+    L = Himg * Wimg
+    q, k, v, dout = (torch.randn(B, V, H, L, D, generator=g) for _ in range(4))
+    q, k, v, dout = ((t * f).half() for t, f in zip((q, k, v, dout), (qk, qk, v_size, dout_size)))
+    coords = torch.rand(B, V, L, V, P, 2, generator=g) * 1.2 - 0.1
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    deform_sdpa_triton(*leaves, coords.cuda(), Wimg, Himg, scale).backward(dout.cuda())
+    torch.cuda.synchronize()
+    want = oracle_bwd(*(t.float().numpy() for t in (q, k, v, coords, dout)), Wimg, Himg, scale)
+    for leaf, b, name in zip(leaves, want, ("dq", "dk", "dv")):
+        if name not in names:
+            continue
+        a, b = leaf.grad.double().cpu().numpy(), np.asarray(b, dtype=np.float64)
+        assert np.abs(b).max() < 65504 and np.isfinite(a).all(), name
+        rms = lambda x: math.sqrt(np.mean(x * x))
+        stored = rms(b.astype(np.float16).astype(np.float64) - b)
+        assert rms(a - b) <= 2 * stored + 1e-3 * rms(b), (name, rms(a - b), stored, rms(b))
+
+
+@pytest.fixture(params=[True], ids=["deterministic"])
+def mode(request):
+    prev = torch.are_deterministic_algorithms_enabled()
+    torch.use_deterministic_algorithms(request.param)
+    yield request.param
+    torch.use_deterministic_algorithms(prev)
+
+
+# D = 128 and 256 on maps that do not fit in LDS, lists too long for patches: cells with the pairs handed on
+@pytest.mark.parametrize("dout", [1.0, 1e-3, 1e-4, 1e-5])
+@pytest.mark.parametrize("D", [128, 256])
+def test_small_gradients(D, dout, mode):
+    check(1, 4, 2, 18, 19, D, 16, 1.0 / math.sqrt(D), 1.0, 1.0, dout)
+
+
+# sm_scale * ds beyond 65504 where q and k are small, dq, dk and dv all finite
+def test_coefficients_beyond_the_largest_fp16(mode):
+    check(1, 4, 2, 18, 19, 128, 16, 100.0, 0.015, 2.0, 5e3, names=("dq", "dk", "dv"))
