@@ -614,6 +614,10 @@ __device__ __forceinline__ void cell_sums(
             const unsigned *r = list + 3u * min(cstart + (unsigned)lane, hi - 1u);
             return CellEntry{r[0], __uint_as_float(r[1]), __uint_as_float(r[2])};
         };
+        // fp16: what the coefficients of ds are multiplied by at the split (lower_scale). The ring holds them as they are, so
+        // that a scale lowered for a new block holds for what is left of the old ones too; the sums are brought down to it.
+        constexpr bool kScaled = !S::kBf16;
+        float scale_ds = kScaled ? kScaleDs : 1.0f;
         auto prepare = [&](unsigned cstart, int tail, unsigned sid, float2 ff, float2 pdv) -> int {
             const unsigned ql = dm.divP.div(sid);                                  // ql = s1*L + l
             const unsigned s1 = dm.divL.div(ql), l = ql - s1 * (unsigned)dm.L;
@@ -641,6 +645,8 @@ __device__ __forceinline__ void cell_sums(
                 const float pairsum = fmaf(m1, __shfl_down(c[i], 1, kWave), c[i]);
                 c[i] = fmaf(m2, __shfl_down(pairsum, 2, kWave), pairsum);
             }
+            float top = 0.f;
+            if constexpr (kScaled) top = lead ? fmaxf(fmaxf(fabsf(c[0]), fabsf(c[1])), fmaxf(fabsf(c[2]), fabsf(c[3]))) : 0.f;
             const unsigned row = (s1 * view_rows + l) * kRowBytes;
             const unsigned qrow = (s1 * (unsigned)dm.q_sv + l * (unsigned)dm.q_sl) * S::kBytes;
             float *ck = s_ckq[wave], *cv = s_cvq[wave];
@@ -659,6 +665,13 @@ __device__ __forceinline__ void cell_sums(
                 for (int tpi = 0; tpi < 4; ++tpi) { ck[tpi * kRing + at] = 0.f; cv[tpi * kRing + at] = 0.f; }
                 s_rowq[wave][at] = (unsigned)__builtin_amdgcn_readfirstlane((int)row);
                 s_qrowq[wave][at] = (unsigned)__builtin_amdgcn_readfirstlane((int)qrow);
+            }
+            if constexpr (kScaled) {
+                const float by = lower_scale(first_lane(wave_max(top)), scale_ds);
+                if (by != 1.0f) {
+#pragma unroll
+                    for (int d = 0; d < DC; ++d) mK[d] *= by;
+                }
             }
             return n;
         };
@@ -706,8 +719,9 @@ __device__ __forceinline__ void cell_sums(
                 const int at = (head & (kRing - 1)) >> 2;
                 const float4 ck4 = reinterpret_cast<const float4 *>(s_ckq[wave])[tap_lane + at];
                 const float4 cv4 = reinterpret_cast<const float4 *>(s_cvq[wave])[tap_lane + at];
-                const uint4 sk = split_coefficients<S>(ck4.x, ck4.y, ck4.z, ck4.w);
-                const uint4 sv = split_coefficients<S>(cv4.x, cv4.y, cv4.z, cv4.w);
+                const float by_p = kScaled ? kScaleP : 1.0f;
+                const uint4 sk = split_coefficients<S>(ck4.x * scale_ds, ck4.y * scale_ds, ck4.z * scale_ds, ck4.w * scale_ds);
+                const uint4 sv = split_coefficients<S>(cv4.x * by_p, cv4.y * by_p, cv4.z * by_p, cv4.w * by_p);
                 __builtin_amdgcn_sched_barrier(0);
                 block_blend4_pair<S, DC>(rq, __builtin_bit_cast(shortx4, make_uint2(sk.x, sk.y)),
                                          __builtin_bit_cast(shortx4, make_uint2(sk.z, sk.w)), mK);
@@ -726,6 +740,11 @@ __device__ __forceinline__ void cell_sums(
             tail += prepare(cnext, tail, e_a.id, make_float2(e_a.fx, e_a.fy), pd_a);
             wave_lds_sync();
             e_a = e_n;
+        }
+        if constexpr (kScaled) {
+            const float un = 1.0f / scale_ds;
+#pragma unroll
+            for (int d = 0; d < DC; ++d) { mK[d] *= un; mV[d] *= 1.0f / kScaleP; }
         }
     }
     if constexpr (!kQuad) {

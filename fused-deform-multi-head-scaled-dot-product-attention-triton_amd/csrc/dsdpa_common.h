@@ -450,6 +450,22 @@ __device__ __forceinline__ uint4 split_coefficients(float c0, float c1, float c2
     }
 }
 
+__device__ __forceinline__ float first_lane(float x) { return __uint_as_float((unsigned)__builtin_amdgcn_readfirstlane((int)__float_as_uint(x))); }
+// fp16 has five bits of exponent, fp32 coefficients eight: before they are split they are multiplied by a power of two, and
+// their sums divided by it. p <= 1 (and what one query's samples of a cell add up to) by kScaleP, sm_scale * ds by a scale that
+// follows the largest magnitude seen so far: `scale` is lowered to put `top` between 2^13 and 2^14 where it would pass 2^14,
+// and what the sums made until then have to be multiplied by is returned (1: nothing). From kScaleDs on.
+constexpr float kScaleP = 32768.0f, kScaleDs = 0x1p110f;
+__device__ __forceinline__ float lower_scale(float top, float &scale)
+{
+    if (!(top * scale > 16384.0f)) return 1.0f;
+    const int ex = (int)((__float_as_uint(top) >> 23) & 0xffu) - 127;
+    const float s = __uint_as_float((unsigned)(13 - ex + 127) << 23);              // 2^(13 - ex), ex in [-97, 128]
+    const float by = s / scale;
+    scale = s;
+    return by;
+}
+
 __device__ __forceinline__ uint4 lane_offsets(const uint4 &e, unsigned lane_byte)
 {
     return make_uint4(e.x + lane_byte, e.y + lane_byte, e.z + lane_byte, e.w + lane_byte);

@@ -21,8 +21,7 @@
 //                   product t is element E*n + t: no data crosses lanes). The coefficients are split in a high and a low
 //                   part of the storage type, one product each; two byte permutes make the operand of a pair of rows.
 //   fp32            v_mfma_f32_16x16x4_f32: one entry per lane group and instruction, everything in fp32.
-// fp16 has 5 bits of exponent: its coefficients are scaled by powers of two, p by 2^13 (p <= 1), ds by a scale that
-// follows the largest |ds| seen so far (the sums are rescaled when it grows).
+// fp16 has 5 bits of exponent: its coefficients are scaled by powers of two (lower_scale).
 //
 // A non-finite query row times the zeros of its column would reach all sixteen pixels: where a patch's sums
 // come out non-finite, the workgroup works it out again entry by entry, each for the pixels it touches only.
@@ -183,8 +182,8 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
     floatx4 mK[E], mV[E];
 #pragma unroll
     for (int i = 0; i < E; ++i) { mK[i] = floatx4{0.f, 0.f, 0.f, 0.f}; mV[i] = floatx4{0.f, 0.f, 0.f, 0.f}; }
-    constexpr float kScaleP = kF16 ? 8192.0f : 1.0f;
-    float scale_ds = kF16 ? 0x1p110f : 1.0f, rescale = 1.0f;
+    constexpr float kByP = kF16 ? kScaleP : 1.0f;
+    float scale_ds = kF16 ? kScaleDs : 1.0f, rescale = 1.0f;
     (void)rescale;
 
     // C of one block of 64 entries, and the entries' row offsets. The places written are kept for the clearing.
@@ -199,17 +198,10 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
         const unsigned rows = (r >= 1 ? 3u : 0u) | (r <= 3 ? 12u : 0u), cols = (c >= 1 ? 5u : 0u) | (c <= 3 ? 10u : 0u);
         float ds = f.pd.y;
         if constexpr (kF16) {
-            const float top = wave_max(live ? fabsf(ds) : 0.f);
-            rescale = 1.0f;
-            if (top * scale_ds > 16384.0f) {
-                const int ex = (int)((__float_as_uint(top) >> 23) & 0xffu) - 127;
-                const float s = __uint_as_float((unsigned)(13 - ex + 127) << 23);      // 2^(13 - ex), ex in [-97, 128]
-                rescale = s / scale_ds;
-                scale_ds = s;
-            }
+            rescale = lower_scale(first_lane(wave_max(live ? fabsf(ds) : 0.f)), scale_ds);
             ds *= scale_ds;
         }
-        const float p = f.pd.x * kScaleP;
+        const float p = f.pd.x * kByP;
         zmask = live ? rows & cols : 0u;
         zat = ((r - 1) * kPatchSide + (c - 1)) * kPatchPitch + lane;
 #pragma unroll
@@ -347,7 +339,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
     if constexpr (kF16) {
         const float uk = 1.0f / scale_ds;
 #pragma unroll
-        for (int i = 0; i < E; ++i) { mK[i] *= uk; mV[i] *= 1.0f / kScaleP; }
+        for (int i = 0; i < E; ++i) { mK[i] *= uk; mV[i] *= 1.0f / kByP; }
     }
 
     // Sum of the waves through LDS, and the stores: the patch as [pixel][column], dk and then dv.

@@ -38,7 +38,7 @@ def check(B, V, H, Himg, Wimg, D, P, scale, qk, v_size, dout_size, names=("dk", 
         assert rms(a - b) <= 2 * stored + 1e-3 * rms(b), (name, rms(a - b), stored, rms(b))
 
 
-@pytest.fixture(params=[True], ids=["deterministic"])
+@pytest.fixture(params=[False, True], ids=["default", "deterministic"])
 def mode(request):
     prev = torch.are_deterministic_algorithms_enabled()
     torch.use_deterministic_algorithms(request.param)
