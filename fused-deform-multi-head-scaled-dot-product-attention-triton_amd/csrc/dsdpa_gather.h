@@ -909,10 +909,18 @@ __global__ __launch_bounds__(kGatherWaves *kWave, (WIN && !CG && DC <= 8) ? 4 : 
                 atomicAdd(&tA[te.z], (double)(ds * w2));
                 atomicAdd(&tA[te.w], (double)(ds * w3));
                 wave_lds_sync();
+                float c0f = 0.f, c1f = 0.f, c2f = 0.f, c3f = 0.f, un = 1.0f;
                 if (lane < nquads) {
                     const uint4 ent = *reinterpret_cast<const uint4 *>(q_ent + 4 * lane);
-                    const float c0f = (float)tA[ent.x], c1f = (float)tA[ent.y];
-                    const float c2f = (float)tA[ent.z], c3f = (float)tA[ent.w];
+                    c0f = (float)tA[ent.x]; c1f = (float)tA[ent.y]; c2f = (float)tA[ent.z]; c3f = (float)tA[ent.w];
+                }
+                if constexpr (kBlock && !S::kBf16) {               // (fp16: the chunk's own scale, see lower_scale)
+                    float scale = kScaleDs;
+                    (void)lower_scale(first_lane(wave_max(fmaxf(fmaxf(fabsf(c0f), fabsf(c1f)), fmaxf(fabsf(c2f), fabsf(c3f))))), scale);
+                    c0f *= scale; c1f *= scale; c2f *= scale; c3f *= scale;
+                    un = 1.0f / scale;
+                }
+                if (lane < nquads) {
                     if constexpr (kBlock) {
                         tC[2 * lane] = split_coefficients<S>(c0f, c1f, c2f, c3f);
                         tC[2 * lane + 1] = make_uint4(0u, 0u, 0u, 0u);
@@ -940,7 +948,7 @@ __global__ __launch_bounds__(kGatherWaves *kWave, (WIN && !CG && DC <= 8) ? 4 : 
                     step(0, std::true_type{});
                     for (int q0 = NS; q0 < nquads; q0 += NS) step(q0, std::false_type{});
 #pragma unroll
-                    for (int d = 0; d < DC; ++d) dqa[d] += macc[d][0] + macc[d][1];
+                    for (int d = 0; d < DC; ++d) dqa[d] = fmaf(macc[d][0] + macc[d][1], un, dqa[d]);
                 } else {
                     for (int q0 = 0; q0 < nquads; q0 += NS) {
                         const int qd = min(q0 + slot, nquads - 1);

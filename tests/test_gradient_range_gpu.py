@@ -17,13 +17,15 @@ from ops.triton import deform_sdpa_triton
 pytestmark = pytest.mark.gpu
 
 
-def check(B, V, H, Himg, Wimg, D, P, scale, qk, v_size, dout_size, names=("dk", "dv")):
+def check(B, V, H, Himg, Wimg, D, P, scale, qk, v_size, dout_size, names=("dk", "dv"), clustered=False):
     print(f"[case] range B{B} V{V} H{H} {Himg}x{Wimg} D{D} P{P} qk {qk} dout {dout_size}", flush=True)
     g = torch.Generator().manual_seed(D + P)
     L = Himg * Wimg
     q, k, v, dout = (torch.randn(B, V, H, L, D, generator=g) for _ in range(4))
     q, k, v, dout = ((t * f).half() for t, f in zip((q, k, v, dout), (qk, qk, v_size, dout_size)))
     coords = torch.rand(B, V, L, V, P, 2, generator=g) * 1.2 - 0.1
+    if clustered:
+        coords = 0.4 + 0.2 * torch.rand(B, V, L, V, 1, 2, generator=g) + 0.03 * torch.randn(B, V, L, V, P, 2, generator=g)
     leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
     deform_sdpa_triton(*leaves, coords.cuda(), Wimg, Himg, scale).backward(dout.cuda())
     torch.cuda.synchronize()
@@ -56,3 +58,10 @@ def test_small_gradients(D, dout, mode):
 # sm_scale * ds beyond 65504 where q and k are small, dq, dk and dv all finite
 def test_coefficients_beyond_the_largest_fp16(mode):
     check(1, 4, 2, 18, 19, 128, 16, 100.0, 0.015, 2.0, 5e3, names=("dq", "dk", "dv"))
+
+
+# 64 samples around one place: dq by the pixels of a query's window (a scale of one: sm_scale multiplies the sums, after them)
+@pytest.mark.parametrize("dout", [1.0, 1e-4, 1e-5])
+@pytest.mark.parametrize("D", [64, 128])
+def test_small_gradients_of_clustered_samples(D, dout, mode):
+    check(1, 2, 2, 31, 33, D, 64, 1.0, 1.0 / D ** 0.25, 1.0, dout, names=("dq", "dk", "dv"), clustered=True)
