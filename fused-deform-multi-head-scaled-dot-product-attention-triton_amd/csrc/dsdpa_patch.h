@@ -18,8 +18,12 @@
 // ahead, straight from memory into the layout of the B operand -- are multiplied:
 //   16-bit storage  v_mfma_f32_16x16x32: lane group lane/16 holds eight entries, lane % 16 = column n: E = D/16
 //                   consecutive elements of each row, element t of every lane in product t (so output column n of
-//                   product t is element E*n + t: no data crosses lanes). The coefficients are split in a high and a low
-//                   part of the storage type, one product each; two byte permutes make the operand of a pair of rows.
+//                   product t is element E*n + t: no data crosses lanes). The coefficients are split in parts of the storage
+//                   type, one product each: two in fp16 (good to 2^-23), three in bf16 (two are good to 2^-17, which rows
+//                   that cancel show); two byte permutes make the operand of a pair of rows. The third part costs a third of
+//                   the tables' LDS, 13.7 KB a wave for 9.4. us a step, cells / two parts / three, bf16: 18x18, 32 heads, D = 32, 6 views x 6
+//                   samples 351 / 274 / 292, 12 x 4 797 / 670 / 701; 20x20, 4 x 6, D = 64 229 / 182 / 186; 40x28, 4 x 8,
+//                   coherent, D = 128 581 / 425 / 441.
 //   fp32            v_mfma_f32_16x16x4_f32: one entry per lane group and instruction, everything in fp32.
 // fp16 has 5 bits of exponent: its coefficients are scaled by powers of two (lower_scale).
 //
@@ -42,8 +46,10 @@ constexpr int kPatchSide = 4, kPatchPixels = kPatchSide * kPatchSide;
 constexpr int kPatchMaxWaves = 4;
 constexpr int kPatchPitch = kWave + 4;             // dwords between two rows of C: 16-byte reads of 16 rows cover all banks
 constexpr int kPatchC = kPatchPixels * kPatchPitch;
-constexpr int kPatchWaveDwords = 2 * kPatchC + 2 * kWave + 5 * 8 + 4;   // C of ds, C of p, row offsets in q and dout, list bounds, a flag
-constexpr size_t patch_lds_bytes(int waves) { return (size_t)waves * kPatchWaveDwords * 4; }
+// per wave: C of ds, C of p (bf16: and their third parts), row offsets in q and dout, list bounds, a flag
+template <typename S> constexpr int kPatchTables = S::kBf16 ? 3 : 2;
+template <typename S> constexpr int kPatchWaveDwords = kPatchTables<S> * kPatchC + 2 * kWave + 5 * 8 + 4;
+template <typename S> constexpr size_t patch_lds_bytes(int waves) { return (size_t)waves * kPatchWaveDwords<S> * 4; }
 
 struct PatchGrid {
     int npx, npatch;                        // patches per row and per plane
@@ -63,24 +69,28 @@ __device__ __forceinline__ void load_piece(const char *p, uint32_t (&w)[(BYTES +
     else load_words<BYTES / 4>(p, w);
 }
 
-// A coefficient as (high part | low part << 16) of the storage type; high + low is good to 2^-17 (bf16) or 2^-22 (fp16).
+// A coefficient as (high part | low part << 16) of the storage type, and in `rest` what they leave of it: nothing that
+// matters in fp16 (good to 2^-23), a third part in bf16 (2^-17 without it).
 template <typename S>
-__device__ __forceinline__ uint32_t split_pack(float c)
+__device__ __forceinline__ uint32_t split_pack(float c, float &rest)
 {
     using T = std::conditional_t<S::kBf16, __bf16, _Float16>;
     typedef T pair_t __attribute__((ext_vector_type(2)));
     const T hi = (T)c;
-    return __builtin_bit_cast(uint32_t, pair_t{hi, (T)(c - (float)hi)});
+    const float r = c - (float)hi;
+    const T lo = (T)r;
+    rest = r - (float)lo;
+    return __builtin_bit_cast(uint32_t, pair_t{hi, lo});
 }
 
 template <typename S, int D, int DP>
-__global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_dkdv_patch_kernel(
+__global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 : 4) void bwd_dkdv_patch_kernel(
     const void *__restrict__ q_, const void *__restrict__ dout_, const unsigned *__restrict__ start,
     const unsigned *__restrict__ sorted, const unsigned *__restrict__ left, const float2 *__restrict__ handed_,
     void *__restrict__ dk_, void *__restrict__ dv_, float *__restrict__ dk_acc, float *__restrict__ dv_acc, Dims dm, int NC,
     PatchGrid pg)
 {
-    constexpr bool k16 = S::kBytes == 2, kF16 = k16 && !S::kBf16;
+    constexpr bool k16 = S::kBytes == 2, kBf16 = S::kBf16, kF16 = k16 && !kBf16;
     constexpr int E = DP / 16;                        // elements of a row per lane
     constexpr int EPL = k16 ? 8 : 4;                  // entries per lane group and step
     constexpr int STEP = 4 * EPL, NSTEP = kWave / STEP;
@@ -90,9 +100,9 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
 
     const int nw = (int)(blockDim.x >> 6);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    unsigned *const base = smem_patch + wave * kPatchWaveDwords;
-    unsigned *const ck = base, *const cv = base + kPatchC;
-    unsigned *const s_qrow = base + 2 * kPatchC, *const s_row = s_qrow + kWave, *const s_bnd = s_row + kWave;
+    unsigned *const base = smem_patch + wave * kPatchWaveDwords<S>;
+    unsigned *const ck = base, *const cv = base + kPatchC, *const cl = base + 2 * kPatchC;       // cl: bf16's third parts, ds | p << 16
+    unsigned *const s_qrow = base + kPatchTables<S> * kPatchC, *const s_row = s_qrow + kWave, *const s_bnd = s_row + kWave;
 
     // plane-major: (b, h, s2, patch)
     const unsigned work = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x);
@@ -209,8 +219,10 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
             if (zmask & (1u << i)) {
                 const int at = zat + ((i >> 1) * kPatchSide + (i & 1)) * kPatchPitch;
                 if constexpr (k16) {
-                    ck[at] = split_pack<S>(w[i] * ds);
-                    cv[at] = split_pack<S>(w[i] * p);
+                    float rk, rv;
+                    ck[at] = split_pack<S>(w[i] * ds, rk);
+                    cv[at] = split_pack<S>(w[i] * p, rv);
+                    if constexpr (kBf16) cl[at] = __builtin_bit_cast(uint32_t, dsdpa_bf16x2{(__bf16)rk, (__bf16)rv});
                 } else {
                     ck[at] = __float_as_uint(w[i] * ds);
                     cv[at] = __float_as_uint(w[i] * p);
@@ -229,6 +241,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
                 const int at = zat + ((i >> 1) * kPatchSide + (i & 1)) * kPatchPitch;
                 ck[at] = 0u;
                 cv[at] = 0u;
+                if constexpr (kBf16) cl[at] = 0u;
             }
         }
     };
@@ -253,14 +266,15 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
         for (int i = 0; i < EPL / 4; ++i) f.x[i] = src[i];
         return f;
     };
-    auto multiply = [&](const Coefs &f, const uint32_t (&r)[EPL][WORDS], floatx4 (&acc)[E]) {
+    // (g, half: bf16's third parts, in the low or the high halves)
+    auto multiply = [&](const Coefs &f, const Coefs &g, unsigned half, const uint32_t (&r)[EPL][WORDS], floatx4 (&acc)[E]) {
         if constexpr (k16) {
-            const uint4 a = f.x[0], c = f.x[EPL / 4 - 1];
             auto pick = [](unsigned y, unsigned x, unsigned sel) { return __builtin_amdgcn_perm(y, x, sel); };
-            const uint4 hi = make_uint4(pick(a.y, a.x, 0x05040100u), pick(a.w, a.z, 0x05040100u),
-                                        pick(c.y, c.x, 0x05040100u), pick(c.w, c.z, 0x05040100u));
-            const uint4 lo = make_uint4(pick(a.y, a.x, 0x07060302u), pick(a.w, a.z, 0x07060302u),
-                                        pick(c.y, c.x, 0x07060302u), pick(c.w, c.z, 0x07060302u));
+            auto part = [&](const Coefs &t, unsigned sel) {
+                const uint4 a = t.x[0], c = t.x[EPL / 4 - 1];
+                return make_uint4(pick(a.y, a.x, sel), pick(a.w, a.z, sel), pick(c.y, c.x, sel), pick(c.w, c.z, sel));
+            };
+            const uint4 hi = part(f, 0x05040100u), lo = part(f, 0x07060302u), third = kBf16 ? part(g, half) : hi;
 #pragma unroll
             for (int i = 0; i < E; ++i) {
                 const unsigned sel = (i & 1) ? 0x07060302u : 0x05040100u;
@@ -268,6 +282,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
                                            pick(r[EPL - 3][i / 2], r[EPL - 4][i / 2], sel), pick(r[EPL - 1][i / 2], r[EPL - 2][i / 2], sel));
                 acc[i] = mfma_16x16x32<S>(hi, x, acc[i]);
                 acc[i] = mfma_16x16x32<S>(lo, x, acc[i]);
+                if constexpr (kBf16) acc[i] = mfma_16x16x32<S>(third, x, acc[i]);
             }
         } else {
             const uint32_t a[4] = { f.x[0].x, f.x[0].y, f.x[0].z, f.x[0].w };
@@ -280,7 +295,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
         }
     };
 
-    for (int i = lane; i < 2 * kPatchC / 4; i += kWave) reinterpret_cast<uint4 *>(base)[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = lane; i < kPatchTables<S> * kPatchC / 4; i += kWave) reinterpret_cast<uint4 *>(base)[i] = make_uint4(0u, 0u, 0u, 0u);
     const unsigned stride = (unsigned)nw * kWave;
     unsigned first = (unsigned)wave * kWave;                      // the waves take the blocks of 64 entries in turn
     if (first < total) {
@@ -305,7 +320,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
             __builtin_amdgcn_sched_barrier(0);                    // (requested here, not where they are used)
 #pragma unroll
             for (int s = 0; s < NSTEP; ++s) {
-                const Coefs fk = read_coefs(ck, s), fv = read_coefs(cv, s);
+                const Coefs fk = read_coefs(ck, s), fv = read_coefs(cv, s), fl = kBf16 ? read_coefs(cl, s) : Coefs{};
                 if (s == NSTEP - 1 && more) {                     // this block's C has been read: the next block's
                     wave_lds_sync();
                     clear_tables();
@@ -314,11 +329,11 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
                 }
                 const int next = (s + 1) % NSTEP;
                 __builtin_amdgcn_sched_barrier(0);
-                multiply(fk, rq, mK);
+                multiply(fk, fl, 0x05040100u, rq, mK);
                 __builtin_amdgcn_sched_barrier(0);
                 issue(q_bh, s_qrow, next, rq);                    // (behind the last block: rows that nothing uses)
                 __builtin_amdgcn_sched_barrier(0);
-                multiply(fv, rd, mV);
+                multiply(fv, fl, 0x07060302u, rd, mV);
                 __builtin_amdgcn_sched_barrier(0);
                 issue(do_bh, s_row, next, rd);
                 __builtin_amdgcn_sched_barrier(0);
@@ -343,7 +358,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
     }
 
     // Sum of the waves through LDS, and the stores: the patch as [pixel][column], dk and then dv.
-    unsigned &s_bad = smem_patch[kPatchWaveDwords - 1];
+    unsigned &s_bad = smem_patch[kPatchWaveDwords<S> - 1];
     if (threadIdx.x == 0) s_bad = 0u;
     float z = 0.f;
 #pragma unroll
@@ -372,7 +387,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP <= 64 ? 4 : 2) void bwd_d
             for (int d = 0; d < VE; ++d) sum[d] = all[i * VE + d];
             for (int w = 1; w < nw; ++w) {
 #pragma unroll
-                for (int d = 0; d < VE; ++d) sum[d] += all[w * kPatchWaveDwords + i * VE + d];
+                for (int d = 0; d < VE; ++d) sum[d] += all[w * kPatchWaveDwords<S> + i * VE + d];
             }
             size_t elem;
             if (pixel_at(m, elem)) store_chunk<S, VE>((char *)(which == 0 ? dk_ : dv_) + (elem + c) * S::kBytes, sum);

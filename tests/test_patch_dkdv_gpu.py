@@ -75,3 +75,42 @@ def test_non_finite_rows_stay_with_their_pixels(bad, dtype):
         assert 0 < (~np.isfinite(b)).sum() < 2000, name
         ok = np.isfinite(b)
         assert np.abs(a[ok] - b[ok]).max() < BAR[dtype] * np.abs(b[ok]).max(), name
+
+
+# Coefficients (weight times p) to fp32's precision: three queries look at one place, with different p, and the rows of dout
+# cancel down to 2^-13 of their size. What is left takes the storage type's rounding (1.7e-3 in bf16) and that of p and the sums (2^-23 of the
+# terms, a few of them: 2^-10 of the rest); coefficients good to 2^-17 would leave 2^-4 times a third of it (1.5e-2).
+@pytest.mark.parametrize("dtype,kept", [(torch.bfloat16, 2.0 ** -4), (torch.float16, 0.5)], ids=str)
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+def test_coefficients_are_not_rounded_to_16_bits(D, dtype, kept):
+    H, W = 64, 16
+    L, T, scale = W * W, W * W // 3, 1.0 / math.sqrt(D)
+    g = torch.Generator().manual_seed(D)
+    q, k, v, d = (torch.randn(1, 1, H, L, D, generator=g).to(dtype) for _ in range(4))
+    coords = torch.full((1, 1, L, 1, 2, 2), -1.0)                # the second sample: outside, its logit 0
+    place = torch.rand(T, 2, generator=g) * 0.9 + 0.05
+    coords[0, 0, :3 * T, 0, 0] = place.repeat_interleave(3, 0)
+    x, y = (place.double() * (W - 1)).unbind(-1)
+    x0, y0 = x.floor().long(), y.floor().long()
+    fx, fy = x - x0, y - y0
+    taps = [((y0 + j) * W + x0 + i, (fx if i else 1 - fx) * (fy if j else 1 - fy)) for j in (0, 1) for i in (0, 1)]
+    at = sum(w[:, None] * k[0, 0].double()[:, p] for p, w in taps)                                   # (H, T, D): k at the places
+    p = torch.sigmoid(scale * (q[0, 0, :, :3 * T].double().view(H, T, 3, D) * at[:, :, None]).sum(-1))
+    p = [p[..., m, None] for m in range(3)]
+    rows = d[0, 0, :, :3 * T].double().view(H, T, 3, D)[:, :, 0]
+    second = (-p[0] / p[1] * rows).to(dtype)
+    left = p[0] * rows + p[1] * second.double()
+    third = (-(1 - kept) * left / p[2]).to(dtype)
+    left = left + p[2] * third.double()
+    dout = torch.zeros_like(d)
+    dout[0, 0, :, :3 * T] = torch.stack([rows.to(dtype), second, third], 2).view(H, 3 * T, D)
+    want = torch.zeros(H, L, D, dtype=torch.float64)
+    for pix, w in taps:
+        want.index_add_(1, pix, w[:, None] * left)
+    print(f"[case] cancelling rows D{D} {dtype}", flush=True)
+    vd = v.cuda().requires_grad_(True)
+    deform_sdpa_triton(q.cuda(), k.cuda(), vd, coords.cuda(), W, W, scale).backward(dout.cuda())
+    torch.cuda.synchronize()
+    err = float((vd.grad[0, 0].double().cpu() - want).norm() / want.norm())
+    print("error", err, "of", float(left.norm() / rows.norm()))
+    assert err < 8e-3, err
