@@ -225,7 +225,7 @@ __device__ __forceinline__ void scan_keys(const unsigned (&v)[kScanKeys], int c0
     if (lane == kWave - 1) s_wave[wave] = make_uint2(incl, pincl);
     __syncthreads();
     unsigned excl = carry.entries + incl - sum, pexcl = carry.pieces + pincl - psum;
-#pragma unroll
+#pragma unroll 4                                                      // (unrolled whole: 100 bytes of scratch a lane at 64 registers)
     for (int w = 0; w < THREADS / kWave; ++w) {
         const uint2 t = s_wave[w];
         excl += w < wave ? t.x : 0u;

@@ -354,7 +354,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
 
     // per row block: this slot's row and its state
     bool have_s[ROWS];
-    size_t row_s[ROWS], crow_s[ROWS];
+    unsigned qc_s[ROWS];
     float qf_s[ROWS][DC], acc_s[ROWS][DC], m_s[ROWS], lsum_s[ROWS];
     uint32_t qp_s[ROWS][kPacked ? DC / 2 : 1];
 #pragma unroll
@@ -363,8 +363,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
         have_s[rb] = qidx < nq;
         const unsigned qc = (unsigned)(have_s[rb] ? qidx : nq - 1);
         const unsigned s1 = dm.divL.div(qc), l = qc - s1 * (unsigned)dm.L;
-        row_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l;
-        crow_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.L + l) * (size_t)dm.N;
+        qc_s[rb] = qc;
         if constexpr (kPacked) {
             load_packed<S, DC>((const char *)q_ + dm.q_row(pb.b, (int)s1, pb.h, (int)l) * S::kBytes + lane_byte, qp_s[rb]);
         } else {
@@ -386,7 +385,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
         __syncthreads();
 #pragma unroll
         for (int rb = 0; rb < ROWS; ++rb) {
-        const size_t crow = crow_s[rb];
+        const size_t crow = ((size_t)pb.b * nq + qc_s[rb]) * (size_t)dm.N;
         const float (&qf)[DC] = qf_s[rb];
         const uint32_t (&qp)[kPacked ? DC / 2 : 1] = qp_s[rb];
         float (&acc)[DC] = acc_s[rb];
@@ -470,8 +469,10 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void fwd_slot_kernel(
             const float inv = 1.0f / lsum_s[rb];
 #pragma unroll
             for (int d = 0; d < DC; ++d) acc_s[rb][d] *= inv;
-            Lane::store((char *)out_ + row_s[rb] * (size_t)kRow, lane_byte, acc_s[rb]);
-            if (g == 0) lse_[row_s[rb]] = m_s[rb] + __log2f(lsum_s[rb]);
+            const unsigned s1 = dm.divL.div(qc_s[rb]), l = qc_s[rb] - s1 * (unsigned)dm.L;
+            const size_t row = (((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l;
+            Lane::store((char *)out_ + row * (size_t)kRow, lane_byte, acc_s[rb]);
+            if (g == 0) lse_[row] = m_s[rb] + __log2f(lsum_s[rb]);
         }
     }
 }
@@ -496,6 +497,9 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
     constexpr int G = D / DC, NS = kWave / G;
     constexpr int kRow = D * S::kBytes;
     constexpr bool kPacked = S::kBytes == 2 && !CG;
+    // The scheduler requests a trip's taps all together, which at 16 waves a workgroup, 128 registers a lane, spills in these
+    // forms; they, and the coordinate gradient, are held to one pair of taps, or one tap, at a time.
+    constexpr bool kTight = (DC == 16 && S::kBytes == 2) || (HAND && ROWS == 2 && S::kBytes * DC == 32);
     static_assert(G >= 2 && G <= 16 && G * DC == D, "lane split");
     extern __shared__ __attribute__((aligned(kPlaneLdsAlign))) unsigned char smem[];
     const int img_bytes = plane_lds_bytes<S, D>(dm.L);
@@ -518,7 +522,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
 
     // per row block: this slot's row and its state
     bool have_s[ROWS];
-    size_t crow_s[ROWS], roff_s[ROWS], hrow_s[ROWS];
+    unsigned qc_s[ROWS];
     float qf_s[ROWS][DC], dof_s[ROWS][DC], dqa_s[ROWS][DC], delta_s[ROWS], lse_s[ROWS];
     uint32_t dop_s[ROWS][kPacked ? DC / 2 : 1];
 #pragma unroll
@@ -528,10 +532,8 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         const unsigned qc = (unsigned)(have_s[rb] ? qidx : nq - 1);
         const unsigned s1 = dm.divL.div(qc), l = qc - s1 * (unsigned)dm.L;
         const size_t row = (((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l;
-        crow_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.L + l) * (size_t)dm.N;
-        hrow_s[rb] = ((size_t)(pb.b * dm.H + pb.h - bh0) * nq + qc) * (size_t)dm.N;
+        qc_s[rb] = qc;
         const size_t roff = row * (size_t)kRow;
-        roff_s[rb] = roff;
         float of[DC];
         Lane::load((const char *)q_ + dm.q_row(pb.b, (int)s1, pb.h, (int)l) * S::kBytes, lane_byte, qf_s[rb]);
         Lane::load((const char *)dout_ + roff, lane_byte, dof_s[rb]);
@@ -554,7 +556,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
 #pragma unroll
         for (int rb = 0; rb < ROWS; ++rb) {
         const bool have = have_s[rb];
-        const size_t crow = crow_s[rb];
+        const size_t crow = ((size_t)pb.b * nq + qc_s[rb]) * (size_t)dm.N;
         const float (&qf)[DC] = qf_s[rb];
         const float (&dof)[DC] = dof_s[rb];
         const uint32_t (&dop)[kPacked ? DC / 2 : 1] = dop_s[rb];
@@ -580,19 +582,26 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                     for (int d = 0; d < DC; ++d) kk[d] = 0.f;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        float tk[DC], tv[DC];
+                        float tk[DC];
                         Lane::read(kp[i], (i & 1) * 2 * kRow, tk);
-                        Lane::read(vp[i], (i & 1) * 2 * kRow, tv);
                         dk_t[i] = 0.f;
-                        dv_t[i] = 0.f;
 #pragma unroll
                         for (int d = 0; d < DC; ++d) {
                             dk_t[i] = fmaf(qf[d], tk[d], dk_t[i]);
-                            dv_t[i] = fmaf(dof[d], tv[d], dv_t[i]);
                             kk[d] = fmaf(wt[i], tk[d], kk[d]);
                         }
                         dot = fmaf(wt[i], dk_t[i], dot);
+                        if (DC == 16 || (i & 1)) __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float tv[DC];
+                        Lane::read(vp[i], (i & 1) * 2 * kRow, tv);
+                        dv_t[i] = 0.f;
+#pragma unroll
+                        for (int d = 0; d < DC; ++d) dv_t[i] = fmaf(dof[d], tv[d], dv_t[i]);
                         dp = fmaf(wt[i], dv_t[i], dp);
+                        if (DC == 16 || (i & 1)) __builtin_amdgcn_sched_barrier(0);
                     }
                     dot = group_sum<G>(dot);
                     dp = group_sum<G>(dp);
@@ -613,7 +622,11 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                     float gy = fmaf(gf.x, (g3 - g1) - dy0, dy0) * (float)(dm.Himg - 1);
                     gx = group_sum<G>(gx);
                     gy = group_sum<G>(gy);
-                    if (t == my_trip) { my_gx = gx; my_gy = gy; my_p = p; my_ds = ds; }
+                    const bool mine = t == my_trip;                     // (selects: behind a branch the compiler spilled 276 bytes a lane)
+                    my_gx = mine ? gx : my_gx;
+                    my_gy = mine ? gy : my_gy;
+                    my_p = mine ? p : my_p;
+                    my_ds = mine ? ds : my_ds;
                     continue;
                 }
                 const uint32_t at = e.x + lbase, ab = e.y + lbase;
@@ -622,42 +635,48 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                 float dot = 0.f, dp = 0.f;
                 {
                     float t0[DC], t1[DC], t2[DC], t3[DC];
-                    Lane::read(at, 0, t0);
-                    Lane::read(at ^ kRow, 2 * kRow, t1);
                     Lane::read(ab, 0, t2);
                     Lane::read(ab ^ kRow, 2 * kRow, t3);
 #pragma unroll
+                    for (int d = 0; d < DC; ++d) kk[d] = fmaf(w.z, t2[d], w.w * t3[d]);
+                    if constexpr (kTight) __builtin_amdgcn_sched_barrier(0);
+                    Lane::read(at, 0, t0);
+                    Lane::read(at ^ kRow, 2 * kRow, t1);
+#pragma unroll
                     for (int d = 0; d < DC; ++d) {
-                        kk[d] = fmaf(w.x, t0[d], fmaf(w.y, t1[d], fmaf(w.z, t2[d], w.w * t3[d])));
+                        kk[d] = fmaf(w.x, t0[d], fmaf(w.y, t1[d], kk[d]));
                         dot = fmaf(qf[d], kk[d], dot);
                     }
                 }
+                if constexpr (kTight) __builtin_amdgcn_sched_barrier(0);
                 if constexpr (kPacked) {
                     dp = tap_dot16<S, DC>(lds_at(at ^ kRow), lds_at(at + 2 * kRow), lds_at(ab ^ kRow), lds_at(ab + 2 * kRow), w, dop);
                 } else {
                     float u0[DC], u1[DC], u2[DC], u3[DC];
-                    Lane::read(at ^ kRow, 0, u0);
-                    Lane::read(at, 2 * kRow, u1);
                     Lane::read(ab ^ kRow, 0, u2);
                     Lane::read(ab, 2 * kRow, u3);
 #pragma unroll
-                    for (int d = 0; d < DC; ++d) {
-                        const float vv = fmaf(w.x, u0[d], fmaf(w.y, u1[d], fmaf(w.z, u2[d], w.w * u3[d])));
-                        dp = fmaf(dof[d], vv, dp);
-                    }
+                    for (int d = 0; d < DC; ++d) u3[d] = fmaf(w.z, u2[d], w.w * u3[d]);
+                    if constexpr (kTight) __builtin_amdgcn_sched_barrier(0);
+                    Lane::read(at ^ kRow, 0, u0);
+                    Lane::read(at, 2 * kRow, u1);
+#pragma unroll
+                    for (int d = 0; d < DC; ++d) dp = fmaf(dof[d], fmaf(w.x, u0[d], fmaf(w.y, u1[d], u3[d])), dp);
                 }
                 dot = group_sum<G>(dot);
                 dp = group_sum<G>(dp);
                 const float p = __builtin_amdgcn_exp2f(dot * qscale - lse);
                 const float ds = p * (dp - delta);
                 if constexpr (HAND) {
-                    if (t == my_trip) { my_p = p; my_ds = ds; }
+                    my_p = t == my_trip ? p : my_p;
+                    my_ds = t == my_trip ? ds : my_ds;
                 }
 #pragma unroll
                 for (int d = 0; d < DC; ++d) dqa[d] = fmaf(ds, kk[d], dqa[d]);
             }
             if (HAND && have && c0 + g < dm.P)
-                handed_[hrow_s[rb] + (size_t)(s2 * dm.P + my_n)] = make_float2(my_p, my_ds * dm.sm_scale);
+                handed_[((size_t)(pb.b * dm.H + pb.h - bh0) * nq + qc_s[rb]) * (size_t)dm.N + (size_t)(s2 * dm.P + my_n)] =
+                    make_float2(my_p, my_ds * dm.sm_scale);
             if (CG && have && c0 + g < dm.P) {
                 float *dst = dcoords_ + 2 * (crow + (size_t)s2 * dm.P + (size_t)my_n);
                 atomicAdd(dst, my_gx);
@@ -672,7 +691,8 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         if (have_s[rb]) {
 #pragma unroll
             for (int d = 0; d < DC; ++d) dqa_s[rb][d] *= dm.sm_scale;
-            Lane::store((char *)dq_ + roff_s[rb], lane_byte, dqa_s[rb]);
+            const unsigned s1 = dm.divL.div(qc_s[rb]), l = qc_s[rb] - s1 * (unsigned)dm.L;
+            Lane::store((char *)dq_ + ((((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l) * (size_t)kRow, lane_byte, dqa_s[rb]);
         }
     }
 }

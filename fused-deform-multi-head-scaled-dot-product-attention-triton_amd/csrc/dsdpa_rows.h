@@ -255,6 +255,7 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
                     if constexpr (CG) dk_t[i] = fmaf(qf[d], tk[d], dk_t[i]);
                 }
                 if constexpr (CG) dot = fmaf(wt[i], dk_t[i], dot);
+                if constexpr (CG && S::kBf16) __builtin_amdgcn_sched_barrier(0);   // (widening tap by tap: 107 registers for 130, four waves a SIMD)
                 if constexpr (kPacked) {
                     dp = fmaf(wt[i], packed_dot<S, DC>(dop, vr[i]), dp);
                 } else {

@@ -1,0 +1,44 @@
+"""Scratch memory (register spills) and waves per SIMD of the built kernels, from the metadata that the compiler wrote into the
+library: the staged, row, patch and binning kernels run from registers, apart from the forms named here, whose state is two query
+rows or rows of 256 elements in 128 registers (16 waves a workgroup)."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from ops import _native
+
+READELF = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-readelf")
+# bytes a lane; fwd_slot_kernel<storage, D, elements a lane, row blocks>
+SPILLED = {"fwd_slot_kernel<BF16, 64, 8, 2>": 80, "fwd_slot_kernel<BF16, 256, 16, 1>": 8, "fwd_slot_kernel<F32, 256, 16, 1>": 52,
+           "fwd_slot_kernel<F32, 64, 8, 1>": 8}
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    if not (os.path.exists(_native.LIB_PATH) and os.path.exists(READELF)):
+        pytest.skip("no built library, or no llvm-readelf")
+    blob, out = open(_native.LIB_PATH, "rb").read(), {}
+    for m in re.finditer(rb"\x7fELF\x02\x01\x01\x40", blob):           # (64: the AMD GPU ABI)
+        part = tmp_path_factory.mktemp("co") / "code.o"
+        part.write_bytes(blob[m.start():])
+        notes = subprocess.run([READELF, "--notes", str(part)], capture_output=True, text=True).stdout
+        for entry in notes.split("- .agpr_count:")[1:]:
+            field = lambda name: re.search(r"\." + name + r":\s+(\S+)", entry).group(1)
+            out[field("name")] = (int(field("private_segment_fixed_size")), int(field("vgpr_count")))
+    names = subprocess.run(["c++filt"], input="\n".join(out), capture_output=True, text=True).stdout.splitlines()
+    short = lambda n: re.sub(r"\(.*", "", n.replace("dsdpa::", "").replace("void ", "")).strip()
+    return {short(n): v for n, v in zip(names, out.values())}
+
+
+def test_main_kernels_do_not_spill(kernels):
+    ours = {n: v for n, v in kernels.items() if re.match(r"(fwd_slot|bwd_dq_slot|fwd_rows|bwd_dq_rows|bwd_dkdv_patch|bin_)", n)}
+    assert len(ours) > 100
+    over = {n: v[0] for n, v in ours.items() if v[0] > SPILLED.get(n, 0)}
+    assert not over, over
+
+
+def test_row_kernels_keep_four_waves_a_simd(kernels):
+    over = {n: v[1] for n, v in kernels.items() if re.match(r"(fwd_rows|bwd_dq_rows)", n) and v[1] > 128}
+    assert not over, over
