@@ -304,7 +304,7 @@ __global__ __launch_bounds__(THREADS, THREADS == 512 ? 8 : 4) void bin_scan_kern
 // no faster; 11664 34.8 against 24.1, 17871 59 against 19.
 // Keys: one per cell, (Himg + 1)(Wimg + 1) <= 2 Himg Wimg + 2 of them, in LDS; the query views are one group (their rows
 // take at most 2 * 2048 * 256 * 4 bytes, below where views_per_group splits them).
-constexpr int kBinOneSamples = 2 * 1024, kBinOneKeys = 2 * kBinOneSamples + 2, kBinOneKeyBits = 13;
+constexpr int kBinOneKeys = 2 * kBinOneSamples + 2, kBinOneKeyBits = 13;
 static_assert(kBinOneKeys < (1 << kBinOneKeyBits), "a key fits below its rank");
 static_assert(2ull * kBinOneSamples * 256 * 4 <= kGroupRowsBytes, "one group of query views");
 template <int PER>

@@ -224,7 +224,8 @@ inline bool slab_path_fits(size_t V, size_t Himg, size_t Wimg, size_t D, size_t 
 //   handed   bhg*V*L*(V*P) x 8 bytes         (p, sm_scale*ds) per query*sample of one GROUP of bhg (batch, head) pairs,
 //                                            dq kernel -> dk/dv kernel (shapes on the gather kernels, and short lists);
 //                                            at most kHandedCapBytes whatever the shape
-//   acc      2*n floats                      fp32 dk/dv accumulators (16-bit storage only)
+//   acc      2*n floats                      fp32 dk/dv accumulators (16-bit storage, not deterministic; in the place of `handed` where
+//                                            patches of few samples need none)
 //   desc     20 bytes per coordinate pair    descriptor table (only when the plane kernels apply); 36 with
 //                                            the coordinate gradient
 // deterministic backward only (DSDPA_FLAG_DETERMINISTIC):
@@ -237,6 +238,9 @@ size_t sort_temp_bytes(size_t n, size_t segments);                       // dsdp
 int sort_cell_lists(void *temp, size_t temp_bytes, const unsigned *ids_in, unsigned *ids_out, size_t n,
                     size_t segments, const unsigned *seg_begin, const unsigned *seg_end, unsigned id_bits,
                     hipStream_t st);
+
+// Samples of a (batch, key view) up to which the binning is one launch (bin_one_kernel).
+constexpr int kBinOneSamples = 2 * 1024;
 
 struct WorkspaceLayout {
     size_t delta, counters, start, sorted, frac, items, handed, handed_bytes, acc, desc, sorted2, seg, sorttmp, sorttmp_bytes, taps, total;
@@ -330,7 +334,7 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
     w.NC = (int)((Himg + 1) * (Wimg + 1));
     size_t off = 0;
     w.delta = off; off += round256(rows * 8);           // (lse, delta) per row
-    const size_t L = Himg * Wimg, esize = storage16 ? 2 : 4, acc_bytes = storage16 ? round256(2 * rows * D * 4) : 0;
+    const size_t L = Himg * Wimg, esize = storage16 ? 2 : 4, acc_bytes = storage16 && !deterministic ? round256(2 * rows * D * 4) : 0;
     const bool planes = plane_path_fits(L, D, esize);
     w.patch = patch_path(B, V, H, Himg, Wimg, P, esize, deterministic);
     w.bh_group = planes && !w.patch ? 0 : handed_group(B, V, H, L, P);
@@ -349,8 +353,11 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
     // dk/dv kernel (see handed_group)
     w.handed = off;
     w.handed_bytes = round256((size_t)w.bh_group * V * L * (V * P) * 8);
-    off += w.handed_bytes;
-    w.acc = off; off += acc_bytes;
+    // (the few samples of 16-bit patches that no cell kernel follows: one room for the pairs, or for the accumulators of a
+    // path that was forced, whichever is in use. 18x18, 2 views x 2 samples, 32 heads, D = 32, batch 2: 12 -> 10.6 MB)
+    const bool shared = w.patch && storage16 && V * L * P <= kBinOneSamples;
+    w.acc = shared ? off : off + w.handed_bytes;
+    off = shared ? off + (w.handed_bytes > acc_bytes ? w.handed_bytes : acc_bytes) : w.acc + acc_bytes;
     // with the coordinate gradient the staged dq kernel needs more LDS; where it no longer fits, dq takes the
     // gather kernel and no table is needed
     w.dl = desc_layout(B, V, Himg, Wimg, D, P, storage16 ? 2 : 4, coords_grad);
@@ -364,21 +371,14 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
         w.seg = off; off += round256(2 * segs * 4);
         w.sorttmp_bytes = round256(sort_temp_bytes(ids, segs));
         w.sorttmp = off; off += w.sorttmp_bytes;
-        // dk and dv as four taps each: groups of equal size, at most kTapsCapBytes or one plane, in the place of the
-        // accumulators, which this backward does not use, as far as that goes
+        // dk and dv as four taps each: groups of equal size, at most kTapsCapBytes or one plane (there are no accumulators)
         const size_t per = 8 * L * D * 4, planes_all = B * H * V;
         size_t g = kTapsCapBytes / per;
         g = g < 1 ? 1 : g > planes_all ? planes_all : g;
         g = g > 32768 ? 32768 : g;                          // (a dimension of the grid)
         const size_t ngroups = (planes_all + g - 1) / g;
         w.tap_planes = (int)((planes_all + ngroups - 1) / ngroups);
-        const size_t taps_bytes = round256((size_t)w.tap_planes * per);
-        if (taps_bytes <= acc_bytes) {
-            w.taps = w.acc;
-        } else {
-            w.taps = off;
-            off += taps_bytes;
-        }
+        w.taps = off; off += round256((size_t)w.tap_planes * per);
     }
     w.total = off;
     return w;

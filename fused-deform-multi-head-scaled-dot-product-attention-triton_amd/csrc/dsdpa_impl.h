@@ -858,7 +858,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     // (neither dk/dv kernel needs the statistics then. The few samples that are binned in one launch are the patches' wherever
     // they lie in 16-bit storage: 18x18, 2 views x 2 samples, clustered, step 58 us with cells, 49 with patches; fp32 50 / 60)
     unsigned *left = patch && !(S::kBytes == 2 && bin_in_one_launch(dm)) ? (unsigned *)stats : nullptr;
-    float2 *handed = patch || (wl.handed_bytes && cell_binned && !staged) ? (float2 *)(ws + wl.handed) : nullptr;
+    float2 *handed = patch || (wl.handed_bytes && wl.acc != wl.handed && cell_binned && !staged) ? (float2 *)(ws + wl.handed) : nullptr;
     // fp32 storage: dk and dv are their own accumulators; 16-bit: fp32 accumulators in the workspace
     float *dk_acc = S::kBytes == 4 ? (float *)dk : (float *)(ws + wl.acc);
     float *dv_acc = S::kBytes == 4 ? (float *)dv : dk_acc + n;

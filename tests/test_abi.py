@@ -116,6 +116,40 @@ def test_workspace_bytes():
     assert fits == expect(1, 2, 1, 21, 22, 32, 4, False) and nofit == fits - table(1, 2, 21, 22, 32, 4, False)
 
 
+def test_backward_workspace_of_short_lists_and_of_the_fixed_order():
+    """What the hand-over of short lists and the taps of the deterministic backward add is bounded."""
+    lib = _native.load()
+    MB = 1 << 20
+
+    def beside(B, V, H, Himg, Wimg, D, P, table):
+        """statistics, lists and tap table, an upper bound within 2 kB of padding"""
+        L, NC, M = Himg * Wimg, (Himg + 1) * (Wimg + 1), V * Himg * Wimg * P
+        return B * V * H * L * 8 + B * V * (2 * NC + 1) * 4 + B * V * M * 12 + B * V * (NC + M // 768 + 1) * 16 + (B * V * M * 20 if table else 0) + 2048
+
+    def pairs_and_sums(code, B, V, H, Himg, Wimg, D, P, table):
+        return lib.dsdpa_bwd_workspace_bytes(code, B, V, H, Himg, Wimg, D, P, 0) - beside(B, V, H, Himg, Wimg, D, P, table)
+
+    # the pairs of all samples (no more than 128 MiB) and, in 16-bit storage, the fp32 sums of the views whose lists are long
+    rows = 2 * 6 * 32 * 324
+    assert pairs_and_sums(_native.DSDPA_F32, 2, 6, 32, 18, 18, 32, 2, True) <= rows * 12 * 8
+    assert pairs_and_sums(_native.DSDPA_BF16, 2, 6, 32, 18, 18, 32, 6, True) <= rows * 36 * 8 + rows * 32 * 8
+    assert pairs_and_sums(_native.DSDPA_BF16, 4, 6, 64, 18, 18, 32, 8, True) <= 128 * MB + 4 * rows * 32 * 8
+    # few samples, which are the patches' wherever they lie: the larger of the two
+    assert pairs_and_sums(_native.DSDPA_BF16, 2, 2, 32, 18, 18, 32, 2, True) <= 2 * 2 * 32 * 324 * 32 * 8
+    assert pairs_and_sums(_native.DSDPA_F16, 1, 2, 64, 32, 16, 16, 2, True) <= 1 * 2 * 64 * 512 * 16 * 8
+
+    # the taps: 8 floats per element of dk, of at most 256 MiB of planes or one plane, and no accumulators
+    def taps(code, B, V, H, Himg, Wimg, D, P, table):
+        det = lib.dsdpa_bwd_workspace_bytes(code, B, V, H, Himg, Wimg, D, P, _native.FLAG_DETERMINISTIC)
+        M, NC = V * Himg * Wimg * P, (Himg + 1) * (Wimg + 1)
+        pairs = 0 if table else min(128 * MB, B * V * H * Himg * Wimg * V * P * 8)
+        return det - beside(B, V, H, Himg, Wimg, D, P, table) - B * V * M * 4 - 2 * B * V * NC * 4 - pairs - 4096
+    assert taps(_native.DSDPA_F32, 2, 6, 8, 18, 18, 32, 32, True) <= 2 * 6 * 8 * 324 * 32 * 32 + 64 * 1024
+    assert taps(_native.DSDPA_F32, 1, 1, 17, 46, 46, 256, 4, False) <= 256 * MB + 64 * 1024
+    assert taps(_native.DSDPA_BF16, 1, 4, 8, 64, 64, 128, 16, False) <= 256 * MB + 64 * 1024
+    assert taps(_native.DSDPA_F32, 1, 1, 2, 256, 256, 256, 2, False) <= 256 * 256 * 256 * 32 + 64 * 1024
+
+
 def test_argument_validation_before_launch():
     """Bad arguments are rejected with an error code before anything touches the GPU."""
     lib = _native.load()
