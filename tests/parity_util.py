@@ -55,3 +55,13 @@ def spread_slices(B, H, n=4):
         if len(out) == n:
             break
     return out
+
+
+def kernels_of(call):
+    """The names of the library's kernels that `call` launches (with template arguments, without parameters)."""
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    names = (e.key for e in prof.key_averages())
+    return {n.replace("dsdpa::", "").replace("void ", "").split("(")[0].strip() for n in names if "dsdpa::" in n}

@@ -51,10 +51,10 @@ CASES = [
     (42, 2, 3, 2, 6, 4, 32, 23, -0.1, 1.1),
     (43, 1, 4, 3, 7, 9, 32, 32, 0.0, 1.0),
     (44, 1, 2, 2, 5, 6, 64, 17, -0.5, 1.5),
-    (45, 1, 2, 1, 1, 1, 16, 1, 0.0, 1.0),        # 1x1 image: every colour pass but one is empty of pixels
+    (45, 1, 2, 1, 1, 1, 16, 1, 0.0, 1.0),        # 1x1 image: every cell has one tap inside
     (46, 1, 3, 2, 1, 11, 128, 5, -0.2, 1.2),
     (47, 1, 2, 1, 40, 40, 16, 4, 0.45, 0.55),    # clustered: a few very long cell lists
-    (48, 1, 2, 2, 20, 20, 64, 16, -0.1, 1.1),    # fp32: dq by the slab kernel (no pairs handed over on this path)
+    (48, 1, 2, 2, 20, 20, 64, 16, -0.1, 1.1),    # fp32: dq by the slab kernel, which hands its pairs on
 ]
 
 
@@ -112,6 +112,26 @@ def test_deterministic_backward_c5_full_size(deterministic):
     for (b, h), (_, rdq, rdk, rdv) in ref.items():
         for got, want in zip(first, (rdq, rdk, rdv)):
             assert rel(slice_bh(got, b, h), want) < TOL[torch.bfloat16], (b, h)
+
+
+def test_deterministic_backward_in_two_groups_of_planes(deterministic):
+    """17 planes whose taps take 295 MB, 256 at a time: groups of nine and of eight."""
+    say("[case] deterministic in two groups of planes")
+    B, V, H, Himg, Wimg, D, P = 1, 1, 17, 46, 46, 256, 4
+    assert 15 * 32 * Himg * Wimg * D <= 256 << 20 < 16 * 32 * Himg * Wimg * D
+    g = torch.Generator().manual_seed(49)
+    q, k, v, do = (torch.randn(B, V, H, Himg * Wimg, D, generator=g) for _ in range(4))
+    c = torch.rand(B, V, Himg * Wimg, V, P, 2, generator=g) * 1.2 - 0.1
+    dev = [t.cuda() for t in (q, k, v, c, do)]
+    first = grads(*dev, Wimg, Himg, 0.1)
+    again = grads(*dev, Wimg, Himg, 0.1)
+    for a, b in zip(first, again):
+        assert torch.equal(a, b)
+    slices = [(0, 0), (0, 8), (0, 9), (0, 16)]
+    ref = oracle_on_slices(q, k, v, c, do, Wimg, Himg, 0.1, slices, forward=False)
+    for (b, h), (_, *want) in ref.items():
+        for got, w in zip(first, want):
+            assert rel(slice_bh(got, b, h), w) < TOL[torch.float32], h
 
 
 def test_deterministic_with_coords_gradient_is_refused(deterministic):

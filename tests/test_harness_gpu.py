@@ -86,7 +86,7 @@ def test_non_default_stream_and_back_to_back_calls():
     assert rel(qg.grad, rdq) < 1e-3 and rel(kg.grad, rdk) < 1e-3 and rel(vg.grad, rdv) < 1e-3
 
 
-def test_large_image_uses_global_binning_path():
+def test_large_image_with_more_cells_than_samples_of_a_run():
     """A 96x128 image with 2 views: 12513 cells, more than a binning workgroup's samples (images beyond its counters in
     LDS: test_binning_runs_gpu.py); planes are too big for LDS too."""
     print("[case] large image", flush=True)

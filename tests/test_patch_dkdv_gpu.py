@@ -10,7 +10,7 @@ import torch
 
 from oracle import oracle_bwd
 from ops.triton import deform_sdpa_triton
-from parity_util import rel
+from parity_util import kernels_of, oracle_on_slices, rel
 
 pytestmark = pytest.mark.gpu
 BAR = {torch.float32: 1e-3, torch.bfloat16: 2e-2, torch.float16: 2e-2}
@@ -44,7 +44,7 @@ def test_patches_against_the_oracle(B, V, H, Himg, Wimg, D, P, dtype):
         assert rel(a, b) < BAR[dtype], name
 
 
-# mean list length up to 48 in 16 bits and 12 in fp32: lists of several blocks of 64 entries a patch, two and four waves
+# mean list length up to 48 in 16 bits and 12 in fp32: lists of several blocks of 64 entries a patch, one and two waves
 @pytest.mark.parametrize("P,dtype", [(7, torch.float32), (40, torch.bfloat16), (40, torch.float16)], ids=str)
 def test_several_blocks_a_patch(P, dtype):
     q, k, v, dout, coords = inputs(1, 1, 114, 11, 9, 32, P, dtype, 8)
@@ -53,8 +53,24 @@ def test_several_blocks_a_patch(P, dtype):
         assert rel(a, b) < BAR[dtype], name
 
 
+# 1350 visits a patch: four waves
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+def test_four_waves_a_patch(dtype):
+    B, V, H, side, D, P = 1, 6, 7, 20, 32, 9
+    assert V * side * side * P * 25 // 16 // (side // 4) ** 2 > 1280
+    q, k, v, dout, coords = inputs(B, V, H, side, side, D, P, dtype, 15)
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    print(f"[case] four waves a patch {dtype}", flush=True)
+    out = deform_sdpa_triton(*leaves, coords.cuda(), side, side, 0.18)
+    names = kernels_of(lambda: out.backward(dout.cuda()))
+    assert any(n.startswith("bwd_dkdv_patch_kernel") for n in names), names
+    want = oracle_bwd(*(t.float().numpy() for t in (q, k, v, coords, dout)), side, side, 0.18)
+    for leaf, b, name in zip(leaves, want, ("dq", "dk", "dv")):
+        assert rel(leaf.grad, b) < BAR[dtype], name
+
+
 # samples of one key view in one cell: its lists are left to the cell kernel, the other views' are not
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
 def test_one_view_clustered(dtype):
     q, k, v, dout, coords = inputs(2, 3, 12, 20, 18, 64, 2, dtype, 9)
     coords[:, :, :, 1] = (coords[:, :, :, 1] + 0.1) / 1.2 / 40 + 0.5
@@ -63,7 +79,7 @@ def test_one_view_clustered(dtype):
         assert rel(a, b) < BAR[dtype], name
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_non_finite_rows_stay_with_their_pixels(bad, dtype):
     q, k, v, dout, coords = inputs(1, 2, 64, 9, 10, 32, 2, dtype, 11)
@@ -114,3 +130,48 @@ def test_coefficients_are_not_rounded_to_16_bits(D, dtype, kept):
     err = float((vd.grad[0, 0].double().cpu() - want).norm() / want.norm())
     print("error", err, "of", float(left.norm() / rows.norm()))
     assert err < 8e-3, err
+
+
+# What leaves the pairs: the staged dq kernel (narrow, and eight fp32 elements a lane), with the coordinate gradient, and the row
+# kernel, which takes few samples and planes beyond LDS; q, k, v as projections leave them
+@pytest.mark.parametrize("B,V,H,Himg,Wimg,D,P,dtype,coords_grad,dq", [
+    (2, 2, 32, 18, 18, 32, 4, torch.float32, False, "bwd_dq_slot_kernel<F32, 32, 8, false, 1, true>"),
+    (2, 2, 32, 12, 13, 64, 4, torch.float32, False, "bwd_dq_slot_kernel<F32, 64, 8, false, 1, true>"),
+    (2, 2, 32, 18, 18, 32, 4, torch.float32, True, "bwd_dq_slot_kernel<F32, 32, 4, true, 1, true>"),
+    (2, 2, 32, 18, 18, 32, 4, torch.bfloat16, True, "bwd_dq_slot_kernel<BF16, 32, 8, true, 1, true>"),
+    (2, 2, 32, 18, 17, 64, 5, torch.float16, True, "bwd_dq_slot_kernel<F16, 64, 8, true, 1, true>"),
+    (1, 4, 64, 9, 10, 256, 4, torch.bfloat16, True, "bwd_dq_slot_kernel<BF16, 256, 16, true, 1, true>"),
+    (1, 2, 12, 23, 29, 128, 2, torch.float32, True, "bwd_dq_rows_kernel<F32, 128, "),
+    (1, 2, 12, 23, 29, 128, 5, torch.float16, False, "bwd_dq_rows_kernel<F16, 128, "),
+    (1, 2, 12, 23, 29, 256, 3, torch.bfloat16, True, "bwd_dq_rows_kernel<BF16, 256, "),
+], ids=str)
+@pytest.mark.parametrize("projection", [False, True])
+def test_patches_behind_every_dq_kernel(B, V, H, Himg, Wimg, D, P, dtype, coords_grad, dq, projection):
+    q, k, v, dout, coords = inputs(B, V, H, Himg, Wimg, D, P, dtype, 12)
+    scale = 1.0 / math.sqrt(D)
+    print(f"[case] patches behind {dq} B{B} V{V} H{H} {Himg}x{Wimg} D{D} P{P} {projection}", flush=True)
+    turn = (lambda t: t.permute(0, 1, 3, 2, 4)) if projection else (lambda t: t)
+    leaves = [turn(t).contiguous().cuda().requires_grad_(True) for t in (q, k, v)]
+    cdev = coords.cuda().requires_grad_(coords_grad)
+    out = deform_sdpa_triton(*(turn(t) for t in leaves), cdev, Wimg, Himg, scale, coords_grad)
+    names = kernels_of(lambda: out.backward(dout.cuda()))
+    assert any(n.startswith(dq) for n in names) and any(n.startswith("bwd_dkdv_patch_kernel") for n in names), names
+    want = oracle_bwd(*(t.float().numpy() for t in (q, k, v, coords, dout)), Wimg, Himg, scale, with_coords=coords_grad)
+    got = [turn(t.grad) for t in leaves] + ([cdev.grad] if coords_grad else [])
+    for a, b, name in zip(got, want, ("dq", "dk", "dv", "dcoords")):
+        assert rel(a, b) < BAR[dtype], name
+
+
+# 138 MB of pairs, 128 at a time: two groups of (batch, head) pairs
+def test_patches_in_groups_of_pairs():
+    q, k, v, dout, coords = inputs(1, 4, 270, 20, 20, 32, 10, torch.bfloat16, 13)
+    assert 4 * 270 * 400 * 40 * 8 > 128 << 20
+    print("[case] patches in two groups", flush=True)
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    out = deform_sdpa_triton(*leaves, coords.cuda(), 20, 20, 0.25)
+    names = kernels_of(lambda: out.backward(dout.cuda()))
+    assert any(n.startswith("bwd_dkdv_patch_kernel") for n in names), names
+    slices = [(0, 0), (0, 134), (0, 135), (0, 269)]
+    for (b, h), (_, *want) in oracle_on_slices(q, k, v, coords, dout, 20, 20, 0.25, slices, forward=False).items():
+        for leaf, w, name in zip(leaves, want, ("dq", "dk", "dv")):
+            assert rel(leaf.grad[b:b + 1, :, h:h + 1], w) < BAR[torch.bfloat16], (name, h)

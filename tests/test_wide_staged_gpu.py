@@ -1,6 +1,6 @@
 """Staged forward and dq with eight fp32 elements a lane (D = 32 and 64, launches of many query rows): query rows that end inside a
-wave and a workgroup, passes that end inside a run of samples, strided inputs, the pairs handed on to dk/dv. Against the CPU
-oracle at the bars of the other fp32 parity tests."""
+wave and a workgroup, passes that end inside a run of samples, strided inputs. (These lists are long: the form that hands its
+pairs on is among the tests of dk/dv by patches.) Against the CPU oracle at the bars of the other fp32 parity tests."""
 import math
 
 import pytest
@@ -8,7 +8,7 @@ import torch
 
 from oracle import oracle_bwd, oracle_fwd
 from ops.triton import deform_sdpa_triton
-from parity_util import rel
+from parity_util import kernels_of, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -26,8 +26,8 @@ def test_wide_split_against_the_oracle(B, V, H, Himg, Wimg, D, P, projection):
     dev = [t.to("cuda:0").requires_grad_(True) for t in leaves]
     view = (lambda t: t.permute(0, 1, 3, 2, 4)) if projection else (lambda t: t)
     out = deform_sdpa_triton(*(view(t) for t in dev), coords.to("cuda:0"), Wimg, Himg, scale)
-    out.backward(dout.to("cuda:0"))
-    torch.cuda.synchronize()
+    names = kernels_of(lambda: out.backward(dout.to("cuda:0")))
+    assert f"bwd_dq_slot_kernel<F32, {D}, 8, false, 1, false>" in names, names
     n = [view(t).contiguous().numpy() for t in leaves]
     assert rel(out, oracle_fwd(*n, coords.numpy(), Wimg, Himg, scale)[0]) < 1e-4
     want = oracle_bwd(*n, coords.numpy(), dout.numpy(), Wimg, Himg, scale)
