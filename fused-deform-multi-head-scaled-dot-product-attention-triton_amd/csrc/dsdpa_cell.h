@@ -248,19 +248,33 @@ __device__ __forceinline__ void scan_keys(const unsigned (&v)[kScanKeys], int c0
     }
 }
 
-// after the last turn: the total, the empty slots behind the items, and (where `spread` is asked for) whether the lists are
-// the patch kernel's (kSpreadLongest entries at most and `mean` or fewer on average): 0 if they are, else the number of items
-struct Spread { unsigned *items, mean; };
-constexpr unsigned kSpreadLongest = 1024;
+// after the last turn: the total, the empty slots behind the items, and (where `spread` is asked for) the number of items, with
+// kSpreadLong set unless the lists are the patch kernel's: `mean` or fewer entries a non-empty list and at most kSpreadLongest
+// in the longest, or where the lists are fewer than `few`, `mean` in the longest
+struct Spread { unsigned *items, mean, few; };
+constexpr unsigned kSpreadLongest = 1024, kSpreadLong = 0x80000000u;
+// Whether more than a third of the n groups (b, s2) have long lists: then all are the cell kernel's. (Half the views by
+// patches and half by cells fill the chip twice by half: 40x28, batch 2, 4 views x 8 heads, P = 1, clustered, D = 128, bf16, all by cells
+// 133 us a step, by patches 175, so mixed 185; 18x18, 6 x 16, P = 6 around the query's place, D = 32 183 / 192 / 206.)
+__device__ __forceinline__ bool mostly_long(const unsigned *__restrict__ left, int n)
+{
+    const int lane = threadIdx.x & 63;
+    int longs = 0;
+    for (int i = 0; i < n; i += kWave) longs += __popcll(__ballot(i + lane < n && (left[min(i + lane, n - 1)] & kSpreadLong) != 0u));
+    return 3 * longs > n;
+}
+// items that the cell kernel has to do in the planes of a group with left[] = l, 0 if they are the patch kernel's
+__device__ __forceinline__ unsigned items_left(unsigned l, bool all) { return all || (l & kSpreadLong) ? l & ~kSpreadLong : 0u; }
 template <int THREADS>
 __device__ __forceinline__ void scan_end(const ScanCarry &carry, int NC, unsigned wmax, unsigned *__restrict__ st, uint4 *__restrict__ it,
                                          const Spread &spread, unsigned longest)
 {
     if (spread.items) {
-        const int any_long = __syncthreads_or(longest > kSpreadLongest);
-        if (threadIdx.x == 0)
-            spread.items[blockIdx.x] = !any_long && (unsigned long long)carry.entries <= (unsigned long long)spread.mean * carry.pieces
-                                     ? 0u : min(carry.pieces, wmax);
+        const int any_long = __syncthreads_or(longest > (carry.pieces < spread.few ? spread.mean : kSpreadLongest));
+        if (threadIdx.x == 0) {
+            const bool is_long = any_long || (unsigned long long)carry.entries > (unsigned long long)spread.mean * carry.pieces;
+            spread.items[blockIdx.x] = min(carry.pieces, wmax) | (is_long ? kSpreadLong : 0u);
+        }
     }
     if (threadIdx.x == 0) st[NC] = carry.entries;
     for (unsigned i = min(carry.pieces, wmax) + threadIdx.x; i < wmax; i += THREADS) it[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -1046,13 +1060,14 @@ __global__ __launch_bounds__(256) void combine_taps_kernel(const float *__restri
 }
 
 // The planes that the patch kernel has left: a loop over their work lists, at once over where there are none. left[grp]:
-// items of the list, 0 where the patch kernel has done the planes of this (batch, key view). Every XCD takes one contiguous
+// see scan_end. Every XCD takes one contiguous
 // part of the planes. (A loop costs registers and, over whole launches, time: one wave per SIMD less.)
 template <typename S, int D, int DC>
 __global__ __launch_bounds__(kCellWaves *kWave) void bwd_dkdv_cell_rest_kernel(const unsigned *__restrict__ left, DSDPA_CELL_ARGS)
 {
+    const bool all = mostly_long(left, dm.B * dm.V);
     unsigned most = 0u;
-    for (int i = threadIdx.x & 63; i < dm.B * dm.V; i += kWave) most = max(most, left[i]);
+    for (int i = threadIdx.x & 63; i < dm.B * dm.V; i += kWave) most = max(most, items_left(left[i], all));
     most = (unsigned)__builtin_amdgcn_readfirstlane((int)wave_all(most, [](unsigned x, unsigned y) { return max(x, y); }));
     if (most == 0u) return;
     const unsigned planes = cg.nwork / (unsigned)cg.ncells, total = planes * most, parts = gridDim.x / kXcds;
@@ -1060,7 +1075,7 @@ __global__ __launch_bounds__(kCellWaves *kWave) void bwd_dkdv_cell_rest_kernel(c
     for (unsigned i = (unsigned)((unsigned long long)total * x / kXcds) + blockIdx.x / kXcds; i < end; i += parts) {
         const unsigned t = i / most, ci = i - t * most;
         const unsigned bhl = cg.div_v.div(t), b = cg.div_h.div((unsigned)cg.bh0 + bhl);
-        if (ci < left[b * (unsigned)dm.V + t - bhl * (unsigned)dm.V])
+        if (ci < items_left(left[b * (unsigned)dm.V + t - bhl * (unsigned)dm.V], all))
             cell_sums<S, D, DC, true, false>(t, (int)ci, q_, k_, v_, stats_, dout_, start, sorted, items, handed_, dk_acc, dv_acc,
                                             dm, NC, cg);
     }

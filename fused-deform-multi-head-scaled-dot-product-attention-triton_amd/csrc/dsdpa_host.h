@@ -247,7 +247,7 @@ struct WorkspaceLayout {
     int tap_planes;             // planes (b, h, s2) whose taps the buffer of the deterministic backward holds at a time
     int bh_group;               // (batch, head) pairs whose pairs the handed buffer holds at a time; 0: nothing is handed over
     bool patch;                 // dk/dv by patches where the lists are short (DSDPA_PATH_AUTO)
-    unsigned spread_mean;       // ... up to so many entries a non-empty list on average
+    unsigned spread_mean, spread_few;   // ... up to so many entries a non-empty list on average; few such lists
     DescLayout dl;
     size_t counters_bytes;
     int NC;                     // cells of the grid
@@ -312,18 +312,34 @@ inline int handed_group(size_t B, size_t V, size_t H, size_t L, size_t P)
     return (int)((B * H + ngroups - 1) / ngroups);
 }
 // dk/dv by patches of 4x4 pixels (dsdpa_patch.h) where the lists are short: what the cell kernel pays per list -- 300
-// instructions and 8*D float atomics, which the memory side takes at 0.3 a ns -- is then most of its time. Up to 48
-// entries a list over the whole grid in 16-bit storage, where the products run at 16 times the vector rate, and 12 in fp32,
-// where they run at twice; from 1024 patches, which fill the chip. us a step, cells / patches, 20x20, V = 4, P = 2, 6, 18 (7, 22,
-// 65 entries): bf16 D = 32 118 / 88, 150 / 129, 273 / 255; D = 64 178 / 123, 230 / 193, 474 / 413; D = 128 114 / 82, 142 / 113,
-// 234 / 227; fp32 D = 32 115 / 98, 150 / 153, 269 / 300; D = 64 185 / 147, 277 / 289, 612 / 704. At 184 entries (48x48, D = 64,
-// bf16) the kernels take 1150 / 1680, at 223 (14x14, D = 32, fp32) 235 / 500.
-// The lists are counted when they are made: spread_mean is the mean of the non-empty ones up to which the patches go ahead.
-inline unsigned spread_mean(size_t esize) { return esize == 2 ? 64u : 16u; }
-inline bool patch_path(size_t B, size_t V, size_t H, size_t Himg, size_t Wimg, size_t P, size_t esize, bool deterministic)
+// instructions and 8*D float atomics, which the memory side takes at 0.3 a ns -- is then most of its time. From 1024 patches,
+// which fill the chip, and up to 48 entries a list over the whole grid in 16-bit storage (32 at D = 16, where a row's products are
+// the least of a visit), where the products run at 16 times the vector rate; 12 in fp32, where they run at twice. us a step,
+// cells / patches, 40x28, batch 2, 4 views, 8 heads, P = 4, 8, 10 (15, 30, 38 entries): bf16 D = 16 136 / 118, 170 / 162, 181 / 185;
+// D = 32 161 / 135, 225 / 217, 262 / 260; D = 64 232 / 166, 312 / 270, 353 / 325; D = 128 426 / 261, 580 / 448, 657 / 543; D = 256
+// 902 / 529, 1330 / 1028, 1510 / 1249; fp32 P = 1, 3 (4, 11) D = 32 114 / 81, 149 / 134; D = 64 184 / 114, 256 / 218. bf16 18x18,
+// 6 views x 8, 16 heads (43): D = 16 167 / 181, D = 32 213 / 211, D = 64 383 / 321. At 184 entries (48x48, D = 64, bf16) the kernels
+// take 1150 / 1680, at 223 (14x14, D = 32, fp32) 235 / 500.
+//
+// The lists are counted when they are made: spread_mean is the mean of the non-empty ones up to which the patches go ahead. Behind
+// it the second launch works by cells, which with the launch of patches that only clear costs up to 7 % more than cells alone. us a
+// step, cells by that second launch / patches, bf16, the first shape with samples in the middle 0.7 of the image each way, P = 4, 6,
+// 8, 10 (34, 50, 66, 82): D = 16 116 / 115, 133 / 141, 153 / 166, 173 / 192; D = 32 142 / 132, 176 / 173, 212 / 215, 248 / 256; D = 64
+// 192 / 163, 236 / 220, 282 / 273, 330 / 329; D = 128 330 / 256, 408 / 357, 482 / 451, 565 / 551; D = 256 637 / 470, 852 / 711, 1007 / 891,
+// 1190 / 1093 (105: even). P = 8 around the query's own place (56): D = 64 cells alone 271, patches 275; D = 128 474 / 439.
+// Where few cells hold samples (spread_few, less than 1024 patches' worth in a launch) the longest list takes the mean's place, since
+// the patch around it is most of the launch. The first shape with P = 1, bf16, 121 such cells of 37 entries, the longest 120
+// (clustered): cells alone / patches D = 64 95 / 120, D = 128 133 / 175, D = 256 257 / 236; 117 cells of 38, the longest 59: D = 128
+// 132 / 135, D = 256 255 / 202.
+inline unsigned spread_mean(size_t D, size_t esize)
+{
+    return esize == 4 ? 16u : D == 16 ? 36u : D == 32 ? 52u : D == 64 ? 72u : D == 128 ? 80u : 128u;
+}
+inline unsigned spread_few(size_t planes) { return (unsigned)((1024 * 16 + planes - 1) / planes); }
+inline bool patch_path(size_t B, size_t V, size_t H, size_t Himg, size_t Wimg, size_t D, size_t P, size_t esize, bool deterministic)
 {
     const size_t L = Himg * Wimg, mean = V * L * P / ((Himg + 1) * (Wimg + 1));
-    return !deterministic && L >= 16 && mean <= (esize == 2 ? 48 : 12) && B * V * H * L * V * P >= ((size_t)1 << 15) &&
+    return !deterministic && L >= 16 && mean <= (esize == 4 ? 12 : D == 16 ? 32 : 48) && B * V * H * L * V * P >= ((size_t)1 << 15) &&
            B * V * H * ((Himg + 3) / 4) * ((Wimg + 3) / 4) >= 1024;
 }
 inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Himg, size_t Wimg, size_t D, size_t P,
@@ -336,10 +352,11 @@ inline WorkspaceLayout workspace_layout(size_t B, size_t V, size_t H, size_t Him
     w.delta = off; off += round256(rows * 8);           // (lse, delta) per row
     const size_t L = Himg * Wimg, esize = storage16 ? 2 : 4, acc_bytes = storage16 && !deterministic ? round256(2 * rows * D * 4) : 0;
     const bool planes = plane_path_fits(L, D, esize);
-    w.patch = patch_path(B, V, H, Himg, Wimg, P, esize, deterministic);
+    w.patch = patch_path(B, V, H, Himg, Wimg, D, P, esize, deterministic);
     w.bh_group = planes && !w.patch ? 0 : handed_group(B, V, H, L, P);
     w.patch = w.patch && w.bh_group > 0;
-    w.spread_mean = spread_mean(esize);
+    w.spread_mean = spread_mean(D, esize);
+    w.spread_few = w.patch ? spread_few((size_t)w.bh_group * V) : 0;
     const bool grouped = w.bh_group > 0 && !planes && !deterministic;
     w.vpg = views_per_group(V, L, D, esize, P, (size_t)w.NC, grouped);
     w.NK = w.NC * (int)((V + w.vpg - 1) / w.vpg);       // (short lists are never split: NK = NC where there are patches)

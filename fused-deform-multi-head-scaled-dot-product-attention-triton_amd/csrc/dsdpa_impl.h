@@ -65,15 +65,16 @@ __global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ ds
     }
 }
 
-// The same for dk and dv of the planes (b, view) whose sums are in the accumulators: those with left[] items
+// The same for dk and dv of the planes (b, view) whose sums are in the accumulators: those that the patch kernel has left
 // (n8 = elements of a (batch, view, head) over 8). At once over where there are none.
 template <typename S>
 __global__ void cast_rest_kernel(const unsigned *__restrict__ left, const float *__restrict__ dk_acc, const float *__restrict__ dv_acc,
                                  void *__restrict__ dk, void *__restrict__ dv, Dims dm, size_t n8)
 {
     const size_t per = n8 * dm.H, stride = (size_t)gridDim.x * blockDim.x;
+    const bool all = mostly_long(left, dm.B * dm.V);
     for (int g = 0; g < dm.B * dm.V; ++g) {
-        if (left[g] == 0u) continue;
+        if (items_left(left[g], all) == 0u) continue;
         for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < 2 * per; i += stride) {
             const size_t at = g * per + (i < per ? i : i - per);
             const float4 *s4 = reinterpret_cast<const float4 *>(i < per ? dk_acc : dv_acc) + 2 * at;
@@ -904,7 +905,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
                            stats, (size_t)dm.rows, D);
         if ((rc = check_launch()) != DSDPA_OK) return rc;
     }
-    if (cell_binned && (rc = launch_binning(coords, dm, wl, ws, deterministic ? 0 : 1, Spread{left, wl.spread_mean},
+    if (cell_binned && (rc = launch_binning(coords, dm, wl, ws, deterministic ? 0 : 1, Spread{left, wl.spread_mean, wl.spread_few},
                                               side_on && !deterministic, bst)) != DSDPA_OK)
         return rc;
     if (deterministic && (rc = launch_list_ordering(coords, dm, wl, ws, bst)) != DSDPA_OK) return rc;

@@ -32,9 +32,9 @@
 //
 // Short lists only. A patch costs its visits; the cell kernel costs its lists (300 instructions and 8*D atomics each) and
 // entries, and is ahead where lists are long. The host asks for patches where the lists would be short with the samples
-// spread over the image, and the binning, which counts them, decides per (batch, key view), by the mean of the
-// non-empty lists and the longest. Where they are not short (samples that cluster leave most cells empty and the others
-// full), left[] holds the number of work items, the patch kernel only clears its pixels' accumulators, and a second
+// spread over the image, and the binning, which counts them, decides by the mean of the non-empty lists and the longest, per
+// (batch, key view) or, where many are long, for all (mostly_long). Where they are not short (samples that cluster leave
+// most cells empty and the others full), the patch kernel only clears its pixels' accumulators, and a second
 // launch, the cell kernel as a loop over the work list, does the sums.
 #pragma once
 #include "dsdpa_cell.h"
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
         elem = plane_base + (size_t)(y * dm.Wimg + x) * D + col0;
         return y < dm.Himg && x < dm.Wimg;
     };
-    if (left && left[grp] != 0u) {
+    if (left && items_left(left[grp], mostly_long(left, dm.B * dm.V)) != 0u) {
         for (int i = threadIdx.x; i < kPatchPixels * DP / 4; i += (int)blockDim.x) {
             size_t elem;
             if (pixel_at(i * 4 / DP, elem)) {

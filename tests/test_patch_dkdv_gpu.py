@@ -79,6 +79,29 @@ def test_one_view_clustered(dtype):
         assert rel(a, b) < BAR[dtype], name
 
 
+# few cells hold samples and one of them many: left to the cell kernel by the longest list, at a mean that is the patches'
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
+def test_few_cells_and_a_long_list(dtype):
+    q, k, v, dout, coords = inputs(1, 2, 45, 19, 21, 16, 2, dtype, 10)
+    coords = 0.5 + 0.07 * torch.randn(coords.shape, generator=torch.Generator().manual_seed(10))
+    at = (coords[0, :, :, 0].reshape(-1, 2) * torch.tensor([20, 18])).floor().long()
+    lists = torch.unique(at[:, 1] * 22 + at[:, 0], return_counts=True)[1]
+    assert len(lists) * 90 < 16384 and lists.double().mean() < 31 and lists.max() > 40, lists
+    got, want = gradients(q, k, v, coords, dout, 21, 19)
+    for a, b, name in zip(got, want, ("dq", "dk", "dv")):
+        assert rel(a, b) < BAR[dtype], name
+
+
+# samples of two key views of three in a few cells each: the third one's lists are left to the cell kernel too, although they are short
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+def test_most_views_clustered(dtype):
+    q, k, v, dout, coords = inputs(2, 3, 12, 20, 18, 32, 2, dtype, 14)
+    coords[:, :, :, :2] = (coords[:, :, :, :2] + 0.1) / 1.2 / 40 + 0.5
+    got, want = gradients(q, k, v, coords, dout, 18, 20)
+    for a, b, name in zip(got, want, ("dq", "dk", "dv")):
+        assert rel(a, b) < BAR[dtype], name
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_non_finite_rows_stay_with_their_pixels(bad, dtype):
