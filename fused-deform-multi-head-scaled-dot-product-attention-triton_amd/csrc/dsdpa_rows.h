@@ -58,7 +58,7 @@ __global__ __launch_bounds__(kRowWaves *kWave) void fwd_rows_kernel(
 {
     constexpr int G = D / DC, NS = kWave / G;
     constexpr bool kPacked = S::kBytes == 2;
-    constexpr int U = DC * S::kBytes <= 16 ? 2 : 1;               // samples per step: their eight taps in flight together
+    constexpr int kStep = DC * S::kBytes <= 16 ? 2 : 1;           // samples per step: their eight taps in flight together
     constexpr int RW = kPacked ? DC / 2 : DC;                    // 32-bit words of a tap held by one lane
     static_assert(G >= 2 && G <= 32 && G * DC == D, "lane split");
     __shared__ float4 s_w[kRowWaves][NS * (G + 1)];             // (a pad place per slot: neither side has bank conflicts)
@@ -87,6 +87,64 @@ __global__ __launch_bounds__(kRowWaves *kWave) void fwd_rows_kernel(
 #pragma unroll
     for (int d = 0; d < DC; ++d) acc[d] = 0.f;
 
+    // the n samples of a pass from the t-th on
+    auto step = [&](auto n, int t) {
+        constexpr int U = decltype(n)::value;
+        float4 wt[U];
+        uint32_t kr[U][4][RW], vr[U][4][RW];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            wt[u] = my_w[t + u];
+            const uint4 o = lane_offsets(my_e[t + u], lane_byte);
+            load_words<RW>(kb + o.x, kr[u][0]);
+            load_words<RW>(kb + o.y, kr[u][1]);
+            load_words<RW>(kb + o.z, kr[u][2]);
+            load_words<RW>(kb + o.w, kr[u][3]);
+            load_words<RW>(vb + o.x, vr[u][0]);
+            load_words<RW>(vb + o.y, vr[u][1]);
+            load_words<RW>(vb + o.z, vr[u][2]);
+            load_words<RW>(vb + o.w, vr[u][3]);
+        }
+        float s[U], mc = m;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float4 x = wt[u];
+            float dot = 0.f;
+            if constexpr (kPacked) {
+                const float d0 = packed_dot<S, DC>(qp, kr[u][0]), d1 = packed_dot<S, DC>(qp, kr[u][1]);
+                const float d2 = packed_dot<S, DC>(qp, kr[u][2]), d3 = packed_dot<S, DC>(qp, kr[u][3]);
+                dot = qscale * fmaf(x.x, d0, fmaf(x.y, d1, fmaf(x.z, d2, x.w * d3)));
+            } else {
+#pragma unroll
+                for (int d = 0; d < DC; ++d) {
+                    const float kk = fmaf(x.x, __uint_as_float(kr[u][0][d]), fmaf(x.y, __uint_as_float(kr[u][1][d]),
+                                     fmaf(x.z, __uint_as_float(kr[u][2][d]), x.w * __uint_as_float(kr[u][3][d]))));
+                    dot = fmaf(qf[d], kk, dot);
+                }
+            }
+            s[u] = group_sum<G>(dot);
+            mc = fmaxf(mc, s[u]);
+        }
+        const float alpha = __builtin_amdgcn_exp2f(m - mc);
+        m = mc;
+        lsum *= alpha;
+#pragma unroll
+        for (int d = 0; d < DC; ++d) acc[d] *= alpha;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float p = __builtin_amdgcn_exp2f(s[u] - mc);
+            lsum += p;
+            const float c[4] = { p * wt[u].x, p * wt[u].y, p * wt[u].z, p * wt[u].w };
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float x[DC];
+                widen_words<S, DC>(vr[u][i], x);
+#pragma unroll
+                for (int d = 0; d < DC; ++d) acc[d] = fmaf(c[i], x[d], acc[d]);
+            }
+        }
+    };
+
     float2 xy = crow[min(g, dm.N - 1)];
     for (int c0 = 0; c0 < dm.N; c0 += G) {
         const int n = c0 + g, cnt = min(G, dm.N - c0);
@@ -99,63 +157,10 @@ __global__ __launch_bounds__(kRowWaves *kWave) void fwd_rows_kernel(
         my_w[g] = w;
         my_e[g] = e;
         wave_lds_sync();
-        for (int t = 0; t < cnt; t += U) {
-            float4 wt[U];
-            uint32_t kr[U][4][RW], vr[U][4][RW];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                wt[u] = my_w[t + u];
-                const uint4 o = lane_offsets(my_e[t + u], lane_byte);
-                load_words<RW>(kb + o.x, kr[u][0]);
-                load_words<RW>(kb + o.y, kr[u][1]);
-                load_words<RW>(kb + o.z, kr[u][2]);
-                load_words<RW>(kb + o.w, kr[u][3]);
-                load_words<RW>(vb + o.x, vr[u][0]);
-                load_words<RW>(vb + o.y, vr[u][1]);
-                load_words<RW>(vb + o.z, vr[u][2]);
-                load_words<RW>(vb + o.w, vr[u][3]);
-            }
-            float s[U], mc = m;
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const float4 x = wt[u];
-                float dot = 0.f;
-                if constexpr (kPacked) {
-                    const float d0 = packed_dot<S, DC>(qp, kr[u][0]), d1 = packed_dot<S, DC>(qp, kr[u][1]);
-                    const float d2 = packed_dot<S, DC>(qp, kr[u][2]), d3 = packed_dot<S, DC>(qp, kr[u][3]);
-                    dot = qscale * fmaf(x.x, d0, fmaf(x.y, d1, fmaf(x.z, d2, x.w * d3)));
-                } else {
-#pragma unroll
-                    for (int d = 0; d < DC; ++d) {
-                        const float kk = fmaf(x.x, __uint_as_float(kr[u][0][d]), fmaf(x.y, __uint_as_float(kr[u][1][d]),
-                                         fmaf(x.z, __uint_as_float(kr[u][2][d]), x.w * __uint_as_float(kr[u][3][d]))));
-                        dot = fmaf(qf[d], kk, dot);
-                    }
-                }
-                s[u] = group_sum<G>(dot);
-                if (U > 1 && t + u >= cnt) s[u] = kNegBig;        // (beyond the row: weight 0 in the sums below)
-                mc = fmaxf(mc, s[u]);
-            }
-            const float alpha = __builtin_amdgcn_exp2f(m - mc);
-            m = mc;
-            lsum *= alpha;
-#pragma unroll
-            for (int d = 0; d < DC; ++d) acc[d] *= alpha;
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                float p = __builtin_amdgcn_exp2f(s[u] - mc);
-                if (U > 1 && t + u >= cnt) p = 0.f;
-                lsum += p;
-                const float c[4] = { p * wt[u].x, p * wt[u].y, p * wt[u].z, p * wt[u].w };
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float x[DC];
-                    widen_words<S, DC>(vr[u][i], x);
-#pragma unroll
-                    for (int d = 0; d < DC; ++d) acc[d] = fmaf(c[i], x[d], acc[d]);
-                }
-            }
-        }
+        // (an odd sample on its own: a second one of weight 0 would make NaN of an infinite V)
+        int t = 0;
+        for (; t + kStep <= cnt; t += kStep) step(std::integral_constant<int, kStep>{}, t);
+        if (kStep > 1 && t < cnt) step(std::integral_constant<int, 1>{}, t);
     }
     if (!rs.have) return;
     const size_t row = (((size_t)rs.b * dm.V + rs.s1) * dm.H + rs.h) * dm.L + rs.l;

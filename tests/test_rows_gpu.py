@@ -3,6 +3,7 @@ of one sample, of an odd number and of a whole pass, strided inputs, the coordin
 dk/dv. Against the CPU oracle at the bars of the other parity tests."""
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -56,3 +57,19 @@ def test_rows_with_the_coordinate_gradient(D, P, dtype):
 @pytest.mark.parametrize("V,H,P,dtype", [(2, 10, 12, torch.float32), (2, 20, 10, torch.bfloat16), (3, 14, 21, torch.bfloat16)], ids=str)
 def test_many_rows(V, H, P, dtype):
     check(1, V, H, 30, 31, 64, P, dtype)
+
+
+# infinite V at the taps of a row's last sample, rows of an odd number of samples: infinite, not NaN
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("V,P", [(1, 1), (3, 1), (1, 5)])
+def test_infinite_values(V, P, dtype):
+    print(f"[case] rows, infinite V, {V} x {P} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(V + P)
+    L = 18 * 17
+    q, k, v = (torch.randn(1, V, 2, L, 32, generator=g).to(dtype) for _ in range(3))
+    coords = torch.rand(1, V, L, V, P, 2, generator=g) * 0.9 + 0.05            # (no tap outside)
+    v[0, V - 1, :, 3 * 17 + 5] = float("inf")
+    out = deform_sdpa_triton(*(t.cuda() for t in (q, k, v, coords)), 17, 18, 0.2).double().cpu().numpy()
+    want = oracle_fwd(*(t.float().numpy() for t in (q, k, v, coords)), 17, 18, 0.2)[0]
+    assert 0 < np.isinf(want).sum() < want.size // 4 and not np.isnan(want).any()
+    assert np.array_equal(np.isinf(out), np.isinf(want)) and not np.isnan(out).any()
