@@ -1060,8 +1060,8 @@ __global__ __launch_bounds__(256) void combine_taps_kernel(const float *__restri
 }
 
 // The planes that the patch kernel has left: a loop over their work lists, at once over where there are none. left[grp]:
-// see scan_end. Every XCD takes one contiguous
-// part of the planes. (A loop costs registers and, over whole launches, time: one wave per SIMD less.)
+// see scan_end. Every XCD takes one contiguous part of the planes. (A loop costs registers and, over whole launches, time: one
+// wave per SIMD less.)
 template <typename S, int D, int DC>
 __global__ __launch_bounds__(kCellWaves *kWave) void bwd_dkdv_cell_rest_kernel(const unsigned *__restrict__ left, DSDPA_CELL_ARGS)
 {

@@ -454,7 +454,10 @@ __device__ __forceinline__ float first_lane(float x) { return __uint_as_float((u
 // fp16 has five bits of exponent, fp32 coefficients eight: before they are split they are multiplied by a power of two, and
 // their sums divided by it. p <= 1 (and what one query's samples of a cell add up to) by kScaleP, sm_scale * ds by a scale that
 // follows the largest magnitude seen so far: `scale` is lowered to put `top` between 2^13 and 2^14 where it would pass 2^14,
-// and what the sums made until then have to be multiplied by is returned (1: nothing). From kScaleDs on.
+// and what the sums made until then have to be multiplied by is returned (1: nothing). From kScaleDs on. Two fp16 parts of a
+// scaled coefficient are good to 2^-23 of it, and where that is below half of fp16's smallest step to 2^-25: for weight times p 2^-23 from
+// 2^-17 up and 2^-40 below (times dout of 65504, the smallest step of dv itself), for weight times ds 2^-23 from 2^-15 of the
+// largest ds up and 2^-38 of the largest below.
 constexpr float kScaleP = 32768.0f, kScaleDs = 0x1p110f;
 __device__ __forceinline__ float lower_scale(float top, float &scale)
 {

@@ -868,7 +868,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     // enqueued; joined after the dk/dv kernel (before the casts of 16-bit storage, which need both).
     // Only for shapes on the staged dq kernel, whose one 16-wave workgroup per CU leaves half the wave slots
     // free. The gather dq kernel (planes too large for LDS) fills every CU with small workgroups: beside it the
-    // binning workgroups (1024 threads, up to 135 KB of LDS) wait until it ends, and with the binning done
+    // binning workgroups (512 threads, up to 80 KB of LDS) wait until it ends, and with the binning done
     // first the dq and dk/dv kernels only take turns (measured at 64x64, D = 128: 14.2 ms against 14.5 for the
     // step, each kernel stretched to the sum of both) -- those shapes run the backward on the caller's stream.
     // So do small problems: the fork and join cost about 0.05 ms of host time per call, which a backward of

@@ -19,11 +19,11 @@
 //   16-bit storage  v_mfma_f32_16x16x32: lane group lane/16 holds eight entries, lane % 16 = column n: E = D/16
 //                   consecutive elements of each row, element t of every lane in product t (so output column n of
 //                   product t is element E*n + t: no data crosses lanes). The coefficients are split in parts of the storage
-//                   type, one product each: two in fp16 (good to 2^-23), three in bf16 (two are good to 2^-17, which rows
-//                   that cancel show); two byte permutes make the operand of a pair of rows. The third part costs a third of
-//                   the tables' LDS, 13.7 KB a wave for 9.4. us a step, cells / two parts / three, bf16: 18x18, 32 heads, D = 32, 6 views x 6
-//                   samples 351 / 274 / 292, 12 x 4 797 / 670 / 701; 20x20, 4 x 6, D = 64 229 / 182 / 186; 40x28, 4 x 8,
-//                   coherent, D = 128 581 / 425 / 441.
+//                   type, one product each: two in fp16 (good to 2^-23 down to a floor, see lower_scale), three in bf16 (two
+//                   are good to 2^-17, which rows that cancel show); two byte permutes make the operand of a pair of rows.
+//                   The third part costs a third of the tables' LDS, 13.7 KB a wave for 9.4. us a step, cells / two parts /
+//                   three, bf16: 18x18, 32 heads, D = 32, 6 views x 6 samples 351 / 274 / 292, 12 x 4 797 / 670 / 701; 20x20,
+//                   4 x 6, D = 64 229 / 182 / 186; 40x28, 4 x 8, coherent, D = 128 581 / 425 / 441.
 //   fp32            v_mfma_f32_16x16x4_f32: one entry per lane group and instruction, everything in fp32.
 // fp16 has 5 bits of exponent: its coefficients are scaled by powers of two (lower_scale).
 //
@@ -69,8 +69,8 @@ __device__ __forceinline__ void load_piece(const char *p, uint32_t (&w)[(BYTES +
     else load_words<BYTES / 4>(p, w);
 }
 
-// A coefficient as (high part | low part << 16) of the storage type, and in `rest` what they leave of it: nothing that
-// matters in fp16 (good to 2^-23), a third part in bf16 (2^-17 without it).
+// A coefficient as (high part | low part << 16) of the storage type, and in `rest` what they leave of it: a third part in
+// bf16 (2^-17 without it), not used in fp16.
 template <typename S>
 __device__ __forceinline__ uint32_t split_pack(float c, float &rest)
 {

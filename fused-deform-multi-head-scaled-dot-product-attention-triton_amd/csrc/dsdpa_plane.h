@@ -35,7 +35,7 @@
 
 namespace dsdpa {
 
-constexpr int kPlaneWaves = 16;          // at most; see plane_waves for the number a launch uses
+constexpr int kPlaneWaves = 16;          // at most; see plane_config for the number a launch uses
 
 // LDS addresses as plain 32-bit numbers: the tap addresses are sums and XORs of byte offsets, and a
 // pointer made from the finished number costs no instruction (adding offsets to a generic pointer to

@@ -13,6 +13,7 @@ import torch
 
 from oracle import oracle_bwd
 from ops.triton import deform_sdpa_triton
+from parity_util import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +66,37 @@ def test_coefficients_beyond_the_largest_fp16(mode):
 @pytest.mark.parametrize("D", [64, 128])
 def test_small_gradients_of_clustered_samples(D, dout, mode):
     check(1, 2, 2, 31, 33, D, 64, 1.0, 1.0 / D ** 0.25, 1.0, dout, names=("dq", "dk", "dv"), clustered=True)
+
+
+# Pixels whose samples all have small weights (e^-12 and e^-17 of the others') in the same patches as pixels of large ones, large
+# gradients: dv of every single pixel, not of the largest. Storing the result takes 2^-12 of an element or half of 2^-24; p is good
+# to 2^-18 (logits of 17 in fp32); the coefficients' last bit is 2^-40 of p = 1, with dout of 2000 2^-29 an entry. Twice that.
+# Coefficients without their scale would miss the bar by 50 times. (dk takes the saved output's rounding through the row sums, which
+# hides what its coefficients lose.)
+@pytest.mark.parametrize("gap", [12.0, 17.0])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+def test_small_pixels_beside_large_ones_by_patches(D, gap):
+    print(f"[case] small pixels D{D} gap {gap}", flush=True)
+    V, H, Himg, Wimg = 2, 64, 9, 10
+    L, g = Himg * Wimg, torch.Generator().manual_seed(D)
+    u = torch.nn.functional.normalize(torch.randn(D, generator=g), dim=0)
+    far = (torch.arange(L) % Wimg >= 5).float()[:, None]                       # the columns of small weights
+    q = 4.0 * u + 0.1 * torch.randn(1, V, H, L, D, generator=g)
+    k = (1.0 - far * gap / 4.0) * u + 0.1 * torch.randn(1, V, H, L, D, generator=g)
+    v, dout = torch.randn(1, V, H, L, D, generator=g), 2000.0 * torch.randn(1, V, H, L, D, generator=g)
+    q, k, v, dout = (t.half() for t in (q, k, v, dout))
+    coords = torch.rand(1, V, L, V, 2, 2, generator=g)
+    coords[..., 0, 0] *= 4.0 / 9.0                                             # the first sample left of them, the second inside
+    coords[..., 1, 0] = coords[..., 1, 0] * 4.0 / 9.0 + 5.0 / 9.0
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v)]
+    out = deform_sdpa_triton(*leaves, coords.cuda(), Wimg, Himg, 1.0)
+    names = kernels_of(lambda: out.backward(dout.cuda()))
+    assert any(n.startswith("bwd_dkdv_patch_kernel") for n in names), names
+    want = oracle_bwd(*(t.float().numpy() for t in (q, k, v, coords, dout)), Wimg, Himg, 1.0)
+    a, b = leaves[2].grad.double().cpu().numpy(), np.asarray(want[2], dtype=np.float64)
+    small = np.broadcast_to(far.numpy()[:, 0] > 0, b.shape[:-1])
+    size, err = np.linalg.norm(b, axis=-1), np.linalg.norm(a - b, axis=-1)
+    assert 0 < size[small].max() < 1e-2 * np.median(size[~small])
+    over = err / (2.0 ** -11 * size + math.sqrt(D) * 2.0 ** -24)
+    print("worst of the bar", over[small].max(), over[~small].max())
+    assert over.max() <= 1.0, (over[small].max(), over[~small].max())
