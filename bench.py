@@ -42,9 +42,9 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-# HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (two runs per workload), each
+# HBM bytes per step measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (two runs per workload), each
 # counter scaled by its reading for a plain 256 MiB copy in the same run. The figures, the scale factors and
-# the commands are in profiles/hbm_traffic_*.md; profiles/traffic.json holds the bytes per launch by workload
+# the commands are in profiles/cases_traffic.md; profiles/traffic.json holds the bytes per step by workload
 # and kernel, and is rewritten whenever the counters are collected again.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 
@@ -54,7 +54,7 @@ KERNEL_SLOTS = ("fwd", "bwd_dkdv", "bwd_dq", "bwd_bin", "desc_table")     # the 
 
 
 def load_traffic(workload, which):
-    """Measured HBM bytes per launch of a kernel of a workload, or None when it was not measured."""
+    """Measured HBM bytes per step of a kernel of a workload, or None when it was not measured."""
     try:
         with open(TRAFFIC_FILE) as f:
             table = json.load(f)
