@@ -123,8 +123,8 @@ int dsdpa_fwd_noalloc(int dtype, const void *q, const void *k, const void *v, co
 /* Flags of the backward. The reference has one backward, with float atomics (ops/triton.py:345-360).
  * DSDPA_FLAG_DETERMINISTIC: bitwise reproducible dq, dk, dv: the samples of every bilinear cell are
  * added up in ascending order of their index, and the sums of every cell's four taps are stored apart and then
- * added pixel by pixel in a fixed order instead of by float atomics. Needs a larger
- * workspace (pass the same flags to dsdpa_bwd_workspace_bytes) and cannot be combined with dcoords. */
+ * added pixel by pixel in a fixed order instead of by float atomics. Needs a workspace of another
+ * size (pass the same flags to dsdpa_bwd_workspace_bytes) and cannot be combined with dcoords. */
 enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SINGLE_STREAM = 4 };
 /* B*V*H*L * V*P from which the backward may use its second stream; below it DSDPA_FLAG_SINGLE_STREAM changes nothing */
 #define DSDPA_TWO_STREAMS_FROM (1ll << 21)
@@ -132,8 +132,9 @@ enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SING
  * (clearing the accumulators, delta, the cell binning, the dk/dv kernel) runs on a second stream of the
  * library's beside the tap table and the dq kernel: neither side reads what the other writes, and the two
  * main kernels leave each other idle issue slots (C2: 7 % off the fwd+bwd step). Only on shapes whose K/V planes
- * fit in LDS, and only from DSDPA_TWO_STREAMS_FROM query*samples (B*V*H*L * V*P) up: below that the fork and join cost more host
- * time than the overlap saves. Same results either way. */
+ * fit in LDS and whose cell lists are not short (there dk/dv reads what dq hands over), and only from DSDPA_TWO_STREAMS_FROM
+ * query*samples (B*V*H*L * V*P) up: below that the fork and join cost more host time than the overlap saves. Same results either
+ * way. */
 /* DSDPA_FLAG_COORDS_GRAD: the workspace has room for the coordinate gradient's part of the per-coordinate
  * table (16 more bytes per coordinate pair where the staged kernels run), so that a backward given dcoords
  * stays on the staged dq kernel. Pass the same flags to dsdpa_bwd_workspace_bytes and to dsdpa_bwd_*;
@@ -155,14 +156,15 @@ enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SING
  * the per-row delta = dout.out (one float per query row, the reference's `delta`,
  * ops/triton.py:430), the per-(batch, key view) ordering of the samples by
  * bilinear cell (one u32 and the position inside the cell, 8 bytes, per coordinate pair, plus the cell
- * offsets; it depends on coords only and is shared by all heads) and, for bf16/fp16, the fp32 dk/dv
- * accumulators that are rounded to the storage type at the end (fp32: dk and dv
- * are themselves the accumulators), and the same per-coordinate table as the forward's -- or, on shapes
- * whose K/V planes do not fit in LDS, a buffer in which the dq kernel leaves the softmax weight and its
+ * offsets; it depends on coords only and is shared by all heads) and, for bf16/fp16 without
+ * DSDPA_FLAG_DETERMINISTIC, the fp32 dk/dv accumulators that are rounded to the storage type at the end (fp32: dk and dv
+ * are themselves the accumulators), and the same per-coordinate table as the forward's -- and, on shapes
+ * whose K/V planes do not fit in LDS or whose cell lists are short, a buffer in which the dq kernel leaves the softmax weight and its
  * gradient (8 bytes per (query row, sample)) for the dk/dv kernel: the backward runs in groups of (batch,
  * head) pairs and the buffer holds one group's, at most 128 MiB whatever the shape. The workspace is therefore
  * O(N) + O(coords) + a constant: the reference's own temporaries (dk32, dv32, delta, ops/triton.py:427-432)
- * plus 12 to 32 bytes per coordinate pair, plus at most 128 MiB; nothing in it grows with (query rows) x
+ * plus 12 to 32 bytes per coordinate pair, plus at most 128 MiB (with DSDPA_FLAG_DETERMINISTIC 8 floats per
+ * element of dk of as many (batch, head, view) planes as 256 MiB hold, at least one); nothing in it grows with (query rows) x
  * (samples) or with samples x D. Without
  * DSDPA_FLAG_DETERMINISTIC the accumulation order into dk/dv is not deterministic (float atomics,
  * as in the reference, ops/triton.py:345-360).
