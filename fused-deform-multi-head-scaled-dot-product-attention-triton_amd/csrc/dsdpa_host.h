@@ -142,21 +142,37 @@ inline bool few_samples_prefer_rows(size_t V, size_t P, size_t esize) { return P
 // Row kernels (dsdpa_rows.h) against the gather kernels, a wave per row, for fewer than 64 samples per view. The less samples
 // a row has the more the latter's empty lanes and the merge of its slots cost; the more it has the more its eight or four samples
 // in flight per row pay where the launch has few rows to fill the chip with. us, gather / rows, forward: 40x40, D = 32, fp32, N = 8
-// samples a row, 400 / 1600 waves of rows: 5 / 4, 10 / 6; N = 24, 1200 / 2400 / 4800: 12 / 16, 21 / 21, 37 / 34; N = 40, 400 / 1600: 9 / 14,
-// 21 / 22; 44x20, 14080 waves: N = 8 59 / 33, 24 94 / 84, 80 277 / 264. Beyond 64 samples 16-bit rows and narrow heads are even or
-// behind (56x50, N = 150: D = 16 fp32 801 / 840, dq 808 / 1019; D = 32 bf16 800 / 861; 48x48, N = 192, D = 64 bf16 1440 / 1450), dq with
-// D >= 64 and fp32 ahead (1716 / 1636 there; fp32 D = 64 1833 / 1364). Rows of a wave sample all views at once: with the K and
-// V planes of a (batch, head) well beyond an XCD's 4 MB of L2 that costs misses (D = 128, 56x50, V = 5: bf16, 7 MB, forward
-// 563 / 632, dq 930 / 689; fp32, 14 MB, 1851 / 2227 and 1023 / 2182).
+// samples a row, 400 / 1600 waves of rows: 5 / 4, 10 / 6; N = 24, 1200: 12 / 16; N = 40, 400 / 1600: 9 / 14, 21 / 22; 44x20, 14080
+// waves: N = 8 59 / 33. Rows of a wave sample all views at once: with the K and V planes of a (batch, head) well beyond an XCD's 4 MB of L2
+// that costs misses (D = 128, 56x50, V = 5: bf16, 7 MB, forward 563 / 632, dq 930 / 689; fp32, 14 MB, 1851 / 2227 and 1023 / 2182; V = 4, dq,
+// 5.5 MB, N = 100 over the image 0.82 to 0.95 of the gather kernel's speed).
+//
+// A workgroup of rows is long and its CU's share of the work: what the CU with the most of them has to do sets the launch's time,
+// and `fill`, the mean over the most, is what is left of the rows' advantage. Gather's time over that of rows where the workgroups
+// fill the CUs evenly, lower tenth and median over 2 to 12 views x 3 to 50 samples, 31x9 to 56x50, samples over the image, clustered
+// and around the query's place:
+//                       fp32, D = 32     64 and 128     256            bf16, D = 32     64             128 and 256
+//   N <= 32, forward    1.14 1.27        1.07 1.14      1.16 1.66      1.41 1.85        1.34 1.46      1.21 1.30
+//            dq         1.25 1.38        1.06 1.15      1.46 1.94      1.50 1.86        1.38 1.54      1.38 1.54
+//   N <= 64, forward    1.05 1.10        1.03 1.07                     1.04 1.28        1.13 1.20      1.06 1.15
+//            dq         1.10 1.18        1.02 1.08      1.58 1.88      1.20 1.39        1.14 1.26      1.20 1.38
+//   beyond,  forward    1.02 1.05        1.01 1.04      1.47 1.81      0.97 1.08        1.02 1.08      1.01 1.06 (D = 256 1.08 1.15)
+//            dq         1.03 1.09        1.00 1.03      1.54 2.07      1.13 1.19        1.04 1.12      1.12 1.22
+// The fill that a launch needs is about the inverse of the medians. (One workgroup over five a CU, fp32, D = 64, 43x24, N = 40 to 200: 0.82 to 0.99
+// without it; fp32, D = 64, 43x24, 4 views x 50 samples, clustered, 8.1 workgroups a CU: step 1035 us by rows, 948 by gather.)
 inline bool row_path(size_t rows, size_t V, size_t L, size_t D, size_t P, size_t esize, bool dq)
 {
-    const size_t N = V * P, lanes = D * esize >= 512 ? 32 : D * esize / 16, waves = rows * lanes / 64;
+    const size_t N = V * P, lanes = D * esize >= 512 ? 32 : D * esize / 16, waves = rows * lanes / 64, MB = (size_t)1 << 20;
+    const bool fp32 = esize == 4;
     if (P >= 64) return false;
     if (N <= 16) return true;
-    if (2 * V * L * D * esize > ((size_t)(dq ? 8 : 4) << 20)) return false;
-    if (N <= 32) return waves >= 2048;
-    if (N <= 64) return waves >= 4096 && (esize == 2 || D >= 32);
-    return waves >= 8192 && D >= 64 && (dq || esize == 4 || D == 256);
+    if (2 * V * L * D * esize > (!dq ? 4 : fp32 && D == 128 ? 5 : 8) * MB) return false;
+    if (waves < (N <= 32 ? 2048 : N <= 64 ? 4096 : 8192)) return false;
+    if (N > 32 && fp32 && D < 32) return false;
+    if (N > 64 && (D < 64 || (!dq && !fp32 && D < 256))) return false;
+    const size_t per = 4 * (64 / lanes), groups = rows / (V * L) * ((V * L + per - 1) / per);     // workgroups, 256 CUs
+    const size_t fill = 100 * groups / ((groups + 255) / 256 * 256);
+    return fill >= (fp32 && D == 256 ? 65 : N <= 32 ? (fp32 && D >= 64 ? 88 : 80) : N <= 64 ? (fp32 ? 95 : 85) : fp32 ? 97 : 93);
 }
 
 // Descriptor table of the plane kernels: per coordinate pair 16 bytes of weights and 4 of packed slot

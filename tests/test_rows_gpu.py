@@ -9,7 +9,7 @@ import torch
 
 from oracle import oracle_bwd, oracle_fwd
 from ops.triton import deform_sdpa_triton
-from parity_util import rel
+from parity_util import kernels_of, oracle_on_slices, rel
 
 pytestmark = pytest.mark.gpu
 BAR = {torch.float32: (1e-4, 1e-3), torch.bfloat16: (2e-2, 2e-2), torch.float16: (2e-2, 2e-2)}
@@ -57,6 +57,23 @@ def test_rows_with_the_coordinate_gradient(D, P, dtype):
 @pytest.mark.parametrize("V,H,P,dtype", [(2, 10, 12, torch.float32), (2, 20, 10, torch.bfloat16), (3, 14, 21, torch.bfloat16)], ids=str)
 def test_many_rows(V, H, P, dtype):
     check(1, V, H, 30, 31, 64, P, dtype)
+
+
+# 5.94 workgroups of rows a CU, and 5.03, which leave a sixth of the last one's time empty: rows and a wave per row
+@pytest.mark.parametrize("H,kernels", [(13, ("fwd_rows_kernel", "bwd_dq_rows_kernel")), (11, ("fwd_gather_kernel", "bwd_dq_gather_kernel"))])
+def test_rows_where_their_workgroups_fill_the_cus(H, kernels):
+    print(f"[case] rows or a wave per row, H {H}", flush=True)
+    g = torch.Generator().manual_seed(H)
+    L, dev = 30 * 31, [torch.randn(1, 2, H, 30 * 31, 64, generator=g).cuda().requires_grad_(True) for _ in range(3)]
+    coords, dout = torch.rand(1, 2, L, 2, 20, 2, generator=g), torch.randn(1, 2, H, L, 64, generator=g)
+    out = []
+    names = kernels_of(lambda: out.append(deform_sdpa_triton(*dev, coords.cuda(), 31, 30, 0.125)))
+    names |= kernels_of(lambda: out[0].backward(dout.cuda()))
+    assert all(any(n.startswith(k) for n in names) for k in kernels), names
+    slices = [(0, 0), (0, H - 1)]
+    for (b, h), (ro, *want) in oracle_on_slices(*(t.detach().cpu() for t in dev), coords, dout, 31, 30, 0.125, slices).items():
+        for a, w, bar in zip([out[0]] + [t.grad for t in dev], [ro] + want, (1e-4, 1e-3, 1e-3, 1e-3)):
+            assert rel(a[b:b + 1, :, h:h + 1], w) < bar, h
 
 
 # infinite V at the taps of a row's last sample, rows of an odd number of samples: infinite, not NaN
