@@ -497,9 +497,11 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
     constexpr int G = D / DC, NS = kWave / G;
     constexpr int kRow = D * S::kBytes;
     constexpr bool kPacked = S::kBytes == 2 && !CG;
-    // The scheduler requests a trip's taps all together, which at 16 waves a workgroup, 128 registers a lane, spills in these
-    // forms; they, and the coordinate gradient, are held to one pair of taps, or one tap, at a time.
-    constexpr bool kTight = (DC == 16 && S::kBytes == 2) || (HAND && ROWS == 2 && S::kBytes * DC == 32);
+    // The scheduler requests a trip's taps all together, which at 16 waves a workgroup, 128 registers a lane, spills up to 372 bytes
+    // in these forms; they are held to one pair of taps, or one tap, at a time, and to the row index alone (9x10, 4 views x 4 samples,
+    // D = 256, bf16, with the coordinate gradient: step 545 -> 202 us). The others lose 2 to 6 % of dq that way (18x18 and less, D = 16 to
+    // 128), also the coordinate gradient in bf16 with the 20 bytes that it spills outside the trips.
+    constexpr bool kTight = CG ? DC == 16 : (DC == 16 && S::kBytes == 2) || (HAND && ROWS == 2 && S::kBytes * DC == 32);
     static_assert(G >= 2 && G <= 16 && G * DC == D, "lane split");
     extern __shared__ __attribute__((aligned(kPlaneLdsAlign))) unsigned char smem[];
     const int img_bytes = plane_lds_bytes<S, D>(dm.L);
@@ -523,6 +525,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
     // per row block: this slot's row and its state
     bool have_s[ROWS];
     unsigned qc_s[ROWS];
+    size_t crow_s[ROWS], roff_s[ROWS], hrow_s[ROWS];               // (kTight: made from qc_s where they are used)
     float qf_s[ROWS][DC], dof_s[ROWS][DC], dqa_s[ROWS][DC], delta_s[ROWS], lse_s[ROWS];
     uint32_t dop_s[ROWS][kPacked ? DC / 2 : 1];
 #pragma unroll
@@ -534,6 +537,9 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         const size_t row = (((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l;
         qc_s[rb] = qc;
         const size_t roff = row * (size_t)kRow;
+        crow_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.L + l) * (size_t)dm.N;
+        hrow_s[rb] = ((size_t)(pb.b * dm.H + pb.h - bh0) * nq + qc) * (size_t)dm.N;
+        roff_s[rb] = roff;
         float of[DC];
         Lane::load((const char *)q_ + dm.q_row(pb.b, (int)s1, pb.h, (int)l) * S::kBytes, lane_byte, qf_s[rb]);
         Lane::load((const char *)dout_ + roff, lane_byte, dof_s[rb]);
@@ -556,7 +562,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
 #pragma unroll
         for (int rb = 0; rb < ROWS; ++rb) {
         const bool have = have_s[rb];
-        const size_t crow = ((size_t)pb.b * nq + qc_s[rb]) * (size_t)dm.N;
+        const size_t crow = kTight ? ((size_t)pb.b * nq + qc_s[rb]) * (size_t)dm.N : crow_s[rb];
         const float (&qf)[DC] = qf_s[rb];
         const float (&dof)[DC] = dof_s[rb];
         const uint32_t (&dop)[kPacked ? DC / 2 : 1] = dop_s[rb];
@@ -580,8 +586,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                     float dot = 0.f, dp = 0.f;
 #pragma unroll
                     for (int d = 0; d < DC; ++d) kk[d] = 0.f;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
+                    auto k_tap = [&](int i) {
                         float tk[DC];
                         Lane::read(kp[i], (i & 1) * 2 * kRow, tk);
                         dk_t[i] = 0.f;
@@ -591,17 +596,27 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                             kk[d] = fmaf(wt[i], tk[d], kk[d]);
                         }
                         dot = fmaf(wt[i], dk_t[i], dot);
-                        if (DC == 16 || (i & 1)) __builtin_amdgcn_sched_barrier(0);
-                    }
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
+                    };
+                    auto v_tap = [&](int i) {
                         float tv[DC];
                         Lane::read(vp[i], (i & 1) * 2 * kRow, tv);
                         dv_t[i] = 0.f;
 #pragma unroll
                         for (int d = 0; d < DC; ++d) dv_t[i] = fmaf(dof[d], tv[d], dv_t[i]);
                         dp = fmaf(wt[i], dv_t[i], dp);
-                        if (DC == 16 || (i & 1)) __builtin_amdgcn_sched_barrier(0);
+                    };
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        k_tap(i);
+                        if constexpr (kTight) __builtin_amdgcn_sched_barrier(0);
+                        else v_tap(i);
+                    }
+                    if constexpr (kTight) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            v_tap(i);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
                     }
                     dot = group_sum<G>(dot);
                     dp = group_sum<G>(dp);
@@ -635,16 +650,19 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                 float dot = 0.f, dp = 0.f;
                 {
                     float t0[DC], t1[DC], t2[DC], t3[DC];
+                    if constexpr (!kTight) { Lane::read(at, 0, t0); Lane::read(at ^ kRow, 2 * kRow, t1); }
                     Lane::read(ab, 0, t2);
                     Lane::read(ab ^ kRow, 2 * kRow, t3);
+                    if constexpr (kTight) {
 #pragma unroll
-                    for (int d = 0; d < DC; ++d) kk[d] = fmaf(w.z, t2[d], w.w * t3[d]);
-                    if constexpr (kTight) __builtin_amdgcn_sched_barrier(0);
-                    Lane::read(at, 0, t0);
-                    Lane::read(at ^ kRow, 2 * kRow, t1);
+                        for (int d = 0; d < DC; ++d) t3[d] = fmaf(w.z, t2[d], w.w * t3[d]);
+                        __builtin_amdgcn_sched_barrier(0);
+                        Lane::read(at, 0, t0);
+                        Lane::read(at ^ kRow, 2 * kRow, t1);
+                    }
 #pragma unroll
                     for (int d = 0; d < DC; ++d) {
-                        kk[d] = fmaf(w.x, t0[d], fmaf(w.y, t1[d], kk[d]));
+                        kk[d] = fmaf(w.x, t0[d], fmaf(w.y, t1[d], kTight ? t3[d] : fmaf(w.z, t2[d], w.w * t3[d])));
                         dot = fmaf(qf[d], kk[d], dot);
                     }
                 }
@@ -653,15 +671,21 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                     dp = tap_dot16<S, DC>(lds_at(at ^ kRow), lds_at(at + 2 * kRow), lds_at(ab ^ kRow), lds_at(ab + 2 * kRow), w, dop);
                 } else {
                     float u0[DC], u1[DC], u2[DC], u3[DC];
+                    if constexpr (!kTight) { Lane::read(at ^ kRow, 0, u0); Lane::read(at, 2 * kRow, u1); }
                     Lane::read(ab ^ kRow, 0, u2);
                     Lane::read(ab, 2 * kRow, u3);
+                    if constexpr (kTight) {
 #pragma unroll
-                    for (int d = 0; d < DC; ++d) u3[d] = fmaf(w.z, u2[d], w.w * u3[d]);
-                    if constexpr (kTight) __builtin_amdgcn_sched_barrier(0);
-                    Lane::read(at ^ kRow, 0, u0);
-                    Lane::read(at, 2 * kRow, u1);
+                        for (int d = 0; d < DC; ++d) u3[d] = fmaf(w.z, u2[d], w.w * u3[d]);
+                        __builtin_amdgcn_sched_barrier(0);
+                        Lane::read(at ^ kRow, 0, u0);
+                        Lane::read(at, 2 * kRow, u1);
+                    }
 #pragma unroll
-                    for (int d = 0; d < DC; ++d) dp = fmaf(dof[d], fmaf(w.x, u0[d], fmaf(w.y, u1[d], u3[d])), dp);
+                    for (int d = 0; d < DC; ++d) {
+                        const float vv = fmaf(w.x, u0[d], fmaf(w.y, u1[d], kTight ? u3[d] : fmaf(w.z, u2[d], w.w * u3[d])));
+                        dp = fmaf(dof[d], vv, dp);
+                    }
                 }
                 dot = group_sum<G>(dot);
                 dp = group_sum<G>(dp);
@@ -675,7 +699,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
                 for (int d = 0; d < DC; ++d) dqa[d] = fmaf(ds, kk[d], dqa[d]);
             }
             if (HAND && have && c0 + g < dm.P)
-                handed_[((size_t)(pb.b * dm.H + pb.h - bh0) * nq + qc_s[rb]) * (size_t)dm.N + (size_t)(s2 * dm.P + my_n)] =
+                handed_[(kTight ? ((size_t)(pb.b * dm.H + pb.h - bh0) * nq + qc_s[rb]) * (size_t)dm.N : hrow_s[rb]) + (size_t)(s2 * dm.P + my_n)] =
                     make_float2(my_p, my_ds * dm.sm_scale);
             if (CG && have && c0 + g < dm.P) {
                 float *dst = dcoords_ + 2 * (crow + (size_t)s2 * dm.P + (size_t)my_n);
@@ -691,8 +715,12 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         if (have_s[rb]) {
 #pragma unroll
             for (int d = 0; d < DC; ++d) dqa_s[rb][d] *= dm.sm_scale;
-            const unsigned s1 = dm.divL.div(qc_s[rb]), l = qc_s[rb] - s1 * (unsigned)dm.L;
-            Lane::store((char *)dq_ + ((((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l) * (size_t)kRow, lane_byte, dqa_s[rb]);
+            size_t roff = roff_s[rb];
+            if constexpr (kTight) {
+                const unsigned s1 = dm.divL.div(qc_s[rb]), l = qc_s[rb] - s1 * (unsigned)dm.L;
+                roff = ((((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l) * (size_t)kRow;
+            }
+            Lane::store((char *)dq_ + roff, lane_byte, dqa_s[rb]);
         }
     }
 }
