@@ -132,6 +132,20 @@ inline bool plane_path_fits(size_t L, size_t D, size_t esize, bool coords_grad =
     return (L + 2) * 2 * D * esize + kPlaneDescLdsBytes + (coords_grad ? kPlaneGradLdsBytes : 0) <= kLdsBytes;
 }
 
+// Whether the staged dq kernel leaves dk/dv's workgroups, of some KB of LDS each, room beside its own, of which a CU holds one. Where it
+// leaves little, they come in as its workgroups end, and a second round of those finds no CU with enough LDS free before dk/dv
+// runs out. Backward on one stream over that on two, mean and range of 260 shapes (2 to 12 views x 4 to 63 samples, all types): one round
+// of dq with 0 to 8 KB left 0.98 (0.94 to 1.05), 8 to 24 KB 1.05 (0.98 to 1.13), 24 KB and more 1.17 (0.99 to 1.50); more rounds with 0
+// to 20 KB 0.93 (0.85 to 1.00), 24 KB and more 1.05 (1.00 to 1.11). A round: 256 workgroups of at most 16 waves and two blocks
+// of rows (one with the coordinate gradient or 16 elements a lane).
+inline bool dq_leaves_room(size_t planes, size_t V, size_t L, size_t D, size_t esize, bool coords_grad)
+{
+    const size_t lanes = D * esize / 16 < 16 ? D * esize / 16 : 16, rows = (coords_grad || D / lanes > 8 ? 16 : 32) * (64 / lanes);
+    const bool one_round = planes * ((V * L + rows - 1) / rows) <= 256;
+    const size_t used = (L + 2) * 2 * D * esize + kPlaneDescLdsBytes + (coords_grad ? kPlaneGradLdsBytes : 0);
+    return used + (one_round ? 8 : 24) * 1024 <= kLdsBytes;
+}
+
 // With very few samples per view the staged kernels mostly stage: every workgroup loads all V plane pairs for P samples
 // per row and view, while the row kernels touch only the rows they sample, and need no table. us a step, staged / rows, D = 32,
 // 18x14: fp32 V = 8: P = 1 114 / 92, P = 2 165 / 163, P = 3 185 / 195; V = 12: P = 1 242 / 178, 2 293 / 277, 3 341 / 357; V = 4: P = 2

@@ -875,7 +875,9 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     // under two million query*samples (0.15 ms of kernels) does not win back.
     hipStream_t bst = st;
     const bool worth_forking = (long long)dm.rows * dm.N >= DSDPA_TWO_STREAMS_FROM;
-    SideLane *side = cell_binned && staged && !patch && worth_forking && !(flags & DSDPA_FLAG_SINGLE_STREAM) ? side_lane() : nullptr;
+    const bool forks = cell_binned && staged && !patch && worth_forking && !(flags & DSDPA_FLAG_SINGLE_STREAM) &&
+                       dq_leaves_room((size_t)dm.B * dm.H, V, dm.L, D, S::kBytes, dcoords != nullptr);
+    SideLane *side = forks ? side_lane() : nullptr;
     const size_t ncounters = cell_binned && !bin_in_one_launch(dm) ? wl.counters_bytes / 4 : 0;
     SideJoin joiner;
     if (side && hipEventRecord(side->fork, st) == hipSuccess &&

@@ -132,7 +132,7 @@ enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SING
  * (clearing the accumulators, delta, the cell binning, the dk/dv kernel) runs on a second stream of the
  * library's beside the tap table and the dq kernel: neither side reads what the other writes, and the two
  * main kernels leave each other idle issue slots (C2: 7 % off the fwd+bwd step). Only on shapes whose K/V planes
- * fit in LDS and whose cell lists are not short (there dk/dv reads what dq hands over), and only from DSDPA_TWO_STREAMS_FROM
+ * fit in LDS with room to spare and whose cell lists are not short (there dk/dv reads what dq hands over), and only from DSDPA_TWO_STREAMS_FROM
  * query*samples (B*V*H*L * V*P) up: below that the fork and join cost more host time than the overlap saves. Same results either
  * way. */
 /* DSDPA_FLAG_COORDS_GRAD: the workspace has room for the coordinate gradient's part of the per-coordinate

@@ -13,6 +13,7 @@ import torch
 
 from ops import _native
 from ops.triton import deform_sdpa_triton
+from parity_util import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -100,6 +101,21 @@ def test_lists_made_beside_dq(dims):
     tol = 1e-5 if dtype == torch.float32 else 1e-2         # order of the float atomics / one rounding to 16 bits
     assert torch.equal(one[1], two[1])
     assert rel(two[2], one[2]) < tol and rel(two[3], one[3]) < tol
+
+
+# 15 KB of LDS left beside a workgroup of dq: two streams where dq is one round of workgroups (160), one where it is more (260). The
+# (lse, delta) pairs are a launch of their own on the second stream only
+@pytest.mark.parametrize("H,two", [(40, True), (65, False)])
+def test_second_stream_where_dq_leaves_room(H, two):
+    say(f"[case] room beside dq H{H}")
+    q, k, v, c, do = make(60, 1, 2, H, 36, 12, 64, 39, torch.float16)
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    out = deform_sdpa_triton(*leaves, c, 12, 36, 0.3)
+    names = kernels_of(lambda: out.backward(do))
+    assert any(n.startswith("delta_kernel") for n in names) == two, names
+    one = c_abi_backward(*(t.detach() for t in leaves), c, do, 36, 12, _native.FLAG_SINGLE_STREAM)
+    for t, w in zip(leaves, one[1:4]):
+        assert rel(t.grad, w) < 1e-2                       # float atomics / one rounding to 16 bits
 
 
 def test_caller_stream_is_ordered_before_and_after():
