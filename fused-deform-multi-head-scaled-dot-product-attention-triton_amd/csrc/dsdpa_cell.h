@@ -462,7 +462,7 @@ __device__ __forceinline__ void cell_sums(
     const float2 *__restrict__ stats_,
     const void *__restrict__ dout_, const unsigned *__restrict__ start, const unsigned *__restrict__ sorted,
     const uint4 *__restrict__ items, const float2 *__restrict__ handed_,
-    float *__restrict__ dk_acc, float *__restrict__ dv_acc, const Dims &dm, int NC, const CellGrid &cg)
+    float *__restrict__ dk_acc, float *__restrict__ dv_acc, const GradDims &dm, int NC, const CellGrid &cg)
 {
     constexpr int G = D / DC;
     constexpr int NS = kWave / G;
@@ -524,7 +524,7 @@ __device__ __forceinline__ void cell_sums(
     }
     const int tpix[4] = { y0 * dm.Wimg + x0, y0 * dm.Wimg + x0 + 1, (y0 + 1) * dm.Wimg + x0,
                           (y0 + 1) * dm.Wimg + x0 + 1 };
-    const size_t plane_base = ((grp * dm.H) + h) * (size_t)dm.L * D;          // elements in dk/dv; grp = b*V + s2
+    const size_t plane_base = dm.acc_plane<S, D>(b, s2, h);                     // elements in dk/dv
     const size_t kv_base = dm.kv_plane(b, s2, h);                               // ... in k and v
     const char *kb = (const char *)k_ + kv_base * S::kBytes;
     const char *vb = (const char *)v_ + kv_base * S::kBytes;
@@ -1008,7 +1008,7 @@ __device__ __forceinline__ void cell_sums(
             const float val = fl[idx];
             if (ok) {
                 if constexpr (FIXED) tap_place(which, r, pix)[dd] = val;
-                else atomicAdd(acc + (size_t)pix * D + dd, val);
+                else atomicAdd(acc + (size_t)pix * dm.acc_pixel<S, D>() + dd, val);
             }
         }
     }
@@ -1018,7 +1018,7 @@ __device__ __forceinline__ void cell_sums(
     const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_,                                 \
     const float2 *__restrict__ stats_, const void *__restrict__ dout_, const unsigned *__restrict__ start,                  \
     const unsigned *__restrict__ sorted, const uint4 *__restrict__ items, const float2 *__restrict__ handed_,               \
-    float *__restrict__ dk_acc, float *__restrict__ dv_acc, Dims dm, int NC, CellGrid cg
+    float *__restrict__ dk_acc, float *__restrict__ dv_acc, GradDims dm, int NC, CellGrid cg
 
 template <typename S, int D, int DC, bool HANDED, bool FIXED>
 __global__ __launch_bounds__(kCellWaves *kWave, HANDED ? (DC <= 4 ? 5 : (S::kBytes == 2 ? 3 : 4))
@@ -1037,7 +1037,7 @@ void bwd_dkdv_cell_kernel(DSDPA_CELL_ARGS)
 // eight floats read per element of dk and dv.
 template <typename S, int D>
 __global__ __launch_bounds__(256) void combine_taps_kernel(const float *__restrict__ dk_taps, const float *__restrict__ dv_taps,
-                                                           void *__restrict__ dk_, void *__restrict__ dv_, Dims dm, CellGrid cg)
+                                                           void *__restrict__ dk_, void *__restrict__ dv_, GradDims dm, CellGrid cg)
 {
     constexpr int VE = S::kBytes == 4 ? 4 : 8;
     const unsigned per = (unsigned)dm.L * (D / VE);                          // threads per plane
@@ -1045,7 +1045,8 @@ __global__ __launch_bounds__(256) void combine_taps_kernel(const float *__restri
     if (at >= per) return;
     const unsigned bhl = cg.div_v.div(t + cg.t0), s2 = t + cg.t0 - bhl * (unsigned)dm.V, bh = (unsigned)cg.bh0 + bhl;
     const unsigned b = cg.div_h.div(bh), h = bh - b * (unsigned)dm.H;
-    const size_t dst = (((size_t)b * dm.V + s2) * dm.H + h) * dm.L * D + (size_t)at * VE;
+    const unsigned pix = at / (D / VE);
+    const size_t dst = dm.dkv_plane((int)b, (int)s2, (int)h) + pix * (unsigned)dm.dkv_sl + (at - pix * (D / VE)) * VE;
     const size_t tap = (size_t)cg.nplanes * dm.L * D;
 #pragma unroll
     for (int which = 0; which < 2; ++which) {

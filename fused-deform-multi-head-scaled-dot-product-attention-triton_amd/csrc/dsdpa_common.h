@@ -38,8 +38,9 @@ struct Dims {
     float sm_scale;
     FastDiv divP, divL;                 // for decoding sample ids (s1*L + l)*P + p
     // Element strides of the inputs q and k/v (k and v share one set) over (batch, view, head, pixel); the head
-    // dimension itself is contiguous. Everything else (out, lse, dout, the gradients) is contiguous
-    // [B][V][H][L][D]. Offsets inside one (batch, head) -- view*sv + pixel*sl -- fit 32 bits.
+    // dimension itself is contiguous. Everything else (out, lse, dout) is contiguous [B][V][H][L][D], and so are the
+    // gradients unless the caller asked for dq laid out as q and dk, dv as k. Offsets inside one (batch, head) --
+    // view*sv + pixel*sl -- fit 32 bits.
     long long q_sb, q_sh, kv_sb, kv_sh;
     int q_sv, q_sl, kv_sv, kv_sl;
     __device__ __forceinline__ size_t q_row(int b, int s1, int h, int l) const
@@ -50,6 +51,27 @@ struct Dims {
     {
         return (size_t)((long long)b * kv_sb + (long long)h * kv_sh) + (size_t)((unsigned)view * (unsigned)kv_sv);
     }
+};
+
+// What the backward's kernels take: also the strides of dq, and of dk and dv.
+struct GradDims : Dims {
+    long long dq_sb, dq_sh, dkv_sb, dkv_sh;
+    int dq_sv, dq_sl, dkv_sv, dkv_sl;
+    // a row of dq inside its (batch, head), and the (batch, head)
+    __device__ __forceinline__ unsigned dq_at(unsigned s1, unsigned l) const { return s1 * (unsigned)dq_sv + l * (unsigned)dq_sl; }
+    __device__ __forceinline__ size_t dq_bh(int b, int h) const { return (size_t)((long long)b * dq_sb + (long long)h * dq_sh); }
+    __device__ __forceinline__ size_t dkv_plane(int b, int view, int h) const
+    {
+        return (size_t)((long long)b * dkv_sb + (long long)h * dkv_sh) + (size_t)((unsigned)view * (unsigned)dkv_sv);
+    }
+    // The same of what dk and dv are summed in: themselves in fp32, contiguous accumulators in 16-bit storage.
+    template <typename S, int D>
+    __device__ __forceinline__ size_t acc_plane(int b, int view, int h) const
+    {
+        return S::kBytes == 4 ? dkv_plane(b, view, h) : (((size_t)b * V + view) * H + h) * (size_t)L * D;
+    }
+    template <typename S, int D>
+    __device__ __forceinline__ unsigned acc_pixel() const { return S::kBytes == 4 ? (unsigned)dkv_sl : (unsigned)D; }
 };
 
 // ------------------------------------------------------------------ storage types

@@ -753,7 +753,7 @@ __global__ __launch_bounds__(kGatherWaves *kWave, (WIN && !CG && DC <= 8) ? 4 : 
     const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_,
     const float *__restrict__ coords_, const void *__restrict__ out_, const float *__restrict__ lse_,
     const void *__restrict__ dout_, void *__restrict__ dq_, float2 *__restrict__ stats_,
-    float *__restrict__ dcoords_, float2 *__restrict__ handed_, Dims dm, int work0, int work_end)
+    float *__restrict__ dcoords_, float2 *__restrict__ handed_, GradDims dm, int work0, int work_end)
 {
     constexpr int G = D / DC;
     constexpr int NS = kWave / G;
@@ -1071,9 +1071,11 @@ __global__ __launch_bounds__(kGatherWaves *kWave, (WIN && !CG && DC <= 8) ? 4 : 
         for (int d = 0; d < DC; ++d) dqa[d] += __shfl_xor(dqa[d], off, kWave);
     }
     if (slot == 0) {
+        const int t1 = work / dm.L, t2 = t1 / dm.V, t3 = t2 / dm.H;              // (b, h, s1, l), as decode_row
+        const size_t dq_row = dm.dq_bh(t3, t2 - t3 * dm.H) + dm.dq_at((unsigned)(t1 - t2 * dm.V), (unsigned)(work - t1 * dm.L));
 #pragma unroll
         for (int d = 0; d < DC; ++d) dqa[d] *= dm.sm_scale;
-        store_chunk<S, DC>((char *)dq_ + roff, dqa);
+        store_chunk<S, DC>((char *)dq_ + (dq_row + lane_elem) * S::kBytes, dqa);
     }
 }
 

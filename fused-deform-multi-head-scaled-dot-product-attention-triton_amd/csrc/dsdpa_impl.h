@@ -49,9 +49,23 @@ int allow_full_lds(K kern, std::atomic<unsigned long long> &done)
     return DSDPA_OK;
 }
 
+// Where the 8 elements `i` of the contiguous accumulators go in dk and dv (elements; per8: 8 elements of a row of D).
+struct GradPlace {
+    FastDiv div_per8, div_v, div_h;
+    bool plain;                                  // contiguous gradients: at their own place
+};
+__device__ __forceinline__ size_t grad_place(const GradPlace &gp, const GradDims &dm, unsigned per8, size_t i)
+{
+    if (gp.plain) return i * 8;
+    const unsigned row = gp.div_per8.div((unsigned)i), c = (unsigned)i - row * per8;       // (rows * D / 8 < 2^31: checked by the host)
+    const unsigned t = dm.divL.div(row), l = row - t * (unsigned)dm.L;
+    const unsigned bv = gp.div_h.div(t), h = t - bv * (unsigned)dm.H, b = gp.div_v.div(bv);
+    return dm.dkv_plane((int)b, (int)(bv - b * (unsigned)dm.V), (int)h) + l * (unsigned)dm.dkv_sl + c * 8u;
+}
+
 // fp32 accumulators -> 16-bit storage, 8 elements per thread
 template <typename S>
-__global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ dst, size_t n8)
+__global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ dst, size_t n8, GradDims dm, GradPlace gp, unsigned per8)
 {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -61,7 +75,7 @@ __global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ ds
         float4 a = s4[0], b = s4[1];
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
         v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-        store_chunk<S, 8>((char *)dst + i * 16, v);
+        store_chunk<S, 8>((char *)dst + grad_place(gp, dm, per8, i) * 2, v);
     }
 }
 
@@ -69,7 +83,7 @@ __global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ ds
 // (n8 = elements of a (batch, view, head) over 8). At once over where there are none.
 template <typename S>
 __global__ void cast_rest_kernel(const unsigned *__restrict__ left, const float *__restrict__ dk_acc, const float *__restrict__ dv_acc,
-                                 void *__restrict__ dk, void *__restrict__ dv, Dims dm, size_t n8)
+                                 void *__restrict__ dk, void *__restrict__ dv, GradDims dm, size_t n8, GradPlace gp, unsigned per8)
 {
     const size_t per = n8 * dm.H, stride = (size_t)gridDim.x * blockDim.x;
     const bool all = mostly_long(left, dm.B * dm.V);
@@ -80,7 +94,7 @@ __global__ void cast_rest_kernel(const unsigned *__restrict__ left, const float 
             const float4 *s4 = reinterpret_cast<const float4 *>(i < per ? dk_acc : dv_acc) + 2 * at;
             const float4 a = s4[0], b = s4[1];
             const float v[8] = { a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w };
-            store_chunk<S, 8>((char *)(i < per ? dk : dv) + at * 16, v);
+            store_chunk<S, 8>((char *)(i < per ? dk : dv) + grad_place(gp, dm, per8, at) * 2, v);
         }
     }
 }
@@ -155,6 +169,41 @@ static inline int apply_strides(const long long *st, int D, int esize, Dims *dm,
     return DSDPA_OK;
 }
 
+// Whether element strides over (batch, view, head, pixel), a row of D being contiguous, place the elements without holes or overlaps.
+static inline bool dense_strides(const Dims &dm, int D, long long sb, long long sv, long long sh, long long sl)
+{
+    const long long size[4] = { dm.B, dm.V, dm.H, dm.L };
+    long long stride[4] = { sb, sv, sh, sl }, want = D;
+    bool used[4] = { size[0] == 1, size[1] == 1, size[2] == 1, size[3] == 1 };
+    for (int n = 0; n < 4; ++n) {
+        int next = -1;
+        for (int i = 0; i < 4; ++i)
+            if (!used[i] && stride[i] == want) next = i;
+        if (next < 0) break;
+        used[next] = true;
+        want *= size[next];
+    }
+    return used[0] && used[1] && used[2] && used[3];
+}
+
+// DSDPA_FLAG_GRADS_AS_INPUTS: dq laid out as q, dk and dv as k and v. Each fills a block of memory of its tensor's size (fp32 dk and dv
+// are cleared as such a block).
+static inline int apply_grad_strides(int D, bool as_inputs, GradDims *dm)
+{
+    const long long L = dm->L, H = dm->H;
+    dm->dq_sl = dm->dkv_sl = D;
+    dm->dq_sh = dm->dkv_sh = L * D;
+    dm->dq_sv = dm->dkv_sv = (int)(H * L * D);
+    dm->dq_sb = dm->dkv_sb = (long long)dm->V * H * L * D;
+    if (!as_inputs) return DSDPA_OK;
+    if (!dense_strides(*dm, D, dm->q_sb, dm->q_sv, dm->q_sh, dm->q_sl) || !dense_strides(*dm, D, dm->kv_sb, dm->kv_sv, dm->kv_sh, dm->kv_sl))
+        return DSDPA_ERR_BAD_STRIDES;
+    if ((long long)dm->rows * D / 8 > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;
+    dm->dq_sb = dm->q_sb; dm->dq_sv = dm->q_sv; dm->dq_sh = dm->q_sh; dm->dq_sl = dm->q_sl;
+    dm->dkv_sb = dm->kv_sb; dm->dkv_sv = dm->kv_sv; dm->dkv_sh = dm->kv_sh; dm->dkv_sl = dm->kv_sl;
+    return DSDPA_OK;
+}
+
 // lanes per sample are D/DC; DC is chosen so that a lane moves 16 bytes per tap
 // (32 or 64 for the widest heads) and a sample never spans more than 16 lanes.
 template <typename S, int D> struct Chunk {
@@ -196,7 +245,7 @@ int launch_fwd_rows(const void *q, const void *k, const void *v, const float *co
 }
 template <typename S, int D>
 int launch_bwd_dq_rows(const void *q, const void *k, const void *v, const float *coords, const void *out, const float *lse,
-                       const void *dout, void *dq, float2 *stats, float *dcoords, float2 *handed, const Dims &dm, int bh0, int nbh,
+                       const void *dout, void *dq, float2 *stats, float *dcoords, float2 *handed, const GradDims &dm, int bh0, int nbh,
                        hipStream_t st)
 {
     constexpr int DC = RowChunk<S, D>::value;
@@ -268,7 +317,7 @@ int launch_fwd_slab(const void *q, const void *k, const void *v, const float *co
 template <typename S, int D, bool CG>
 int launch_bwd_dq_slab_cg(const void *q, const void *k, const void *v, const float *coords, const void *out,
                           const float *lse, const void *dout, void *dq, float2 *stats, float2 *handed, float *dcoords,
-                          const Dims &dm, int bh0, int nbh, hipStream_t st)
+                          const GradDims &dm, int bh0, int nbh, hipStream_t st)
 {
     if constexpr (S::kBytes != 4 || (D != 32 && D != 64 && D != 128)) {
         return DSDPA_ERR_UNSUPPORTED;
@@ -297,7 +346,7 @@ int launch_bwd_dq_slab_cg(const void *q, const void *k, const void *v, const flo
 template <typename S, int D>
 int launch_bwd_dq_slab(const void *q, const void *k, const void *v, const float *coords, const void *out,
                        const float *lse, const void *dout, void *dq, float2 *stats, float2 *handed, float *dcoords,
-                       const Dims &dm, int bh0, int nbh, hipStream_t st)
+                       const GradDims &dm, int bh0, int nbh, hipStream_t st)
 {
     return dcoords ? launch_bwd_dq_slab_cg<S, D, true>(q, k, v, coords, out, lse, dout, dq, stats, handed, dcoords, dm, bh0, nbh, st)
                    : launch_bwd_dq_slab_cg<S, D, false>(q, k, v, coords, out, lse, dout, dq, stats, handed, dcoords, dm, bh0, nbh, st);
@@ -349,7 +398,7 @@ int launch_bwd_gather(const void *q, const void *k, const void *v, const float *
 template <typename S, int D>
 int launch_bwd_dq_gather(const void *q, const void *k, const void *v, const float *coords, const void *out,
                          const float *lse, const void *dout, void *dq, float2 *stats, float *dcoords,
-                         float2 *handed, const Dims &dm, int bh0, int nbh, hipStream_t st)
+                         float2 *handed, const GradDims &dm, int bh0, int nbh, hipStream_t st)
 {
     constexpr int DC = Chunk<S, D>::value;
     const int work0 = bh0 * dm.V * dm.L, work_end = (bh0 + nbh) * dm.V * dm.L;      // (at most dm.rows)
@@ -415,7 +464,7 @@ static inline TileGeom make_tile_geom(const Dims &dm, int D)
 
 template <typename S, int D>
 int launch_bwd_dkdv_tile(const void *q, const void *k, const void *v, const float *coords,
-                         const float2 *stats, const void *dout, float *dk_acc, float *dv_acc, const Dims &dm,
+                         const float2 *stats, const void *dout, float *dk_acc, float *dv_acc, const GradDims &dm,
                          hipStream_t st)
 {
     constexpr int DC = Chunk<S, D>::value;
@@ -502,7 +551,7 @@ int launch_fwd_plane(const void *q, const void *k, const void *v, const float4 *
 template <typename S, int D, int DC>
 int launch_bwd_dq_plane_as(const void *q, const void *k, const void *v, const float4 *desc_w, const uint32_t *desc_e,
                            const void *out, const float *lse, const void *dout, void *dq, float2 *stats, const float4 *desc_g,
-                           float *dcoords, float2 *handed, const Dims &dm, int bh0, int nbh, const PlaneConfig &pc, hipStream_t st)
+                           float *dcoords, float2 *handed, const GradDims &dm, int bh0, int nbh, const PlaneConfig &pc, hipStream_t st)
 {
     const size_t smem = (size_t)plane_lds_bytes<S, D>(dm.L) + kPlaneDescBytes + (dcoords ? kPlaneGradBytes : 0);
     const int rows_per_block = pc.row_blocks * pc.waves * (kWave / (D / DC));
@@ -526,7 +575,7 @@ int launch_bwd_dq_plane_as(const void *q, const void *k, const void *v, const fl
 template <typename S, int D>
 int launch_bwd_dq_plane(const void *q, const void *k, const void *v, const float4 *desc_w, const uint32_t *desc_e, const void *out,
                         const float *lse, const void *dout, void *dq, float2 *stats, const float4 *desc_g,
-                        float *dcoords, float2 *handed, const Dims &dm, int bh0, int nbh, hipStream_t st)
+                        float *dcoords, float2 *handed, const GradDims &dm, int bh0, int nbh, hipStream_t st)
 {
     constexpr int DC = Chunk<S, D>::value, WDC = WideChunk<S, D>::value;
     // (two row blocks and the wide form only without the coordinate gradient, two blocks up to 8 elements per lane: registers)
@@ -697,7 +746,7 @@ static inline int make_cell_grid(const Dims &dm, int ncells, int bh0, long long 
 template <typename S, int D>
 int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const float2 *stats, const void *dout, const unsigned *start, const unsigned *sorted,
                          const uint4 *items, unsigned wmax, const float2 *handed,
-                         float *dk_acc, float *dv_acc, const Dims &dm, int NC, int bh0, int nbh, hipStream_t st)
+                         float *dk_acc, float *dv_acc, const GradDims &dm, int NC, int bh0, int nbh, hipStream_t st)
 {
     constexpr int DC = CellChunk<S, D>::value;
     CellGrid cg;
@@ -715,7 +764,7 @@ int launch_bwd_dkdv_cell(const void *q, const void *k, const void *v, const floa
 template <typename S, int D>
 int launch_bwd_dkdv_fixed(const void *q, const void *k, const void *v, const float2 *stats, const void *dout, const unsigned *start,
                           const unsigned *sorted, const float2 *handed, float *taps, int tap_planes, void *dk, void *dv,
-                          const Dims &dm, int NC, int bh0, int nbh, hipStream_t st)
+                          const GradDims &dm, int NC, int bh0, int nbh, hipStream_t st)
 {
     constexpr int DC = CellChunk<S, D>::value;
     const long long all = (long long)nbh * dm.V;
@@ -743,7 +792,7 @@ template <typename S, int D>
 int launch_bwd_dkdv_patch(const void *q, const void *k, const void *v, const void *dout, const unsigned *start,
                           const unsigned *sorted, const uint4 *items, unsigned wmax,
                           const unsigned *left, const float2 *handed, void *dk, void *dv, float *dk_acc, float *dv_acc,
-                          const Dims &dm, int NC, int bh0, int nbh, hipStream_t st)
+                          const GradDims &dm, int NC, int bh0, int nbh, hipStream_t st)
 {
     constexpr int DP = D < 128 ? D : 128;
     PatchGrid pg;
@@ -824,15 +873,18 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
 {
     if (!q || !k || !v || !coords || !out || !lse || !dout || !dq || !dk || !dv || !workspace)
         return DSDPA_ERR_NULL_POINTER;
-    if (flags & ~(unsigned)(DSDPA_FLAG_DETERMINISTIC | DSDPA_FLAG_COORDS_GRAD | DSDPA_FLAG_SINGLE_STREAM)) return DSDPA_ERR_UNSUPPORTED;
+    if (flags & ~(unsigned)(DSDPA_FLAG_DETERMINISTIC | DSDPA_FLAG_COORDS_GRAD | DSDPA_FLAG_SINGLE_STREAM | DSDPA_FLAG_GRADS_AS_INPUTS))
+        return DSDPA_ERR_UNSUPPORTED;
     const bool deterministic = (flags & DSDPA_FLAG_DETERMINISTIC) != 0;
     if (deterministic && dcoords) return DSDPA_ERR_UNSUPPORTED;   // dcoords sums over heads with float atomics
-    Dims dm;
+    GradDims dm;
     int rc = make_dims(B, V, H, Himg, Wimg, D, P, sm_scale, &dm);
     if (rc != DSDPA_OK) return rc;
     if ((long long)dm.L * dm.N > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;   // sample ids are 32-bit
     bool contiguous;
     if ((rc = apply_strides(strides, D, S::kBytes, &dm, &contiguous)) != DSDPA_OK) return rc;
+    const bool as_inputs = !contiguous && (flags & DSDPA_FLAG_GRADS_AS_INPUTS) != 0;
+    if ((rc = apply_grad_strides(D, as_inputs, &dm)) != DSDPA_OK) return rc;
     hipStream_t st = (hipStream_t)stream;
     const size_t n = (size_t)dm.rows * D;
     // the staged dq kernel computes dcoords only when the caller sized the workspace for it (same flags)
@@ -963,19 +1015,25 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     }
 #undef DSDPA_BWD_CASE
     if (rc != DSDPA_OK) return rc;
+    GradPlace gp;
+    gp.plain = !as_inputs;
+    gp.div_per8 = FastDiv::make((unsigned)D / 8);
+    gp.div_v = FastDiv::make((unsigned)V);
+    gp.div_h = FastDiv::make((unsigned)H);
     if (S::kBytes != 4 && left) {
         const size_t n8 = (size_t)dm.L * D / 8;                     // of a plane
         size_t blocks = (n8 * B * V * H + 255) / 256;
         if (blocks > 256 * 8) blocks = 256 * 8;
-        hipLaunchKernelGGL((cast_rest_kernel<S>), dim3((unsigned)blocks), dim3(256), 0, st, left, dk_acc, dv_acc, dk, dv, dm, n8);
+        hipLaunchKernelGGL((cast_rest_kernel<S>), dim3((unsigned)blocks), dim3(256), 0, st, left, dk_acc, dv_acc, dk, dv, dm, n8, gp,
+                           (unsigned)D / 8);
         rc = check_launch();
     } else if (S::kBytes != 4 && !patch && !deterministic) {
         const size_t n8 = n / 8;
         const int threads = 256;
         size_t blocks = (n8 + threads - 1) / threads;
         if (blocks > 256 * 16) blocks = 256 * 16;
-        hipLaunchKernelGGL((cast_kernel<S>), dim3((unsigned)blocks), dim3(threads), 0, st, dk_acc, dk, n8);
-        hipLaunchKernelGGL((cast_kernel<S>), dim3((unsigned)blocks), dim3(threads), 0, st, dv_acc, dv, n8);
+        hipLaunchKernelGGL((cast_kernel<S>), dim3((unsigned)blocks), dim3(threads), 0, st, dk_acc, dk, n8, dm, gp, (unsigned)D / 8);
+        hipLaunchKernelGGL((cast_kernel<S>), dim3((unsigned)blocks), dim3(threads), 0, st, dv_acc, dv, n8, dm, gp, (unsigned)D / 8);
         rc = check_launch();
     }
     return rc;

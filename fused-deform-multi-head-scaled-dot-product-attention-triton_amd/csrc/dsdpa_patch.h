@@ -87,7 +87,7 @@ template <typename S, int D, int DP>
 __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 : 4) void bwd_dkdv_patch_kernel(
     const void *__restrict__ q_, const void *__restrict__ dout_, const unsigned *__restrict__ start,
     const unsigned *__restrict__ sorted, const unsigned *__restrict__ left, const float2 *__restrict__ handed_,
-    void *__restrict__ dk_, void *__restrict__ dv_, float *__restrict__ dk_acc, float *__restrict__ dv_acc, Dims dm, int NC,
+    void *__restrict__ dk_, void *__restrict__ dv_, float *__restrict__ dk_acc, float *__restrict__ dv_acc, GradDims dm, int NC,
     PatchGrid pg)
 {
     constexpr bool k16 = S::kBytes == 2, kBf16 = S::kBf16, kF16 = k16 && !kBf16;
@@ -127,17 +127,24 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
     const char *handed_bh = (const char *)(handed_ + (size_t)bhl * dm.V * dm.L * (size_t)dm.N);
     const unsigned view_rows = (unsigned)dm.H * (unsigned)dm.L;
 
-    const size_t plane_base = (grp * dm.H + h) * (size_t)dm.L * D;
+    const size_t plane_base = dm.dkv_plane(b, s2, h);
     constexpr int VE = k16 ? 8 : 4;                               // elements of a 16-byte store
-    auto pixel_at = [&](int m, size_t &elem) -> bool {
+    auto pixel_of = [&](int m, unsigned &pix) -> bool {
         const int y = kPatchSide * py + (m >> 2), x = kPatchSide * px + (m & 3);
-        elem = plane_base + (size_t)(y * dm.Wimg + x) * D + col0;
+        pix = (unsigned)(y * dm.Wimg + x);
         return y < dm.Himg && x < dm.Wimg;
+    };
+    auto pixel_at = [&](int m, size_t &elem) -> bool {
+        unsigned pix;
+        const bool in = pixel_of(m, pix);
+        elem = plane_base + pix * (unsigned)dm.dkv_sl + col0;
+        return in;
     };
     if (left && items_left(left[grp], mostly_long(left, dm.B * dm.V)) != 0u) {
         for (int i = threadIdx.x; i < kPatchPixels * DP / 4; i += (int)blockDim.x) {
-            size_t elem;
-            if (pixel_at(i * 4 / DP, elem)) {
+            unsigned pix;
+            if (pixel_of(i * 4 / DP, pix)) {
+                const size_t elem = dm.acc_plane<S, D>(b, s2, h) + pix * dm.acc_pixel<S, D>() + col0;
                 *reinterpret_cast<float4 *>(dk_acc + elem + i * 4 % DP) = make_float4(0.f, 0.f, 0.f, 0.f);
                 *reinterpret_cast<float4 *>(dv_acc + elem + i * 4 % DP) = make_float4(0.f, 0.f, 0.f, 0.f);
             }

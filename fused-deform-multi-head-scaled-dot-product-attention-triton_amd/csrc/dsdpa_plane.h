@@ -492,7 +492,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
     const float4 *__restrict__ desc_w, const uint32_t *__restrict__ desc_e, const void *__restrict__ out_,
     const float *__restrict__ lse_, const void *__restrict__ dout_, void *__restrict__ dq_,
     float2 *__restrict__ stats_, const float4 *__restrict__ desc_g, float *__restrict__ dcoords_,
-    float2 *__restrict__ handed_, int bh0, Dims dm)
+    float2 *__restrict__ handed_, int bh0, GradDims dm)
 {
     constexpr int G = D / DC, NS = kWave / G;
     constexpr int kRow = D * S::kBytes;
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
     // per row block: this slot's row and its state
     bool have_s[ROWS];
     unsigned qc_s[ROWS];
-    size_t crow_s[ROWS], roff_s[ROWS], hrow_s[ROWS];               // (kTight: made from qc_s where they are used)
+    size_t crow_s[ROWS], hrow_s[ROWS];                             // (kTight: made from qc_s where they are used)
     float qf_s[ROWS][DC], dof_s[ROWS][DC], dqa_s[ROWS][DC], delta_s[ROWS], lse_s[ROWS];
     uint32_t dop_s[ROWS][kPacked ? DC / 2 : 1];
 #pragma unroll
@@ -539,7 +539,6 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         const size_t roff = row * (size_t)kRow;
         crow_s[rb] = (((size_t)pb.b * dm.V + s1) * dm.L + l) * (size_t)dm.N;
         hrow_s[rb] = ((size_t)(pb.b * dm.H + pb.h - bh0) * nq + qc) * (size_t)dm.N;
-        roff_s[rb] = roff;
         float of[DC];
         Lane::load((const char *)q_ + dm.q_row(pb.b, (int)s1, pb.h, (int)l) * S::kBytes, lane_byte, qf_s[rb]);
         Lane::load((const char *)dout_ + roff, lane_byte, dof_s[rb]);
@@ -715,12 +714,14 @@ __global__ __launch_bounds__(kPlaneWaves *kWave) void bwd_dq_slot_kernel(
         if (have_s[rb]) {
 #pragma unroll
             for (int d = 0; d < DC; ++d) dqa_s[rb][d] *= dm.sm_scale;
-            size_t roff = roff_s[rb];
-            if constexpr (kTight) {
-                const unsigned s1 = dm.divL.div(qc_s[rb]), l = qc_s[rb] - s1 * (unsigned)dm.L;
-                roff = ((((size_t)pb.b * dm.V + s1) * dm.H + pb.h) * dm.L + l) * (size_t)kRow;
+            unsigned qc = qc_s[rb];
+            if constexpr (CG && !HAND) {                     // (made anew from the slot: not kept in registers through the views)
+                int slot_here = slot;
+                asm volatile("" : "+v"(slot_here));
+                qc = (unsigned)(pb.qbase + rb * rows_block + wave * NS + slot_here);
             }
-            Lane::store((char *)dq_ + roff, lane_byte, dqa_s[rb]);
+            const unsigned s1 = dm.divL.div(qc), l = qc - s1 * (unsigned)dm.L;
+            Lane::store((char *)dq_ + (dm.dq_bh(pb.b, pb.h) + dm.dq_at(s1, l)) * S::kBytes, lane_byte, dqa_s[rb]);
         }
     }
 }

@@ -178,7 +178,7 @@ template <typename S, int D, int DC, bool CG>
 __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
     const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_, const float *__restrict__ coords_,
     const void *__restrict__ out_, const float *__restrict__ lse_, const void *__restrict__ dout_, void *__restrict__ dq_,
-    float2 *__restrict__ stats_, float *__restrict__ dcoords_, float2 *__restrict__ handed_, Dims dm, RowGrid rg)
+    float2 *__restrict__ stats_, float *__restrict__ dcoords_, float2 *__restrict__ handed_, GradDims dm, RowGrid rg)
 {
     constexpr int G = D / DC, NS = kWave / G;
     constexpr bool kPacked = S::kBytes == 2 && !CG;
@@ -302,9 +302,13 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
         }
     }
     if (rs.have) {
+        // (decoded anew: the row's place in dq is not kept in registers through the loop)
+        int slot_here = slot;
+        asm volatile("" : "+v"(slot_here));
+        const RowSlot re = decode_row_slot<NS>(dm, rg, wave, slot_here);
 #pragma unroll
         for (int d = 0; d < DC; ++d) dqa[d] *= dm.sm_scale;
-        store_chunk<S, DC>((char *)dq_ + roff, dqa);
+        store_chunk<S, DC>((char *)dq_ + (dm.dq_bh((int)re.b, (int)re.h) + dm.dq_at(re.s1, re.l) + lane_elem) * S::kBytes, dqa);
     }
 }
 

@@ -388,7 +388,7 @@ __global__ __launch_bounds__(NW *kWave) void bwd_dq_slab_kernel(
     const float *__restrict__ q_, const float *__restrict__ k_, const float *__restrict__ v_,
     const float *__restrict__ coords_, const float *__restrict__ out_, const float *__restrict__ lse_,
     const float *__restrict__ dout_, float *__restrict__ dq_, float2 *__restrict__ stats_,
-    float2 *__restrict__ handed_, float *__restrict__ dcoords_, Dims dm, int bh0, int nblk, int pitch, unsigned buf_bytes)
+    float2 *__restrict__ handed_, float *__restrict__ dcoords_, GradDims dm, int bh0, int nblk, int pitch, unsigned buf_bytes)
 {
     constexpr int NSLAB = D / kSlabCols;
     constexpr int NR = IT / KB, RW = 4 * NR, RB = NW * RW;       // query rows per lane, wave, workgroup (see the forward)
@@ -590,9 +590,10 @@ __global__ __launch_bounds__(NW *kWave) void bwd_dq_slab_kernel(
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
         if (!live[r]) continue;
-        const size_t row = row_of(rb * RB + wave * RW + 4 * r + rg);
+        const int rr = rb * RB + wave * RW + 4 * r + rg, s1 = rr / dm.L;
+        float *dst = dq_ + dm.dq_bh(b, h) + dm.dq_at((unsigned)s1, (unsigned)(rr - s1 * dm.L)) + col;
 #pragma unroll
-        for (int s = 0; s < NSLAB; ++s) dq_[row * D + s * kSlabCols + col] = acc[r][s] * dm.sm_scale;
+        for (int s = 0; s < NSLAB; ++s) dst[s * kSlabCols] = acc[r][s] * dm.sm_scale;
     }
 }
 

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(kTileWaves *kWave) void bwd_dkdv_tile_kernel(
     const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_,
     const float *__restrict__ coords_, const float2 *__restrict__ stats_,
     const void *__restrict__ dout_, float *__restrict__ dk_acc, float *__restrict__ dv_acc,
-    Dims dm, TileGeom tg)
+    GradDims dm, TileGeom tg)
 {
     constexpr int G = D / DC;
     constexpr int NS = kWave / G;
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kTileWaves *kWave) void bwd_dkdv_tile_kernel(
     for (int i = threadIdx.x; i < 2 * tile_elems; i += blockDim.x) tileK[i] = 0.0;
     __syncthreads();
 
-    const size_t plane_base = (((size_t)b * dm.V + s2) * dm.H + h) * (size_t)dm.L * D;   // elements in dk/dv
+    const size_t plane_base = dm.acc_plane<S, D>(b, s2, h);             // elements in dk/dv
     const char *kb = (const char *)k_ + dm.kv_plane(b, s2, h) * S::kBytes;
     const char *vb = (const char *)v_ + dm.kv_plane(b, s2, h) * S::kBytes;
     const int g = lane % G, slot = lane / G, lane_elem = g * DC;
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kTileWaves *kWave) void bwd_dkdv_tile_kernel(
         const int ly = px / tg.lw, lx = px % tg.lw;
         const int y = ya + ly, x = xa + lx;
         if (y < dm.Himg && x < dm.Wimg) {
-            const size_t gi = ((size_t)y * dm.Wimg + x) * D + d;
+            const size_t gi = ((size_t)y * dm.Wimg + x) * dm.acc_pixel<S, D>() + d;
             const float a = (float)tileK[i], c = (float)tileV[i];
             if (a != 0.f) atomicAdd(dkb + gi, a);
             if (c != 0.f) atomicAdd(dvb + gi, c);

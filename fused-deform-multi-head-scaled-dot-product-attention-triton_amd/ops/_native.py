@@ -25,6 +25,7 @@ PATH_AUTO, PATH_GATHER, PATH_LDS = 0, 1, 2
 FLAG_DETERMINISTIC = 1
 FLAG_COORDS_GRAD = 2
 FLAG_SINGLE_STREAM = 4
+FLAG_GRADS_AS_INPUTS = 16
 ERR_HEAD_DIM = 3
 ERR_SCRATCH = 8
 ERR_BAD_STRIDES = 9

@@ -125,7 +125,7 @@ int dsdpa_fwd_noalloc(int dtype, const void *q, const void *k, const void *v, co
  * added up in ascending order of their index, and the sums of every cell's four taps are stored apart and then
  * added pixel by pixel in a fixed order instead of by float atomics. Needs a workspace of another
  * size (pass the same flags to dsdpa_bwd_workspace_bytes) and cannot be combined with dcoords. */
-enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SINGLE_STREAM = 4 };
+enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SINGLE_STREAM = 4, DSDPA_FLAG_GRADS_AS_INPUTS = 16 };
 /* B*V*H*L * V*P from which the backward may use its second stream; below it DSDPA_FLAG_SINGLE_STREAM changes nothing */
 #define DSDPA_TWO_STREAMS_FROM (1ll << 21)
 /* DSDPA_FLAG_SINGLE_STREAM: enqueue every launch of the backward on `stream` itself. By default the dk/dv side
@@ -139,6 +139,10 @@ enum { DSDPA_FLAG_DETERMINISTIC = 1, DSDPA_FLAG_COORDS_GRAD = 2, DSDPA_FLAG_SING
  * table (16 more bytes per coordinate pair where the staged kernels run), so that a backward given dcoords
  * stays on the staged dq kernel. Pass the same flags to dsdpa_bwd_workspace_bytes and to dsdpa_bwd_*;
  * dcoords without the bit is computed by the slower gather dq kernel, the bit without dcoords does nothing. */
+/* DSDPA_FLAG_GRADS_AS_INPUTS: dq has the strides of q, dk and dv those of k and v (`strides`; NULL: all contiguous, the
+ * bit does nothing) instead of being contiguous, so that the gradients of permuted inputs need no copy on their way back
+ * through the permutation. The strides have to place B*V*H*L rows of D elements without holes or overlaps
+ * (DSDPA_ERR_BAD_STRIDES otherwise). Does not change the workspace. */
 
 /*
  * Backward: replaces everything `_fused_deform_sdpa.backward` enqueues,
