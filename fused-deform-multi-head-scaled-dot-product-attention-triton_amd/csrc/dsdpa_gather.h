@@ -787,16 +787,19 @@ __global__ __launch_bounds__(kGatherWaves *kWave, (WIN && !CG && DC <= 8) ? 4 : 
     // 16-bit storage: packed pairs for the dot-product instructions -- in the window mode always, tap by tap only
     // without the coordinate gradient (whose per-tap products take the widened rows)
     constexpr bool kPackedWin = S::kBytes == 2 && WIN;
-    constexpr bool kPacked = S::kBytes == 2 && !CG;
+    // dout, and q, as packed pairs; with the coordinate gradient tap by tap only in bf16, where widening costs an instruction an element (127
+    // registers for 94; 19x54, D = 128 62 us for 65): fp16's halves are widened by the multiply-add that takes them
+    constexpr bool kPackedTaps = S::kBytes == 2 && (!CG || S::kBf16);
+    constexpr bool kPacked = kPackedTaps || (S::kBytes == 2 && WIN), kPackedQ = S::kBytes == 2 && (WIN || (CG && S::kBf16));
     float qf[DC], dof[DC], of[DC];
-    uint32_t dop[(kPacked || kPackedWin) ? DC / 2 : 1], qp[kPackedWin ? DC / 2 : 1];
+    uint32_t dop[kPacked ? DC / 2 : 1], qp[kPackedQ ? DC / 2 : 1];
     const size_t roff = (rc.row * D + lane_elem) * S::kBytes;
     const size_t q_roff = (rc.q_off + lane_elem) * S::kBytes;
     load_chunk<S, DC>((const char *)q_ + q_roff, qf);
     load_chunk<S, DC>((const char *)dout_ + roff, dof);
     load_chunk<S, DC>((const char *)out_ + roff, of);
-    if constexpr (kPacked || kPackedWin) load_packed<S, DC>((const char *)dout_ + roff, dop);
-    if constexpr (kPackedWin) load_packed<S, DC>((const char *)q_ + q_roff, qp);
+    if constexpr (kPacked) load_packed<S, DC>((const char *)dout_ + roff, dop);
+    if constexpr (kPackedQ) load_packed<S, DC>((const char *)q_ + q_roff, qp);
     float delta = 0.f;
 #pragma unroll
     for (int d = 0; d < DC; ++d) delta = fmaf(dof[d], of[d], delta);
@@ -990,26 +993,36 @@ __global__ __launch_bounds__(kGatherWaves *kWave, (WIN && !CG && DC <= 8) ? 4 : 
                 float kk[DC];
                 float dot = 0.f, dp = 0.f;
                 if constexpr (CG) {
-                    float t[4][DC], u[4][DC];
+                    constexpr int RW = DC * S::kBytes / 4;
+                    uint32_t kr[4][RW], vr[4][RW];
                     const unsigned eo[4] = { e.x, e.y, e.z, e.w };
                     const float wt[4] = { w.x, w.y, w.z, w.w };
                     float dk_t[4], dv_t[4];
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        load_chunk<S, DC>(kb + eo[i], t[i]);
-                        load_chunk<S, DC>(vb + eo[i], u[i]);
+                        load_words<RW>(kb + eo[i], kr[i]);
+                        load_words<RW>(vb + eo[i], vr[i]);
                     }
 #pragma unroll
                     for (int d = 0; d < DC; ++d) kk[d] = 0.f;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        dk_t[i] = 0.f;
-                        dv_t[i] = 0.f;
+                        float tk[DC];
+                        widen_words<S, DC>(kr[i], tk);
 #pragma unroll
-                        for (int d = 0; d < DC; ++d) {
-                            dk_t[i] = fmaf(qf[d], t[i][d], dk_t[i]);
-                            dv_t[i] = fmaf(dof[d], u[i][d], dv_t[i]);
-                            kk[d] = fmaf(wt[i], t[i][d], kk[d]);
+                        for (int d = 0; d < DC; ++d) kk[d] = fmaf(wt[i], tk[d], kk[d]);
+                        if constexpr (kPackedTaps) {                       // (products of 16-bit pairs are exact in fp32)
+                            dk_t[i] = packed_dot<S, DC>(qp, kr[i]);
+                            dv_t[i] = packed_dot<S, DC>(dop, vr[i]);
+                        } else {
+                            float tv[DC];
+                            widen_words<S, DC>(vr[i], tv);
+                            dk_t[i] = dv_t[i] = 0.f;
+#pragma unroll
+                            for (int d = 0; d < DC; ++d) {
+                                dk_t[i] = fmaf(qf[d], tk[d], dk_t[i]);
+                                dv_t[i] = fmaf(dof[d], tv[d], dv_t[i]);
+                            }
                         }
                         dot = fmaf(wt[i], dk_t[i], dot);
                         dp = fmaf(wt[i], dv_t[i], dp);

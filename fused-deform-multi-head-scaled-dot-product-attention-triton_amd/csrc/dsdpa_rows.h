@@ -181,7 +181,10 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
     float2 *__restrict__ stats_, float *__restrict__ dcoords_, float2 *__restrict__ handed_, GradDims dm, RowGrid rg)
 {
     constexpr int G = D / DC, NS = kWave / G;
-    constexpr bool kPacked = S::kBytes == 2 && !CG;
+    // dot products of 16-bit pairs as they are stored; with the coordinate gradient in bf16 only, where widening costs an instruction an
+    // element (107 registers for 99): fp16's halves are widened by the multiply-add that takes them, and its forms differ by 5 % either
+    // way (us, pairs / widened: 40x28, 4 views x 8, D = 64 99 / 104, 32x19, 2 x 3 21.8 / 19.9)
+    constexpr bool kPacked = S::kBytes == 2 && (!CG || S::kBf16);
     constexpr int RW = DC * S::kBytes / 4;
     static_assert(G >= 2 && G <= 32 && G * DC == D, "lane split");
     __shared__ float4 s_w[kRowWaves][NS * (G + 1)];
@@ -201,7 +204,7 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
     const size_t row = (((size_t)rs.b * dm.V + rs.s1) * dm.H + rs.h) * dm.L + rs.l;
     const size_t roff = (row * D + lane_elem) * S::kBytes;
     float qf[DC], dof[DC], dqa[DC];
-    uint32_t dop[kPacked ? DC / 2 : 1];
+    uint32_t dop[kPacked ? DC / 2 : 1], qp[kPacked && CG ? DC / 2 : 1];
     float delta = 0.f;
     {
         float of[DC];
@@ -209,6 +212,8 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
         load_chunk<S, DC>((const char *)dout_ + roff, dof);
         load_chunk<S, DC>((const char *)out_ + roff, of);
         if constexpr (kPacked) load_packed<S, DC>((const char *)dout_ + roff, dop);
+        if constexpr (kPacked && CG)
+            load_packed<S, DC>((const char *)q_ + (dm.q_row((int)rs.b, (int)rs.s1, (int)rs.h, (int)rs.l) + lane_elem) * S::kBytes, qp);
 #pragma unroll
         for (int d = 0; d < DC; ++d) { delta = fmaf(dof[d], of[d], delta); dqa[d] = 0.f; }
         delta = group_sum<G>(delta);
@@ -257,12 +262,14 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
 #pragma unroll
                 for (int d = 0; d < DC; ++d) {
                     kk[d] = i == 0 ? wt[0] * tk[d] : fmaf(wt[i], tk[d], kk[d]);
-                    if constexpr (CG) dk_t[i] = fmaf(qf[d], tk[d], dk_t[i]);
+                    if constexpr (CG && !kPacked) dk_t[i] = fmaf(qf[d], tk[d], dk_t[i]);
                 }
+                if constexpr (CG && kPacked) dk_t[i] = packed_dot<S, DC>(qp, kr[i]);
                 if constexpr (CG) dot = fmaf(wt[i], dk_t[i], dot);
                 if constexpr (CG && S::kBf16) __builtin_amdgcn_sched_barrier(0);   // (widening tap by tap: 107 registers for 130, four waves a SIMD)
                 if constexpr (kPacked) {
-                    dp = fmaf(wt[i], packed_dot<S, DC>(dop, vr[i]), dp);
+                    dv_t[i] = packed_dot<S, DC>(dop, vr[i]);
+                    dp = fmaf(wt[i], dv_t[i], dp);
                 } else {
                     float tv[DC];
                     widen_words<S, DC>(vr[i], tv);
