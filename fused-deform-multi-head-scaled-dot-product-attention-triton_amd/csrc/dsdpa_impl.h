@@ -813,7 +813,7 @@ int launch_bwd_dkdv_patch(const void *q, const void *k, const void *v, const voi
     if (int rc = make_cell_grid(dm, (int)wmax, bh0, 0, (long long)nbh * dm.V, &cg)) return rc;
     const unsigned rest = 32u * (unsigned)device_cus();
     ScopedKernelTimer timer(1, st);
-    DSDPA_LAUNCH((bwd_dkdv_patch_kernel<S, D, DP>), dim3((unsigned)blocks, D / DP), dim3(waves * kWave), patch_lds_bytes<S>(waves), st,
+    DSDPA_LAUNCH((bwd_dkdv_patch_kernel<S, D, DP>), dim3((unsigned)blocks, D / DP), dim3(waves * kWave), (patch_lds_bytes<S, DP>(waves)), st,
                  timer.start(), left ? nullptr : timer.stop(), q, dout, start, sorted, left, handed, dk, dv, dk_acc, dv_acc, dm, NC, pg);
     if (!left) return check_launch();
     DSDPA_LAUNCH((bwd_dkdv_cell_rest_kernel<S, D, CellChunk<S, D>::value>), dim3(rest), dim3(kCellWaves * kWave), 0, st, nullptr,

@@ -13,7 +13,7 @@
 // (25/16 visits on average) and that four of a column's sixteen places are used; the matrix unit has that to spare.
 //
 // Per 64 entries: one lane per entry fetches its record and pair, forms the four weights times p and ds and scatters
-// them into the wave's C matrices in LDS ([pixel][entry], the rest of which is zero and is made zero again afterwards);
+// them into the wave's C matrices in LDS ([pixel][entry], all 64 columns or half at a time; the rest is zero and is made zero again);
 // then steps of STEP entries: the lanes read their row of C as the A operand, and the query rows -- requested a step
 // ahead, straight from memory into the layout of the B operand -- are multiplied:
 //   16-bit storage  v_mfma_f32_16x16x32: lane group lane/16 holds eight entries, lane % 16 = column n: E = D/16
@@ -21,8 +21,8 @@
 //                   product t is element E*n + t: no data crosses lanes). The coefficients are split in parts of the storage
 //                   type, one product each: two in fp16 (good to 2^-23 down to a floor, see lower_scale), three in bf16 (two
 //                   are good to 2^-17, which rows that cancel show); two byte permutes make the operand of a pair of rows.
-//                   The third part costs a third of the tables' LDS, 13.7 KB a wave for 9.4. us a step, cells / two parts /
-//                   three, bf16: 18x18, 32 heads, D = 32, 6 views x 6 samples 351 / 274 / 292, 12 x 4 797 / 670 / 701; 20x20,
+//                   The third part costs a third of the tables' LDS. us a step with 64 columns in LDS (kPatchColumns), cells / two
+//                   parts / three, bf16: 18x18, 32 heads, D = 32, 6 views x 6 samples 351 / 274 / 292, 12 x 4 797 / 670 / 701; 20x20,
 //                   4 x 6, D = 64 229 / 182 / 186; 40x28, 4 x 8, coherent, D = 128 581 / 425 / 441.
 //   fp32            v_mfma_f32_16x16x4_f32: one entry per lane group and instruction, everything in fp32.
 // fp16 has 5 bits of exponent: its coefficients are scaled by powers of two (lower_scale).
@@ -44,12 +44,22 @@ namespace dsdpa {
 
 constexpr int kPatchSide = 4, kPatchPixels = kPatchSide * kPatchSide;
 constexpr int kPatchMaxWaves = 4;
-constexpr int kPatchPitch = kWave + 4;             // dwords between two rows of C: 16-byte reads of 16 rows cover all banks
-constexpr int kPatchC = kPatchPixels * kPatchPitch;
-// per wave: C of ds, C of p (bf16: and their third parts), row offsets in q and dout, list bounds, a flag
+// Entries whose columns of C are in LDS at a time: a block of 64, or half of it, where the tables' LDS is what limits the waves on
+// a CU (bf16's three tables with 64 columns leave room for 11, with 32 for 21). dk/dv, us, 64 / 32: bf16 D = 32, 18x18, 6 views x 6
+// samples, 32 heads 117 / 105, 50x50, 4 x 4 171 / 148; bf16 D = 16, 40x28, 4 x 2, 24 heads 73 / 55; fp32 D = 16, same 62 / 52. Elsewhere
+// registers limit them, and the second turn of writing and clearing is not won back: a step, D = 64, 40x28, 4 x 8, bf16 273 / 275, fp16 265 /
+// 269; D = 128, 4 x 4 271 / 276; fp16 D = 32, 18x18, 6 x 6 268 / 269.
+template <typename S, int DP> constexpr int kPatchColumns = DP <= (S::kBf16 ? 32 : S::kBytes == 4 ? 16 : 0) ? kWave / 2 : kWave;
+// dwords between two rows of C: 16-byte reads of 16 rows cover all banks
+template <typename S, int DP> constexpr int kPatchPitch = kPatchColumns<S, DP> + 4;
+// per wave: C of ds, C of p (bf16: and their third parts), over which the sums of DP columns pass at the end; row offsets in q and
+// dout, list bounds, a flag
+template <typename S, int DP> constexpr int kPatchC = kPatchPixels * kPatchPitch<S, DP>;
 template <typename S> constexpr int kPatchTables = S::kBf16 ? 3 : 2;
-template <typename S> constexpr int kPatchWaveDwords = kPatchTables<S> * kPatchC + 2 * kWave + 5 * 8 + 4;
-template <typename S> constexpr size_t patch_lds_bytes(int waves) { return (size_t)waves * kPatchWaveDwords<S> * 4; }
+template <typename S, int DP>
+constexpr int kPatchRoom = kPatchTables<S> * kPatchC<S, DP> > kPatchPixels * DP ? kPatchTables<S> * kPatchC<S, DP> : kPatchPixels * DP;
+template <typename S, int DP> constexpr int kPatchWaveDwords = kPatchRoom<S, DP> + 2 * kWave + 5 * 8 + 4;
+template <typename S, int DP> constexpr size_t patch_lds_bytes(int waves) { return (size_t)waves * kPatchWaveDwords<S, DP> * 4; }
 
 struct PatchGrid {
     int npx, npatch;                        // patches per row and per plane
@@ -84,7 +94,7 @@ __device__ __forceinline__ uint32_t split_pack(float c, float &rest)
 }
 
 template <typename S, int D, int DP>
-__global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 : 4) void bwd_dkdv_patch_kernel(
+__global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : DP > 32 && S::kBf16 ? 3 : 4) void bwd_dkdv_patch_kernel(
     const void *__restrict__ q_, const void *__restrict__ dout_, const unsigned *__restrict__ start,
     const unsigned *__restrict__ sorted, const unsigned *__restrict__ left, const float2 *__restrict__ handed_,
     void *__restrict__ dk_, void *__restrict__ dv_, float *__restrict__ dk_acc, float *__restrict__ dv_acc, GradDims dm, int NC,
@@ -94,15 +104,16 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
     constexpr int E = DP / 16;                        // elements of a row per lane
     constexpr int EPL = k16 ? 8 : 4;                  // entries per lane group and step
     constexpr int STEP = 4 * EPL, NSTEP = kWave / STEP;
+    constexpr int PITCH = kPatchPitch<S, DP>, COLS = kPatchColumns<S, DP>, SPC = COLS / STEP;     // steps of the columns in LDS
     constexpr int PIECE = E * S::kBytes, WORDS = (PIECE + 3) / 4;
     static_assert(DP % 16 == 0 && D % DP == 0 && DP <= 128, "columns of a workgroup");
     extern __shared__ __attribute__((aligned(16))) unsigned smem_patch[];
 
     const int nw = (int)(blockDim.x >> 6);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    unsigned *const base = smem_patch + wave * kPatchWaveDwords<S>;
-    unsigned *const ck = base, *const cv = base + kPatchC, *const cl = base + 2 * kPatchC;       // cl: bf16's third parts, ds | p << 16
-    unsigned *const s_qrow = base + kPatchTables<S> * kPatchC, *const s_row = s_qrow + kWave, *const s_bnd = s_row + kWave;
+    unsigned *const base = smem_patch + wave * kPatchWaveDwords<S, DP>;
+    unsigned *const ck = base, *const cv = base + kPatchC<S, DP>, *const cl = base + 2 * kPatchC<S, DP>;       // cl: bf16's third parts, ds | p << 16
+    unsigned *const s_qrow = base + kPatchRoom<S, DP>, *const s_row = s_qrow + kWave, *const s_bnd = s_row + kWave;
 
     // plane-major: (b, h, s2, patch)
     const unsigned work = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x);
@@ -203,9 +214,11 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
     float scale_ds = kF16 ? kScaleDs : 1.0f, rescale = 1.0f;
     (void)rescale;
 
-    // C of one block of 64 entries, and the entries' row offsets. The places written are kept for the clearing.
+    // The coefficients of a block of 64 entries, a lane each, and the entries' row offsets. They go into C COLS entries at a time, the
+    // `part`-th COLS lanes' at once, and are cleared when they have been read.
     int zat = 0;
     unsigned zmask = 0u;
+    uint32_t zk[4], zv[4], zl[kBf16 ? 4 : 1];
     auto tables = [&](unsigned first, const PatchEntry &e, const Fetched &f) {
         const bool live = first + (unsigned)lane < total;
         const float2 ff = make_float2(e.fx, e.fy);
@@ -220,20 +233,17 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
         }
         const float p = f.pd.x * kByP;
         zmask = live ? rows & cols : 0u;
-        zat = ((r - 1) * kPatchSide + (c - 1)) * kPatchPitch + lane;
+        zat = ((r - 1) * kPatchSide + (c - 1)) * PITCH + (lane & (COLS - 1));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            if (zmask & (1u << i)) {
-                const int at = zat + ((i >> 1) * kPatchSide + (i & 1)) * kPatchPitch;
-                if constexpr (k16) {
-                    float rk, rv;
-                    ck[at] = split_pack<S>(w[i] * ds, rk);
-                    cv[at] = split_pack<S>(w[i] * p, rv);
-                    if constexpr (kBf16) cl[at] = __builtin_bit_cast(uint32_t, dsdpa_bf16x2{(__bf16)rk, (__bf16)rv});
-                } else {
-                    ck[at] = __float_as_uint(w[i] * ds);
-                    cv[at] = __float_as_uint(w[i] * p);
-                }
+            if constexpr (k16) {
+                float rk, rv;
+                zk[i] = split_pack<S>(w[i] * ds, rk);
+                zv[i] = split_pack<S>(w[i] * p, rv);
+                if constexpr (kBf16) zl[i] = __builtin_bit_cast(uint32_t, dsdpa_bf16x2{(__bf16)rk, (__bf16)rv});
+            } else {
+                zk[i] = __float_as_uint(w[i] * ds);
+                zv[i] = __float_as_uint(w[i] * p);
             }
         }
         unsigned qrow, row;
@@ -241,14 +251,15 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
         s_qrow[lane] = qrow;
         s_row[lane] = row;
     };
-    auto clear_tables = [&]() {
+    auto put_tables = [&](int part, bool clear) {
+        const unsigned here = lane / COLS == part ? zmask : 0u;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            if (zmask & (1u << i)) {
-                const int at = zat + ((i >> 1) * kPatchSide + (i & 1)) * kPatchPitch;
-                ck[at] = 0u;
-                cv[at] = 0u;
-                if constexpr (kBf16) cl[at] = 0u;
+            if (here & (1u << i)) {
+                const int at = zat + ((i >> 1) * kPatchSide + (i & 1)) * PITCH;
+                ck[at] = clear ? 0u : zk[i];
+                cv[at] = clear ? 0u : zv[i];
+                if constexpr (kBf16) cl[at] = clear ? 0u : zl[i];
             }
         }
     };
@@ -268,7 +279,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
     struct Coefs { uint4 x[EPL / 4]; };
     auto read_coefs = [&](const unsigned *c, int s) -> Coefs {
         Coefs f;
-        const uint4 *src = reinterpret_cast<const uint4 *>(c + (lane & 15) * kPatchPitch + s * STEP + (lane >> 4) * EPL);
+        const uint4 *src = reinterpret_cast<const uint4 *>(c + (lane & 15) * PITCH + s * STEP % COLS + (lane >> 4) * EPL);
 #pragma unroll
         for (int i = 0; i < EPL / 4; ++i) f.x[i] = src[i];
         return f;
@@ -302,7 +313,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
         }
     };
 
-    for (int i = lane; i < kPatchTables<S> * kPatchC / 4; i += kWave) reinterpret_cast<uint4 *>(base)[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = lane; i < kPatchTables<S> * kPatchC<S, DP> / 4; i += kWave) reinterpret_cast<uint4 *>(base)[i] = make_uint4(0u, 0u, 0u, 0u);
     const unsigned stride = (unsigned)nw * kWave;
     unsigned first = (unsigned)wave * kWave;                      // the waves take the blocks of 64 entries in turn
     if (first < total) {
@@ -316,6 +327,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
             const Fetched f0 = fetch(e0.id);
             f1 = fetch(e1.id);
             tables(first, e0, f0);
+            put_tables(0, false);
         }
         wave_lds_sync();
         issue(q_bh, s_qrow, 0, rq);
@@ -328,10 +340,11 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
 #pragma unroll
             for (int s = 0; s < NSTEP; ++s) {
                 const Coefs fk = read_coefs(ck, s), fv = read_coefs(cv, s), fl = kBf16 ? read_coefs(cl, s) : Coefs{};
-                if (s == NSTEP - 1 && more) {                     // this block's C has been read: the next block's
+                if (s % SPC == SPC - 1 && (s < NSTEP - 1 || more)) {      // C has been read: the next columns
                     wave_lds_sync();
-                    clear_tables();
-                    tables(first + stride, e1, f1);
+                    put_tables(s / SPC, true);
+                    if (s == NSTEP - 1) tables(first + stride, e1, f1);
+                    put_tables((s + 1) % NSTEP / SPC, false);
                     wave_lds_sync();
                 }
                 const int next = (s + 1) % NSTEP;
@@ -365,7 +378,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
     }
 
     // Sum of the waves through LDS, and the stores: the patch as [pixel][column], dk and then dv.
-    unsigned &s_bad = smem_patch[kPatchWaveDwords<S> - 1];
+    unsigned &s_bad = smem_patch[kPatchWaveDwords<S, DP> - 1];
     if (threadIdx.x == 0) s_bad = 0u;
     float z = 0.f;
 #pragma unroll
@@ -394,7 +407,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : S::kBf16 ? 3 :
             for (int d = 0; d < VE; ++d) sum[d] = all[i * VE + d];
             for (int w = 1; w < nw; ++w) {
 #pragma unroll
-                for (int d = 0; d < VE; ++d) sum[d] += all[w * kPatchWaveDwords<S> + i * VE + d];
+                for (int d = 0; d < VE; ++d) sum[d] += all[w * kPatchWaveDwords<S, DP> + i * VE + d];
             }
             size_t elem;
             if (pixel_at(m, elem)) store_chunk<S, VE>((char *)(which == 0 ? dk_ : dv_) + (elem + c) * S::kBytes, sum);

@@ -53,6 +53,15 @@ def test_several_blocks_a_patch(P, dtype):
         assert rel(a, b) < BAR[dtype], name
 
 
+# 16 columns: C in LDS by halves of a block; lists that end in a first half, in a second one and behind one
+@pytest.mark.parametrize("P,dtype", [(3, torch.float32), (7, torch.float32), (3, torch.bfloat16), (20, torch.bfloat16)], ids=str)
+def test_half_blocks(P, dtype):
+    q, k, v, dout, coords = inputs(1, 1, 114, 11, 9, 16, P, dtype, 16)
+    got, want = gradients(q, k, v, coords, dout, 9, 11)
+    for a, b, name in zip(got, want, ("dq", "dk", "dv")):
+        assert rel(a, b) < BAR[dtype], name
+
+
 # 1350 visits a patch: four waves
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
 def test_four_waves_a_patch(dtype):
