@@ -189,6 +189,18 @@ inline bool row_path(size_t rows, size_t V, size_t L, size_t D, size_t P, size_t
     return fill >= (fp32 && D == 256 ? 65 : N <= 32 ? (fp32 && D >= 64 ? 88 : 80) : N <= 64 ? (fp32 ? 95 : 85) : fp32 ? 97 : 93);
 }
 
+// Samples whose taps the row dq kernel has in flight together. Two hold more registers, and in fp32 4 workgroups a CU instead of 6: there the
+// number whose last round of workgroups is the fuller, two where they are even. dq, us, one / two: bf16 48x48, 6 views x 32 samples, D = 64
+// 1889 / 1842; 60x50, 4 x 8, D = 16 160 / 143; 44x44, 6 x 20, D = 64 bf16 896 / 876, fp16 911 / 880, fp32 (11616 workgroups) 1653 /
+// 1600; fp32 40x28, 4 x 8, D = 64 (4480: 2.9 and 4.4 rounds) 172 / 177, 37x23, 3 x 7, D = 128, one batch (1600: 1.04 and 1.6 rounds)
+// 49.7 / 46.8. With the coordinate gradient one: 40x28, 4 x 8, D = 64 bf16 101 / 106, fp16 109 / 120.
+inline int row_step(size_t esize, long long groups)
+{
+    if (esize == 2) return 2;
+    auto full = [&](long long at_once) { return (double)groups / (double)((groups + at_once - 1) / at_once * at_once); };
+    return full(6 * 256) > full(4 * 256) ? 1 : 2;
+}
+
 // Descriptor table of the plane kernels: per coordinate pair 16 bytes of weights and 4 of packed slot
 // codes (plus, for the coordinate gradient, 16 bytes of derivative weights), computed once per call by
 // plane_descriptor_kernel. Empty when the plane kernels do not apply.

@@ -252,7 +252,9 @@ int launch_bwd_dq_rows(const void *q, const void *k, const void *v, const float 
     const RowGrid rg = make_row_grid<kWave * DC / D>(dm, bh0);
     const long long blocks = (long long)nbh * rg.nblk;
     if (blocks > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;
-    auto kern = dcoords ? bwd_dq_rows_kernel<S, D, DC, true> : bwd_dq_rows_kernel<S, D, DC, false>;
+    constexpr int kTwo = DC * S::kBytes <= 16 ? 2 : 1, kOne = S::kBytes == 2 ? kTwo : 1;
+    auto kern = dcoords ? bwd_dq_rows_kernel<S, D, DC, true, 1>
+                : row_step(S::kBytes, blocks) == 2 ? bwd_dq_rows_kernel<S, D, DC, false, kTwo> : bwd_dq_rows_kernel<S, D, DC, false, kOne>;
     ScopedKernelTimer timer(2, st);
     DSDPA_LAUNCH(kern, dim3((unsigned)blocks), dim3(kRowWaves * kWave), 0, st, timer.start(), timer.stop(), q, k, v, coords, out,
                  lse, dout, dq, stats, dcoords, handed, dm, rg);

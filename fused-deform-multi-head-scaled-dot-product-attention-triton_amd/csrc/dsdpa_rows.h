@@ -174,7 +174,9 @@ __global__ __launch_bounds__(kRowWaves *kWave) void fwd_rows_kernel(
 // dq, the rows' (lse, delta) (stats_ may be null), the pairs for the dk/dv kernel (handed_ may be null; see
 // bwd_dq_gather_kernel) and, with CG, the gradient of the coordinates: per-tap dot products instead of blend-then-dot, each
 // lane's part of the two derivatives summed over the slot, and one pair of atomics per pass from the lane that owns the sample.
-template <typename S, int D, int DC, bool CG>
+// STEP samples have their taps in flight together: two (112 registers in fp32, 4 waves a SIMD; 118 to 125 in 16 bits) or one (80, 6 waves;
+// 80 to 92), see row_step.
+template <typename S, int D, int DC, bool CG, int STEP>
 __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
     const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_, const float *__restrict__ coords_,
     const void *__restrict__ out_, const float *__restrict__ lse_, const void *__restrict__ dout_, void *__restrict__ dq_,
@@ -240,18 +242,7 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
         xy = crow[min(n + G, dm.N - 1)];
         wave_lds_sync();
         float my_p = 0.f, my_ds = 0.f, my_gx = 0.f, my_gy = 0.f;
-        for (int t = 0; t < cnt; ++t) {
-            const float4 x = my_w[t];
-            const uint4 o = lane_offsets(my_e[t], lane_byte);
-            uint32_t kr[4][RW], vr[4][RW];
-            load_words<RW>(kb + o.x, kr[0]);
-            load_words<RW>(kb + o.y, kr[1]);
-            load_words<RW>(kb + o.z, kr[2]);
-            load_words<RW>(kb + o.w, kr[3]);
-            load_words<RW>(vb + o.x, vr[0]);
-            load_words<RW>(vb + o.y, vr[1]);
-            load_words<RW>(vb + o.z, vr[2]);
-            load_words<RW>(vb + o.w, vr[3]);
+        auto one = [&](int t, const float4 &x, const uint32_t (&kr)[4][RW], const uint32_t (&vr)[4][RW]) {
             const float wt[4] = { x.x, x.y, x.z, x.w };
             float kk[DC], dot = 0.f, dp = 0.f, dk_t[4], dv_t[4];
 #pragma unroll
@@ -298,7 +289,32 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
                 const float gy = group_sum<G>(fmaf(ay.x, g0, fmaf(ay.y, g1, fmaf(ay.z, g2, ay.w * g3))));
                 if (t == g) { my_gx = gx; my_gy = gy; }
             }
-        }
+        };
+        // the n samples from the t-th on: their taps in flight together
+        auto step = [&](auto n, int t) {
+            constexpr int U = decltype(n)::value;
+            float4 xs[U];
+            uint32_t kr[U][4][RW], vr[U][4][RW];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                xs[u] = my_w[t + u];
+                const uint4 o = lane_offsets(my_e[t + u], lane_byte);
+                load_words<RW>(kb + o.x, kr[u][0]);
+                load_words<RW>(kb + o.y, kr[u][1]);
+                load_words<RW>(kb + o.z, kr[u][2]);
+                load_words<RW>(kb + o.w, kr[u][3]);
+                load_words<RW>(vb + o.x, vr[u][0]);
+                load_words<RW>(vb + o.y, vr[u][1]);
+                load_words<RW>(vb + o.z, vr[u][2]);
+                load_words<RW>(vb + o.w, vr[u][3]);
+            }
+            if constexpr (U > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) one(t + u, xs[u], kr[u], vr[u]);
+        };
+        int t = 0;
+        for (; t + STEP <= cnt; t += STEP) step(std::integral_constant<int, STEP>{}, t);
+        if (STEP > 1 && t < cnt) step(std::integral_constant<int, 1>{}, t);
         if (rs.have && n < dm.N) {
             if (handed_row) handed_row[n] = make_float2(my_p, my_ds * dm.sm_scale);
             if constexpr (CG) {
