@@ -267,13 +267,13 @@ __device__ __forceinline__ bool mostly_long(const unsigned *__restrict__ left, i
 __device__ __forceinline__ unsigned items_left(unsigned l, bool all) { return all || (l & kSpreadLong) ? l & ~kSpreadLong : 0u; }
 template <int THREADS>
 __device__ __forceinline__ void scan_end(const ScanCarry &carry, int NC, unsigned wmax, unsigned *__restrict__ st, uint4 *__restrict__ it,
-                                         const Spread &spread, unsigned longest)
+                                         const Spread &spread, unsigned grp, unsigned longest)
 {
     if (spread.items) {
         const int any_long = __syncthreads_or(longest > (carry.pieces < spread.few ? spread.mean : kSpreadLongest));
         if (threadIdx.x == 0) {
             const bool is_long = any_long || (unsigned long long)carry.entries > (unsigned long long)spread.mean * carry.pieces;
-            spread.items[blockIdx.x] = min(carry.pieces, wmax) | (is_long ? kSpreadLong : 0u);
+            spread.items[grp] = min(carry.pieces, wmax) | (is_long ? kSpreadLong : 0u);
         }
     }
     if (threadIdx.x == 0) st[NC] = carry.entries;
@@ -306,11 +306,11 @@ __global__ __launch_bounds__(THREADS, THREADS == 512 ? 8 : 4) void bin_scan_kern
             at += v[i];
         }
     }
-    scan_end<THREADS>(carry, NC, wmax, st, it, spread, longest);
+    scan_end<THREADS>(carry, NC, wmax, st, it, spread, blockIdx.x, longest);
 }
 
-// Count, scan and fill in one launch, for lists short enough that one workgroup holds all samples of a (b, s2) in
-// its registers, PER of them a thread: every sample's rank in its list comes from the counting atomic itself, so
+// Count, scan and fill by one workgroup, for lists short enough that one workgroup holds all samples of a (b, s2) in
+// its registers, kBinOneSamples / THREADS of them a thread: every sample's rank in its list comes from the counting atomic itself, so
 // the coordinates are read once and there is one round of LDS atomics, no counters in memory (nothing to clear)
 // and no wait between launches. Bound by that chain of latencies (a few workgroups on the whole chip), as the three
 // launches are: 1296 samples a list group (18x18, 2 views x 2 samples) 6.2 us against 13.7 for the three and the gaps
@@ -321,50 +321,55 @@ __global__ __launch_bounds__(THREADS, THREADS == 512 ? 8 : 4) void bin_scan_kern
 constexpr int kBinOneKeys = 2 * kBinOneSamples + 2, kBinOneKeyBits = 13;
 static_assert(kBinOneKeys < (1 << kBinOneKeyBits), "a key fits below its rank");
 static_assert(2ull * kBinOneSamples * 256 * 4 <= kGroupRowsBytes, "one group of query views");
-template <int PER>
-__global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__ coords_, Dims dm, int NC,
-                                                       unsigned *__restrict__ start, unsigned piece, unsigned wmax,
-                                                       uint4 *__restrict__ items, unsigned *__restrict__ sorted, int records,
-                                                       Spread spread)
+// What it makes of coords: lists (starts, entries, as ids or `records`), work list, and the counts for the patch kernel (see above).
+// `groups` of them; 0: nothing to do.
+struct BinJob { unsigned groups; int NC; unsigned piece, wmax; unsigned *start; uint4 *items; unsigned *sorted; int records; Spread spread; };
+// One (b, s2) = grp, by a workgroup of THREADS threads. s_hist: NC words of LDS.
+template <int THREADS>
+__device__ __forceinline__ void bin_one_group(const float *__restrict__ coords_, const Dims &dm, const BinJob &bj, unsigned grp, unsigned *s_hist)
 {
-    __shared__ unsigned s_hist[kBinOneKeys];                       // list lengths, then starts
-    __shared__ uint2 s_wave[16];
-    const int s2 = blockIdx.x % dm.V, b = blockIdx.x / dm.V;       // blockIdx.x = (b, s2), as the scan's
+    constexpr int PER = kBinOneSamples / THREADS;
+    __shared__ uint2 s_wave[THREADS / kWave];
+    const int NC = bj.NC;
+    const unsigned s2 = grp % (unsigned)dm.V, b = grp / (unsigned)dm.V;
     const unsigned M = (unsigned)dm.V * (unsigned)dm.L * (unsigned)dm.P;
     const float2 *crd = reinterpret_cast<const float2 *>(coords_) + ((size_t)b * dm.V * dm.L * dm.V + s2) * (size_t)dm.P;
+    unsigned tid = threadIdx.x;
+    auto fetch = [&](int i) {
+        const unsigned id = min((unsigned)(i * THREADS) + tid, M - 1u);                // id = ql * P + p
+        const unsigned ql = dm.divP.div(id), p = id - ql * (unsigned)dm.P;
+        return crd[(size_t)ql * dm.N + p];
+    };
     float2 xy[PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const unsigned id = min((unsigned)i * 1024u + threadIdx.x, M - 1u);            // id = ql * P + p
-        const unsigned ql = dm.divP.div(id), p = id - ql * (unsigned)dm.P;
-        xy[i] = crd[(size_t)ql * dm.N + p];
-    }
-    for (int i = threadIdx.x; i < NC; i += 1024) s_hist[i] = 0u;
+    for (int i = 0; i < PER; ++i) xy[i] = fetch(i);
+    for (int i = threadIdx.x; i < NC; i += THREADS) s_hist[i] = 0u;
     __syncthreads();
     unsigned key_rank[PER];                                        // key, rank above; all ones: in no list
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        const unsigned id = (unsigned)i * 1024u + threadIdx.x;
+        const unsigned id = (unsigned)(i * THREADS) + threadIdx.x;
         const Taps tp = make_taps(xy[i].x, xy[i].y, dm.Wimg, dm.Himg);
         key_rank[i] = 0xffffffffu;
         if (id < M && taps_any(tp)) {
             const unsigned key = (unsigned)cell_of(tp, dm.Wimg);
             key_rank[i] = key | (atomicAdd(&s_hist[key], 1u) << kBinOneKeyBits);
         }
+        if (PER > 2) __builtin_amdgcn_sched_barrier(0);            // (one after the other: registers)
     }
     __syncthreads();
     ScanCarry carry{0u, 0u};
     unsigned longest = 0u;
-    unsigned *st = start + (size_t)blockIdx.x * (NC + 1);
-    uint4 *it = items + (size_t)blockIdx.x * wmax;
-    for (int base = 0; base < NC; base += 1024 * kScanKeys) {
+    unsigned *st = bj.start + (size_t)grp * (NC + 1);
+    uint4 *it = bj.items + (size_t)grp * bj.wmax;
+    for (int base = 0; base < NC; base += THREADS * kScanKeys) {
         const int c0 = base + (int)threadIdx.x * kScanKeys;
         unsigned v[kScanKeys], at;
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) v[i] = c0 + i < NC ? s_hist[c0 + i] : 0u;
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) longest = max(longest, v[i]);
-        scan_keys<1024>(v, c0, NC, NC, piece, wmax, st, it, s_wave, carry, at);
+        scan_keys<THREADS>(v, c0, NC, NC, bj.piece, bj.wmax, st, it, s_wave, carry, at);
 #pragma unroll
         for (int i = 0; i < kScanKeys; ++i) {
             if (c0 + i < NC) s_hist[c0 + i] = at;                  // (this thread's own keys)
@@ -372,13 +377,28 @@ __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__
         }
     }
     __syncthreads();
+    if constexpr (PER > 2) asm volatile("" : "+v"(tid)::"memory");       // (coordinates and ids made anew: not held through the scan)
+    constexpr int AT_ONCE = PER > 2 ? PER / 2 : PER;
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        if (key_rank[i] != 0xffffffffu)
-            store_cell_entry(sorted, (size_t)blockIdx.x * M + s_hist[key_rank[i] & ((1u << kBinOneKeyBits) - 1u)] + (key_rank[i] >> kBinOneKeyBits),
-                             (unsigned)i * 1024u + threadIdx.x, cell_fraction(xy[i], dm), records);
+    for (int i0 = 0; i0 < PER; i0 += AT_ONCE) {
+#pragma unroll
+        for (int i = i0; PER > 2 && i < i0 + AT_ONCE; ++i) xy[i] = fetch(i);
+#pragma unroll
+        for (int i = i0; i < i0 + AT_ONCE; ++i) {
+            if (key_rank[i] != 0xffffffffu)
+                store_cell_entry(bj.sorted, (size_t)grp * M + s_hist[key_rank[i] & ((1u << kBinOneKeyBits) - 1u)] + (key_rank[i] >> kBinOneKeyBits),
+                                 (unsigned)(i * THREADS) + tid, cell_fraction(xy[i], dm), bj.records);
+        }
+        if (PER > 2) __builtin_amdgcn_sched_barrier(0);
     }
-    scan_end<1024>(carry, NC, wmax, st, it, spread, longest);
+    scan_end<THREADS>(carry, NC, bj.wmax, st, it, bj.spread, grp, longest);
+}
+
+// In a launch of its own: before the dq kernels that take no BinJob (the row kernel does), and before the sort of the deterministic backward.
+static __global__ __launch_bounds__(1024) void bin_one_kernel(const float *__restrict__ coords_, Dims dm, BinJob bj)
+{
+    __shared__ unsigned s_hist[kBinOneKeys];                       // list lengths, then starts
+    bin_one_group<1024>(coords_, dm, bj, blockIdx.x, s_hist);
 }
 
 // Deterministic backward: begin / end of every cell list as positions in the flat id array

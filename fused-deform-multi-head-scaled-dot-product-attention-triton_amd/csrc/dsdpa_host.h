@@ -201,6 +201,9 @@ inline int row_step(size_t esize, long long groups)
     return full(6 * 256) > full(4 * 256) ? 1 : 2;
 }
 
+// Whether the row dq kernel has a form that bins beside its rows: all but the one of 1 KB rows with the coordinate gradient, which would spill.
+constexpr bool row_takes_bins(size_t D, size_t esize, bool coords_grad) { return !(coords_grad && D * esize >= 1024); }
+
 // Descriptor table of the plane kernels: per coordinate pair 16 bytes of weights and 4 of packed slot
 // codes (plus, for the coordinate gradient, 16 bytes of derivative weights), computed once per call by
 // plane_descriptor_kernel. Empty when the plane kernels do not apply.

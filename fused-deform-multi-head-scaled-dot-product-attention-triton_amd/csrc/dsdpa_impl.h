@@ -245,19 +245,24 @@ int launch_fwd_rows(const void *q, const void *k, const void *v, const float *co
 }
 template <typename S, int D>
 int launch_bwd_dq_rows(const void *q, const void *k, const void *v, const float *coords, const void *out, const float *lse,
-                       const void *dout, void *dq, float2 *stats, float *dcoords, float2 *handed, const GradDims &dm, int bh0, int nbh,
-                       hipStream_t st)
+                       const void *dout, void *dq, float2 *stats, float *dcoords, float2 *handed, const BinJob &bj, const GradDims &dm,
+                       int bh0, int nbh, hipStream_t st)
 {
     constexpr int DC = RowChunk<S, D>::value;
     const RowGrid rg = make_row_grid<kWave * DC / D>(dm, bh0);
     const long long blocks = (long long)nbh * rg.nblk;
-    if (blocks > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;
+    if (blocks > 0x7fffffffll - 65536) return DSDPA_ERR_TOO_LARGE;
     constexpr int kTwo = DC * S::kBytes <= 16 ? 2 : 1, kOne = S::kBytes == 2 ? kTwo : 1;
-    auto kern = dcoords ? bwd_dq_rows_kernel<S, D, DC, true, 1>
-                : row_step(S::kBytes, blocks) == 2 ? bwd_dq_rows_kernel<S, D, DC, false, kTwo> : bwd_dq_rows_kernel<S, D, DC, false, kOne>;
+    auto pick = [&](auto bin) {
+        constexpr bool BIN = decltype(bin)::value;
+        return dcoords ? bwd_dq_rows_kernel<S, D, DC, true, 1, BIN && row_takes_bins(D, S::kBytes, true)>
+               : row_step(S::kBytes, blocks) == 2 ? bwd_dq_rows_kernel<S, D, DC, false, kTwo, BIN> : bwd_dq_rows_kernel<S, D, DC, false, kOne, BIN>;
+    };
+    auto kern = bj.groups ? pick(std::true_type{}) : pick(std::false_type{});
+    const unsigned bins = bin_blocks(bj.groups);
     ScopedKernelTimer timer(2, st);
-    DSDPA_LAUNCH(kern, dim3((unsigned)blocks), dim3(kRowWaves * kWave), 0, st, timer.start(), timer.stop(), q, k, v, coords, out,
-                 lse, dout, dq, stats, dcoords, handed, dm, rg);
+    DSDPA_LAUNCH(kern, dim3((unsigned)blocks + bins), dim3(kRowWaves * kWave), bins ? bj.NC * sizeof(unsigned) : 0, st, timer.start(),
+                 timer.stop(), q, k, v, coords, out, lse, dout, dq, stats, dcoords, handed, dm, rg, bj);
     return check_launch();
 }
 
@@ -667,6 +672,12 @@ static inline bool bin_in_one_launch(const Dims &dm)
     return (long long)dm.V * dm.L * dm.P <= kBinOneSamples;
 }
 
+static inline BinJob bin_job(const Dims &dm, const WorkspaceLayout &wl, char *ws, int records, const Spread &spread)
+{
+    return BinJob{(unsigned)(dm.B * dm.V), wl.NC, wl.piece, wl.wmax, (unsigned *)(ws + wl.start), (uint4 *)(ws + wl.items),
+                  (unsigned *)(ws + wl.sorted), records, spread};
+}
+
 // spread: flags to set for the patch kernel, or none. beside_dq: the staged dq kernel runs at the same time and dk/dv is next, so
 // take workgroups that fit beside its waves.
 // records: the lists as 12-byte records (id and position in the cell) from wl.sorted on, through the room of
@@ -679,9 +690,8 @@ static inline int launch_binning(const float *coords, const Dims &dm, const Work
     unsigned *sorted = (unsigned *)(ws + wl.sorted);
     if (bin_in_one_launch(dm)) {
         ScopedKernelTimer timer(3, st);
-        auto kern = bin_one_kernel<kBinOneSamples / 1024>;
-        DSDPA_LAUNCH(kern, dim3((unsigned)(dm.B * dm.V)), dim3(1024), 0, st, timer.start(), timer.stop(),
-                     coords, dm, wl.NC, start, wl.piece, wl.wmax, (uint4 *)(ws + wl.items), sorted, records, spread);
+        DSDPA_LAUNCH(bin_one_kernel, dim3((unsigned)(dm.B * dm.V)), dim3(1024), 0, st, timer.start(), timer.stop(), coords, dm,
+                     bin_job(dm, wl, ws, records, spread));
         return check_launch();
     }
     const long long total = (long long)dm.B * dm.V * dm.L * dm.N;
@@ -961,8 +971,17 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
                            stats, (size_t)dm.rows, D);
         if ((rc = check_launch()) != DSDPA_OK) return rc;
     }
-    if (cell_binned && (rc = launch_binning(coords, dm, wl, ws, deterministic ? 0 : 1, Spread{left, wl.spread_mean, wl.spread_few},
-                                              side_on && !deterministic, bst)) != DSDPA_OK)
+    const bool slab = path == DSDPA_PATH_AUTO && !staged && slab_path_fits(V, Himg, Wimg, D, P, S::kBytes);
+    const bool rows = path == DSDPA_PATH_AUTO && !staged && !slab &&
+                      ((plane_path_fits(dm.L, D, S::kBytes) && few_samples_prefer_rows(V, P, S::kBytes)) ||
+                       row_path((size_t)dm.rows, V, dm.L, D, P, S::kBytes, true));
+    // (the deterministic backward orders the lists before dq)
+    const Spread spread{left, wl.spread_mean, wl.spread_few};
+    const bool bin_in_dq = cell_binned && rows && !deterministic && bin_in_one_launch(dm) && dm.B * dm.V <= 32768 &&
+                           row_takes_bins(D, S::kBytes, dcoords != nullptr);
+    const BinJob bins = bin_in_dq ? bin_job(dm, wl, ws, 1, spread) : BinJob{};
+    if (cell_binned && !bin_in_dq &&
+        (rc = launch_binning(coords, dm, wl, ws, deterministic ? 0 : 1, spread, side_on && !deterministic, bst)) != DSDPA_OK)
         return rc;
     if (deterministic && (rc = launch_list_ordering(coords, dm, wl, ws, bst)) != DSDPA_OK) return rc;
     float2 *dq_stats = side_on || patch ? nullptr : stats;       // the dq kernel writes them only when dk/dv runs behind it
@@ -970,10 +989,6 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     // group's pairs (workspace_layout), and the dk/dv kernel of a group finds them where the dq kernel of the same
     // group has just left them. Otherwise one launch each covers all pairs.
     const int nbh_all = dm.B * dm.H, bh_step = handed ? wl.bh_group : nbh_all;
-    const bool slab = path == DSDPA_PATH_AUTO && !staged && slab_path_fits(V, Himg, Wimg, D, P, S::kBytes);
-    const bool rows = path == DSDPA_PATH_AUTO && !staged && !slab &&
-                      ((plane_path_fits(dm.L, D, S::kBytes) && few_samples_prefer_rows(V, P, S::kBytes)) ||
-                       row_path((size_t)dm.rows, V, dm.L, D, P, S::kBytes, true));
 #define DSDPA_BWD_CASE(DD)                                                                                      \
     case DD:                                                                                                    \
         if (fused_atomics && !dcoords) {                                                                        \
@@ -987,7 +1002,7 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
                  : slab ? launch_bwd_dq_slab<S, DD>(q, k, v, coords, out, lse, dout, dq, dq_stats, handed, dcoords,\
                                                     dm, bh0, nbh, st)                                           \
                  : rows ? launch_bwd_dq_rows<S, DD>(q, k, v, coords, out, lse, dout, dq, dq_stats, dcoords, handed,\
-                                                    dm, bh0, nbh, st)                                           \
+                                                    bh0 == 0 ? bins : BinJob{}, dm, bh0, nbh, st)               \
                         : launch_bwd_dq_gather<S, DD>(q, k, v, coords, out, lse, dout, dq, dq_stats, dcoords,   \
                                                       handed, dm, bh0, nbh, st);                                \
             if (rc == DSDPA_OK && patch)                                                                        \

@@ -12,6 +12,7 @@
 // staged kernels: every tap is a row from L1 or L2, 8 * D * e bytes a sample at 64 a clock and CU where LDS gives 128, but
 // no table, no staging and no barrier.
 #pragma once
+#include "dsdpa_cell.h"
 #include "dsdpa_gather.h"
 
 namespace dsdpa {
@@ -20,12 +21,16 @@ constexpr int kRowWaves = 4;
 
 struct RowGrid { int nblk; FastDiv div_nblk, div_h; int bh0; };       // workgroups per (batch, head); first pair of the launch
 
+// workgroups before the rows': whole rounds over the XCDs, so that the rows' stay where xcd_logical_block takes them to be
+__host__ __device__ inline unsigned bin_blocks(unsigned groups) { return (groups + kXcds - 1) / kXcds * kXcds; }
+
 // A slot's place: its row, clamped to the last of the (batch, head) for the slots beyond it.
 struct RowSlot { bool have; unsigned bhl, b, h, s1, l, qidx; };
+// (`skip`: workgroups of the launch, a multiple of 8, before those of the rows)
 template <int NS>
-__device__ __forceinline__ RowSlot decode_row_slot(const Dims &dm, const RowGrid &rg, int wave, int slot)
+__device__ __forceinline__ RowSlot decode_row_slot(const Dims &dm, const RowGrid &rg, int wave, int slot, unsigned skip = 0u)
 {
-    const unsigned bid = (unsigned)xcd_logical_block(blockIdx.x, gridDim.x);
+    const unsigned bid = (unsigned)xcd_logical_block((int)(blockIdx.x - skip), (int)(gridDim.x - skip));
     RowSlot r;
     r.bhl = rg.div_nblk.div(bid);
     const unsigned bh = r.bhl + (unsigned)rg.bh0, nq = (unsigned)(dm.V * dm.L);
@@ -174,13 +179,17 @@ __global__ __launch_bounds__(kRowWaves *kWave) void fwd_rows_kernel(
 // dq, the rows' (lse, delta) (stats_ may be null), the pairs for the dk/dv kernel (handed_ may be null; see
 // bwd_dq_gather_kernel) and, with CG, the gradient of the coordinates: per-tap dot products instead of blend-then-dot, each
 // lane's part of the two derivatives summed over the slot, and one pair of atomics per pass from the lane that owns the sample.
+// BIN: the binning of few samples, which reads coords only and is wanted by the kernel behind this one, takes the launch's first workgroups,
+// one a (batch, key view): a launch less, and its chain of waits beside the rows'. Binning and dq, us, in two launches / in one: 18x18,
+// 2 views x 2 samples, 32 heads, D = 32, fp32 6.6 + 13.1 / 12.5, bf16 6.2 + 8.3 / 9.8; 20x20, 2 x 2, 8 heads, D = 128, fp32
+// 6.1 + 14.8 / 14.8; 20x18, 4 x 1, 8 heads, D = 16, fp32 6.9 + 5.1 / 7.6.
 // STEP samples have their taps in flight together: two (112 registers in fp32, 4 waves a SIMD; 118 to 125 in 16 bits) or one (80, 6 waves;
 // 80 to 92), see row_step.
-template <typename S, int D, int DC, bool CG, int STEP>
-__global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
+template <typename S, int D, int DC, bool CG, int STEP, bool BIN>
+__global__ __launch_bounds__(kRowWaves *kWave, BIN && S::kBytes == 4 ? 4 : 1) void bwd_dq_rows_kernel(
     const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_, const float *__restrict__ coords_,
     const void *__restrict__ out_, const float *__restrict__ lse_, const void *__restrict__ dout_, void *__restrict__ dq_,
-    float2 *__restrict__ stats_, float *__restrict__ dcoords_, float2 *__restrict__ handed_, GradDims dm, RowGrid rg)
+    float2 *__restrict__ stats_, float *__restrict__ dcoords_, float2 *__restrict__ handed_, GradDims dm, RowGrid rg, BinJob bj)
 {
     constexpr int G = D / DC, NS = kWave / G;
     // dot products of 16-bit pairs as they are stored; with the coordinate gradient in bf16 only, where widening costs an instruction an
@@ -194,7 +203,15 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
     __shared__ float4 s_gx[CG ? kRowWaves : 1][CG ? NS * (G + 1) : 1], s_gy[CG ? kRowWaves : 1][CG ? NS * (G + 1) : 1];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int g = lane % G, slot = lane / G, lane_elem = g * DC;
-    const RowSlot rs = decode_row_slot<NS>(dm, rg, wave, slot);
+    const unsigned skip = BIN ? bin_blocks(bj.groups) : 0u;
+    if constexpr (BIN) {
+        if (blockIdx.x < skip) {
+            extern __shared__ unsigned s_hist[];
+            if (blockIdx.x < bj.groups) bin_one_group<kRowWaves * kWave>(coords_, dm, bj, blockIdx.x, s_hist);
+            return;
+        }
+    }
+    const RowSlot rs = decode_row_slot<NS>(dm, rg, wave, slot, skip);
     const unsigned lane_byte = (unsigned)lane_elem * S::kBytes;
     const size_t kv_base = dm.kv_plane((int)rs.b, 0, (int)rs.h) * S::kBytes;
     const char *kb = (const char *)k_ + kv_base, *vb = (const char *)v_ + kv_base;
@@ -328,7 +345,7 @@ __global__ __launch_bounds__(kRowWaves *kWave) void bwd_dq_rows_kernel(
         // (decoded anew: the row's place in dq is not kept in registers through the loop)
         int slot_here = slot;
         asm volatile("" : "+v"(slot_here));
-        const RowSlot re = decode_row_slot<NS>(dm, rg, wave, slot_here);
+        const RowSlot re = decode_row_slot<NS>(dm, rg, wave, slot_here, skip);
 #pragma unroll
         for (int d = 0; d < DC; ++d) dqa[d] *= dm.sm_scale;
         store_chunk<S, DC>((char *)dq_ + (dm.dq_bh((int)re.b, (int)re.h) + dm.dq_at(re.s1, re.l) + lane_elem) * S::kBytes, dqa);

@@ -59,6 +59,19 @@ def test_many_rows(V, H, P, dtype):
     check(1, V, H, 30, 31, 64, P, dtype)
 
 
+# the binning of few samples beside the rows of dq: all its places taken, two short of it, more groups than XCDs, a workgroup's threads
+# and one more; 2052 samples are binned in launches of their own
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("B,V,H,Himg,Wimg,D,P", [(1, 2, 3, 16, 32, 64, 2), (5, 2, 1, 11, 31, 32, 3), (1, 1, 2, 16, 16, 128, 1),
+                                                 (1, 1, 2, 1, 257, 16, 1), (2, 2, 2, 10, 12, 256, 3), (1, 2, 2, 19, 18, 64, 3)])
+def test_binning_beside_the_rows(B, V, H, Himg, Wimg, D, P, dtype):
+    if dtype == torch.float32 and V * Himg * Wimg * P >= 2048:
+        names = kernels_of(lambda: check(B, V, H, Himg, Wimg, D, P, dtype))
+        assert any(n.startswith("bin_") for n in names) == (V * Himg * Wimg * P > 2048), names
+    else:
+        check(B, V, H, Himg, Wimg, D, P, dtype)
+
+
 # 5.94 workgroups of rows a CU, and 5.03, which leave a sixth of the last one's time empty: rows and a wave per row
 @pytest.mark.parametrize("H,kernels", [(13, ("fwd_rows_kernel", "bwd_dq_rows_kernel")), (11, ("fwd_gather_kernel", "bwd_dq_gather_kernel"))])
 def test_rows_where_their_workgroups_fill_the_cus(H, kernels):
