@@ -327,6 +327,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : DP > 32 && S::
             const Fetched f0 = fetch(e0.id);
             f1 = fetch(e1.id);
             tables(first, e0, f0);
+            wave_lds_sync();                                      // (the zeros above are other lanes')
             put_tables(0, false);
         }
         wave_lds_sync();
@@ -344,6 +345,7 @@ __global__ __launch_bounds__(kPatchMaxWaves *kWave, DP > 64 ? 2 : DP > 32 && S::
                     wave_lds_sync();
                     put_tables(s / SPC, true);
                     if (s == NSTEP - 1) tables(first + stride, e1, f1);
+                    if constexpr (COLS < kWave) wave_lds_sync();      // (lanes l and l + 32 share a column: the zeros before the coefficients)
                     put_tables((s + 1) % NSTEP / SPC, false);
                     wave_lds_sync();
                 }

@@ -62,6 +62,18 @@ def test_half_blocks(P, dtype):
         assert rel(a, b) < BAR[dtype], name
 
 
+# C in LDS by halves of a block, every entry at the same four pixels: what one lane clears, the lane 32 places on writes next. (Few samples,
+# binned in one launch, are the patches' wherever they lie in 16-bit storage. They are spread over their cell: at one point dp - delta, and
+# with it ds, cancels down to what the rounding of the saved output, 2^-9 of delta, leaves of it.)
+@pytest.mark.parametrize("D,P", [(16, 3), (16, 20), (32, 3), (32, 20)])
+def test_half_blocks_of_one_cell(D, P):
+    q, k, v, dout, coords = inputs(1, 1, 114, 11, 9, D, P, torch.bfloat16, 18)
+    coords = 0.5 + (coords + 0.1) / 1.2 * torch.tensor([0.124, 0.099])
+    got, want = gradients(q, k, v, coords, dout, 9, 11)
+    for a, b, name in zip(got, want, ("dq", "dk", "dv")):
+        assert rel(a, b) < BAR[torch.bfloat16], name
+
+
 # 1350 visits a patch: four waves
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=str)
 def test_four_waves_a_patch(dtype):
