@@ -26,6 +26,9 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/accumulate_grad.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -35,6 +38,7 @@ namespace {
 
 using at::Tensor;
 using torch::autograd::AutogradContext;
+using torch::autograd::Node;
 using torch::autograd::variable_list;
 
 struct Strides {
@@ -202,6 +206,38 @@ void usable(variable_list &saved, const Tensor &dout, PyObject *bound)
     lse = packed(lse);
 }
 
+// Whether somebody is shown the gradient that goes into `node`: hooks of the tensor or the node, retain_grad, or a caller
+// of torch.autograd.grad that asked for it. (A leaf's node hands it to no hook behind it: those, a data-parallel wrapper's, read .grad.)
+bool shown(Node &node)
+{
+    const auto *exec = torch::autograd::get_current_graph_task_exec_info();
+    if (exec && !exec->empty()) {
+        const auto at = exec->find(&node);
+        if (at != exec->end() && at->second.captures_) return true;
+    }
+    return !node.pre_hooks().empty() || !node.tensor_pre_hooks().empty() || !node.retains_grad_hooks().empty() ||
+           (!node.post_hooks().empty() && !dynamic_cast<torch::autograd::AccumulateGrad *>(&node));
+}
+
+// Whether the gradients of those of q, k, v that are not contiguous go straight into the backward of the permutation that made them,
+// and neither they nor what comes out of it is shown to anybody. Everyone else gets contiguous gradients, of which views can
+// be made, whatever q, k and v look like.
+bool only_permuted(const Tensor &q, const Tensor &k)
+{
+    const std::shared_ptr<Node> self = torch::autograd::get_current_node();
+    if (!self || !self->post_hooks().empty()) return false;
+    for (uint32_t i = 0; i < 3; ++i) {
+        if ((i == 0 ? q : k).is_contiguous()) continue;
+        Node *fn = self->next_edge(i).function.get();
+        if (!fn) continue;                               // (no gradient asked for)
+        const std::string name = fn->name();
+        if ((name != "PermuteBackward0" && name != "TransposeBackward0") || shown(*fn)) return false;
+        Node *from = fn->next_edge(0).function.get();
+        if (from && shown(*from)) return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 // The autograd node. Outside the namespace for a plain name in graphs (torch::autograd::CppNode<fused_deform_sdpa>); the
@@ -249,7 +285,7 @@ struct fused_deform_sdpa : public torch::autograd::Function<fused_deform_sdpa> {
         readable_in_place(q, k, v, &st);
         // (of permuted inputs -- a linear layer's output split into heads -- the gradients go back through the permutation as they
         // are: contiguous ones would each be copied there, 10 us apiece of a step of 322 at 4 views of 40x28, 8 heads, D = 64, fp16)
-        const bool as_inputs = st.given && q.is_non_overlapping_and_dense() && k.is_non_overlapping_and_dense();
+        const bool as_inputs = st.given && q.is_non_overlapping_and_dense() && k.is_non_overlapping_and_dense() && only_permuted(q, k);
         if (as_inputs) flags |= DSDPA_FLAG_GRADS_AS_INPUTS;
         Tensor dq = fresh_as(q, as_inputs), dk = fresh_as(k, as_inputs), dv = fresh_as(v, as_inputs);
         Tensor dcoords = want_dcoords ? fresh(coords.sizes(), at::kFloat, dev) : Tensor();

@@ -9,18 +9,19 @@ import torch
 
 from ops import _native
 from ops.triton import deform_sdpa_triton
+from parity_util import kernels_of
 
 CASES = [
-    # B, V, H, Himg, Wimg, D, P, how the samples lie           which kernels
-    (2, 2, 3, 6, 5, 32, 2, "unit"),                          # rows, cells
-    (2, 2, 32, 10, 9, 32, 2, "unit"),                        # rows, patches
-    (1, 3, 2, 9, 7, 64, 12, "unit"),                         # staged planes, cells
-    (1, 2, 24, 13, 21, 32, 4, "border"),                     # staged planes, patches
-    (2, 3, 16, 23, 21, 16, 4, "point"),                      # patches left to the cells behind them
-    (1, 2, 2, 32, 32, 64, 16, "border"),                     # slabs (fp32)
-    (1, 2, 1, 37, 23, 128, 40, "border"),                    # a wave per row
-    (1, 2, 1, 34, 36, 128, 64, "point"),                     # windows
-    (1, 1, 1, 1, 1, 256, 1, "unit"),
+    # B, V, H, Himg, Wimg, D, P, how the samples lie, dq and dk/dv kernels (slabs: fp32; deterministic: cells)
+    (2, 2, 3, 6, 5, 32, 2, "unit", "rows", "cell"),
+    (2, 2, 32, 10, 9, 32, 2, "unit", "rows", "patch"),
+    (1, 3, 2, 9, 7, 64, 12, "unit", "slot", "cell"),
+    (1, 2, 24, 13, 21, 32, 4, "border", "slot", "patch"),
+    (2, 3, 16, 23, 21, 16, 4, "point", "slot", "patch"),     # left to the cells behind them
+    (1, 2, 2, 32, 32, 64, 16, "border", "slab", "cell"),
+    (1, 2, 1, 37, 23, 128, 40, "border", "gather", "cell"),
+    (1, 2, 1, 34, 36, 128, 64, "point", "gather", "cell"),   # windows
+    (1, 1, 1, 1, 1, 256, 1, "unit", "rows", "cell"),
 ]
 
 
@@ -39,12 +40,18 @@ def layouts(kind, t):
     return leaf, leaf
 
 
+def as_given(kind, grad, H):
+    """a leaf's gradient as one of the operator's (B, V, H, L, D) argument"""
+    return (grad.permute(0, 1, 3, 2, 4) if kind == "projection" else grad.permute(0, 2, 3, 1, 4) if kind == "pixels first"
+            else grad[:, :, :H] if kind == "sliced" else grad)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["plain", "coords", "deterministic"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
 @pytest.mark.parametrize("case", CASES, ids=[f"{c[3]}x{c[4]}-D{c[5]}-P{c[6]}" for c in CASES])
 def test_gradients_follow_the_inputs_layout(case, dtype, mode):
-    B, V, H, Himg, Wimg, D, P, where = case
+    B, V, H, Himg, Wimg, D, P, where, dq_kernel, dkdv_kernel = case
     L = Himg * Wimg
     print(f"[case] gradient layout {case} {dtype} {mode}", flush=True)
     g = torch.Generator().manual_seed(L + P)
@@ -62,11 +69,12 @@ def test_gradients_follow_the_inputs_layout(case, dtype, mode):
             c = coords.clone().requires_grad_(mode == "coords")
             out = deform_sdpa_triton(qv, kv, vv, c, Wimg, Himg, 1.0 / math.sqrt(D), mode == "coords")
             assert out.is_contiguous()
-            grads = torch.autograd.grad(out, (qv, kv, vv) + ((c,) if mode == "coords" else ()), dout)
-            if "sliced" not in (kq, kk):
-                for t, d in ((qv, grads[0]), (kv, grads[1]), (vv, grads[2])):
-                    assert all(s == u for s, u, n in zip(t.stride(), d.stride(), t.shape) if n > 1)
-            results[kq, kk] = [x.contiguous() for x in grads]
+            names = kernels_of(lambda: out.backward(dout))
+            grads = [as_given(kind, leaf.grad, H) for kind, leaf in ((kq, ql), (kk, kl), (kk, vl))]
+            results[kq, kk] = [x.contiguous() for x in grads] + ([c.grad] if mode == "coords" else [])
+            dq_by = "gather" if dq_kernel == "slab" and dtype != torch.float32 else dq_kernel
+            dkdv_by = "cell" if mode == "deterministic" else dkdv_kernel
+            assert all(any(n.startswith(by) for n in names) for by in (f"bwd_dq_{dq_by}_kernel", f"bwd_dkdv_{dkdv_by}_kernel")), names
     finally:
         torch.use_deterministic_algorithms(False)
     ref = results.pop(("contiguous", "contiguous"))
@@ -93,6 +101,54 @@ def test_leaf_gradients_are_not_copied():
     assert not any(e.key in ("aten::copy_", "aten::clone") for e in prof.key_averages())
     for t in leaves:
         assert t.grad.is_contiguous()
+
+
+# Only a gradient that nobody sees lies as its tensor does. Whoever is shown that of q, or what the permutation's backward makes of it,
+# gets it contiguous as (B, V, H, L, D), whatever q's strides are.
+@pytest.mark.gpu
+@pytest.mark.parametrize("who", ["grad", "hook", "retain", "prehook", "node", "own node", "leaf grad", "leaf hook", "behind", "permuted leaf", "nobody"])
+def test_gradients_that_are_shown_are_contiguous(who):
+    print(f"[case] shown gradients: {who}", flush=True)
+    B, V, H, Himg, Wimg, D, P = 1, 2, 4, 10, 9, 32, 2
+    seen = []
+
+    def see(g):
+        seen.append(g.detach())
+    leaf = torch.randn(B, V, Himg * Wimg, H, D, device="cuda").requires_grad_(True)
+    back = lambda g: g.permute(0, 1, 3, 2, 4)
+    q = back(leaf + 1.0) if who == "behind" else back(leaf)
+    if who == "permuted leaf":
+        q = back(leaf.detach()).requires_grad_(True)
+    k, v = torch.randn(2, B, V, H, Himg * Wimg, D, device="cuda").requires_grad_(True).unbind(0)
+    out = deform_sdpa_triton(q, k, v, torch.rand(B, V, Himg * Wimg, V, P, 2, device="cuda"), Wimg, Himg, 0.2)
+    dout = torch.randn(out.shape, device="cuda")
+    if who in ("grad", "permuted leaf"):
+        see(torch.autograd.grad(out, q, dout)[0])
+    elif who == "leaf grad":
+        see(back(torch.autograd.grad(out, leaf, dout)[0]))
+    else:
+        if who == "hook":
+            q.register_hook(see)
+        elif who == "retain":
+            q.retain_grad()
+        elif who == "prehook":
+            q.grad_fn.register_prehook(lambda go: see(go[0]))
+        elif who == "node":
+            q.grad_fn.register_hook(lambda gi, go: see(go[0]))
+        elif who == "own node":
+            out.grad_fn.register_hook(lambda gi, go: see(gi[0]))
+        elif who == "leaf hook":
+            leaf.register_hook(lambda g: see(back(g)))
+        elif who == "behind":
+            q.grad_fn.next_functions[0][0].register_prehook(lambda go: see(back(go[0])))
+        out.backward(dout)
+        if who == "retain":
+            see(q.grad)
+    if who == "nobody":
+        assert leaf.grad.is_contiguous() and not seen
+    else:
+        assert len(seen) == 1 and seen[0].is_contiguous()
+        seen[0].view(-1)
 
 
 def test_strides_that_do_not_fill_a_block_are_refused():
