@@ -49,15 +49,16 @@ int allow_full_lds(K kern, std::atomic<unsigned long long> &done)
     return DSDPA_OK;
 }
 
-// Where the 8 elements `i` of the contiguous accumulators go in dk and dv (elements; per8: 8 elements of a row of D).
+// Where the 8 elements `i` of the contiguous accumulators go in dk and dv (elements).
 struct GradPlace {
-    FastDiv div_per8, div_v, div_h;
+    FastDiv div_v, div_h;
+    unsigned log_per8;                           // of D / 8, a power of two: `i` itself may not fit 32 bits, a row does
     bool plain;                                  // contiguous gradients: at their own place
 };
-__device__ __forceinline__ size_t grad_place(const GradPlace &gp, const GradDims &dm, unsigned per8, size_t i)
+__device__ __forceinline__ size_t grad_place(const GradPlace &gp, const GradDims &dm, size_t i)
 {
     if (gp.plain) return i * 8;
-    const unsigned row = gp.div_per8.div((unsigned)i), c = (unsigned)i - row * per8;       // (rows * D / 8 < 2^31: checked by the host)
+    const unsigned row = (unsigned)(i >> gp.log_per8), c = (unsigned)i & ((1u << gp.log_per8) - 1u);
     const unsigned t = dm.divL.div(row), l = row - t * (unsigned)dm.L;
     const unsigned bv = gp.div_h.div(t), h = t - bv * (unsigned)dm.H, b = gp.div_v.div(bv);
     return dm.dkv_plane((int)b, (int)(bv - b * (unsigned)dm.V), (int)h) + l * (unsigned)dm.dkv_sl + c * 8u;
@@ -65,7 +66,7 @@ __device__ __forceinline__ size_t grad_place(const GradPlace &gp, const GradDims
 
 // fp32 accumulators -> 16-bit storage, 8 elements per thread
 template <typename S>
-__global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ dst, size_t n8, GradDims dm, GradPlace gp, unsigned per8)
+__global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ dst, size_t n8, GradDims dm, GradPlace gp)
 {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -75,7 +76,7 @@ __global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ ds
         float4 a = s4[0], b = s4[1];
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
         v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-        store_chunk<S, 8>((char *)dst + grad_place(gp, dm, per8, i) * 2, v);
+        store_chunk<S, 8>((char *)dst + grad_place(gp, dm, i) * 2, v);
     }
 }
 
@@ -83,7 +84,7 @@ __global__ void cast_kernel(const float *__restrict__ src, void *__restrict__ ds
 // (n8 = elements of a (batch, view, head) over 8). At once over where there are none.
 template <typename S>
 __global__ void cast_rest_kernel(const unsigned *__restrict__ left, const float *__restrict__ dk_acc, const float *__restrict__ dv_acc,
-                                 void *__restrict__ dk, void *__restrict__ dv, GradDims dm, size_t n8, GradPlace gp, unsigned per8)
+                                 void *__restrict__ dk, void *__restrict__ dv, GradDims dm, size_t n8, GradPlace gp)
 {
     const size_t per = n8 * dm.H, stride = (size_t)gridDim.x * blockDim.x;
     const bool all = mostly_long(left, dm.B * dm.V);
@@ -94,7 +95,7 @@ __global__ void cast_rest_kernel(const unsigned *__restrict__ left, const float 
             const float4 *s4 = reinterpret_cast<const float4 *>(i < per ? dk_acc : dv_acc) + 2 * at;
             const float4 a = s4[0], b = s4[1];
             const float v[8] = { a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w };
-            store_chunk<S, 8>((char *)(i < per ? dk : dv) + grad_place(gp, dm, per8, at) * 2, v);
+            store_chunk<S, 8>((char *)(i < per ? dk : dv) + grad_place(gp, dm, at) * 2, v);
         }
     }
 }
@@ -198,7 +199,6 @@ static inline int apply_grad_strides(int D, bool as_inputs, GradDims *dm)
     if (!as_inputs) return DSDPA_OK;
     if (!dense_strides(*dm, D, dm->q_sb, dm->q_sv, dm->q_sh, dm->q_sl) || !dense_strides(*dm, D, dm->kv_sb, dm->kv_sv, dm->kv_sh, dm->kv_sl))
         return DSDPA_ERR_BAD_STRIDES;
-    if ((long long)dm->rows * D / 8 > 0x7fffffffll) return DSDPA_ERR_TOO_LARGE;
     dm->dq_sb = dm->q_sb; dm->dq_sv = dm->q_sv; dm->dq_sh = dm->q_sh; dm->dq_sl = dm->q_sl;
     dm->dkv_sb = dm->kv_sb; dm->dkv_sv = dm->kv_sv; dm->dkv_sh = dm->kv_sh; dm->dkv_sl = dm->kv_sl;
     return DSDPA_OK;
@@ -1034,23 +1034,22 @@ int bwd_impl(const void *q, const void *k, const void *v, const float *coords, c
     if (rc != DSDPA_OK) return rc;
     GradPlace gp;
     gp.plain = !as_inputs;
-    gp.div_per8 = FastDiv::make((unsigned)D / 8);
+    gp.log_per8 = (unsigned)__builtin_ctz((unsigned)D / 8);
     gp.div_v = FastDiv::make((unsigned)V);
     gp.div_h = FastDiv::make((unsigned)H);
     if (S::kBytes != 4 && left) {
         const size_t n8 = (size_t)dm.L * D / 8;                     // of a plane
         size_t blocks = (n8 * B * V * H + 255) / 256;
         if (blocks > 256 * 8) blocks = 256 * 8;
-        hipLaunchKernelGGL((cast_rest_kernel<S>), dim3((unsigned)blocks), dim3(256), 0, st, left, dk_acc, dv_acc, dk, dv, dm, n8, gp,
-                           (unsigned)D / 8);
+        hipLaunchKernelGGL((cast_rest_kernel<S>), dim3((unsigned)blocks), dim3(256), 0, st, left, dk_acc, dv_acc, dk, dv, dm, n8, gp);
         rc = check_launch();
     } else if (S::kBytes != 4 && !patch && !deterministic) {
         const size_t n8 = n / 8;
         const int threads = 256;
         size_t blocks = (n8 + threads - 1) / threads;
         if (blocks > 256 * 16) blocks = 256 * 16;
-        hipLaunchKernelGGL((cast_kernel<S>), dim3((unsigned)blocks), dim3(threads), 0, st, dk_acc, dk, n8, dm, gp, (unsigned)D / 8);
-        hipLaunchKernelGGL((cast_kernel<S>), dim3((unsigned)blocks), dim3(threads), 0, st, dv_acc, dv, n8, dm, gp, (unsigned)D / 8);
+        hipLaunchKernelGGL((cast_kernel<S>), dim3((unsigned)blocks), dim3(threads), 0, st, dk_acc, dk, n8, dm, gp);
+        hipLaunchKernelGGL((cast_kernel<S>), dim3((unsigned)blocks), dim3(threads), 0, st, dv_acc, dv, n8, dm, gp);
         rc = check_launch();
     }
     return rc;

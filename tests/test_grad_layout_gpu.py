@@ -162,3 +162,15 @@ def test_strides_that_do_not_fill_a_block_are_refused():
     call = [fake] * 10 + [None, fake, 1, V, H, 3, 4, D, 2, 0.5]
     for q, kv in ((holes, dense), (dense, holes), (shared, dense)):
         assert lib.dsdpa_bwd_f32(*call, ll8(*q, *kv), _native.FLAG_GRADS_AS_INPUTS, None) == _native.ERR_BAD_STRIDES
+
+
+# 2^34 elements and more are addressed like fewer. (Where there is no GPU, what passes the checks ends at the first launch.)
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="the pointers are made up")
+def test_size_is_no_reason_to_refuse_the_layout():
+    lib = _native.load()
+    fake, ll8 = ctypes.c_void_p(0x1000), ctypes.c_longlong * 8
+    B, V, H, side, D = 8200, 1, 2, 64, 256
+    strides = ll8(*2 * (V * H * side * side * D, H * side * side * D, D, H * D))
+    call = [fake] * 10 + [None, fake, B, V, H, side, side, D, 2, 0.5, strides]
+    rc = [lib.dsdpa_bwd_bf16(*call, flags, None) for flags in (0, _native.FLAG_GRADS_AS_INPUTS)]
+    assert rc[0] == rc[1], rc
