@@ -233,6 +233,7 @@ __device__ __forceinline__ void scan_keys(const unsigned (&v)[kScanKeys], int c0
         carry.entries += t.x;
         carry.pieces += t.y;
     }
+    asm volatile("" : "+v"(excl), "+v"(pexcl));                    // (summed here, not from two dozen parts behind each branch below)
     first = excl;
 #pragma unroll
     for (int i = 0; i < kScanKeys; ++i) {

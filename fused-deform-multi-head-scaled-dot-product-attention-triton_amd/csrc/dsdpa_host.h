@@ -184,8 +184,8 @@ inline bool row_path(size_t rows, size_t V, size_t L, size_t D, size_t P, size_t
     if (waves < (N <= 32 ? 2048 : N <= 64 ? 4096 : 8192)) return false;
     if (N > 32 && fp32 && D < 32) return false;
     if (N > 64 && (D < 64 || (!dq && !fp32 && D < 256))) return false;
-    const size_t per = 4 * (64 / lanes), groups = rows / (V * L) * ((V * L + per - 1) / per);     // workgroups, 256 CUs
-    const size_t fill = 100 * groups / ((groups + 255) / 256 * 256);
+    const size_t per = 4 * (64 / lanes), groups = rows / (V * L) * ((V * L + per - 1) / per);     // workgroups
+    const size_t cus = (size_t)device_cus(), fill = 100 * groups / ((groups + cus - 1) / cus * cus);
     return fill >= (fp32 && D == 256 ? 65 : N <= 32 ? (fp32 && D >= 64 ? 88 : 80) : N <= 64 ? (fp32 ? 95 : 85) : fp32 ? 97 : 93);
 }
 
@@ -197,8 +197,9 @@ inline bool row_path(size_t rows, size_t V, size_t L, size_t D, size_t P, size_t
 inline int row_step(size_t esize, long long groups)
 {
     if (esize == 2) return 2;
+    const long long cus = device_cus();
     auto full = [&](long long at_once) { return (double)groups / (double)((groups + at_once - 1) / at_once * at_once); };
-    return full(6 * 256) > full(4 * 256) ? 1 : 2;
+    return full(6 * cus) > full(4 * cus) ? 1 : 2;
 }
 
 // Whether the row dq kernel has a form that bins beside its rows: all but the one of 1 KB rows with the coordinate gradient, which would spill.

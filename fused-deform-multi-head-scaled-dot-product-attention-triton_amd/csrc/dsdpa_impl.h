@@ -253,13 +253,13 @@ int launch_bwd_dq_rows(const void *q, const void *k, const void *v, const float 
     const long long blocks = (long long)nbh * rg.nblk;
     if (blocks > 0x7fffffffll - 65536) return DSDPA_ERR_TOO_LARGE;
     constexpr int kTwo = DC * S::kBytes <= 16 ? 2 : 1, kOne = S::kBytes == 2 ? kTwo : 1;
+    const unsigned bins = bin_blocks(bj.groups);
     auto pick = [&](auto bin) {
         constexpr bool BIN = decltype(bin)::value;
         return dcoords ? bwd_dq_rows_kernel<S, D, DC, true, 1, BIN && row_takes_bins(D, S::kBytes, true)>
-               : row_step(S::kBytes, blocks) == 2 ? bwd_dq_rows_kernel<S, D, DC, false, kTwo, BIN> : bwd_dq_rows_kernel<S, D, DC, false, kOne, BIN>;
+               : row_step(S::kBytes, blocks + bins) == 2 ? bwd_dq_rows_kernel<S, D, DC, false, kTwo, BIN> : bwd_dq_rows_kernel<S, D, DC, false, kOne, BIN>;
     };
     auto kern = bj.groups ? pick(std::true_type{}) : pick(std::false_type{});
-    const unsigned bins = bin_blocks(bj.groups);
     ScopedKernelTimer timer(2, st);
     DSDPA_LAUNCH(kern, dim3((unsigned)blocks + bins), dim3(kRowWaves * kWave), bins ? bj.NC * sizeof(unsigned) : 0, st, timer.start(),
                  timer.stop(), q, k, v, coords, out, lse, dout, dq, stats, dcoords, handed, dm, rg, bj);

@@ -183,17 +183,25 @@ __global__ __launch_bounds__(kRowWaves *kWave) void fwd_rows_kernel(
 // one a (batch, key view): a launch less, and its chain of waits beside the rows'. Binning and dq, us, in two launches / in one: 18x18,
 // 2 views x 2 samples, 32 heads, D = 32, fp32 6.6 + 13.1 / 12.5, bf16 6.2 + 8.3 / 9.8; 20x20, 2 x 2, 8 heads, D = 128, fp32
 // 6.1 + 14.8 / 14.8; 20x18, 4 x 1, 8 heads, D = 16, fp32 6.9 + 5.1 / 7.6.
-// STEP samples have their taps in flight together: two (112 registers in fp32, 4 waves a SIMD; 118 to 125 in 16 bits) or one (80, 6 waves;
-// 80 to 92), see row_step.
+// STEP samples have their taps in flight together: two (fp32 112 to 114 registers, 16 bits 102 to 127: 4 waves a SIMD; also with the
+// coordinate gradient and the binning) or one (fp32 up to D = 128 80, 6 waves; with the coordinate gradient 96, 5 waves, but bf16 121 and fp16, D =
+// 16 107), see row_step.
+// Waves a SIMD that the compiler is held to: six in fp32 with one sample and D <= 128 also where it bins (held to four it took 84 registers,
+// five waves, where row_step counts six; dq of 18x18, 2 views x 2 samples, 16 to 96 heads, D = 32, is the same with either). Rows of 1 KB
+// that bin get four and no more, the taps of a sample all in flight (16x20, 2 x 3, D = 256, us, with four / five 30 / 34).
+template <typename S, int D, bool CG, int STEP, bool BIN>
+constexpr int kRowDqWaves = !BIN || S::kBytes == 2 ? 1 : !CG && STEP == 1 && D <= 128 ? 6 : 4;
+template <typename S, int D, bool BIN> constexpr int kRowDqWavesMost = BIN && D * S::kBytes >= 1024 ? 4 : 8;
 template <typename S, int D, int DC, bool CG, int STEP, bool BIN>
-__global__ __launch_bounds__(kRowWaves *kWave, BIN && S::kBytes == 4 ? 4 : 1) void bwd_dq_rows_kernel(
+__global__ __launch_bounds__(kRowWaves *kWave) __attribute__((
+    amdgpu_waves_per_eu(kRowDqWaves<S, D, CG, STEP, BIN>, kRowDqWavesMost<S, D, BIN>))) void bwd_dq_rows_kernel(
     const void *__restrict__ q_, const void *__restrict__ k_, const void *__restrict__ v_, const float *__restrict__ coords_,
     const void *__restrict__ out_, const float *__restrict__ lse_, const void *__restrict__ dout_, void *__restrict__ dq_,
     float2 *__restrict__ stats_, float *__restrict__ dcoords_, float2 *__restrict__ handed_, GradDims dm, RowGrid rg, BinJob bj)
 {
     constexpr int G = D / DC, NS = kWave / G;
     // dot products of 16-bit pairs as they are stored; with the coordinate gradient in bf16 only, where widening costs an instruction an
-    // element (107 registers for 99): fp16's halves are widened by the multiply-add that takes them, and its forms differ by 5 % either
+    // element: fp16's halves are widened by the multiply-add that takes them, and its forms differ by 5 % either
     // way (us, pairs / widened: 40x28, 4 views x 8, D = 64 99 / 104, 32x19, 2 x 3 21.8 / 19.9)
     constexpr bool kPacked = S::kBytes == 2 && (!CG || S::kBf16);
     constexpr int RW = DC * S::kBytes / 4;
@@ -274,7 +282,7 @@ __global__ __launch_bounds__(kRowWaves *kWave, BIN && S::kBytes == 4 ? 4 : 1) vo
                 }
                 if constexpr (CG && kPacked) dk_t[i] = packed_dot<S, DC>(qp, kr[i]);
                 if constexpr (CG) dot = fmaf(wt[i], dk_t[i], dot);
-                if constexpr (CG && S::kBf16) __builtin_amdgcn_sched_barrier(0);   // (widening tap by tap: 107 registers for 130, four waves a SIMD)
+                if constexpr (CG && S::kBf16) __builtin_amdgcn_sched_barrier(0);   // (widening tap by tap: registers for four waves a SIMD)
                 if constexpr (kPacked) {
                     dv_t[i] = packed_dot<S, DC>(dop, vr[i]);
                     dp = fmaf(wt[i], dv_t[i], dp);
@@ -325,7 +333,8 @@ __global__ __launch_bounds__(kRowWaves *kWave, BIN && S::kBytes == 4 ? 4 : 1) vo
                 load_words<RW>(vb + o.z, vr[u][2]);
                 load_words<RW>(vb + o.w, vr[u][3]);
             }
-            if constexpr (U > 1) __builtin_amdgcn_sched_barrier(0);
+            // (the second: 96 registers for 100, five waves; 50x50, 4 views x 4 samples, D = 32, 16 heads, coordinate gradient, fp16 197 -> 185 us)
+            if constexpr (U > 1 || (CG && S::kBytes == 2 && !S::kBf16 && D <= 32 && !BIN)) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int u = 0; u < U; ++u) one(t + u, xs[u], kr[u], vr[u]);
         };

@@ -41,6 +41,27 @@ def test_main_kernels_do_not_spill(kernels):
     assert not over, over
 
 
+def test_row_dq_keeps_the_waves_that_its_rules_count_on(kernels):
+    """bwd_dq_rows_kernel<storage, D, elements a lane, coordinate gradient, samples a step, bins>: registers for six waves a SIMD
+    (80 of 512) in fp32 with one sample a step, for five (96) with the coordinate gradient, in fp16 where it does not bin."""
+    name = r"bwd_dq_rows_kernel<(\w+), (\d+), \d+, (true|false), (\d), (true|false)>"
+    over, seen = {}, 0
+    for n, (_, regs) in kernels.items():
+        m = re.match(name, n)
+        if not m:
+            continue
+        storage, D, coords, step, bins = m[1], int(m[2]), m[3] == "true", int(m[4]), m[5] == "true"
+        most = 128
+        if storage == "F32" and not coords and step == 1 and (D <= 128 or not bins):
+            most = 80
+        elif coords and not bins and ((storage == "F32" and D <= 128) or (storage == "F16" and D >= 32)):
+            most = 96
+        seen += most < 128
+        if regs > most:
+            over[n] = regs
+    assert not over and seen == 4 + 5 + 4 + 4, (seen, over)
+
+
 def test_row_kernels_keep_four_waves_a_simd(kernels):
     over = {n: v[1] for n, v in kernels.items() if re.match(r"(fwd_rows|bwd_dq_rows)", n) and v[1] > 128}
     assert not over, over
