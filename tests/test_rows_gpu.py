@@ -60,16 +60,17 @@ def test_many_rows(V, H, P, dtype):
 
 
 # the binning of few samples beside the rows of dq: all its places taken, two short of it, more groups than XCDs, a workgroup's threads
-# and one more; 2052 samples are binned in launches of their own
+# and one more; 2052 samples, and rows of 1 KB with the coordinate gradient, are binned in launches of their own
+@pytest.mark.parametrize("coords_grad", [False, True], ids=["plain", "coords"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
 @pytest.mark.parametrize("B,V,H,Himg,Wimg,D,P", [(1, 2, 3, 16, 32, 64, 2), (5, 2, 1, 11, 31, 32, 3), (1, 1, 2, 16, 16, 128, 1),
                                                  (1, 1, 2, 1, 257, 16, 1), (2, 2, 2, 10, 12, 256, 3), (1, 2, 2, 19, 18, 64, 3)])
-def test_binning_beside_the_rows(B, V, H, Himg, Wimg, D, P, dtype):
-    if dtype == torch.float32 and V * Himg * Wimg * P >= 2048:
-        names = kernels_of(lambda: check(B, V, H, Himg, Wimg, D, P, dtype))
-        assert any(n.startswith("bin_") for n in names) == (V * Himg * Wimg * P > 2048), names
-    else:
-        check(B, V, H, Himg, Wimg, D, P, dtype)
+def test_binning_beside_the_rows(B, V, H, Himg, Wimg, D, P, dtype, coords_grad):
+    names = kernels_of(lambda: check(B, V, H, Himg, Wimg, D, P, dtype, coords_grad))
+    beside = V * Himg * Wimg * P <= 2048 and not (coords_grad and D == 256 and dtype == torch.float32)
+    rows = [n for n in names if n.startswith("bwd_dq_rows_kernel")]
+    assert len(rows) == 1 and rows[0].endswith("true>" if beside else "false>"), names      # (last argument: bins)
+    assert any(n.startswith("bin_") for n in names) == (not beside), names
 
 
 # 5.94 workgroups of rows a CU, and 5.03, which leave a sixth of the last one's time empty: rows and a wave per row
