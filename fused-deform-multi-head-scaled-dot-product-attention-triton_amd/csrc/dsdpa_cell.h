@@ -312,8 +312,8 @@ __global__ __launch_bounds__(THREADS, THREADS == 512 ? 8 : 4) void bin_scan_kern
 
 // Count, scan and fill by one workgroup, for lists short enough that one workgroup holds all samples of a (b, s2) in
 // its registers, kBinOneSamples / THREADS of them a thread: every sample's rank in its list comes from the counting atomic itself, so
-// the coordinates are read once and there is one round of LDS atomics, no counters in memory (nothing to clear)
-// and no wait between launches. Bound by that chain of latencies (a few workgroups on the whole chip), as the three
+// there is one round of LDS atomics, no counters in memory (nothing to clear) and no wait between launches; 1024 threads read the coordinates
+// once, 256 (in the row dq launch, whose registers do not hold them and the scan) again for the fill. Bound by that chain of latencies (a few workgroups on the whole chip), as the three
 // launches are: 1296 samples a list group (18x18, 2 views x 2 samples) 6.2 us against 13.7 for the three and the gaps
 // between them. One workgroup's throughput then takes over: 5184 (4 x 4, six samples a thread) 13.9 against 17.4, a step
 // no faster; 11664 34.8 against 24.1, 17871 59 against 19.
